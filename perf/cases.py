@@ -265,3 +265,102 @@ def tolerance(case):
     if op == "bf16_step":
         return {"rel": 2e-3, "max": 0.016}
     return {"rel": 7e-4 if op in ("swiglu_step", "experts_step") else 3e-3, "max": 0.13}
+
+
+def exact(case, seed):
+    """What run() returns, in 64-bit arithmetic and plain torch: scales and values unrounded, codes the FP8 value
+    nearest to the 64-bit quotient."""
+    s, f64, fp8, fmax = prepare(case, seed), torch.float64, torch.float8_e4m3fn, 448.0
+    op, pow2 = case["op"], case.get("pow2", False)
+
+    def scale_of(amax):
+        scale = (amax / fmax).clamp_min(1e-30)
+        return torch.exp2(torch.ceil(torch.log2(scale))) if pow2 else scale
+
+    def codes(v):
+        return v.to(fp8).to(f64)
+
+    def rows(v):  # codes [M, n], scales [M, n/128]
+        g = v.view(v.shape[0], -1, 128)
+        scale = scale_of(g.abs().amax(2))
+        return codes((g / scale[:, :, None]).view(v.shape)), scale
+
+    def columns(v):  # codes [n, M], scales [ceil(M/128), n]
+        M, n = v.shape
+        g = torch.nn.functional.pad(v, (0, 0, 0, -M % 128)).view(-1, 128, n)
+        scale = scale_of(g.abs().amax(1))
+        return codes((g / scale[:, None, :]).view(-1, n)[:M].t().contiguous()), scale
+
+    def both(v):
+        q, scale = rows(v)
+        return q, scale.t().contiguous(), *columns(v)
+
+    def experts(v, splits):  # the flat pieces of the experts one after the other
+        out, pos = [[], [], [], []], 0
+        for p in splits:
+            for k, piece in enumerate(both(v[pos:pos + p]) if p else ()):
+                out[k].append(piece if k in (0, 3) else piece.reshape(-1))
+            pos += p
+        return [torch.cat(o) for o in out]
+
+    def norm(x, gamma):
+        x = x.to(f64)
+        r = 1.0 / torch.sqrt((x * x).mean(1) + 1e-6)
+        return x * r[:, None] * gamma.to(f64), r
+
+    def silu(h, weight=None):
+        h1, h2 = h.to(f64).chunk(2, 1)
+        y = torch.sigmoid(h1) * h1 * h2
+        return y if weight is None else y * weight.to(f64).view(-1, 1)
+
+    def silu_back(dh, h, weight=None):
+        h1, h2 = h.to(f64).chunk(2, 1)
+        sig, d = torch.sigmoid(h1), dh.to(f64)
+        w = 1.0 if weight is None else weight.to(f64).view(-1, 1)
+        dx = torch.cat([d * w * h2 * sig * (1.0 + h1 * (1.0 - sig)), d * w * sig * h1], 1)
+        return dx, None if weight is None else (d * sig * h1 * h2).sum(1).view(weight.shape)
+
+    def swap(t):  # scales of row-wise codes, one row per 128 columns
+        return t[0], t[1].t().contiguous()
+
+    if op == "infer":
+        y, r = norm(s["x"], s["gamma"])
+        return (*swap(rows(y)), r, rows(s["a"].to(f64)), swap(rows(silu(s["h"]))))
+    if op in ("norm_quant", "norm_recompute"):
+        y, r = norm(s["x"], s["gamma"])
+        q, scale, qt, st = both(y)
+        return q, scale, r, qt, st
+    if op == "bf16_step":
+        y, r = norm(s["x"], s["gamma"])
+        dh, dweight = silu_back(s["dh"], s["h"], s["weight"])
+        x, d = s["x"].to(f64), s["dy"].to(f64)
+        xhat, g = x * r[:, None], d * s["gamma"].to(f64)
+        dx = (g - xhat * (g * xhat).mean(1, keepdim=True)) * r[:, None]
+        return y, r, silu(s["h"], s["weight"]), dh, dweight, dx, (d * xhat).sum(0)
+    if op == "swiglu_step":
+        return both(silu(s["h"])), both(silu_back(s["dh"], s["h"])[0])
+    if op == "experts_step":
+        n = case["f"]
+        q, scale, qt, st = experts(silu(s["h"], s["weight"]), s["splits"])
+        dx, dweight = silu_back(s["dh"], s["h"], s["weight"])
+        dq, dscale, dqt, dst = experts(dx, s["splits"])
+        return ((q, scale.view(-1, n // 128), qt.view(-1, n), st),
+                (dq, dscale.view(-1, n // 64), dweight, dqt.view(-1, 2 * n), dst))
+    if op == "dispatch":
+        n, index = case["n"], s["indices"].long()
+        starts = [sum(s["padded"][:e]) for e in range(case["experts"])]
+        real = torch.zeros(len(index), dtype=torch.bool, device="cuda")
+        probs = torch.zeros(len(index), dtype=f64, device="cuda")
+        for e, (at, c) in enumerate(zip(starts, s["splits"])):
+            real[at:at + c] = True
+            probs[at:at + c] = s["probs"][index[at:at + c], e].to(f64)
+        v = torch.where(real[:, None], s["x"][index].to(f64), torch.zeros((), dtype=f64, device="cuda"))
+        q, scale, qt, st = experts(v, s["padded"])
+        dq, dscale, dqt, dst = experts(s["dy"].to(f64), s["padded"])
+        return ((q, scale.view(-1, n // 128), qt.view(-1, n), st, probs), (dq, dscale, dqt, dst.reshape(-1)))
+    if op == "linear":
+        w = s["w"].to(f64).view(case["out"] // 128, 128, case["n"] // 128, 128)
+        scale = scale_of(w.abs().amax((1, 3)))
+        return both(s["x"].to(f64)), (codes(w / scale[:, None, :, None]).view(s["w"].shape), scale)
+    y, r = norm(s["x"], s["gamma"])
+    return (y, r, y @ s["w"].to(f64).t(), *swap(rows(y)))
