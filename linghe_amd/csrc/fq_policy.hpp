@@ -134,10 +134,16 @@ struct Policy {
   static constexpr bool kLoadHintRows = true;
   static constexpr bool kXcdContiguousRowQuant = true;
 
-  // ---- router kernels: hint on the stores of y and the codes, and on the loads of x in the
-  // register-resident kernel
+  // ---- router kernels: hint on the stores of y and the codes
   static constexpr bool kStoreHintRouter = true;
-  static constexpr bool kLoadHintRouter = true;
+  // Which router kernel, by the number of workgroups of 64 rows x 64 logits the call has (us of the kernel
+  // alone at K = 2048, few-rows / 64-logit / 128-logit form).  Up to 80 of them, 256 CUs are mostly idle
+  // and the 16-row form spreads the rows further: 1024 x 256 14.8 / 20.0 / 27.2, 2048 x 256 25.5 / 21.0 / 28.0;
+  // fp32 weight: 1024 x 256 19.6 / 23.4, 2048 x 256 36.4 / 24.8.  As long as the 64-logit workgroups fit
+  // the chip at once they halve a workgroup's work: 4096 x 256 46.9 / 23.8 / 30.0, 8192 x 128 48.6 /
+  // 29.9 / 37.1; beyond, the 128-logit form turns x into operands half as often: 8192 x 256 88.7 / 42.2 / 36.3.
+  static constexpr int kRouterFewRowsMax = 80;
+  static constexpr int kRouterNarrowMax = 256;
 };
 
 }  // namespace fq

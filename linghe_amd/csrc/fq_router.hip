@@ -1,40 +1,26 @@
-// RMSNorm + router GEMM + 1x128 quant in one pass over x
+// RMSNorm + router GEMM + 1x128 quant
 // (linghe/utils/norm.py:616-784, output_mode 0; kernel :616-687):
 //   r = rsqrt(mean(x^2) + eps);  y = (x*r)*gamma  (fp32)
 //   y_bf16 = bf16(y);  logits = y @ W^T (fp32);  q, s = 1x128 quant of y
 //
-// The only contraction on this path, so the only place MFMA is used.  The
-// reference multiplies fp32 y by W with tl.dot; here y is split into two bf16
-// terms, y = hi + lo (hi = bf16(y) is the y_bf16 output itself, lo = bf16(y - hi),
-// what is left is below 2^-17 |y|), W is bf16 already, and the two products go
-// through v_mfma_f32_32x32x16_bf16 with fp32 accumulation: bf16 products are
-// exact in fp32, so the result carries the accuracy of an fp32 GEMM at the bf16
-// MFMA rate.
-//
-// Two kernels share this scheme: the one below streams the rows twice (statistic,
-// then the blocks) and takes any K; rmsnorm_router_quant_resident_kernel further
-// down keeps the rows in registers when they fit.
+// The only contraction on this path, so the only place MFMA is used.  r is a per-row factor of
+// y, hence of the logits:
+//   logits[m, :] = r[m] * sum_k (x[m,k] * gamma[k]) * W[:, k]
+// z = x * gamma is EXACT in fp32 (two 8-bit significands) and so is its split z = hi + lo into
+// two bf16 values; W is bf16 already, and the two products go through the bf16 matrix
+// instructions with fp32 accumulation: bf16 products are exact in fp32, so the result carries
+// only the rounding of the fp32 accumulation and one final multiplication by r, and the
+// contraction does not wait for the statistic.
 //
 // An fp32 router weight (what Megatron keeps) is split the same way, W = hi + lo with
-// hi = bf16(W), lo = bf16(W - hi) (what is left is below 2^-17 |W|), and the two planes
-// are laid side by side as "virtual" columns 2n (hi) and 2n + 1 (lo): the GEMM runs on
-// 2N bf16 columns and the epilogue adds each pair, which sits in neighbouring lanes.
-// More than 512 virtual columns are cut into chunks of at most 512, one launch each;
-// only the first launch writes y, the codes, the scales and the statistic.
+// hi = bf16(W), lo = bf16(W - hi) (what is left is below 2^-17 |W|): two planes, four products
+// into the same accumulators.
 //
-// One workgroup (4 or 8 waves) owns 32 rows and all N <= 512 logits of them and walks K
-// in blocks of 128 (one quantisation group per row):
-//   each thread normalises 2 rows x 8 columns of the block (16 lanes per row, so
-//   every global access is coalesced), quantises them with the row's 1x128 scale
-//   (a DPP reduction over the 16 lanes), stores y_bf16 and the codes, and writes
-//   the hi/lo A operands to LDS in MFMA lane order; after one barrier each wave
-//   multiplies the whole 32x128 block by its N/4 columns of W.
-// Lane l of a wave holds, as MFMA wants it, row l%32 and 8 consecutive k of a
-// 16-wide k step.  Which 16 of the block's 128 columns form step j is free as long
-// as A and B agree: step j takes columns 8j..8j+7 (lanes 0-31) and 64+8j..64+8j+7
-// (lanes 32-63), so that a lane's eight B loads of a block cover one contiguous
-// 128-byte line of its W row; the 32x32 result has column l%32 and rows
-// (v/4)*8 + (l/32)*4 + v%4 in register v.
+// Both kernels below share the work out over (row tile, column chunk) pairs; the workgroups of
+// one row tile sit on one XCD (router_tile), so that x comes from memory once and from that
+// XCD's L2 for the other chunks.  Each of them walks all of K for its columns of the logits,
+// accumulating the row statistic beside it, and then writes y, the codes and the scales for its
+// share of the K / 128 quantisation groups, re-reading that part of x from the L2.
 #include "fq_device.hpp"
 #include "fq_launch.h"
 #include "fq_policy.hpp"
@@ -45,69 +31,35 @@ namespace fq {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float floatx16_t __attribute__((ext_vector_type(16)));
+typedef float floatx4_t __attribute__((ext_vector_type(4)));
 
-constexpr int kRouterRows = 32;
-
-struct RouterShared {
-  uint4 a[2][2][8][64];  // [buffer][hi, lo][k step][lane slot]: A operands of one 32x128 block
-  float rstd[kRouterRows];
-};
-
-// 1/sqrt(mean(x^2) + eps) of four consecutive rows by one wave (their loads in
-// flight together), the arithmetic of the row kernels: 8-element group sums added
-// in double, so the value does not depend on the split
-__device__ __forceinline__ void router_rows_rstd(const uint16_t* rows, int n, float eps, float (&out)[4]) {
-  const int lane = tid_x() & 63;
-  const int chunks = n >> 3;
-  double ss[4] = {0.0, 0.0, 0.0, 0.0};
-  for (int c0 = 0; c0 < chunks; c0 += 256) {
-    uint4 v[4][4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int c = c0 + u * 64 + lane;
-        v[k][u] = make_uint4(0, 0, 0, 0);
-        if (c < chunks) v[k][u] = *(const uint4*)(rows + (int64_t)k * n + c * 8);
-      }
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-#pragma unroll
-      for (int u = 0; u < 4; ++u) ss[k] += (double)sumsq8(v[k][u]);
-  }
-#pragma unroll
-  for (int k = 0; k < 4; ++k) out[k] = 1.0f / sqrtf((float)wave_sum_d(ss[k]) / (float)n + eps);
-}
-
-// W [N, K] -> B operands in the order the main kernel reads them: one 16-byte piece
-// per (k block, 32-column tile, k step, lane), so that every B load of a wave is
-// 1 KB of contiguous memory.  (Read straight from the row-major matrix, each lane of
-// such a load would touch a cache line of its own.)  One launch packs the `vtiles`
-// 32-column tiles of one chunk, starting at virtual column vcol0; with an fp32 weight
-// virtual column v is plane v & 1 (0: bf16(W), 1: bf16 of the rest) of column v >> 1.
+// W [N, K] -> B operands in the order the main kernels read them: one 16-byte piece per (k
+// block of 128, 32-column tile, k step, lane), so that every B load of a wave is 1 KB of
+// contiguous memory.  (Read straight from the row-major matrix, each lane of such a load would
+// touch a cache line of its own.)  Piece j of lane l holds columns 64 (l / 32) + 8 j .. + 7 of
+// the k block of row l % 32 of its tile.  With an fp32 weight the tiles come in pairs: bf16(W) of 32
+// columns, then bf16 of the rest.
 template <bool FP32W>
 __global__ __launch_bounds__(256) void pack_router_weight_kernel(const void* __restrict__ wr,
-                                                                 uint4* __restrict__ packed, int K, int vcol0,
-                                                                 int vtiles) {
-  const int64_t idx = (int64_t)wg_x() * 256 + tid_x();  // piece number inside the chunk
+                                                                 uint4* __restrict__ packed, int K, int vtiles) {
+  const int64_t idx = (int64_t)wg_x() * 256 + tid_x();
   const int64_t total = (int64_t)vtiles * 32 * K / 8;
   if (idx >= total) return;
   const int lane = (int)(idx & 63);
-  int64_t rest = idx >> 6;
-  const int j = (int)(rest & 7);
-  rest >>= 3;
+  const int64_t rest = idx >> 9;
+  const int j = (int)(idx >> 6) & 7;
   const int tile = (int)(rest % vtiles);
   const int kb = (int)(rest / vtiles);
-  const int v = vcol0 + tile * 32 + (lane & 31);
   const int k = kb * kGroup + (lane >> 5) * 64 + j * 8;
   if constexpr (!FP32W) {
-    packed[idx] = *(const uint4*)((const uint16_t*)wr + (int64_t)v * K + k);
+    packed[idx] = *(const uint4*)((const uint16_t*)wr + (int64_t)(tile * 32 + (lane & 31)) * K + k);
   } else {
-    const float4* src = (const float4*)((const float*)wr + (int64_t)(v >> 1) * K + k);
+    const int n = (tile >> 1) * 32 + (lane & 31);
+    const float4* src = (const float4*)((const float*)wr + (int64_t)n * K + k);
     const float4 a = src[0], b = src[1];
     float w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
     const uint4 hi = pack8_bf16(w);
-    if (v & 1) {
+    if (tile & 1) {
       float back[8], lo[8];
       unpack8(hi, back);
 #pragma unroll
@@ -119,342 +71,416 @@ __global__ __launch_bounds__(256) void pack_router_weight_kernel(const void* __r
   }
 }
 
-// Where a launch puts its logits.  A chunk holds `real` columns of the [M, n_logits] matrix
-// starting at col0; with PAIR the accumulator columns come in (hi, lo) pairs in neighbouring
-// lanes and their sum is one real column.
-struct LogitsOut {
-  float* logits;
-  int n_logits;  // row stride
-  int col0;      // first real column of this launch
+struct RouterArgs {
+  const uint16_t* x;      // [M, K]
+  const uint16_t* gamma;  // [K]
+  const uint4* w;         // packed
+  uint16_t* y;            // [M, K]
+  float* rstd;            // [M]
+  float* logits;          // [M, N]
+  uint8_t* q;             // [M, K]
+  float* s;               // [K / 128, M]
+  int M, K, N;
+  int chunks;  // column chunks, i.e. workgroups per row tile
+  float eps;
 };
-template <bool PAIR>
-__device__ __forceinline__ void store_logit(const LogitsOut& o, int64_t row, int vcol, float v) {
-  if constexpr (PAIR) {
-    v += dpp_mov<kDppQuadXor1>(v);  // lanes 2i, 2i+1 hold the two planes of one column
-    if ((vcol & 1) == 0) o.logits[row * o.n_logits + o.col0 + (vcol >> 1)] = v;
+
+// workgroup -> (row tile, column chunk): workgroup i runs on XCD i % 8, so eight row tiles go
+// round the XCDs and the chunks of one tile follow each other there; the last tiles % 8 row tiles do the same
+// in a narrower round
+__device__ __forceinline__ void router_tile(int tiles, int chunks, int& tile, int& chunk) {
+  const int i = (int)wg_x();
+  const int full = (tiles & ~7) * chunks;
+  if (i < full) {
+    const int r = i >> 3;
+    chunk = r % chunks;
+    tile = (r / chunks) * 8 + (i & 7);
   } else {
-    o.logits[row * o.n_logits + o.col0 + vcol] = v;
+    const int left = tiles & 7;
+    chunk = (i - full) / left;
+    tile = (tiles & ~7) + (i - full) % left;
   }
 }
 
-// WAVES waves per workgroup, TPW column tiles (of 32 logits) per wave: N = 32 * WAVES * TPW.
-// With 8 waves a thread owns one row x 8 columns of a k block, with 4 waves two rows.
-// SIDE: this launch also writes y, the codes, the scales and the statistic (the first chunk does)
-template <int KIND, bool ROUND, int TPW, int WAVES, bool PAIR, bool SIDE>
-__global__ __launch_bounds__(64 * WAVES) void rmsnorm_router_quant_kernel(
-    const uint16_t* __restrict__ x, const uint16_t* __restrict__ gamma, const uint4* __restrict__ wpacked,
-    uint16_t* __restrict__ y, float* __restrict__ rstd_out, LogitsOut lout, uint8_t* __restrict__ q,
-    float* __restrict__ s, int64_t M, int K, float eps) {
-  __shared__ RouterShared sh;
-  const int lane = tid_x() & 63;
-  const int wave = tid_x() >> 6;
-  const int64_t row0 = (int64_t)wg_x() * kRouterRows;
+// the two exact terms of x * gamma of 8 columns, as matrix operands
+__device__ __forceinline__ void router_split(const uint4& xr, const uint4& gr, uint4& hi, uint4& lo) {
+  float a[8], g[8], z[8], back[8];
+  unpack8(xr, a);
+  unpack8(gr, g);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) z[i] = a[i] * g[i];
+  hi = pack8_bf16(z);
+  unpack8(hi, back);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) back[i] = z[i] - back[i];
+  lo = pack8_bf16(back);
+}
 
-  constexpr int NT = TPW;
-  constexpr int RPT = 8 / WAVES;  // rows per thread: 2 with 4 waves, 1 with 8
-  // ---- statistic of the 32 rows, four at a time per wave
-#pragma unroll 1
-  for (int u = 0; u < kRouterRows / WAVES; u += 4) {
-    const int r = wave * (kRouterRows / WAVES) + u;
-    float rs[4];
-    router_rows_rstd(x + (row0 + r) * K, K, eps, rs);
-    if (lane < 4) {
-      const float mine = lane == 0 ? rs[0] : lane == 1 ? rs[1] : lane == 2 ? rs[2] : rs[3];
-      sh.rstd[r + lane] = mine;
-      if constexpr (SIDE) rstd_out[row0 + r + lane] = mine;
-    }
+// y, codes and scale of 8 columns; the 16 lanes of a DPP row (the first of them names the scale's place)
+// hold one quantisation group
+template <int KIND, bool ROUND>
+__device__ __forceinline__ void router_emit(uint16_t* y, uint8_t* q, float* s, bool first, const uint4& xr,
+                                            const uint4& gr, float r) {
+  float a[8], g[8], yv[8], m = 0.f;
+  unpack8(xr, a);
+  unpack8(gr, g);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    yv[i] = (a[i] * r) * g[i];
+    m = fmaxf(m, fabsf(yv[i]));
   }
-  __syncthreads();
+  m = row16_max(m);
+  const float sc = make_scale<KIND, ROUND>(m);
+  store16<Policy::kStoreHintRouter>(y, pack8_bf16(yv));
+  store8<Policy::kStoreHintRouter>(q, quantize8<KIND, ROUND>(yv, make_quantum<ROUND>(sc)));
+  if (first) store_f32(s, sc);
+}
 
-  // producer side: thread (rg, cg) holds rows RPT rg .. and columns 8 cg .. 8 cg + 7 of
-  // the k block, so 16 lanes read, and write, 256 (128 for the codes) contiguous bytes
-  const int cg = tid_x() & 15;
-  const int rg = tid_x() >> 4;
-  const float r0 = sh.rstd[RPT * rg], r1 = sh.rstd[RPT * rg + RPT - 1];
-  const uint16_t* xrow = x + (row0 + RPT * rg) * K + cg * 8;
-  uint16_t* yrow = y + (row0 + RPT * rg) * K + cg * 8;
-  uint8_t* qrow = q + (row0 + RPT * rg) * K + cg * 8;
-  // consumer side (MFMA lane order)
-  const int arow = lane & 31;
-  const int half = lane >> 5;
-  floatx16_t acc[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t)
-#pragma unroll
-    for (int v = 0; v < 16; ++v) acc[t][v] = 0.f;
+__device__ __forceinline__ bf16x8_t operand(const uint4& v) { return __builtin_bit_cast(bf16x8_t, v); }
 
-  const int kblocks = K / kGroup;
-  // operands of a k block: this wave's NT column tiles of W (B operands), the
-  // thread's two rows of x and its piece of gamma.  Only one workgroup of these fits
-  // a CU's share of the rows, so the next block's operands are fetched while the
-  // current one is worked on.
-  auto fetch_w = [&](int kb, uint4 (&b)[NT][8]) {
-    const uint4* wp = wpacked + ((int64_t)(kb * WAVES + wave) * NT) * 8 * 64 + lane;
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) b[t][j] = wp[(t * 8 + j) * 64];
-  };
-  auto fetch_x = [&](int kb, uint4 (&xr)[RPT], uint4& gr) {
-#pragma unroll
-    for (int u = 0; u < RPT; ++u) xr[u] = *(const uint4*)(xrow + (int64_t)u * K + kb * kGroup);
-    gr = *(const uint4*)(gamma + kb * kGroup + cg * 8);
-  };
-  // column chunk cg of the block is k step (cg & 7), lanes 32*(cg >> 3).. of the A
-  // operand; the row position is XORed with the k step so that the 16-byte LDS
-  // writes of the eight lanes of a row group fall into different banks
-  const int aj = cg & 7;
-  const int ahalf = cg >> 3;
+// ---------------------------------------------------------------------------
+// 64 rows x 64 VT operand columns per workgroup of eight waves: 64 VT logits of a bf16 weight, 64 of an
+// fp32 one (VT = 2, its two planes).  Per 128-wide k block the threads turn 64 x 128 values of x
+// into A operands in LDS (2 rows x 8 columns each) while the matrix cores work on the block before
+// (double-buffered, one barrier per block).  Wave (wc, kq) multiplies all 64 rows by 32 VT operand columns
+// over a quarter of the block's k, so that A is read from LDS twice per block (64 KB) and W from the L2
+// once (32 KB with VT = 2; an XCD's CUs share about 35 B a clock each); the four k quarters are
+// added up through LDS at the end.
+// Bound by instruction issue: per k block about 1000 clocks of matrix instructions and 900 of operand
+// arithmetic on each SIMD, partly on top of each other, and per block of the second part 1600 clocks of
+// normalising and quantising.  us of the kernel (32-row workgroups with all of W each before / now): 4096 x 256 x 4096
+// with an fp32 weight 84 / 53, 8192 x 256 x 2048 bf16 35.8 / 36.3, 4096 x 512 x 4096 bf16 84 / 51,
+// 16384 x 128 x 2048 bf16 62 / 51; with VT = 1 4096 x 256 x 2048 28.8 / 23.8.
+// ---------------------------------------------------------------------------
+constexpr int kRouterRows = 64;
 
-  // one k block: normalise / quantise / store the thread's piece, publish the A
-  // operands, then multiply the whole block by this wave's columns of W
-  auto step = [&](int kb, const uint4 (&xr)[RPT], const uint4& gr, const uint4 (&b)[NT][8]) {
-    const int buf = kb & 1;
-    float g[8];
-    unpack8(gr, g);
-#pragma unroll
-    for (int u = 0; u < RPT; ++u) {
-      const float r = u ? r1 : r0;
-      float a[8], yv[8];
-      unpack8(xr[u], a);
-      float m = 0.f;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        yv[i] = (a[i] * r) * g[i];
-        m = fmaxf(m, fabsf(yv[i]));
-      }
-      const uint4 hi = pack8_bf16(yv);
-      float back[8], lo[8];
-      unpack8(hi, back);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) lo[i] = yv[i] - back[i];
-      const int slot = ahalf * 32 + ((RPT * rg + u) ^ aj);
-      sh.a[buf][0][aj][slot] = hi;
-      sh.a[buf][1][aj][slot] = pack8_bf16(lo);
-      if constexpr (SIDE) {
-        m = row16_max(m);
-        const float sc = make_scale<KIND, ROUND>(m);
-        store16<Policy::kStoreHintRouter>(yrow + (int64_t)u * K + kb * kGroup, hi);
-        const uint2 pk = quantize8<KIND, ROUND>(yv, make_quantum<ROUND>(sc));
-        store8<Policy::kStoreHintRouter>(qrow + (int64_t)u * K + kb * kGroup, pk);
-        if (cg == 0) s[(int64_t)kb * M + row0 + RPT * rg + u] = sc;
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int slot = half * 32 + (arow ^ j);
-      const bf16x8_t ahi = __builtin_bit_cast(bf16x8_t, sh.a[buf][0][j][slot]);
-      const bf16x8_t alo = __builtin_bit_cast(bf16x8_t, sh.a[buf][1][j][slot]);
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const bf16x8_t bw = __builtin_bit_cast(bf16x8_t, b[t][j]);
-        acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ahi, bw, acc[t], 0, 0, 0);
-        acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(alo, bw, acc[t], 0, 0, 0);
-      }
-    }
-  };
+struct RouterShared {
+  uint4 a[2][2][2][8][64];  // [buffer][hi, lo][32-row tile][k step][lane slot]; afterwards the partial sums
+  uint4 gamma[8192 / 8];
+  float rstd[kRouterRows];
+};
 
-  // x comes from HBM (its second read may still find it in a cache), W from L2: x is
-  // fetched kAhead blocks ahead, W one block ahead.  The loop is unrolled over the
-  // ring of kAhead operand sets so that a set is refilled in place right after it
-  // was used: no register is copied while its load is still in flight.
-  constexpr int kAhead = 4;
-  uint4 b[2][NT][8], xq[kAhead][RPT], gq[kAhead];
-  fetch_w(0, b[0]);
+// The order of a k block's instructions: operand reads, then the matrix instructions with the next
+// block's operand arithmetic between them.  (Left alone the compiler puts the arithmetic behind
+// all of them, and as the waves of a SIMD go in step, matrix cores and arithmetic units take turns:
+// 80 instead of 87 us at 4096 x 256 x 7168.)
+template <int VT>
+__device__ __forceinline__ void router_interleave() {
+  constexpr int kValu = 0x2, kMfma = 0x8, kVmemRead = 0x20, kDsRead = 0x100, kDsWrite = 0x200;
+  __builtin_amdgcn_sched_group_barrier(kDsRead, 5, 0);
+  __builtin_amdgcn_sched_group_barrier(kValu, 12, 0);
 #pragma unroll
-  for (int d = 0; d < kAhead; ++d)
-    if (d < kblocks) fetch_x(d, xq[d], gq[d]);
-#pragma unroll 1
-  for (int kb0 = 0; kb0 < kblocks; kb0 += kAhead) {
+  for (int i = 0; i < 4; ++i) {
 #pragma unroll
-    for (int d = 0; d < kAhead; ++d) {
-      const int kb = kb0 + d;
-      if (kb < kblocks) {
-        if (kb + 1 < kblocks) fetch_w(kb + 1, b[(d + 1) & 1]);
-        step(kb, xq[d], gq[d], b[d & 1]);
-        if (kb + kAhead < kblocks) fetch_x(kb + kAhead, xq[d], gq[d]);
-      }
+    for (int m = 0; m < 2 * VT; ++m) {
+      __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(kValu, 10 / VT, 0);
     }
-  }
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const int col = (wave * NT + t) * 32 + arow;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int row = (v / 4) * 8 + half * 4 + (v % 4);
-      store_logit<PAIR>(lout, row0 + row, col, acc[t][v]);
-    }
+    if (i < 1) __builtin_amdgcn_sched_group_barrier(kDsRead, 4, 0);
+    if (i < 1 + VT) __builtin_amdgcn_sched_group_barrier(kVmemRead, 2, 0);
+    if (i > 0) __builtin_amdgcn_sched_group_barrier(kDsWrite, 2, 0);
   }
 }
 
-
-// The same operation for K == 128 * KB with the workgroup's rows of x held in
-// registers, so that x is read from memory once and the GEMM does not wait for the
-// statistic.  rstd is a per-row factor of y, hence of the logits:
-//   logits[r, :] = rstd[r] * sum_k (x[r,k] * gamma[k]) * W[:, k]
-// and z = x * gamma is EXACT in fp32 (two 8-bit significands), as is its split
-// z = hi + lo into two bf16 values, so the contraction carries only the rounding of
-// the fp32 accumulation and one final multiplication by rstd.
-//   sweep 1, per k block as x arrives: z -> hi/lo A operands in LDS -> MFMA; the sum
-//     of squares accumulates beside it (8-element group sums added in double, the
-//     arithmetic of the row kernels); the next block's W loads are issued between
-//     the MFMAs so that the memory pipeline and the matrix cores work together;
-//   sweep 2, from registers: logits *= rstd; y = (x*rstd)*gamma -> bf16, codes and
-//     scales, streamed out.
-template <int KIND, bool ROUND, int TPW, int WAVES, int KB, int WDEPTH, bool PAIR>
-__global__ __launch_bounds__(64 * WAVES) void rmsnorm_router_quant_resident_kernel(
-    const uint16_t* __restrict__ x, const uint16_t* __restrict__ gamma, const uint4* __restrict__ wpacked,
-    uint16_t* __restrict__ y, float* __restrict__ rstd_out, LogitsOut lout, uint8_t* __restrict__ q,
-    float* __restrict__ s, int64_t M, int K, float eps) {
+template <int KIND, bool ROUND, bool FP32W, int VT>
+__global__ __launch_bounds__(512) void rmsnorm_router_quant_kernel(RouterArgs p) {
   __shared__ RouterShared sh;
-  __shared__ uint4 sgamma[KB * 16];  // gamma, 8 columns per piece
   const int lane = tid_x() & 63;
-  const int wave = tid_x() >> 6;
-  const int64_t row0 = (int64_t)wg_x() * kRouterRows;
-  constexpr int NT = TPW;
-  constexpr int RPT = 8 / WAVES;
-  constexpr int kAhead = 6;  // k blocks of x in flight ahead of the one worked on
-  constexpr int kWAhead = WDEPTH - 1;  // k blocks of W in flight ahead of the one worked on
-  const int cg = tid_x() & 15;
-  const int rg = tid_x() >> 4;
-  const uint16_t* xrow = x + (row0 + RPT * rg) * K + cg * 8;
-  const int aj = cg & 7;
-  const int ahalf = cg >> 3;
-  const int arow = lane & 31;
-  const int half = lane >> 5;
-  constexpr int kblocks = KB;  // a constant trip count lets the compiler schedule across blocks
+  const int wave = uniform32(tid_x() >> 6);
+  const int kq = wave & 3, wc = wave >> 2;
+  const int cg = tid_x() & 15, rg = tid_x() >> 4;
+  const int kblocks = p.K / kGroup;
+  int tile, chunk;
+  router_tile((p.M + kRouterRows - 1) / kRouterRows, p.chunks, tile, chunk);
+  // rows that do not fill a tile are worked on twice, with the same results, by the last two tiles
+  const int row0 = min(tile * kRouterRows, p.M - kRouterRows);
+  const uint16_t* xrow = p.x + (int64_t)(row0 + rg) * p.K + cg * 8;
+  const int64_t half_tile = (int64_t)32 * p.K;
 
-  floatx16_t acc[NT];
+  constexpr int kRing = 4;                // k blocks of x and W in flight or in use
+  constexpr int NACC = FP32W ? 1 : VT;    // 32-column result tiles of a wave
+  uint4 xr[kRing][2], b[kRing][VT][2];    // b: [slot][operand tile][k step]
+  floatx16_t acc[2][NACC];
 #pragma unroll
-  for (int t = 0; t < NT; ++t)
+  for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) acc[t][v] = 0.f;
+    for (int t = 0; t < NACC; ++t)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[rt][t][v] = 0.f;
+  double ss[2] = {0.0, 0.0};
 
-  uint4 xr[KB][RPT], b[WDEPTH][NT][8];
-  double ss[RPT];
+  const int vtiles = p.N / 32 * (FP32W ? 2 : 1);
+  const uint4* wlane = p.w + ((int64_t)(chunk * 2 + wc) * VT * 8 + kq * 2) * 64 + lane;
+  auto fetch_w = [&](int kb, uint4 (&d)[VT][2]) {
+    const uint4* at = wlane + (int64_t)min(kb, kblocks - 1) * vtiles * 512;
 #pragma unroll
-  for (int u = 0; u < RPT; ++u) ss[u] = 0.0;
-  const uint4* wlane = wpacked + (int64_t)wave * NT * 8 * 64 + lane;
-  auto w_piece = [&](int kb, int t, int j) { return wlane[((int64_t)kb * WAVES * NT + t) * 8 * 64 + j * 64]; };
-  auto fetch_x = [&](int kb, uint4 (&xk)[RPT]) {
+    for (int t = 0; t < VT; ++t)
 #pragma unroll
-    for (int u = 0; u < RPT; ++u) xk[u] = load16<Policy::kLoadHintRouter>(xrow + (int64_t)u * K + kb * kGroup);
+      for (int j = 0; j < 2; ++j) d[t][j] = at[t * 512 + j * 64];
   };
+  auto fetch_x = [&](int kb, uint4 (&d)[2]) {
+    const uint16_t* at = xrow + min(kb, kblocks - 1) * kGroup;
+    d[0] = *(const uint4*)at;
+    d[1] = *(const uint4*)(at + half_tile);
+  };
+  // the row position is XORed with the k step so that the 16-byte LDS writes of the eight lanes
+  // of a row group fall into different banks
+  const int aj = cg & 7;
+  const int aslot = (cg >> 3) * 32 + (rg ^ aj);
+  auto produce = [&](int kb, const uint4 (&xk)[2]) {
+    const uint4 g = sh.gamma[kb * 16 + cg];
 #pragma unroll
-  for (int d = 0; d < kWAhead; ++d)
-    if (d < kblocks) {
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) b[d][t][j] = w_piece(d, t, j);
-    }
-#pragma unroll
-  for (int d = 0; d < kAhead; ++d)
-    if (d < kblocks) fetch_x(d, xr[d]);
-  for (int p = tid_x(); p < kblocks * 16; p += 64 * WAVES) sgamma[p] = *(const uint4*)(gamma + p * 8);
-  __syncthreads();
-
-  // ---- sweep 1, software pipelined: the A operands of block kb + 1 are produced
-  // while the matrix cores work on block kb (double-buffered in LDS, one barrier
-  // per block)
-  auto produce = [&](int kb, const uint4 (&xk)[RPT]) {
-    float g[8];
-    unpack8(sgamma[kb * 16 + cg], g);
-#pragma unroll
-    for (int u = 0; u < RPT; ++u) {
-      float a[8], z[8], back[8], lo[8];
-      unpack8(xk[u], a);
+    for (int u = 0; u < 2; ++u) {
       ss[u] += (double)sumsq8(xk[u]);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) z[i] = a[i] * g[i];
-      const uint4 hi = pack8_bf16(z);
-      unpack8(hi, back);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) lo[i] = z[i] - back[i];
-      const int slot = ahalf * 32 + ((RPT * rg + u) ^ aj);
-      sh.a[kb & 1][0][aj][slot] = hi;
-      sh.a[kb & 1][1][aj][slot] = pack8_bf16(lo);
+      uint4 hi, lo;
+      router_split(xk[u], g, hi, lo);
+      sh.a[kb & 1][0][u][aj][aslot] = hi;
+      sh.a[kb & 1][1][u][aj][aslot] = lo;
     }
   };
-  produce(0, xr[0]);
-  if (kAhead < kblocks) fetch_x(kAhead, xr[kAhead]);
+  auto multiply = [&](int buf, const uint4 (&w)[VT][2]) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int step = kq * 2 + j;
+      const int slot = (lane & 32) + ((lane & 31) ^ step);
+#pragma unroll
+      for (int rt = 0; rt < 2; ++rt) {
+        const bf16x8_t hi = operand(sh.a[buf][0][rt][step][slot]);
+        const bf16x8_t lo = operand(sh.a[buf][1][rt][step][slot]);
+#pragma unroll
+        for (int t = 0; t < VT; ++t) {
+          floatx16_t& c = acc[rt][FP32W ? 0 : t];
+          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(hi, operand(w[t][j]), c, 0, 0, 0);
+          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lo, operand(w[t][j]), c, 0, 0, 0);
+        }
+      }
+    }
+  };
+
+  // gamma (at most 1024 pieces) is asked for first, so that waiting for it waits for nothing else
+  uint4 g2[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    g2[i] = *(const uint4*)(p.gamma + min((int)tid_x() + 512 * i, kblocks * 16 - 1) * 8);
+#pragma unroll
+  for (int d = 0; d < kRing; ++d) fetch_x(d, xr[d]);
+#pragma unroll
+  for (int d = 0; d < kRing - 1; ++d) fetch_w(d, b[d]);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) sh.gamma[tid_x() + 512 * i] = g2[i];
   __syncthreads();
+  produce(0, xr[0]);
+  fetch_x(kRing, xr[0]);
+  __syncthreads();
+  // rings of kRing operand sets: a set is refilled in place once it was used.  Fetches beyond the last block
+  // repeat it; all but the last 1 .. kRing blocks run without a condition
+  int kb = 0;
+#pragma unroll 1
+  for (; kb + kRing < kblocks; kb += kRing) {
 #pragma unroll
-  for (int kb = 0; kb < kblocks; ++kb) {
-    const int buf = kb & 1;
-    const bool more = kb + kWAhead < kblocks;
-    const int kNext = (kb + kWAhead) % WDEPTH;
-    if (kb + 1 < kblocks) {
-      produce(kb + 1, xr[kb + 1]);
-      if (kb + 1 + kAhead < kblocks) fetch_x(kb + 1 + kAhead, xr[kb + 1 + kAhead]);
+    for (int d = 0; d < kRing; ++d) {
+      fetch_w(kb + d + kRing - 1, b[(d + kRing - 1) % kRing]);
+      multiply(d & 1, b[d]);
+      produce(kb + d + 1, xr[(d + 1) % kRing]);
+      fetch_x(kb + d + 1 + kRing, xr[(d + 1) % kRing]);
+      router_interleave<VT>();
+      __syncthreads();
+      __builtin_amdgcn_sched_barrier(0);  // the order is laid out block by block
     }
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      if (more) {
-#pragma unroll
-        for (int t = 0; t < NT; ++t) b[kNext][t][j] = w_piece(kb + kWAhead, t, j);
-      }
-      const int slot = half * 32 + (arow ^ j);
-      const bf16x8_t ahi = __builtin_bit_cast(bf16x8_t, sh.a[buf][0][j][slot]);
-      const bf16x8_t alo = __builtin_bit_cast(bf16x8_t, sh.a[buf][1][j][slot]);
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const bf16x8_t bw = __builtin_bit_cast(bf16x8_t, b[kb % WDEPTH][t][j]);
-        acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ahi, bw, acc[t], 0, 0, 0);
-        acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(alo, bw, acc[t], 0, 0, 0);
-      }
-    }
-    __syncthreads();
   }
+#pragma unroll
+  for (int d = 0; d < kRing; ++d) {
+    if (kb + d < kblocks) {
+      if (d == 0) fetch_w(kb + kRing - 1, b[kRing - 1]);
+      multiply(d & 1, b[d]);
+      if (kb + d + 1 < kblocks) produce(kb + d + 1, xr[(d + 1) % kRing]);
+      __syncthreads();
+    }
+  }
+
+  // ---- this workgroup's share of the quantisation groups: its first rows of x leave now
+  const int q0 = chunk * kblocks / p.chunks;
+  const int q1 = (chunk + 1) * kblocks / p.chunks;
+  constexpr int kEmit = 4 * NACC;  // k blocks at a time: no load waits behind a store
+  uint4 xe[kEmit][2];
+#pragma unroll
+  for (int d = 0; d < kEmit; ++d) fetch_x(q0 + d, xe[d]);
 
   // ---- statistic
-  float rs[RPT];
+  float rs[2];
 #pragma unroll
-  for (int u = 0; u < RPT; ++u) {
-    rs[u] = 1.0f / sqrtf((float)row16_sum_d(ss[u]) / (float)K + eps);
+  for (int u = 0; u < 2; ++u) {
+    rs[u] = 1.0f / sqrtf((float)row16_sum_d(ss[u]) / (float)p.K + p.eps);
     if (cg == 0) {
-      sh.rstd[RPT * rg + u] = rs[u];
-      rstd_out[row0 + RPT * rg + u] = rs[u];
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const int col = (wave * NT + t) * 32 + arow;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int row = (v / 4) * 8 + half * 4 + (v % 4);
-      store_logit<PAIR>(lout, row0 + row, col, acc[t][v] * sh.rstd[row]);
+      sh.rstd[u * 32 + rg] = rs[u];
+      if (chunk == 0) p.rstd[row0 + u * 32 + rg] = rs[u];
     }
   }
 
-  // ---- sweep 2
-  uint16_t* yrow = y + (row0 + RPT * rg) * K + cg * 8;
-  uint8_t* qrow = q + (row0 + RPT * rg) * K + cg * 8;
+  // ---- the four k quarters: waves kq and kq ^ 2 exchange a row tile, then kq and kq ^ 1 half of
+  // what they hold, so that all eight waves end up with an equal part of the sums
+  floatx4_t* part = (floatx4_t*)&sh.a[0][0][0][0][0];
+  auto quarter = [](const floatx16_t& c, int i) {
+    floatx4_t o = {c[4 * i], c[4 * i + 1], c[4 * i + 2], c[4 * i + 3]};
+    return o;
+  };
+  // (by value: a conditional between array elements would choose between addresses, and the
+  // arrays would leave the registers)
+  auto pick = [](bool first, floatx4_t a, floatx4_t c) { return first ? a : c; };
+  const bool upper = kq >> 1, odd = kq & 1;
 #pragma unroll
-  for (int kb = 0; kb < kblocks; ++kb) {
-    {
-      float g[8];
-      unpack8(sgamma[kb * 16 + cg], g);
+  for (int t = 0; t < NACC; ++t)
 #pragma unroll
-      for (int u = 0; u < RPT; ++u) {
-        float a[8], yv[8];
-        unpack8(xr[kb][u], a);
-        float m = 0.f;
+    for (int i = 0; i < 4; ++i)
+      part[((wave * NACC + t) * 4 + i) * 64 + lane] = pick(upper, quarter(acc[0][t], i), quarter(acc[1][t], i));
+  __syncthreads();
+  floatx4_t sum[NACC * 4];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          yv[i] = (a[i] * rs[u]) * g[i];
-          m = fmaxf(m, fabsf(yv[i]));
-        }
-        m = row16_max(m);
-        const float sc = make_scale<KIND, ROUND>(m);
-        store16<Policy::kStoreHintRouter>(yrow + (int64_t)u * K + kb * kGroup, pack8_bf16(yv));
-        const uint2 pk = quantize8<KIND, ROUND>(yv, make_quantum<ROUND>(sc));
-        store8<Policy::kStoreHintRouter>(qrow + (int64_t)u * K + kb * kGroup, pk);
-        if (cg == 0) s[(int64_t)kb * M + row0 + RPT * rg + u] = sc;
+  for (int t = 0; t < NACC; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      sum[t * 4 + i] = pick(upper, quarter(acc[1][t], i), quarter(acc[0][t], i)) +
+                       part[(((wave ^ 2) * NACC + t) * 4 + i) * 64 + lane];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NACC * 2; ++i)
+    part[(wave * NACC * 2 + i) * 64 + lane] = pick(odd, sum[i], sum[NACC * 2 + i]);
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NACC * 2; ++i) {
+    const floatx4_t v = pick(odd, sum[NACC * 2 + i], sum[i]) + part[((wave ^ 1) * NACC * 2 + i) * 64 + lane];
+    // register r of a 32x32 result holds row (r / 4) * 8 + (lane / 32) * 4 + r % 4, column lane % 32
+    const int i4 = (odd ? NACC * 2 : 0) + i;
+    const int row = (upper ? 32 : 0) + (i4 & 3) * 8 + (lane >> 5) * 4;
+    const int col = ((chunk * 2 + wc) * NACC + (i4 >> 2)) * 32 + (lane & 31);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      p.logits[(int64_t)(row0 + row + e) * p.N + col] = v[e] * sh.rstd[row + e];
+  }
+
+#pragma unroll 1
+  for (int k0 = q0; k0 < q1; k0 += kEmit) {
+    if (k0 > q0) {
+#pragma unroll
+      for (int d = 0; d < kEmit; ++d) fetch_x(k0 + d, xe[d]);
+    }
+    const int64_t at = (int64_t)(row0 + rg) * p.K + k0 * kGroup + cg * 8;
+    uint16_t* y = p.y + at;
+    uint8_t* q = p.q + at;
+    float* s = p.s + (int64_t)k0 * p.M + row0 + rg;
+#pragma unroll
+    for (int d = 0; d < kEmit; ++d) {
+      if (k0 + d < q1) {
+        const uint4 g = sh.gamma[(k0 + d) * 16 + cg];
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+          router_emit<KIND, ROUND>(y + u * half_tile + d * kGroup, q + u * half_tile + d * kGroup,
+                                   s + (int64_t)d * p.M + u * 32, cg == 0, xe[d][u], g, rs[u]);
       }
     }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Few rows: 16 rows x 32 logits per workgroup.  Every wave takes whole k blocks of its own (block
+// number modulo 8) and makes the A operands in its registers, so there is neither an LDS round
+// trip nor a barrier in the walk over K; the eight partial results meet in LDS at the end.
+// Latency bound: 512 x 256 x 2048 24.9 -> 8.8 us, 512 x 256 x 7168 82 -> 19.5 (32-row workgroups before).
+// ---------------------------------------------------------------------------
+constexpr int kRouterFewRows = 16;
+
+template <int KIND, bool ROUND, bool FP32W>
+__global__ __launch_bounds__(512) void rmsnorm_router_quant_few_rows_kernel(RouterArgs p) {
+  constexpr int NV = FP32W ? 2 : 1;  // operand tiles of 32 columns
+  __shared__ float part[8][512];
+  __shared__ double ssum[32][16];
+  __shared__ float srstd[16];
+  const int lane = tid_x() & 63;
+  const int wave = uniform32(tid_x() >> 6);
+  const int kblocks = p.K / kGroup;
+  int tile, chunk;
+  router_tile(p.M / kRouterFewRows, p.chunks, tile, chunk);
+  const int row0 = tile * kRouterFewRows;
+  const int r = lane & 15, g = lane >> 4;
+  // lane group g of k step s holds 8-column piece 2 s + g % 2 of half g / 2 of the k block
+  const int col0 = (g >> 1) * 64 + (g & 1) * 8;
+  const uint16_t* xl = p.x + (int64_t)(row0 + r) * p.K + col0;
+  const uint16_t* gl = p.gamma + col0;
+  const int vtiles = p.N / 32 * NV;
+  const uint4* wl = p.w + ((int64_t)chunk * NV * 8 + (g & 1)) * 64 + (g >> 1) * 32 + r;
+
+  floatx4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  double ss = 0.0;
+  uint4 xr[2][4], gr[2][4], b[2][NV][4][2];
+  auto fetch = [&](int kb, uint4 (&xd)[4], uint4 (&gd)[4], uint4 (&bd)[NV][4][2]) {
+    const int k = min(kb, kblocks - 1);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      xd[s] = *(const uint4*)(xl + k * kGroup + s * 16);
+      gd[s] = *(const uint4*)(gl + k * kGroup + s * 16);
+    }
+#pragma unroll
+    for (int v = 0; v < NV; ++v)
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) bd[v][s][t] = wl[((int64_t)k * vtiles + v) * 512 + s * 128 + t * 16];
+  };
+  auto multiply = [&](const uint4 (&xd)[4], const uint4 (&gd)[4], const uint4 (&bd)[NV][4][2]) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      ss += (double)sumsq8(xd[s]);
+      uint4 hi, lo;
+      router_split(xd[s], gd[s], hi, lo);
+#pragma unroll
+      for (int v = 0; v < NV; ++v)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(operand(hi), operand(bd[v][s][t]), acc[t], 0, 0, 0);
+          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(operand(lo), operand(bd[v][s][t]), acc[t], 0, 0, 0);
+        }
+    }
+  };
+  fetch(wave, xr[0], gr[0], b[0]);
+#pragma unroll 1
+  for (int kb = wave; kb < kblocks; kb += 16) {
+    fetch(kb + 8, xr[1], gr[1], b[1]);
+    multiply(xr[0], gr[0], b[0]);
+    if (kb + 8 < kblocks) {
+      fetch(kb + 16, xr[0], gr[0], b[0]);
+      multiply(xr[1], gr[1], b[1]);
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < 2; ++t) *(floatx4_t*)&part[wave][t * 256 + lane * 4] = acc[t];
+  ssum[wave * 4 + g][r] = ss;
+  __syncthreads();
+  if (tid_x() < 16) {
+    double total = 0.0;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) total += ssum[i][tid_x()];
+    const float rs = 1.0f / sqrtf((float)total / (float)p.K + p.eps);
+    srstd[tid_x()] = rs;
+    if (chunk == 0) p.rstd[row0 + tid_x()] = rs;
+  }
+  __syncthreads();
+  {
+    // register e of a 16x16 result holds row (lane / 16) * 4 + e, column lane % 16
+    const int col = tid_x() & 31, row = tid_x() >> 5;
+    const int at = (col >> 4) * 256 + ((row >> 2) * 16 + (col & 15)) * 4 + (row & 3);
+    float v = part[0][at];
+#pragma unroll
+    for (int i = 1; i < 8; ++i) v += part[i][at];
+    p.logits[(int64_t)(row0 + row) * p.N + chunk * 32 + col] = v * srstd[row];
+  }
+  const int q0 = chunk * kblocks / p.chunks, q1 = (chunk + 1) * kblocks / p.chunks;
+  const int cg = tid_x() & 15;
+  for (int i = tid_x() >> 4; i < (q1 - q0) * 16; i += 32) {
+    const int row = i & 15, kb = q0 + (i >> 4);
+    const int c = kb * kGroup + cg * 8;
+    const int64_t at = (int64_t)(row0 + row) * p.K + c;
+    router_emit<KIND, ROUND>(p.y + at, p.q + at, p.s + (int64_t)kb * p.M + row0 + row, cg == 0,
+                             *(const uint4*)(p.x + at), *(const uint4*)(p.gamma + c), srstd[row]);
   }
 }
 
@@ -462,25 +488,17 @@ int64_t rmsnorm_router_scratch_bytes(int K, int N, int weight_fp32) {
   return (int64_t)N * K * (weight_fp32 ? 4 : 2);  // the bf16 planes of W in operand order
 }
 
-// W [N, K] (bf16 or fp32) -> the operand order of the main kernels, chunk by chunk of 512 virtual
-// columns.  A router weight changes once per optimiser step, so a caller can pack it once and
-// reuse the result for every forward in between.
+// W [N, K] (bf16 or fp32) -> the operand order of the main kernels.  A router weight changes once
+// per optimiser step, so a caller can pack it once and reuse the result for every forward in between.
 hipError_t launch_pack_router_weight(const void* wr, int weight_fp32, void* wpacked, int K, int N,
                                      hipStream_t stream) {
-  const int vcols = weight_fp32 ? 2 * N : N;  // virtual bf16 columns
-  for (int v0 = 0; v0 < vcols; v0 += 512) {
-    const int vtiles = (vcols - v0 < 512 ? vcols - v0 : 512) / 32;
-    uint4* chunk_w = (uint4*)wpacked + (int64_t)v0 * K / 8;
-    const int64_t pieces = (int64_t)vtiles * 32 * K / 8;
-    const dim3 pgrid((unsigned)((pieces + 255) / 256));
-    if (weight_fp32)
-      hipLaunchKernelGGL(pack_router_weight_kernel<true>, pgrid, dim3(256), 0, stream, wr, chunk_w, K, v0, vtiles);
-    else
-      hipLaunchKernelGGL(pack_router_weight_kernel<false>, pgrid, dim3(256), 0, stream, wr, chunk_w, K, v0, vtiles);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-  }
-  return hipSuccess;
+  const int vtiles = N / 32 * (weight_fp32 ? 2 : 1);
+  const dim3 grid((unsigned)(((int64_t)vtiles * 4 * K + 255) / 256));
+  if (weight_fp32)
+    hipLaunchKernelGGL(pack_router_weight_kernel<true>, grid, dim3(256), 0, stream, wr, (uint4*)wpacked, K, vtiles);
+  else
+    hipLaunchKernelGGL(pack_router_weight_kernel<false>, grid, dim3(256), 0, stream, wr, (uint4*)wpacked, K, vtiles);
+  return hipGetLastError();
 }
 
 // the main kernels on a weight already in operand order
@@ -489,68 +507,43 @@ hipError_t launch_rmsnorm_router_quant_packed(const void* x, const void* gamma, 
                                               float* s, int64_t M, int K, int N, float eps, int round_scale,
                                               int kind, hipStream_t stream) {
   if (M == 0) return hipSuccess;
-  const int vcols = weight_fp32 ? 2 * N : N;  // virtual bf16 columns
-  const dim3 grid((unsigned)(M / kRouterRows));
-#define FQ_ROUTER_ARGS(WAVESV)                                                                                  \
-  grid, dim3(64 * WAVESV), 0, stream, (const uint16_t*)x, (const uint16_t*)gamma, (const uint4*)chunk_w,        \
-      (uint16_t*)y, rstd, lout, (uint8_t*)q, s, M, K, eps
-#define FQ_ROUTER_STREAMED(KINDV, ROUNDV, TPWV, WAVESV)                                                         \
-  if (first)                                                                                                    \
-    hipLaunchKernelGGL((rmsnorm_router_quant_kernel<KINDV, ROUNDV, TPWV, WAVESV, PAIRV, true>),                 \
-                       FQ_ROUTER_ARGS(WAVESV));                                                                 \
-  else                                                                                                          \
-    hipLaunchKernelGGL((rmsnorm_router_quant_kernel<KINDV, ROUNDV, TPWV, WAVESV, PAIRV, false>),                \
-                       FQ_ROUTER_ARGS(WAVESV))
-#define FQ_ROUTER_RESIDENT(KINDV, ROUNDV, TPWV, WAVESV)                                                         \
-  if (single && K == 2048)                                                                                      \
-    hipLaunchKernelGGL((rmsnorm_router_quant_resident_kernel<KINDV, ROUNDV, TPWV, WAVESV, 16, 2, PAIRV>),       \
-                       FQ_ROUTER_ARGS(WAVESV));                                                                 \
-  else if (single && K == 1024)                                                                                 \
-    hipLaunchKernelGGL((rmsnorm_router_quant_resident_kernel<KINDV, ROUNDV, TPWV, WAVESV, 8, 2, PAIRV>),        \
-                       FQ_ROUTER_ARGS(WAVESV));                                                                 \
-  else {                                                                                                        \
-    FQ_ROUTER_STREAMED(KINDV, ROUNDV, TPWV, WAVESV);                                                            \
+  RouterArgs p{(const uint16_t*)x, (const uint16_t*)gamma, (const uint4*)wpacked, (uint16_t*)y, rstd, logits,
+               (uint8_t*)q, s, (int)M, K, N, 0, eps};
+  const int64_t tiles = (M + kRouterRows - 1) / kRouterRows;
+  const int64_t workgroups = tiles * (N / 64);  // of 64 logits
+  const bool few = M < kRouterRows || workgroups <= Policy::kRouterFewRowsMax;
+  const bool narrow = !weight_fp32 && workgroups <= Policy::kRouterNarrowMax;
+  p.chunks = few ? N / 32 : weight_fp32 || narrow ? N / 64 : N / 128;
+  const dim3 grid((unsigned)((few ? M / kRouterFewRows : tiles) * p.chunks));
+#define FQ_ROUTER_GO(KINDV, ROUNDV, FP32V)                                                                           \
+  if (few)                                                                                                           \
+    hipLaunchKernelGGL((rmsnorm_router_quant_few_rows_kernel<KINDV, ROUNDV, FP32V>), grid, dim3(512), 0, stream, p); \
+  else if (!FP32V && narrow)                                                                                         \
+    hipLaunchKernelGGL((rmsnorm_router_quant_kernel<KINDV, ROUNDV, FP32V, FP32V ? 2 : 1>), grid, dim3(512), 0,       \
+                       stream, p);                                                                                   \
+  else                                                                                                               \
+    hipLaunchKernelGGL((rmsnorm_router_quant_kernel<KINDV, ROUNDV, FP32V, 2>), grid, dim3(512), 0, stream, p);
+#define FQ_ROUTER_ROUND(KINDV, FP32V)            \
+  if (round_scale) {                             \
+    FQ_ROUTER_GO(KINDV, true, FP32V)             \
+  } else {                                       \
+    FQ_ROUTER_GO(KINDV, false, FP32V)            \
   }
-#define FQ_ROUTER_KIND(GO, TPWV, WAVESV)                                                                        \
-  if (kind == kE5M2) {                                                                                          \
-    if (round_scale) { GO(kE5M2, true, TPWV, WAVESV); } else { GO(kE5M2, false, TPWV, WAVESV); }                \
-  } else {                                                                                                      \
-    if (round_scale) { GO(kE4M3, true, TPWV, WAVESV); } else { GO(kE4M3, false, TPWV, WAVESV); }                \
+#define FQ_ROUTER_WEIGHT(KINDV)        \
+  if (weight_fp32) {                   \
+    FQ_ROUTER_ROUND(KINDV, true)       \
+  } else {                             \
+    FQ_ROUTER_ROUND(KINDV, false)      \
   }
-  // 8 waves when the column tiles split evenly over them (256, 512 virtual columns), else 4;
-  // rows held in registers when there is one chunk, one column tile per wave (128 or 256
-  // virtual columns) and K is one of the instantiated widths (1024, 2048); streamed twice
-  // otherwise
-#define FQ_ROUTER_TILES()                                                   \
-  switch (vtiles) {                                                         \
-    case 4: FQ_ROUTER_KIND(FQ_ROUTER_RESIDENT, 1, 4) break;                 \
-    case 8: FQ_ROUTER_KIND(FQ_ROUTER_RESIDENT, 1, 8) break;                 \
-    case 12: FQ_ROUTER_KIND(FQ_ROUTER_STREAMED, 3, 4) break;                \
-    case 16: FQ_ROUTER_KIND(FQ_ROUTER_STREAMED, 2, 8) break;                \
-    default: return hipErrorInvalidValue;                                   \
+  if (kind == kE5M2) {
+    FQ_ROUTER_WEIGHT(kE5M2)
+  } else {
+    FQ_ROUTER_WEIGHT(kE4M3)
   }
-  const bool single = vcols <= 512;
-  for (int v0 = 0; v0 < vcols; v0 += 512) {
-    const int vtiles = (vcols - v0 < 512 ? vcols - v0 : 512) / 32;
-    const bool first = v0 == 0;
-    const uint4* chunk_w = (const uint4*)wpacked + (int64_t)v0 * K / 8;
-    const LogitsOut lout{logits, N, weight_fp32 ? v0 / 2 : v0};
-    if (weight_fp32) {
-      constexpr bool PAIRV = true;
-      FQ_ROUTER_TILES()
-    } else {
-      constexpr bool PAIRV = false;
-      FQ_ROUTER_TILES()
-    }
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-  }
-#undef FQ_ROUTER_TILES
-#undef FQ_ROUTER_KIND
-#undef FQ_ROUTER_RESIDENT
-#undef FQ_ROUTER_STREAMED
-#undef FQ_ROUTER_ARGS
-  return hipSuccess;
+#undef FQ_ROUTER_WEIGHT
+#undef FQ_ROUTER_ROUND
+#undef FQ_ROUTER_GO
+  return hipGetLastError();
 }
 
 hipError_t launch_rmsnorm_router_quant(const void* x, const void* gamma, const void* wr, int weight_fp32,

@@ -529,3 +529,43 @@ def test_rms_norm_fp32_gemm_block_quant(gpu, M, N, K, wdtype, round_scale):
     torch.cuda.synchronize()
     assert rms1 is rms
     check_quant_pair("router.col", pin[5], pin[6], qt, st, **EXACT)
+
+
+@pytest.mark.parametrize("M,N,K,wdtype", [
+    # 16-row workgroups: the fewest rows, one k block, the most workgroups of 64 x 64 that still take them (80)
+    (32, 128, 128, torch.bfloat16), (2560, 128, 384, torch.bfloat16), (1280, 256, 1152, torch.float32),
+    # 64 x 64: one more than that, the most that take it (256), a last row tile that is half a tile
+    (2624, 128, 640, torch.bfloat16), (8192, 128, 256, torch.bfloat16), (1312, 256, 128, torch.bfloat16),
+    # 64 x 128 and the fp32 form: k blocks of every remainder modulo the ring of four, half a row tile
+    (8224, 128, 128, torch.bfloat16), (8224, 128, 384, torch.bfloat16), (8256, 128, 640, torch.bfloat16),
+    (2144, 256, 256, torch.float32), (1312, 256, 1920, torch.float32), (2048, 384, 896, torch.float32)])
+def test_router_kernel_choice(gpu, M, N, K, wdtype):
+    """Every form of the router kernel at the edges of its range, rows in the 32s that the C interface takes."""
+    from linghe_amd import _lib
+
+    announce("router kernel choice", M, N, K, wdtype)
+    g = gen(25)
+    x = (torch.randn(M, K, generator=g) ** 2).to(torch.bfloat16)
+    nw = torch.randn(K, generator=g).to(torch.bfloat16)
+    rw = torch.randn(N, K, generator=g).to(wdtype)
+    xd, nwd, rwd = _dev(x, gpu), _dev(nw, gpu), _dev(rw, gpu)
+    fp32 = int(wdtype == torch.float32)
+    scratch = torch.empty(int(_lib.lib.fq_rmsnorm_router_scratch_bytes(K, N, fp32)), dtype=torch.uint8, device=gpu)
+    y = torch.full((M, K), 7.0, dtype=torch.bfloat16, device=gpu)
+    rms = torch.full((M,), 7.0, device=gpu)
+    logits = torch.full((M, N), 7.0, device=gpu)
+    q = torch.zeros((M, K), dtype=torch.float8_e4m3fn, device=gpu)
+    s = torch.full((K // 128, M), 7.0, device=gpu)
+    p = _lib.ptr
+    _lib.check(_lib.lib.fq_rmsnorm_router_quant_fwd(p(xd), p(nwd), p(rwd), fp32, p(scratch), p(y), p(rms), p(logits),
+                                                    p(q), p(s), M, K, N, 1e-6, 0, _lib.FQ_E4M3, _lib.stream_of(xd)))
+    torch.cuda.synchronize()
+    pin = O.rms_gemm_block_quant_forward(x, nw, rw, rstd=rms.cpu())
+    want = 1.0 / torch.sqrt((x.double() ** 2).mean(1) + 1e-6)
+    assert float((rms.cpu().double() / want - 1).abs().max()) < 4 * 2.0 ** -23
+    assert torch.equal(pin[0].view(torch.int16), y.cpu().view(torch.int16))
+    check_quant_pair("router.row", pin[3], pin[4], q, s, **EXACT)
+    # x * gamma enters exactly, an fp32 weight to 2^-17 of each |w|; fp32 accumulation below 2^-16 of sum |y||w|
+    y32 = (x.float() * rms.cpu()[:, None]) * nw.float()
+    err = (logits.cpu().double() - y32.double() @ rw.double().t()).abs()
+    assert bool((err <= 2.0 ** -16 * (y32.abs().double() @ rw.double().abs().t())).all())
