@@ -31,6 +31,12 @@ hipError_t launch_silu_quant_fwd(const void* x, const void* weight, int weight_b
                                  const void* counts, int counts_i64, int n_experts, int64_t row_blocks,
                                  hipStream_t stream, const void* plan = nullptr, const PlanShape* ps = nullptr);
 
+// SwiGLU + row-wise quant of a whole matrix in 16-row workgroups: rows per 16 lanes for a call of this
+// size, 0 where the tile kernel (launch_silu_quant_fwd, mode 0) is the faster one
+int silu_quant_rows_per_team(int64_t M, int n);
+hipError_t launch_silu_quant_rows(const void* x, void* q, float* s, int64_t M, int n, int round_scale, int kind,
+                                  hipStream_t stream);
+
 hipError_t launch_silu_quant_bwd(const void* g, const void* x, const void* weight, int weight_bf16, void* q,
                                  float* s, void* qt, float* st, float* dw_part, void* dw, int64_t M, int n,
                                  int round_scale, int kind, const void* counts, int counts_i64, int n_experts,

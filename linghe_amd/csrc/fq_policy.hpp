@@ -120,6 +120,12 @@ struct Policy {
   // 10.3 / 10.5 / 13.0 us with 1 / 2 / 4 at 8192 x 2048, where a thread has two groups in all
   static constexpr int kGroupQuantUnroll = 1;
 
+  // SwiGLU + row-wise quant, dense: up to so many 1 x 128 groups per row that 16 lanes take, the rows kernel with
+  // one row, then with two.  32768 groups are 2048 workgroups of 256 threads: what 256 CUs hold at once.  Past two
+  // rows the tile kernel is ahead: 4096 x 4096 (131072 groups) 16.29 us, rows kernel 17.3 / 16.5 / 17.0 with 1 / 2 / 4.
+  static constexpr int kSiluRowsGroupsPerRow = 32768;
+  static constexpr int kSiluRowsPerTeamMax = 2;
+
   // ---- the SwiGLU backwards widen row s of their packed inputs after row s-1 is done (fence_values):
   // without it the per-expert form needed 136 registers under its cap of 128 and spilled; with it (and no
   // branch around the arithmetic) 105, the single-matrix form 100

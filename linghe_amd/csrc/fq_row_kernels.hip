@@ -972,4 +972,73 @@ hipError_t launch_block_quant(const void* x, void* q, float* s, int64_t M, int N
   return hipGetLastError();
 }
 
+// ---------------------------------------------------------------------------
+// SwiGLU + row-wise 1x128 quant of a whole matrix (output_mode 0 of the dense form,
+// linghe/utils/silu.py:213-335) for calls of few rows: 16 lanes per row and 128-column group,
+// kR rows each, 16 * kR rows per workgroup, no shared memory and no barrier.  Such calls are
+// bound by latency: the tile kernel, which takes 128 rows per workgroup, runs 12 workgroups at
+// 32 x 1536 (three quarters of their waves without rows) and 288 at 3001 x 1536.  us tile kernel /
+// one row / two rows: 32 x 1536 3.84 / 2.10 / 2.40, 128 x 2048 4.69 / 2.61 / 2.83, 1000 x 4096
+// 6.31 / 5.67 / 5.95, 3001 x 1536 7.98 / 6.98 / 6.44, 4096 x 2048 9.47 / 10.28 / 9.01.
+// ---------------------------------------------------------------------------
+template <int KIND, bool ROUND, int kR>
+__global__ __launch_bounds__(256) void silu_quant_rows_kernel(const uint16_t* __restrict__ x, uint8_t* __restrict__ q,
+                                                              float* __restrict__ s, int64_t M, int n) {
+  const int ncb = n / kGroup;
+  const int rb = wg_x() / ncb, cb = wg_x() - rb * ncb;
+  const int cg = tid_x() & 15;
+  const int64_t row0 = (int64_t)rb * (16 * kR) + (tid_x() >> 4) * kR;
+  const int64_t col = (int64_t)cb * kGroup + cg * 8;
+  // No condition on loads or stores of codes: a row beyond the end repeats the last row (the same
+  // result stored to the same place again).
+  int64_t row[kR];
+  uint4 r1[kR], r2[kR];
+#pragma unroll
+  for (int k = 0; k < kR; ++k) {
+    row[k] = row0 + k < M ? row0 + k : M - 1;
+    r1[k] = ld16(x + row[k] * 2 * n + col);
+    r2[k] = ld16(x + row[k] * 2 * n + n + col);
+  }
+#pragma unroll
+  for (int k = 0; k < kR; ++k) {
+    float a[8], b[8], y[8];
+    unpack8(r1[k], a);
+    unpack8(r2[k], b);
+    float m = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      y[j] = (sigmoid_f32(a[j]) * a[j]) * b[j];
+      m = fmaxf(m, fabsf(y[j]));
+    }
+    m = row16_max(m);
+    const float sc = make_scale<KIND, ROUND>(m);
+    st8(q + row[k] * n + col, quantize8<KIND, ROUND>(y, make_quantum<ROUND>(sc)));
+    if (cg == k) s[(int64_t)cb * M + row[k]] = sc;
+  }
+}
+
+int silu_quant_rows_per_team(int64_t M, int n) {
+  const int64_t groups = M * (n / kGroup);  // 1 x 128 groups of the result
+  for (int rows = 1; rows <= Policy::kSiluRowsPerTeamMax; ++rows)
+    if (groups <= (int64_t)rows * Policy::kSiluRowsGroupsPerRow) return rows;
+  return 0;
+}
+
+hipError_t launch_silu_quant_rows(const void* x, void* q, float* s, int64_t M, int n, int round_scale, int kind,
+                                  hipStream_t stream) {
+  const int rows = silu_quant_rows_per_team(M, n);
+  if (rows == 0) return hipErrorInvalidValue;
+  const int64_t wgs = (M + 16 * rows - 1) / (16 * rows) * (n / kGroup);
+  const dim3 grid((unsigned)wgs), block(256);
+#define FQ_SR(KINDV, ROUNDV)                                                                              \
+  if (rows == 1) hipLaunchKernelGGL((silu_quant_rows_kernel<KINDV, ROUNDV, 1>), grid, block, 0, stream,   \
+                                    (const uint16_t*)x, (uint8_t*)q, s, M, n);                            \
+  else hipLaunchKernelGGL((silu_quant_rows_kernel<KINDV, ROUNDV, 2>), grid, block, 0, stream,             \
+                          (const uint16_t*)x, (uint8_t*)q, s, M, n)
+  if (kind == kE5M2) { if (round_scale) { FQ_SR(kE5M2, true); } else { FQ_SR(kE5M2, false); } }
+  else { if (round_scale) { FQ_SR(kE4M3, true); } else { FQ_SR(kE4M3, false); } }
+#undef FQ_SR
+  return hipGetLastError();
+}
+
 }  // namespace fq

@@ -301,6 +301,25 @@ def test_silu_and_block_quant_fwd(gpu, M, N, coef):
             check_quant_pair(f"silu.{mode}.col", ref[2], ref[3], qt, st, **FUSED)
 
 
+# one row, workgroups of 16 rows and one more or less; the most groups that one row (32768) and two rows (65536)
+# per 16 lanes take, and one row more; last workgroups with one row and with all but one
+@pytest.mark.parametrize("M,n", [(1, 128), (15, 384), (17, 2048), (2048, 2048), (2049, 2048), (4096, 2048),
+                                 (4097, 2048), (2079, 2048)])
+@pytest.mark.parametrize("dtype,round_scale", [(E4M3, False), (E5M2, True)])
+def test_silu_rows_only(gpu, M, n, dtype, round_scale):
+    """Row-wise output alone: the same codes and scales as in the call that writes both layouts."""
+    from linghe_amd.utils.silu import triton_silu_and_block_quant_forward as fwd
+
+    announce("silu rows only", M, n, dtype, round_scale)
+    x = randn_bf16(gen(32), M, 2 * n, scale=3.0)
+    x[:, :128] *= 0.0  # a group of zeros in every row
+    xd = _dev(x, gpu)
+    q, s, _, _ = fwd(xd, round_scale=round_scale, output_mode=0, fp8_dtype=dtype)
+    q2, s2, _, _ = fwd(xd, round_scale=round_scale, output_mode=2, fp8_dtype=dtype)
+    assert torch.equal(s, s2)
+    assert torch.equal(q.view(torch.uint8), q2.view(torch.uint8))
+
+
 @pytest.mark.parametrize("M,N,coef,gcoef", [(2048, 1024, 1.0, 1.0), (1024, 4096, 1.0, 1e-3),
                                             (512, 1536 * 8, 100.0, 100.0), (512, 1536 * 8, 0.0, 0.0)])
 @pytest.mark.parametrize("dtype", [E4M3, E5M2])
