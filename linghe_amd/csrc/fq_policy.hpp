@@ -98,11 +98,15 @@ struct Policy {
   static constexpr bool kStartPriorityRmsnorm = true;
   // RMSNorm + quant in two passes, both passes giving XCD X (workgroup number mod 8) the X-th eighth of the rows,
   // the statistic pass walking its eighth from the end and the tile kernel from the start: what the tile kernel
-  // reads first is what the same XCD's L2 read last.  Rows a multiple of 1024 (the eighths are whole row blocks).
+  // reads first is what the same XCD's L2 read last.  Rows a multiple of 128; where
+  // an eighth is not a whole number of row blocks the two passes' eighths differ by less than one.
   // us without / with: 2048 x 2048 8.8 / 7.9, 4096 x 2048 11.7 / 10.6, 8192 x 2048 17.9 / 16.6, 3072 x 4096
   // 14.6 / 13.3, 4096 x 7168 30.2 / 27.9, 8192 x 4096 33.0 / 32.0, 16384 x 2048 33.2 / 31.7, 8192 x 7168
   // 55.8 / 52.9, 16384 x 4096 63.4 / 62.7, 32768 x 2048 63.6 / 63.3, 16384 x 7168 108.1 / 109.6: up to this
-  // many bytes of input
+  // many bytes of input.  Eighths of broken row blocks: 640 x 4096 8.3 / 8.0, 1152 x 2048 8.0 / 7.6, 2176 x 5120
+  // 15.0 / 14.1, 4224 x 5120 24.2 / 22.7, 8064 x 2048 17.9 / 16.7, 4992 x 7168 35.8 / 34.0, 10112 x 7168 68.6 / 65.2.
+  // With rows that are no multiple of 128 the transposed rows share lines between row blocks and the grid order
+  // is better: 1000 x 2048 8.1 / 8.5, 4104 x 5120 26.9 / 28.8, 6001 x 4096 30.4 / 32.6, 5000 x 7168 42.4 / 45.7
   static constexpr long long kRmsnormByXcdMaxBytes = 160ll << 20;
   // 16-byte chunks per lane, matrix and step in the bf16 SwiGLU backward (three matrices are read):
   // 29.0 / 30.4 / 28.7 / 35.5 us with 2 / 3 / 4 / 8 at 8192 x 4096

@@ -261,8 +261,8 @@ __global__ __launch_bounds__(64 * Policy::kRowstatWaves) void rowstat_kernel(con
   // cache roughly half of the second read never reaches HBM.
   // by_xcd: workgroup w runs on XCD w % 8, and XCD X takes the X-th eighth of the rows, again from its
   // end backwards: the tile kernel hands the same eighth to the same XCD (rmsnorm_passes_by_xcd)
-  const int64_t span = by_xcd ? M >> 3 : M;
-  const int64_t first = by_xcd ? (int64_t)(wg_x() & 7) * span : 0;
+  const int64_t first = by_xcd ? ((int64_t)(wg_x() & 7) * M) >> 3 : 0;
+  const int64_t span = by_xcd ? (((int64_t)(wg_x() & 7) * M + M) >> 3) - first : M;
   const int64_t k0 = by_xcd ? (int64_t)(wg_x() >> 3) * kW + (tid_x() >> 6) : (int64_t)wg_x() * kW + (tid_x() >> 6);
   const int64_t step = by_xcd ? (int64_t)(n_wg_x() >> 3) * kW : (int64_t)n_wg_x() * kW;
   for (int64_t k = k0; k < span; k += step) {
@@ -622,8 +622,10 @@ hipError_t launch_rmsnorm_fwd(const void* x, const void* gamma, void* out, float
                                    scale, rstd, M, n, eps, rows_per_wg);)
   // quant: 0 = bf16 output, 1 = fp8 codes + scales, 2 = statistic only (its own kernel)
   if (quant == 2) {
-    const dim3 sgrid((unsigned)((wgs + Policy::kRowstatWaves - 1) / Policy::kRowstatWaves)), sblock(64 * Policy::kRowstatWaves);
-    const int by_xcd = rmsnorm_passes_by_xcd(M, n) && sgrid.x % 8 == 0;
+    const int by_xcd = rmsnorm_passes_by_xcd(M, n);
+    unsigned swgs = (unsigned)((wgs + Policy::kRowstatWaves - 1) / Policy::kRowstatWaves);
+    if (by_xcd) swgs = (swgs + 7) & ~7u;  // as many workgroups on every XCD
+    const dim3 sgrid(swgs), sblock(64 * Policy::kRowstatWaves);
     if (n <= 2048) hipLaunchKernelGGL(rowstat_kernel<4>, sgrid, sblock, 0, stream, (const uint16_t*)x, rstd, M, n, eps, by_xcd);
     else hipLaunchKernelGGL(rowstat_kernel<8>, sgrid, sblock, 0, stream, (const uint16_t*)x, rstd, M, n, eps, by_xcd);
   } else if (!quant) {
@@ -657,7 +659,7 @@ hipError_t launch_rmsnorm_fwd(const void* x, const void* gamma, void* out, float
 }
 
 bool rmsnorm_passes_by_xcd(int64_t M, int n) {
-  return M % 1024 == 0 && M * n * 2 <= (int64_t)Policy::kRmsnormByXcdMaxBytes;
+  return M % kGroup == 0 && M * n * 2 <= (int64_t)Policy::kRmsnormByXcdMaxBytes;
 }
 
 int64_t rmsnorm_bwd_partials(int64_t M) {

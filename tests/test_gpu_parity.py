@@ -282,6 +282,23 @@ def test_rmsnorm_and_block_quant(gpu, M, N, round_scale):
 
 
 # ------------------------------------------------------------------ SwiGLU
+# whole row blocks that eight XCDs share unevenly: fewer than eight, one more than eight, rows beyond one per wave
+@pytest.mark.parametrize("M,N", [(128, 256), (384, 2048), (1152, 2176), (8320, 128), (16768, 256)])
+def test_rmsnorm_passes_by_xcd(gpu, M, N):
+    """Statistic pass and tile kernel over uneven eighths of the rows: every row is written, the statistic equals the
+    row-wise form's bit for bit and the codes are the oracle's for it."""
+    from linghe_amd.utils.norm import triton_rms_norm_and_block_quant_forward as fn
+
+    announce("rmsnorm passes by xcd", M, N)
+    x, w = randn_bf16(gen(33), M, N), gamma_bf16(gen(34), N)
+    xd, wd = _dev(x, gpu), _dev(w, gpu)
+    q, s, rms, qt, st = fn(xd, wd)
+    assert torch.equal(rms, fn(xd, wd, output_mode=0)[2])
+    ref = O.rms_norm_and_block_quant_forward(x, w, rstd=rms.cpu())
+    check_quant_pair("rms.xcd.row", ref[0], ref[1], q, s, **EXACT)
+    check_quant_pair("rms.xcd.col", ref[3], ref[4], qt, st, **EXACT)
+
+
 @pytest.mark.parametrize("M,N,coef", [(2048, 1024, 1.0), (1024, 4096, 1.0), (1000, 1536, 1.0),
                                       (512, 1536 * 8, 100.0), (512, 1536 * 8, 0.0)])
 def test_silu_and_block_quant_fwd(gpu, M, N, coef):
