@@ -114,8 +114,12 @@ struct Policy {
   // the wide-row (four waves per row) RMSNorm + row-wise quant kernel loads the next row while it works on
   // the current one (122 instead of 84 registers): 68.5 -> 65.5 us at 16384 x 7168
   static constexpr bool kPrefetchRowQuantWide = true;
-  // workgroups per CU of that kernel's launch (it holds four at 122 registers): 64.0 / 65.4 / 64.8 / 64.6 /
-  // 68.0 us with 4 / 5 / 6 / 8 / 12 at 16384 x 7168
+  // Workgroups of that kernel's launch.  Up to 16 rows per CU every row has its own: the hardware hands them out as
+  // others finish, while four looping workgroups per CU leave most of the chip idle in the last round of few
+  // (us 4 / 16 per CU: 1500 x 3072 7.5 / 5.9, 3001 x 4096 11.1 / 9.9, 4000 x 2560 11.3 / 10.4, 4104 x 5120 16.3 / 16.3).
+  // Beyond, 16 looping ones per CU, as they fit (8192 x 4096 22.5 / 21.7, 12000 x 5120 40.0 / 39.0); at n > 6144, where
+  // a CU holds four, exactly those (16384 x 7168: 64.0 / 65.4 / 64.8 / 64.6 / 68.0 with 4 / 5 / 6 / 8 / 12).
+  static constexpr int kRowQuantWideRowPerWg = 16;
   static constexpr int kRowQuantWideWgsPerCu = 4;
   // the same in the wide-row RMSNorm backward with one chunk per thread (2048 < n <= 4096: 70.4 -> 66.9 us at
   // 16384 x 3072, 78.5 -> 76.4 at 16384 x 4096); with two chunks the second register set spills

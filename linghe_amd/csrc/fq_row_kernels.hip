@@ -632,10 +632,11 @@ hipError_t launch_rmsnorm_fwd(const void* x, const void* gamma, void* out, float
     if (reuse_rstd) { FQ_LAUNCH_FWD(true, 0, kE4M3, false) } else { FQ_LAUNCH_FWD(false, 0, kE4M3, false) }
   } else if (n > 2048) {
     // wide rows, quantising form: four waves per row (a wave per row needs up to ~230 registers)
-    int64_t wg4 = M;
-    if (wg4 > 256 * Policy::kRowQuantWideWgsPerCu) wg4 = 256 * Policy::kRowQuantWideWgsPerCu;
-    const dim3 grid4((unsigned)wg4);
     const int nc4 = (n / 8 + 255) / 256;
+    const int64_t one_row = 256 * Policy::kRowQuantWideRowPerWg;
+    int64_t wg4 = M;
+    if (M > one_row) wg4 = nc4 == 4 ? 256 * Policy::kRowQuantWideWgsPerCu : one_row;
+    const dim3 grid4((unsigned)wg4);
 #define FQ_LAUNCH_FWD4(NC, KINDV, ROUNDV)                                                                      \
   hipLaunchKernelGGL((rmsnorm_fwd_kernel<256, NC, false, 1, KINDV, ROUNDV>), grid4, dim3(256), 0, stream,       \
                      (const uint16_t*)x, (const uint16_t*)gamma, out, scale, rstd, M, n, eps, rows_per_wg)
