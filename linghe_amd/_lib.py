@@ -82,6 +82,12 @@ def _load() -> ctypes.CDLL:
 
 lib = _load()
 
+try:  # outputs and launch of the row-wise quantisers in one native call (csrc/fq_torch.cpp)
+    from . import _fq_torch as native
+except ImportError as e:
+    raise ImportError("linghe_amd/_fq_torch.so is missing or was built for another torch: build it with "
+                      "`python -m linghe_amd.build`. There is no fallback path.") from e
+
 
 def check(rc: int) -> None:
     if rc != 0:

@@ -3,7 +3,8 @@
     python -m linghe_amd.build
 
 hipcc cross-compiles for gfx950 without a GPU.  The translation units are
-compiled in parallel and linked into ``linghe_amd/libfq_gfx950.so``.
+compiled in parallel and linked into ``linghe_amd/libfq_gfx950.so``; the host-side
+module ``linghe_amd/_fq_torch.so`` (csrc/fq_torch.cpp) is built behind it.
 """
 from __future__ import annotations
 
@@ -17,6 +18,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB_NAME = "libfq_gfx950.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
+HOST_PATH = os.path.join(HERE, "_fq_torch.so")
 SOURCES = ["fq_api.hip", "fq_tile_kernels.hip", "fq_row_kernels.hip", "fq_router.hip", "fq_stream.hip"]
 
 HIPCC_FLAGS = [
@@ -71,6 +73,24 @@ def build_library(extra_flags=(), verbose: bool = False, csrc: str = CSRC, out: 
         list(pool.map(compile_one, zip(SOURCES, objs)))
     tmp = out + ".tmp"
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", tmp])
+    os.replace(tmp, out)
+    if out == LIB_PATH:
+        build_host_module()
+    return out
+
+
+def build_host_module(out: str = HOST_PATH) -> str:
+    """Compile the host-side module (host code only: g++) against the installed torch and link it to
+    libfq_gfx950.so beside it."""
+    import sysconfig
+
+    from torch.utils import cpp_extension
+
+    includes = [*cpp_extension.include_paths(), sysconfig.get_path("include")]
+    tmp = out + ".tmp"
+    _run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", *("-I" + i for i in includes),
+          os.path.join(CSRC, "fq_torch.cpp"), "-o", tmp, *("-L" + d for d in cpp_extension.library_paths()),
+          "-ltorch_python", "-ltorch_cpu", "-lc10", "-L" + HERE, "-l:" + LIB_NAME, "-Wl,-rpath,$ORIGIN"])
     os.replace(tmp, out)
     return out
 

@@ -126,32 +126,15 @@ def triton_rms_norm_and_block_quant_forward(
     device = x.device
     kind = _lib.fp8_kind(fp8_dtype)
 
-    if out is None and output_mode in (0, 2):
-        out = torch.empty((M, n), device=device, dtype=fp8_dtype)
-    if scale is None and output_mode in (0, 2):
-        scale = torch.empty((n // 128, M), device=device, dtype=torch.float32)
-    # the transposed buffers are always allocated, as in the reference
-    transpose_output = torch.empty((n, M), device=device, dtype=fp8_dtype)
-    transpose_scale = torch.empty(((M + 127) // 128, n), device=device, dtype=torch.float32)
-
+    # a given rms is an input in mode 1; in mode 2 it is ignored and recomputed, as in the reference
     if output_mode == 0:
         assert rms is None
-        rms = torch.empty((M,), dtype=torch.float32, device=device)
     elif output_mode == 1:
         assert rms is not None
-    else:
-        # a given rms is ignored and recomputed, as in the reference
-        rms = torch.empty((M,), dtype=torch.float32, device=device)
-
-    if M > 0:
-        with _lib.on_device(device):
-            _lib.check(_lib.lib.fq_rmsnorm_quant_fwd(
-                _lib.ptr(x), _lib.ptr(weight),
-                _lib.ptr(out) if output_mode != 1 else None,
-                _lib.ptr(scale) if output_mode != 1 else None,
-                _lib.ptr(rms), _lib.ptr(transpose_output), _lib.ptr(transpose_scale),
-                M, n, float(eps), int(bool(round_scale)), output_mode, kind, _lib.stream_of(x)))
-    return out, scale, rms, transpose_output, transpose_scale
+    # the transposed buffers are always allocated, as in the reference
+    with _lib.on_device(device):
+        return _lib.native.rmsnorm_quant(x, weight, out, scale, rms if output_mode == 1 else None, float(eps),
+                                         int(bool(round_scale)), output_mode, fp8_dtype, kind, _lib.stream_of(x))
 
 
 def pack_route_weight(route_weight: torch.Tensor) -> torch.Tensor:

@@ -162,19 +162,9 @@ def triton_silu_and_block_quant_forward(
     assert output_mode in (0, 1, 2)
     assert n % 128 == 0 and N == 2 * n
     device = x.device
-    if out is None:
-        out = torch.empty((M, n), device=device, dtype=fp8_dtype)
-    if scale is None:
-        scale = torch.empty((n // 128, M), device=device, dtype=torch.float32)
-    transpose_output = torch.empty((n, M), device=device, dtype=fp8_dtype)
-    transpose_scale = torch.empty(((M + 127) // 128, n), device=device, dtype=torch.float32)
-    if M > 0:
-        with _lib.on_device(device):
-            _lib.check(_lib.lib.fq_swiglu_quant_fwd(
-                _lib.ptr(x), _lib.ptr(out), _lib.ptr(scale), _lib.ptr(transpose_output),
-                _lib.ptr(transpose_scale), M, n, int(bool(round_scale)), output_mode,
-                _lib.fp8_kind(fp8_dtype), _lib.stream_of(x)))
-    return out, scale, transpose_output, transpose_scale
+    with _lib.on_device(device):
+        return _lib.native.swiglu_quant(x, out, scale, int(bool(round_scale)), output_mode, fp8_dtype,
+                                        _lib.fp8_kind(fp8_dtype) if M else 0, _lib.stream_of(x))
 
 
 def triton_silu_and_block_quant_backward(g, x, round_scale=False, *, fp8_dtype=torch.float8_e4m3fn):

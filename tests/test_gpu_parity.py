@@ -318,6 +318,38 @@ def test_silu_and_block_quant_fwd(gpu, M, N, coef):
             check_quant_pair(f"silu.{mode}.col", ref[2], ref[3], qt, st, **FUSED)
 
 
+def test_row_quantisers_given_outputs_and_no_rows(gpu):
+    """Buffers that a caller passes come back as the same objects, filled; calls without rows return empty outputs of
+    the documented shapes; what the wrappers refuse is still refused."""
+    from linghe_amd.quant.group import triton_group_quant as group
+    from linghe_amd.utils.norm import triton_rms_norm_and_block_quant_forward as norm
+    from linghe_amd.utils.silu import triton_silu_and_block_quant_forward as silu
+
+    x, w = _dev(randn_bf16(gen(35), 40, 256), gpu), _dev(gamma_bf16(gen(36), 256), gpu)
+    for fn, args, n in ((norm, (x, w), 256), (silu, (x,), 128)):
+        out = torch.zeros((40, n), dtype=E4M3, device=gpu)
+        scale = torch.zeros((n // 128, 40), device=gpu)
+        got = fn(*args, out=out, scale=scale, output_mode=0)
+        want = fn(*args, output_mode=0)
+        assert got[0] is out and got[1] is scale
+        assert torch.equal(out.view(torch.uint8), want[0].view(torch.uint8)) and torch.equal(scale, want[1])
+    q, s, rms, qt, st = norm(x, w, rms=want_rms(x), output_mode=1)
+    assert q is None and s is None and qt.shape == (256, 40) and st.shape == (1, 256)
+    none = x[:0]
+    assert [tuple(t.shape) for t in norm(none, w)] == [(0, 256), (2, 0), (0,), (256, 0), (0, 256)]
+    assert [tuple(t.shape) for t in silu(none)] == [(0, 128), (1, 0), (128, 0), (0, 128)]
+    assert [tuple(t.shape) for t in group(none)] == [(0, 256), (0, 2)]
+    for call in (lambda: group(x.float()), lambda: silu(x.float()), lambda: norm(x, w.float())):
+        with pytest.raises(TypeError):
+            call()
+    with pytest.raises(RuntimeError):
+        norm(x[:, :128].contiguous(), w.view(torch.uint8)[2:258].view(torch.bfloat16))  # 2-byte-aligned weight
+
+
+def want_rms(x):
+    return 1.0 / torch.sqrt((x.float() ** 2).mean(1) + 1e-6)
+
+
 # one row, workgroups of 16 rows and one more or less; the most groups that one row (32768) and two rows (65536)
 # per 16 lanes take, and one row more; last workgroups with one row and with all but one
 @pytest.mark.parametrize("M,n", [(1, 128), (15, 384), (17, 2048), (2048, 2048), (2049, 2048), (4096, 2048),
