@@ -514,16 +514,19 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_wave_kernel(const uint16_t* _
   }
 }
 
-// dgamma[c] = sum_p part[p, c] in a fixed order: 16 strided slices of p, each
-// summed sequentially (loads issued eight ahead), then combined 0..15.
-// 64 columns per workgroup of 1024 threads.
-constexpr int kColsumSlices = 16;
+// dgamma[c] = sum_p part[p, c] in a fixed order: 32 strided slices of p, each
+// summed sequentially (loads issued eight ahead), then combined 0..31.
+// 32 columns per workgroup of 1024 threads: bound by the trips to memory of a slice, two at 512
+// partial rows; with 64 columns and 16 slices four, on half the CUs.  us of the whole backward,
+// 64 / 32 / 16 columns: 1000 x 2048 10.8 / 10.0 / 9.7, 4096 x 1024 10.9 / 10.4 / 10.8, 8192 x 2048
+// 23.3 / 22.8 / 23.6, 8192 x 5120 49.0 / 48.6 / 51.5, 16384 x 7168 119.6 / 119.7 / 122.5.
+constexpr int kColsumCols = 32, kColsumSlices = 1024 / kColsumCols;
 __global__ __launch_bounds__(1024) void colsum_kernel(const float* __restrict__ part, float* __restrict__ out,
                                                       int P, int n) {
-  __shared__ float red[kColsumSlices][64];
-  const int lane = tid_x() & 63;
-  const int col = wg_x() * 64 + lane;
-  const int slice = tid_x() >> 6;
+  __shared__ float red[kColsumSlices][kColsumCols];
+  const int lane = tid_x() & (kColsumCols - 1);
+  const int col = wg_x() * kColsumCols + lane;
+  const int slice = tid_x() / kColsumCols;
   float acc = 0.f;
   if (col < n) {
     const float* src = part + col;
@@ -545,6 +548,12 @@ __global__ __launch_bounds__(1024) void colsum_kernel(const float* __restrict__ 
     for (int k = 1; k < kColsumSlices; ++k) tot += red[k][lane];
     out[col] = tot;
   }
+}
+
+static hipError_t launch_colsum(const float* part, float* out, int P, int n, hipStream_t stream) {
+  hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)((n + kColsumCols - 1) / kColsumCols)), dim3(1024), 0, stream, part,
+                     out, P, n);
+  return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
@@ -676,8 +685,7 @@ hipError_t launch_rmsnorm_bwd(const void* dy, const void* x, const void* gamma, 
                               float* dgamma, float* dg_part, int64_t n_partials, int64_t M, int n, float eps,
                               hipStream_t stream) {
   if (M == 0) {  // no rows: dgamma = 0, and no kernel touches dy, x, gamma or dx
-    hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)((n + 63) / 64)), dim3(1024), 0, stream, dg_part, dgamma, 0, n);
-    return hipGetLastError();
+    return launch_colsum(dg_part, dgamma, 0, n, stream);
   }
   const int64_t P = n_partials;
   const int rows_per_wg = (int)((M + P - 1) / P);
@@ -707,9 +715,7 @@ hipError_t launch_rmsnorm_bwd(const void* dy, const void* x, const void* gamma, 
 #undef FQ_LAUNCH_BWD_BLOCK
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return err;
-  hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)((n + 63) / 64)), dim3(1024), 0, stream, dg_part, dgamma, (int)P,
-                     n);
-  return hipGetLastError();
+  return launch_colsum(dg_part, dgamma, (int)P, n, stream);
 }
 
 // ---------------------------------------------------------------------------
