@@ -136,7 +136,7 @@ __device__ __forceinline__ double sumsq_live(const uint4 (&raw)[NCHUNK], int n) 
 #pragma unroll
   for (int k = 0; k < NCHUNK; ++k) {
     const float part = sumsq8(raw[k]);
-    ss += (double)((((int)tid_x() & (T - 1)) + k * T) * 8 < n ? part : 0.f);  // T a power of two; a wave-per-row kernel passes T = 64
+    ss += (double)(((T == 64 ? (int)tid_x() & 63 : (int)tid_x()) + k * T) * 8 < n ? part : 0.f);  // T: threads of the workgroup, or 64 in a wave-per-row kernel
   }
   return ss;
 }
@@ -206,7 +206,7 @@ __global__ __launch_bounds__(T) void rmsnorm_fwd_kernel(const uint16_t* __restri
     }
   };
 
-  if constexpr (OUT == 1 && !(T == 256 && Policy::kPrefetchRowQuantWide)) {
+  if constexpr (OUT == 1 && !(T > 64 && Policy::kPrefetchRowQuantWide)) {
     // the quantising form has enough arithmetic per row to want several waves per SIMD:
     // one row in registers, the other waves cover its loads
     uint4 buf[NCHUNK];
@@ -640,18 +640,21 @@ hipError_t launch_rmsnorm_fwd(const void* x, const void* gamma, void* out, float
   } else if (!quant) {
     if (reuse_rstd) { FQ_LAUNCH_FWD(true, 0, kE4M3, false) } else { FQ_LAUNCH_FWD(false, 0, kE4M3, false) }
   } else if (n > 2048) {
-    // wide rows, quantising form: four waves per row (a wave per row needs up to ~230 registers)
+    // wide rows, quantising form: four waves per row (a wave per row needs up to ~230 registers), three
+    // where two chunks a thread still cover the row with them
     const int nc4 = (n / 8 + 255) / 256;
     const int64_t one_row = 256 * Policy::kRowQuantWideRowPerWg;
     int64_t wg4 = M;
     if (M > one_row) wg4 = nc4 == 4 ? 256 * Policy::kRowQuantWideWgsPerCu : one_row;
     const dim3 grid4((unsigned)wg4);
-#define FQ_LAUNCH_FWD4(NC, KINDV, ROUNDV)                                                                      \
-  hipLaunchKernelGGL((rmsnorm_fwd_kernel<256, NC, false, 1, KINDV, ROUNDV>), grid4, dim3(256), 0, stream,       \
+#define FQ_LAUNCH_FWD4(T, NC, KINDV, ROUNDV)                                                                   \
+  hipLaunchKernelGGL((rmsnorm_fwd_kernel<T, NC, false, 1, KINDV, ROUNDV>), grid4, dim3(T), 0, stream,           \
                      (const uint16_t*)x, (const uint16_t*)gamma, out, scale, rstd, M, n, eps, rows_per_wg)
 #define FQ_LAUNCH_FWD4_NC(KINDV, ROUNDV) \
-  if (nc4 == 2) { FQ_LAUNCH_FWD4(2, KINDV, ROUNDV); } else if (nc4 == 3) { FQ_LAUNCH_FWD4(3, KINDV, ROUNDV); } \
-  else { FQ_LAUNCH_FWD4(4, KINDV, ROUNDV); }
+  if (n <= Policy::kRowQuantThreeWavesMax) { FQ_LAUNCH_FWD4(192, 2, KINDV, ROUNDV); }                          \
+  else if (nc4 == 2) { FQ_LAUNCH_FWD4(256, 2, KINDV, ROUNDV); }                                                \
+  else if (nc4 == 3) { FQ_LAUNCH_FWD4(256, 3, KINDV, ROUNDV); }                                                \
+  else { FQ_LAUNCH_FWD4(256, 4, KINDV, ROUNDV); }
     if (kind == kE5M2) {
       if (round_scale) { FQ_LAUNCH_FWD4_NC(kE5M2, true) } else { FQ_LAUNCH_FWD4_NC(kE5M2, false) }
     } else {

@@ -282,6 +282,20 @@ def test_rmsnorm_and_block_quant(gpu, M, N, round_scale):
 
 
 # ------------------------------------------------------------------ SwiGLU
+# three and four waves per row: the narrowest and widest of each, one workgroup per row and looping ones
+@pytest.mark.parametrize("M,N", [(1, 2176), (4099, 2176), (37, 3072), (4099, 3072), (4099, 3200), (5, 6272), (4099, 6272)])
+def test_rmsnorm_rows_only_wide(gpu, M, N):
+    from linghe_amd.utils.norm import triton_rms_norm_and_block_quant_forward as fn
+
+    announce("rmsnorm rows only, wide", M, N)
+    x, w = randn_bf16(gen(37), M, N), gamma_bf16(gen(38), N)
+    q, s, rms, _, _ = fn(_dev(x, gpu), _dev(w, gpu), output_mode=0)
+    want = 1.0 / torch.sqrt((x.double() ** 2).mean(1) + 1e-6)
+    assert float((rms.cpu().double() / want - 1).abs().max()) < 4 * 2.0 ** -23
+    ref = O.rms_norm_and_block_quant_forward(x, w, rstd=rms.cpu())
+    check_quant_pair("rms.wide.row", ref[0], ref[1], q, s, **EXACT)
+
+
 # whole row blocks that eight XCDs share unevenly: fewer than eight, one more than eight, rows beyond one per wave
 @pytest.mark.parametrize("M,N", [(128, 256), (384, 2048), (1152, 2176), (8320, 128), (16768, 256)])
 def test_rmsnorm_passes_by_xcd(gpu, M, N):
