@@ -114,17 +114,20 @@ struct Policy {
   // the wide-row (three or four waves per row) RMSNorm + row-wise quant kernel loads the next row while it works on
   // the current one (122 instead of 84 registers): 68.5 -> 65.5 us at 16384 x 7168
   static constexpr bool kPrefetchRowQuantWide = true;
-  // Workgroups of that kernel's launch.  Up to 16 rows per CU every row has its own: the hardware hands them out as
-  // others finish, while four looping workgroups per CU leave most of the chip idle in the last round of few
-  // (us 4 / 16 per CU: 1500 x 3072 7.5 / 5.9, 3001 x 4096 11.1 / 9.9, 4000 x 2560 11.3 / 10.4, 4104 x 5120 16.3 / 16.3).
-  // Beyond, 16 looping ones per CU, as they fit (8192 x 4096 22.5 / 21.7, 12000 x 5120 40.0 / 39.0); at n > 6144, where
-  // a CU holds four, exactly those (16384 x 7168: 64.0 / 65.4 / 64.8 / 64.6 / 68.0 with 4 / 5 / 6 / 8 / 12).
-  static constexpr int kRowQuantWideRowPerWg = 16;
+  // Workgroups of that kernel's launch.  Up to 32 rows per CU every row has its own: the hardware hands them out as
+  // others finish, while looping ones leave most of the chip idle in the last round of few (us 4 looping per CU / one
+  // per row: 1500 x 3072 7.5 / 5.9, 3001 x 4096 11.1 / 9.9, 4000 x 2560 11.3 / 10.4; 16 looping per CU / one per row:
+  // 5000 x 7168 23.9 / 23.2, 6001 x 4096 20.8 / 16.7, 8192 x 3072 17.9 / 17.4, 8192 x 4096 21.7 / 21.8, 8192 x 5120
+  // 27.9 / 28.2).  Beyond, 16 looping ones per CU (us with 4 / 16: 12000 x 5120 40.0 / 39.0; with 16 / 32: 38.6 /
+  // 46.5); at n > 6144, where a CU holds four, exactly those (16384 x 7168: 64.0 / 65.4 / 64.8 / 64.6 / 68.0 with
+  // 4 / 5 / 6 / 8 / 12).
+  static constexpr int kRowQuantWideRowPerWg = 32;
+  static constexpr int kRowQuantWideWgsPerCu = 16;
+  static constexpr int kRowQuantWidestWgsPerCu = 4;
   // up to 3072 columns (two chunks on 192 threads) three waves share a row: with four, a quarter and more of the
   // lanes repeat the row's last chunk (us four / three waves: 1500 x 3072 5.89 / 5.79, 3001 x 2560 8.43 / 7.93,
   // 8192 x 3072 19.0 / 17.9; three chunks on 192 are level or behind: 3001 x 3584 9.1 / 10.3, 12000 x 5120 38.9 / 39.7)
   static constexpr int kRowQuantThreeWavesMax = 3072;
-  static constexpr int kRowQuantWideWgsPerCu = 4;
   // the same in the wide-row RMSNorm backward with one chunk per thread (2048 < n <= 4096: 70.4 -> 66.9 us at
   // 16384 x 3072, 78.5 -> 76.4 at 16384 x 4096); with two chunks the second register set spills
   static constexpr bool kPrefetchRowBwdWide = true;

@@ -643,9 +643,9 @@ hipError_t launch_rmsnorm_fwd(const void* x, const void* gamma, void* out, float
     // wide rows, quantising form: four waves per row (a wave per row needs up to ~230 registers), three
     // where two chunks a thread still cover the row with them
     const int nc4 = (n / 8 + 255) / 256;
-    const int64_t one_row = 256 * Policy::kRowQuantWideRowPerWg;
     int64_t wg4 = M;
-    if (M > one_row) wg4 = nc4 == 4 ? 256 * Policy::kRowQuantWideWgsPerCu : one_row;
+    if (M > 256 * Policy::kRowQuantWideRowPerWg)
+      wg4 = 256 * (nc4 == 4 ? Policy::kRowQuantWidestWgsPerCu : Policy::kRowQuantWideWgsPerCu);
     const dim3 grid4((unsigned)wg4);
 #define FQ_LAUNCH_FWD4(T, NC, KINDV, ROUNDV)                                                                   \
   hipLaunchKernelGGL((rmsnorm_fwd_kernel<T, NC, false, 1, KINDV, ROUNDV>), grid4, dim3(T), 0, stream,           \

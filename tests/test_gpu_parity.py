@@ -283,7 +283,7 @@ def test_rmsnorm_and_block_quant(gpu, M, N, round_scale):
 
 # ------------------------------------------------------------------ SwiGLU
 # three and four waves per row: the narrowest and widest of each, one workgroup per row and looping ones
-@pytest.mark.parametrize("M,N", [(1, 2176), (4099, 2176), (37, 3072), (4099, 3072), (4099, 3200), (5, 6272), (4099, 6272)])
+@pytest.mark.parametrize("M,N", [(1, 2176), (8200, 2176), (37, 3072), (4099, 3072), (8195, 3200), (5, 6272), (8195, 6272)])
 def test_rmsnorm_rows_only_wide(gpu, M, N):
     from linghe_amd.utils.norm import triton_rms_norm_and_block_quant_forward as fn
 
