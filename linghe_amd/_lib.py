@@ -87,6 +87,8 @@ try:  # outputs and launch of the row-wise quantisers in one native call (csrc/f
 except ImportError as e:
     raise ImportError("linghe_amd/_fq_torch.so is missing or was built for another torch: build it with "
                       "`python -m linghe_amd.build`. There is no fallback path.") from e
+native.bind(*(ctypes.cast(getattr(lib, name), _P).value
+              for name in ("fq_rmsnorm_quant_fwd", "fq_swiglu_quant_fwd", "fq_group_quant", "fq_last_error")))
 
 
 def check(rc: int) -> None:

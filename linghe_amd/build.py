@@ -80,8 +80,7 @@ def build_library(extra_flags=(), verbose: bool = False, csrc: str = CSRC, out: 
 
 
 def build_host_module(out: str = HOST_PATH) -> str:
-    """Compile the host-side module (host code only: g++) against the installed torch and link it to
-    libfq_gfx950.so beside it."""
+    """Compile the host-side module (host code only: g++) against the installed torch."""
     import sysconfig
 
     from torch.utils import cpp_extension
@@ -90,7 +89,7 @@ def build_host_module(out: str = HOST_PATH) -> str:
     tmp = out + ".tmp"
     _run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", *("-I" + i for i in includes),
           os.path.join(CSRC, "fq_torch.cpp"), "-o", tmp, *("-L" + d for d in cpp_extension.library_paths()),
-          "-ltorch_python", "-ltorch_cpu", "-lc10", "-L" + HERE, "-l:" + LIB_NAME, "-Wl,-rpath,$ORIGIN"])
+          "-ltorch_python", "-ltorch_cpu", "-lc10"])
     os.replace(tmp, out)
     return out
 

@@ -4,6 +4,8 @@
 // with torch.empty and calls the library through ctypes takes 12 us: what bounds a small call is the host.
 // The wrappers keep their checks in Python and hand over here; allocation goes through the dispatcher as
 // torch.empty does (same allocator, pools and modes) and the interpreter lock is released meanwhile.
+// The kernel library is the one that _lib.py loaded: bind() takes its functions' addresses, there is no
+// link-time dependency that could bring a second one into the process.
 // RMSNorm + group + SwiGLU quantiser, three calls: 36.8 -> 21.7 us on 32 rows of 2048, 36.8 -> 23.9 on 3001 of 4096.
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
@@ -14,6 +16,13 @@
 #include "../../include/fq_api.h"
 
 namespace {
+
+struct {
+  decltype(&fq_rmsnorm_quant_fwd) rmsnorm_quant_fwd = nullptr;
+  decltype(&fq_swiglu_quant_fwd) swiglu_quant_fwd = nullptr;
+  decltype(&fq_group_quant) group_quant = nullptr;
+  decltype(&fq_last_error) last_error = nullptr;
+} lib;
 
 at::ScalarType dtype_of(PyObject* o) {
   TORCH_CHECK(THPDtype_Check(o), "expected a torch.dtype");
@@ -42,10 +51,29 @@ at::Tensor empty(const at::Tensor& like, at::ScalarType type, at::IntArrayRef si
 void* data(const at::Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 
 void check(int rc) {
-  TORCH_CHECK(rc == 0, "libfq_gfx950 error ", rc, ": ", fq_last_error());
+  TORCH_CHECK(rc == 0, "libfq_gfx950 error ", rc, ": ", lib.last_error());
 }
 
 void need_args(Py_ssize_t n, Py_ssize_t want) { TORCH_CHECK(n == want, "expected ", want, " arguments, got ", n); }
+
+void need_lib() { TORCH_CHECK(lib.last_error, "bind() was not called"); }
+
+template <typename F>
+F function_at(PyObject* o) {
+  const int64_t address = int_of(o);
+  TORCH_CHECK(address != 0, "a function's address is 0");
+  return reinterpret_cast<F>(static_cast<intptr_t>(address));
+}
+
+// (fq_rmsnorm_quant_fwd, fq_swiglu_quant_fwd, fq_group_quant, fq_last_error): addresses in the loaded library
+PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+  HANDLE_TH_ERRORS
+  need_args(n_args, 4);
+  lib = {function_at<decltype(&fq_rmsnorm_quant_fwd)>(a[0]), function_at<decltype(&fq_swiglu_quant_fwd)>(a[1]),
+         function_at<decltype(&fq_group_quant)>(a[2]), function_at<decltype(&fq_last_error)>(a[3])};
+  Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
+}
 
 // the outputs as a tuple, None for an undefined one
 PyObject* wrap(const std::initializer_list<at::Tensor>& outs) {
@@ -68,6 +96,7 @@ PyObject* wrap(const std::initializer_list<at::Tensor>& outs) {
 PyObject* rmsnorm_quant(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   HANDLE_TH_ERRORS
   need_args(n_args, 11);
+  need_lib();
   const at::Tensor x = tensor_or_none(a[0]), gamma = tensor_or_none(a[1]);
   at::Tensor out = tensor_or_none(a[2]), scale = tensor_or_none(a[3]), rms = tensor_or_none(a[4]), qt, st;
   const double eps = PyFloat_AsDouble(a[5]);
@@ -87,10 +116,10 @@ PyObject* rmsnorm_quant(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     st = empty(x, at::kFloat, {(M + 127) / 128, n});
     if (!rms.defined()) rms = empty(x, at::kFloat, {M});
     if (M > 0)
-      check(fq_rmsnorm_quant_fwd(data(x), data(gamma), mode != 1 ? data(out) : nullptr,
-                                 static_cast<float*>(mode != 1 ? data(scale) : nullptr),
-                                 static_cast<float*>(data(rms)), data(qt), static_cast<float*>(data(st)), M, n,
-                                 static_cast<float>(eps), round, mode, kind, stream));
+      check(lib.rmsnorm_quant_fwd(data(x), data(gamma), mode != 1 ? data(out) : nullptr,
+                                  static_cast<float*>(mode != 1 ? data(scale) : nullptr),
+                                  static_cast<float*>(data(rms)), data(qt), static_cast<float*>(data(st)), M, n,
+                                  static_cast<float>(eps), round, mode, kind, stream));
   }
   return wrap({out, scale, rms, qt, st});
   END_HANDLE_TH_ERRORS
@@ -100,6 +129,7 @@ PyObject* rmsnorm_quant(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
 PyObject* swiglu_quant(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   HANDLE_TH_ERRORS
   need_args(n_args, 8);
+  need_lib();
   const at::Tensor x = tensor_or_none(a[0]);
   at::Tensor out = tensor_or_none(a[1]), scale = tensor_or_none(a[2]), qt, st;
   const int round = static_cast<int>(int_of(a[3])), mode = static_cast<int>(int_of(a[4]));
@@ -114,8 +144,8 @@ PyObject* swiglu_quant(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     qt = empty(x, fp8, {n, M});
     st = empty(x, at::kFloat, {(M + 127) / 128, n});
     if (M > 0)
-      check(fq_swiglu_quant_fwd(data(x), data(out), static_cast<float*>(data(scale)), data(qt),
-                                static_cast<float*>(data(st)), M, n, round, mode, kind, stream));
+      check(lib.swiglu_quant_fwd(data(x), data(out), static_cast<float*>(data(scale)), data(qt),
+                                 static_cast<float*>(data(st)), M, n, round, mode, kind, stream));
   }
   return wrap({out, scale, qt, st});
   END_HANDLE_TH_ERRORS
@@ -125,6 +155,7 @@ PyObject* swiglu_quant(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
 PyObject* group_quant(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   HANDLE_TH_ERRORS
   need_args(n_args, 5);
+  need_lib();
   const at::Tensor x = tensor_or_none(a[0]);
   at::Tensor q, s;
   const int round = static_cast<int>(int_of(a[1]));
@@ -136,14 +167,15 @@ PyObject* group_quant(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     const int64_t M = x.size(0), n = x.size(1);
     q = empty(x, fp8, {M, n});
     s = empty(x, at::kFloat, {M, n / 128});
-    if (M > 0) check(fq_group_quant(data(x), data(q), static_cast<float*>(data(s)), M, n, round, kind, stream));
+    if (M > 0) check(lib.group_quant(data(x), data(q), static_cast<float*>(data(s)), M, n, round, kind, stream));
   }
   return wrap({q, s});
   END_HANDLE_TH_ERRORS
 }
 
 #define FQ_FAST(f) reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(f))
-PyMethodDef methods[] = {{"rmsnorm_quant", FQ_FAST(rmsnorm_quant), METH_FASTCALL, nullptr},
+PyMethodDef methods[] = {{"bind", FQ_FAST(bind), METH_FASTCALL, nullptr},
+                         {"rmsnorm_quant", FQ_FAST(rmsnorm_quant), METH_FASTCALL, nullptr},
                          {"swiglu_quant", FQ_FAST(swiglu_quant), METH_FASTCALL, nullptr},
                          {"group_quant", FQ_FAST(group_quant), METH_FASTCALL, nullptr},
                          {nullptr, nullptr, 0, nullptr}};

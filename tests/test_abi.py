@@ -6,6 +6,10 @@ import ctypes
 import inspect
 import os
 import re
+import shutil
+import subprocess
+import sys
+import textwrap
 
 import pytest
 
@@ -287,3 +291,34 @@ def test_expert_plan_shape_on_host():
     rc = L.fq_batched_pad_permute_quant_planned(None, ctypes.c_void_p(256), good, 4, None, None, 0, None, None, None,
                                                 None, None, 64, 64, 256, 0, 0, None)
     assert rc == -2 and b"padded" in L.fq_last_error()
+
+
+def run_python(code, **env):
+    """A fresh interpreter: which libraries a process maps, and what it can import, is settled at import."""
+    got = subprocess.run([sys.executable, "-c", textwrap.dedent(code)], cwd=ROOT, env={**os.environ, **env},
+                         capture_output=True, text=True, timeout=300)
+    assert got.returncode == 0, got.stderr
+    return got.stdout
+
+
+def test_named_library_serves_every_call(tmp_path):
+    """LINGHE_FQ_LIB names another build: it is the only kernel library in the process, for the calls that go through
+    ctypes and for the native ones alike."""
+    from linghe_amd.build import LIB_PATH
+
+    named = str(tmp_path / "libfq_other_tuning.so")
+    shutil.copyfile(LIB_PATH, named)
+    out = run_python("""
+        import torch
+        from linghe_amd import _lib
+        mapped = {l.split()[-1] for l in open("/proc/self/maps") if "/libfq_" in l}
+        print(*sorted(mapped))
+        # a shape that the library refuses, before any device call: its message is the named library's own
+        try:
+            _lib.native.group_quant(torch.empty(2, 100, dtype=torch.bfloat16), 0, torch.float8_e4m3fn, 0, 0)
+        except RuntimeError as e:
+            assert _lib.lib.fq_last_error().decode() in str(e) and _lib.lib.fq_last_error(), e
+        else:
+            raise SystemExit("not refused")
+    """, LINGHE_FQ_LIB=named)
+    assert out.split() == [os.path.realpath(named)], out
