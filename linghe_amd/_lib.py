@@ -82,13 +82,25 @@ def _load() -> ctypes.CDLL:
 
 lib = _load()
 
-try:  # outputs and launch of the row-wise quantisers in one native call (csrc/fq_torch.cpp)
+
+class _MissingModule:
+    """Stands for csrc/fq_torch.cpp's module where it cannot be imported: the calls that go through it raise."""
+
+    def __init__(self, cause):
+        self._cause = cause
+
+    def __getattr__(self, name):
+        raise ImportError("linghe_amd/_fq_torch.so is missing or was built for another torch: build it with "
+                          "`python -m linghe_amd.build`. There is no fallback path.") from self._cause
+
+
+try:  # outputs and launch of the row-wise quantisers in one native call
     from . import _fq_torch as native
 except ImportError as e:
-    raise ImportError("linghe_amd/_fq_torch.so is missing or was built for another torch: build it with "
-                      "`python -m linghe_amd.build`. There is no fallback path.") from e
-native.bind(*(ctypes.cast(getattr(lib, name), _P).value
-              for name in ("fq_rmsnorm_quant_fwd", "fq_swiglu_quant_fwd", "fq_group_quant", "fq_last_error")))
+    native = _MissingModule(e)
+else:
+    native.bind(*(ctypes.cast(getattr(lib, name), _P).value
+                  for name in ("fq_rmsnorm_quant_fwd", "fq_swiglu_quant_fwd", "fq_group_quant", "fq_last_error")))
 
 
 def check(rc: int) -> None:

@@ -75,19 +75,23 @@ def build_library(extra_flags=(), verbose: bool = False, csrc: str = CSRC, out: 
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", tmp])
     os.replace(tmp, out)
     if out == LIB_PATH:
-        build_host_module()
+        try:
+            build_host_module()
+        except RuntimeError as e:
+            raise RuntimeError(f"{out} is built and serves every call but the row-wise quantisers; "
+                               f"the host module is not (it needs torch's and Python's headers): {e}") from e
     return out
 
 
 def build_host_module(out: str = HOST_PATH) -> str:
-    """Compile the host-side module (host code only: g++) against the installed torch."""
+    """Compile the host-side module (host code only, by the same compiler) against the installed torch."""
     import sysconfig
 
     from torch.utils import cpp_extension
 
     includes = [*cpp_extension.include_paths(), sysconfig.get_path("include")]
     tmp = out + ".tmp"
-    _run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", *("-I" + i for i in includes),
+    _run([_hipcc(), "-x", "c++", "--no-hip-rt", "-O2", "-std=c++17", "-shared", "-fPIC", *("-I" + i for i in includes),
           os.path.join(CSRC, "fq_torch.cpp"), "-o", tmp, *("-L" + d for d in cpp_extension.library_paths()),
           "-ltorch_python", "-ltorch_cpu", "-lc10"])
     os.replace(tmp, out)

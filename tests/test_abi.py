@@ -322,3 +322,33 @@ def test_named_library_serves_every_call(tmp_path):
             raise SystemExit("not refused")
     """, LINGHE_FQ_LIB=named)
     assert out.split() == [os.path.realpath(named)], out
+
+
+def test_only_the_native_calls_need_the_host_module():
+    """Without _fq_torch.so everything else imports and reaches the library; the calls that need it say so."""
+    run_python("""
+        import sys
+        sys.modules["linghe_amd._fq_torch"] = None
+        from linghe_amd import _lib
+        import linghe_amd.facade.norm, linghe_amd.facade.silu, linghe_amd.quant.block, linghe_amd.utils.gather
+        import linghe_amd.quant.group
+        assert _lib.lib.fq_version() >= 100
+        try:
+            _lib.native.group_quant
+        except ImportError as e:
+            assert "_fq_torch.so" in str(e) and e.__cause__ is not None
+        else:
+            raise SystemExit("no error")
+    """)
+
+
+def test_build_needs_one_compiler(monkeypatch):
+    """Every translation unit, the host module's too, is compiled and linked by hipcc."""
+    from linghe_amd import build as B
+
+    commands = []
+    monkeypatch.setattr(B, "_run", commands.append)
+    monkeypatch.setattr(B.os, "replace", lambda src, dst: None)
+    B.build_library()
+    assert len(commands) == len(B.SOURCES) + 2
+    assert {c[0] for c in commands} == {B._hipcc()}
