@@ -91,7 +91,7 @@ def build_host_module(out: str = HOST_PATH) -> str:
 
     includes = [*cpp_extension.include_paths(), sysconfig.get_path("include")]
     tmp = out + ".tmp"
-    _run([_hipcc(), "-x", "c++", "--no-hip-rt", "-O2", "-std=c++17", "-shared", "-fPIC", *("-I" + i for i in includes),
+    _run([_hipcc(), "-x", "c++", "-no-hip-rt", "-O2", "-std=c++17", "-shared", "-fPIC", *("-I" + i for i in includes),
           os.path.join(CSRC, "fq_torch.cpp"), "-o", tmp, *("-L" + d for d in cpp_extension.library_paths()),
           "-ltorch_python", "-ltorch_cpu", "-lc10"])
     os.replace(tmp, out)
