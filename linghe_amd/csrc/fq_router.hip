@@ -134,6 +134,19 @@ __device__ __forceinline__ void router_emit(uint16_t* y, uint8_t* q, float* s, b
   if (first) store_f32(s, sc);
 }
 
+// A row whose squares overflow has the statistic 0, so y = (x * 0) * gamma is 0 where x and gamma are finite and
+// NaN where they are not, and so are its logits.  The products taken before the statistic is known can say neither
+// (x * gamma * W overflows): the factor of such a row's logits is 0 or NaN by its values, and 0 stands
+// for the result itself.
+__device__ __forceinline__ bool router_nonfinite(const uint4& v) {  // any of 8 bf16
+  auto pair = [](unsigned w) { return (w & 0x7f80u) == 0x7f80u || (w & 0x7f800000u) == 0x7f800000u; };
+  return pair(v.x) || pair(v.y) || pair(v.z) || pair(v.w);
+}
+constexpr unsigned kNanBits = 0x7fc00000u;  // as bits throughout: the compiler may take a float for not NaN
+__device__ __forceinline__ float router_logit(float v, unsigned factor) {
+  return __uint_as_float(factor == 0 ? 0u : __float_as_uint(v * __uint_as_float(factor)));
+}
+
 __device__ __forceinline__ bf16x8_t operand(const uint4& v) { return __builtin_bit_cast(bf16x8_t, v); }
 
 // ---------------------------------------------------------------------------
@@ -155,7 +168,7 @@ constexpr int kRouterRows = 64;
 struct RouterShared {
   uint4 a[2][2][2][8][64];  // [buffer][hi, lo][32-row tile][k step][lane slot]; afterwards the partial sums
   uint4 gamma[8192 / 8];
-  float rstd[kRouterRows];
+  unsigned factor[kRouterRows];  // of a row's logits: the bits of its statistic, or see router_logit
 };
 
 // The order of a k block's instructions: operand reads, then the matrix instructions with the next
@@ -309,8 +322,17 @@ __global__ __launch_bounds__(512) void rmsnorm_router_quant_kernel(RouterArgs p)
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
     rs[u] = 1.0f / sqrtf((float)row16_sum_d(ss[u]) / (float)p.K + p.eps);
+    unsigned factor = __float_as_uint(rs[u]);
+    if (factor == 0) {
+      bool bad = false;
+#pragma unroll 1
+      for (int kb = 0; kb < kblocks; ++kb)
+        bad |= router_nonfinite(*(const uint4*)(xrow + u * half_tile + kb * kGroup)) ||
+               router_nonfinite(sh.gamma[kb * 16 + cg]);
+      if (row16_max(bad ? 1.f : 0.f) > 0.f) factor = kNanBits;
+    }
     if (cg == 0) {
-      sh.rstd[u * 32 + rg] = rs[u];
+      sh.factor[u * 32 + rg] = factor;
       if (chunk == 0) p.rstd[row0 + u * 32 + rg] = rs[u];
     }
   }
@@ -353,7 +375,7 @@ __global__ __launch_bounds__(512) void rmsnorm_router_quant_kernel(RouterArgs p)
     const int col = ((chunk * 2 + wc) * NACC + (i4 >> 2)) * 32 + (lane & 31);
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      p.logits[(int64_t)(row0 + row + e) * p.N + col] = v[e] * sh.rstd[row + e];
+      p.logits[(int64_t)(row0 + row + e) * p.N + col] = router_logit(v[e], sh.factor[row + e]);
   }
 
 #pragma unroll 1
@@ -469,7 +491,16 @@ __global__ __launch_bounds__(512) void rmsnorm_router_quant_few_rows_kernel(Rout
     float v = part[0][at];
 #pragma unroll
     for (int i = 1; i < 8; ++i) v += part[i][at];
-    p.logits[(int64_t)(row0 + row) * p.N + chunk * 32 + col] = v * srstd[row];
+    unsigned factor = __float_as_uint(srstd[row]);
+    bool bad = false;
+    if (factor == 0) {
+#pragma unroll 1
+      for (int c = col * 8; c < p.K; c += 256)
+        bad |= router_nonfinite(*(const uint4*)(p.x + (int64_t)(row0 + row) * p.K + c)) ||
+               router_nonfinite(*(const uint4*)(p.gamma + c));
+    }
+    if ((uint32_t)(__ballot(bad) >> (lane & 32))) factor = kNanBits;  // 32 lanes have one row
+    p.logits[(int64_t)(row0 + row) * p.N + chunk * 32 + col] = router_logit(v, factor);
   }
   const int q0 = chunk * kblocks / p.chunks, q1 = (chunk + 1) * kblocks / p.chunks;
   const int cg = tid_x() & 15;

@@ -651,3 +651,34 @@ def test_router_kernel_choice(gpu, M, N, K, wdtype):
     y32 = (x.float() * rms.cpu()[:, None]) * nw.float()
     err = (logits.cpu().double() - y32.double() @ rw.double().t()).abs()
     assert bool((err <= 2.0 ** -16 * (y32.abs().double() @ rw.double().abs().t())).all())
+
+
+# one call of each form of the router kernel: 16-row, 64 x 64, 64 x 128, fp32
+@pytest.mark.parametrize("M,N,K,wdtype", [(128, 128, 640, torch.bfloat16), (2688, 128, 256, torch.bfloat16),
+                                          (8320, 128, 384, torch.bfloat16), (2176, 256, 256, torch.float32),
+                                          (128, 256, 384, torch.float32)])
+def test_router_rows_without_a_statistic(gpu, M, N, K, wdtype):
+    """Rows whose squares overflow: the statistic is 0, hence y and, for finite values, the logits (zeros, not the NaN
+    of overflowed products); an infinity makes the row's logits NaN.  Other rows do not notice."""
+    from linghe_amd.utils.norm import triton_rms_norm_fp32_gemm_block_quant_forward as fn
+
+    announce("router rows without a statistic", M, N, K, wdtype)
+    g = gen(39)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    nw = (1 + torch.rand(K, generator=g)).to(torch.bfloat16)
+    rw = (4 * torch.randn(N, K, generator=g)).to(wdtype)
+    plain = fn(_dev(x, gpu), _dev(nw, gpu), _dev(rw, gpu))[2]
+    low = torch.finfo(torch.bfloat16).min
+    zero, nan = [0, 37, M - 1], [2, M - 33]
+    odd = x.clone()
+    odd[zero] = low
+    odd[37] = x[37]
+    odd[37, K - 1] = low
+    odd[nan, K // 2 + 1] = float("inf")
+    y, rms, logits, _, _, _, _ = fn(_dev(odd, gpu), _dev(nw, gpu), _dev(rw, gpu))
+    assert bool((rms[zero + nan] == 0).all())
+    assert bool((y[zero] == 0).all()) and bool((logits[zero] == 0).all())
+    assert bool(torch.isnan(logits[nan]).all())
+    rest = torch.ones(M, dtype=torch.bool, device=gpu)
+    rest[zero + nan] = False
+    assert torch.equal(logits[rest], plain[rest])
