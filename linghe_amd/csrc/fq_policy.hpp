@@ -114,19 +114,27 @@ struct Policy {
   // the wide-row (three or four waves per row) RMSNorm + row-wise quant kernel loads the next row while it works on
   // the current one (122 instead of 84 registers): 68.5 -> 65.5 us at 16384 x 7168
   static constexpr bool kPrefetchRowQuantWide = true;
-  // Workgroups of that kernel's launch.  Up to 32 rows per CU every row has its own: the hardware hands them out as
-  // others finish, while looping ones leave most of the chip idle in the last round of few (us 4 looping per CU / one
-  // per row: 1500 x 3072 7.5 / 5.9, 3001 x 4096 11.1 / 9.9, 4000 x 2560 11.3 / 10.4; 16 looping per CU / one per row:
-  // 5000 x 7168 23.9 / 23.2, 6001 x 4096 20.8 / 16.7, 8192 x 3072 17.9 / 17.4, 8192 x 4096 21.7 / 21.8, 8192 x 5120
-  // 27.9 / 28.2).  Beyond, 16 looping ones per CU (us with 4 / 16: 12000 x 5120 40.0 / 39.0; with 16 / 32: 38.6 /
-  // 46.5); at n > 6144, where a CU holds four, exactly those (16384 x 7168: 64.0 / 65.4 / 64.8 / 64.6 / 68.0 with
-  // 4 / 5 / 6 / 8 / 12).
-  static constexpr int kRowQuantWideRowPerWg = 32;
+  // Workgroups of that kernel's launch (us at n with: one per row / 4 / 16 looping per CU).  One per row as far as these:
+  // the hardware hands them out as others finish, while looping ones leave most of the chip idle in the last
+  // round of few (2000 x 4096 7.4 / 8.5 / 7.4, 5000 x 4096 14.2 / 15.8 / 20.5, 5000 x 7168 22.6 / 23.5 / 32.7,
+  // 8192 x 7168 34.1 / 34.2 / 35.4).
+  static constexpr int kRowQuantWideRowPerWg = 8192;
+  // Beyond, 16 looping per CU where their last round is full, that is idle for at most M / 12 rows (12000 x 4096
+  // 28.1 / 31.1 / 28.8, 16384 x 2176 26.7 / 29.8 / 25.9, 16384 x 5120 50.8 / 48.6 / 47.2, 50000 x 2176
+  // 74.7 / 80.9 / 70.7), else still one per row up to 4096 columns (9000 x 3072 17.9 / 20.3 / 23.6, 10000 x 4096
+  // 24.3 / 26.7 / 28.5, 18000 x 4096 42.1 / 46.3 / 45.4).
   static constexpr int kRowQuantWideWgsPerCu = 16;
-  static constexpr int kRowQuantWidestWgsPerCu = 4;
+  static constexpr int kRowQuantWideIdleShare = 12;
+  // Rows of three chunks a thread (4096 < n <= 6144; five workgroups on a CU) turn to looping earlier, and to 4 per CU
+  // where 16 do not come out even (6001 x 5120 21.5 / 21.8 / 26.4, 7000 x 4224 23.4 / 22.5 / 24.7, 8192 x 4608
+  // 27.4 / 25.7 / 26.6, 9000 x 5120 29.8 / 29.0 / 35.8, 10000 x 4608 31.7 / 31.0 / 35.6, 14000 x 5632 45.6 / 45.2 / 49.5).
+  static constexpr int kRowQuantThreeChunksRowPerWg = 6144;
+  // Four chunks a thread (n > 6144): exactly the four workgroups that a CU holds (16384 x 7168: 64.0 / 65.4 / 64.8 /
+  // 64.6 / 68.0 with 4 / 5 / 6 / 8 / 12).
+  static constexpr int kRowQuantFewLoopingPerCu = 4;
   // up to 3072 columns (two chunks on 192 threads) three waves share a row: with four, a quarter and more of the
-  // lanes repeat the row's last chunk (us four / three waves: 1500 x 3072 5.89 / 5.79, 3001 x 2560 8.43 / 7.93,
-  // 8192 x 3072 19.0 / 17.9; three chunks on 192 are level or behind: 3001 x 3584 9.1 / 10.3, 12000 x 5120 38.9 / 39.7)
+  // lanes repeat the row's last chunk (us four / three waves, one workgroup per row: 1500 x 3072 5.89 / 5.79,
+  // 3001 x 2560 8.43 / 7.93, 8192 x 3072 19.0 / 17.9; three chunks on 192 are behind: 3001 x 3584 9.1 / 10.3)
   static constexpr int kRowQuantThreeWavesMax = 3072;
   // the same in the wide-row RMSNorm backward with one chunk per thread (2048 < n <= 4096: 70.4 -> 66.9 us at
   // 16384 x 3072, 78.5 -> 76.4 at 16384 x 4096); with two chunks the second register set spills

@@ -614,6 +614,16 @@ static void pick_row_shape(int n, int T, int& nchunk) {
   FQ_ROW_CASE(64, 13, __VA_ARGS__) FQ_ROW_CASE(64, 14, __VA_ARGS__) FQ_ROW_CASE(64, 15, __VA_ARGS__) \
   FQ_ROW_CASE(64, 16, __VA_ARGS__) { return hipErrorInvalidValue; }
 
+// workgroups of the wide-row RMSNorm + row-wise quant kernel; chunks: 16-byte pieces of a row per thread of 256
+static int64_t row_quant_wide_workgroups(int64_t M, int chunks) {
+  if (M <= (chunks == 3 ? Policy::kRowQuantThreeChunksRowPerWg : Policy::kRowQuantWideRowPerWg)) return M;
+  const int64_t few = 256 * Policy::kRowQuantFewLoopingPerCu, looping = 256 * Policy::kRowQuantWideWgsPerCu;
+  if (chunks == 4) return few;
+  const int64_t idle = (M + looping - 1) / looping * looping - M;
+  if (idle * Policy::kRowQuantWideIdleShare <= M) return looping;
+  return chunks == 3 ? few : M;  // M < looping * kRowQuantWideIdleShare here
+}
+
 hipError_t launch_rmsnorm_fwd(const void* x, const void* gamma, void* out, float* scale, float* rstd, int64_t M,
                               int n, float eps, int reuse_rstd, int quant, int round_scale, int kind,
                               hipStream_t stream) {
@@ -643,10 +653,7 @@ hipError_t launch_rmsnorm_fwd(const void* x, const void* gamma, void* out, float
     // wide rows, quantising form: four waves per row (a wave per row needs up to ~230 registers), three
     // where two chunks a thread still cover the row with them
     const int nc4 = (n / 8 + 255) / 256;
-    int64_t wg4 = M;
-    if (M > 256 * Policy::kRowQuantWideRowPerWg)
-      wg4 = 256 * (nc4 == 4 ? Policy::kRowQuantWidestWgsPerCu : Policy::kRowQuantWideWgsPerCu);
-    const dim3 grid4((unsigned)wg4);
+    const dim3 grid4((unsigned)row_quant_wide_workgroups(M, nc4));
 #define FQ_LAUNCH_FWD4(T, NC, KINDV, ROUNDV)                                                                   \
   hipLaunchKernelGGL((rmsnorm_fwd_kernel<T, NC, false, 1, KINDV, ROUNDV>), grid4, dim3(T), 0, stream,           \
                      (const uint16_t*)x, (const uint16_t*)gamma, out, scale, rstd, M, n, eps, rows_per_wg)

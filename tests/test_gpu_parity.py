@@ -283,7 +283,10 @@ def test_rmsnorm_and_block_quant(gpu, M, N, round_scale):
 
 # ------------------------------------------------------------------ SwiGLU
 # three and four waves per row: the narrowest and widest of each, one workgroup per row and looping ones
-@pytest.mark.parametrize("M,N", [(1, 2176), (8200, 2176), (37, 3072), (4099, 3072), (8195, 3200), (5, 6272), (8195, 6272)])
+@pytest.mark.parametrize("M,N", [(1, 2176), (8200, 2176), (37, 3072), (4099, 3072), (8195, 3200), (5, 6272), (8195, 6272),
+                                 # 16 looping per CU (last round full), four, and one more or fewer row than either takes
+                                 (12288, 2176), (12289, 2176), (11343, 3200), (11342, 3200), (6144, 4224), (6145, 4224),
+                                 (8192, 4224)])
 def test_rmsnorm_rows_only_wide(gpu, M, N):
     from linghe_amd.utils.norm import triton_rms_norm_and_block_quant_forward as fn
 
