@@ -520,39 +520,45 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_wave_kernel(const uint16_t* _
 // partial rows; with 64 columns and 16 slices four, on half the CUs.  us of the whole backward,
 // 64 / 32 / 16 columns: 1000 x 2048 10.8 / 10.0 / 9.7, 4096 x 1024 10.9 / 10.4 / 10.8, 8192 x 2048
 // 23.3 / 22.8 / 23.6, 8192 x 5120 49.0 / 48.6 / 51.5, 16384 x 7168 119.6 / 119.7 / 122.5.
-constexpr int kColsumCols = 32, kColsumSlices = 1024 / kColsumCols;
+// Up to 16 partial rows (128 rows of the matrix) 64 columns and 16 slices: the sum over 32 slices, most of them empty,
+// is the longer chain (32 / 64 columns, 1 x 1024 4.78 / 4.58, 64 x 1024 6.11 / 5.88, 9 x 512 5.09 / 4.84).
+constexpr int kColsumFewPartials = 16;
+template <int kCols>
 __global__ __launch_bounds__(1024) void colsum_kernel(const float* __restrict__ part, float* __restrict__ out,
                                                       int P, int n) {
-  __shared__ float red[kColsumSlices][kColsumCols];
-  const int lane = tid_x() & (kColsumCols - 1);
-  const int col = wg_x() * kColsumCols + lane;
-  const int slice = tid_x() / kColsumCols;
+  constexpr int kSlices = 1024 / kCols;
+  __shared__ float red[kSlices][kCols];
+  const int lane = tid_x() & (kCols - 1);
+  const int col = wg_x() * kCols + lane;
+  const int slice = tid_x() / kCols;
   float acc = 0.f;
   if (col < n) {
     const float* src = part + col;
     int p = slice;
-    for (; p + 7 * kColsumSlices < P; p += 8 * kColsumSlices) {
+    for (; p + 7 * kSlices < P; p += 8 * kSlices) {
       float v[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = src[(int64_t)(p + u * kColsumSlices) * n];
+      for (int u = 0; u < 8; ++u) v[u] = src[(int64_t)(p + u * kSlices) * n];
 #pragma unroll
       for (int u = 0; u < 8; ++u) acc += v[u];
     }
-    for (; p < P; p += kColsumSlices) acc += src[(int64_t)p * n];
+    for (; p < P; p += kSlices) acc += src[(int64_t)p * n];
   }
   red[slice][lane] = acc;
   __syncthreads();
   if (slice == 0 && col < n) {
     float tot = red[0][lane];
 #pragma unroll
-    for (int k = 1; k < kColsumSlices; ++k) tot += red[k][lane];
+    for (int k = 1; k < kSlices; ++k) tot += red[k][lane];
     out[col] = tot;
   }
 }
 
 static hipError_t launch_colsum(const float* part, float* out, int P, int n, hipStream_t stream) {
-  hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)((n + kColsumCols - 1) / kColsumCols)), dim3(1024), 0, stream, part,
-                     out, P, n);
+  if (P <= kColsumFewPartials)
+    hipLaunchKernelGGL(colsum_kernel<64>, dim3((unsigned)((n + 63) / 64)), dim3(1024), 0, stream, part, out, P, n);
+  else
+    hipLaunchKernelGGL(colsum_kernel<32>, dim3((unsigned)((n + 31) / 32)), dim3(1024), 0, stream, part, out, P, n);
   return hipGetLastError();
 }
 
