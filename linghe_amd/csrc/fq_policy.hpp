@@ -173,6 +173,17 @@ struct Policy {
   // 29.9 / 37.1; beyond, the 128-logit form turns x into operands half as often: 8192 x 256 88.7 / 42.2 / 36.3.
   static constexpr int kRouterFewRowsMax = 80;
   static constexpr int kRouterNarrowMax = 256;
+  // The 32-row form against these two by rounds (workgroups over 256 CUs, and over what the CUs hold): one of its rounds
+  // costs (k blocks + a) / b of a round of 64-row workgroups, with a, b = 25, 20 where one fits a CU (512 logits,
+  // 256 of an fp32 weight), 12, 20 with 256 of a bf16 weight, 34, 40 (fp32 10, 12) with 128.
+  // One walk over K for all logits is ahead where K is short and where 64 rows are just too many for a round.
+  // us 64-row / 32-row form: 4224 x 512 x 1024 29.5 / 22.0, x 2048 48.4 / 43.4, x 4096 84.7 / 86.3, 4096 x 512 x 1024
+  // 16.9 / 22.4, 12288 x 512 x 2048 81.0 / 95.6; fp32 4224 x 256 x 1024 26.6 / 21.2, 4096 x 256 x 1024 15.3 / 21.2,
+  // 8320 x 128 x 1024 31.6 / 27.0, 8192 x 128 x 1024 18.2 / 22.0; 6144 x 384 x 2048 51.5 / 40.6, 5120 x 384 x 2048
+  // 29.0 / 32.2; 16384 x 256 x 1024 39.4 / 33.1, 8192 x 256 x 1024 20.3 / 18.7, x 2048 36.0 / 41.6.
+  // k blocks up to which it is ahead in one round of either (4096 x 512 x 128 8.9 / 7.4, x 256 10.0 / 9.6, x 512
+  // 12.2 / 13.7; 4096 x 256 x 256 7.7 / 7.4, x 512 9.2 / 9.9)
+  static constexpr int kRouter32ShortK = 2;
 };
 
 }  // namespace fq

@@ -16,7 +16,7 @@
 // hi = bf16(W), lo = bf16(W - hi) (what is left is below 2^-17 |W|): two planes, four products
 // into the same accumulators.
 //
-// Both kernels below share the work out over (row tile, column chunk) pairs; the workgroups of
+// The kernels below share the work out over (row tile, column chunk) pairs; the workgroups of
 // one row tile sit on one XCD (router_tile), so that x comes from memory once and from that
 // XCD's L2 for the other chunks.  Each of them walks all of K for its columns of the logits,
 // accumulating the row statistic beside it, and then writes y, the codes and the scales for its
@@ -145,6 +145,54 @@ __device__ __forceinline__ bool router_nonfinite(const uint4& v) {  // any of 8 
 constexpr unsigned kNanBits = 0x7fc00000u;  // as bits throughout: the compiler may take a float for not NaN
 __device__ __forceinline__ float router_logit(float v, unsigned factor) {
   return __uint_as_float(factor == 0 ? 0u : __float_as_uint(v * __uint_as_float(factor)));
+}
+
+// the factor of a row that the 16 lanes of a DPP row share: r is its statistic, x the lane's first piece, gamma in LDS
+__device__ __forceinline__ unsigned router_factor(float r, const uint16_t* x, const uint4* gamma, int kblocks) {
+  unsigned factor = __float_as_uint(r);
+  if (factor == 0) {
+    bool bad = false;
+#pragma unroll 1
+    for (int kb = 0; kb < kblocks; ++kb)
+      bad |= router_nonfinite(*(const uint4*)(x + kb * kGroup)) || router_nonfinite(gamma[kb * 16]);
+    if (row16_max(bad ? 1.f : 0.f) > 0.f) factor = kNanBits;
+  }
+  return factor;
+}
+
+// EMIT k blocks of the lane's piece of ROWS rows; blocks beyond the last repeat it
+template <int EMIT, int ROWS>
+__device__ __forceinline__ void router_fetch_share(const RouterArgs& p, int row, int row_step, int cg, int k0,
+                                                   uint4 (&xe)[EMIT][ROWS]) {
+#pragma unroll
+  for (int d = 0; d < EMIT; ++d)
+#pragma unroll
+    for (int u = 0; u < ROWS; ++u)
+      xe[d][u] = *(const uint4*)(p.x + (int64_t)(row + u * row_step) * p.K + min(k0 + d, p.K / kGroup - 1) * kGroup +
+                                 cg * 8);
+}
+
+// y, codes and scales of k blocks q0 .. q1 - 1, EMIT at a time (no load waits behind a store); the first are in xe
+template <int KIND, bool ROUND, int EMIT, int ROWS>
+__device__ __forceinline__ void router_emit_share(const RouterArgs& p, const uint4* gamma, int row, int row_step, int cg,
+                                                  int q0, int q1, const float (&rs)[ROWS], uint4 (&xe)[EMIT][ROWS]) {
+#pragma unroll 1
+  for (int k0 = q0; k0 < q1; k0 += EMIT) {
+    if (k0 > q0) router_fetch_share(p, row, row_step, cg, k0, xe);
+    const int64_t at = (int64_t)row * p.K + k0 * kGroup + cg * 8;
+    const int64_t step = (int64_t)row_step * p.K;
+    float* s = p.s + (int64_t)k0 * p.M + row;
+#pragma unroll
+    for (int d = 0; d < EMIT; ++d) {
+      if (k0 + d < q1) {
+        const uint4 g = gamma[(k0 + d) * 16 + cg];
+#pragma unroll
+        for (int u = 0; u < ROWS; ++u)
+          router_emit<KIND, ROUND>(p.y + at + u * step + d * kGroup, p.q + at + u * step + d * kGroup,
+                                   s + (int64_t)d * p.M + u * row_step, cg == 0, xe[d][u], g, rs[u]);
+      }
+    }
+  }
 }
 
 __device__ __forceinline__ bf16x8_t operand(const uint4& v) { return __builtin_bit_cast(bf16x8_t, v); }
@@ -312,25 +360,15 @@ __global__ __launch_bounds__(512) void rmsnorm_router_quant_kernel(RouterArgs p)
   // ---- this workgroup's share of the quantisation groups: its first rows of x leave now
   const int q0 = chunk * kblocks / p.chunks;
   const int q1 = (chunk + 1) * kblocks / p.chunks;
-  constexpr int kEmit = 4 * NACC;  // k blocks at a time: no load waits behind a store
-  uint4 xe[kEmit][2];
-#pragma unroll
-  for (int d = 0; d < kEmit; ++d) fetch_x(q0 + d, xe[d]);
+  uint4 xe[4 * NACC][2];
+  router_fetch_share(p, row0 + rg, 32, cg, q0, xe);
 
   // ---- statistic
   float rs[2];
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
     rs[u] = 1.0f / sqrtf((float)row16_sum_d(ss[u]) / (float)p.K + p.eps);
-    unsigned factor = __float_as_uint(rs[u]);
-    if (factor == 0) {
-      bool bad = false;
-#pragma unroll 1
-      for (int kb = 0; kb < kblocks; ++kb)
-        bad |= router_nonfinite(*(const uint4*)(xrow + u * half_tile + kb * kGroup)) ||
-               router_nonfinite(sh.gamma[kb * 16 + cg]);
-      if (row16_max(bad ? 1.f : 0.f) > 0.f) factor = kNanBits;
-    }
+    const unsigned factor = router_factor(rs[u], xrow + u * half_tile, sh.gamma + cg, kblocks);
     if (cg == 0) {
       sh.factor[u * 32 + rg] = factor;
       if (chunk == 0) p.rstd[row0 + u * 32 + rg] = rs[u];
@@ -378,27 +416,151 @@ __global__ __launch_bounds__(512) void rmsnorm_router_quant_kernel(RouterArgs p)
       p.logits[(int64_t)(row0 + row + e) * p.N + col] = router_logit(v[e], sh.factor[row + e]);
   }
 
-#pragma unroll 1
-  for (int k0 = q0; k0 < q1; k0 += kEmit) {
-    if (k0 > q0) {
+  router_emit_share<KIND, ROUND>(p, sh.gamma, row0 + rg, 32, cg, q0, q1, rs, xe);
+}
+
+// ---------------------------------------------------------------------------
+// 32 rows x 32 WAVES NACC logits per workgroup: all logits of the rows wherever N is 128, 256 or (bf16) 512, so that
+// x becomes operands once. Wave w multiplies the 32 rows by its own VT operand tiles (NACC of logits: VT, or
+// one for the two planes of an fp32 weight) over all of K; nothing is exchanged at the end.
+// W operands come in sets of half a k block (whole blocks cost 165-175 registers instead of 127 with 256 logits, and the
+// second workgroup on a CU: 16384 x 256 x 1024 36.7 / 33.0 us). Three workgroups fit a CU with 128 logits, two with 256
+// of a bf16 weight, one otherwise.
+// ---------------------------------------------------------------------------
+template <int KIND, bool ROUND, bool FP32W, int VT, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 3 : 2) void rmsnorm_router_quant_32_rows_kernel(RouterArgs p) {
+  constexpr int kRows = 32;
+  constexpr int RPT = 8 / WAVES;        // rows per thread
+  constexpr int NACC = FP32W ? 1 : VT;  // 32-column result tiles of a wave
+  constexpr int SETS = 2, STEPS = 8 / SETS;  // sets of W operands per k block, k steps of a set
+  __shared__ struct {
+    uint4 a[2][2][8][64];  // [buffer][hi, lo][k step][lane slot]
+    uint4 gamma[8192 / 8];
+    unsigned factor[kRows];
+  } sh;
+  const int lane = tid_x() & 63;
+  const int wave = uniform32(tid_x() >> 6);
+  const int cg = tid_x() & 15, rg = tid_x() >> 4;
+  const int kblocks = p.K / kGroup;
+  int tile, chunk;
+  router_tile(p.M / kRows, p.chunks, tile, chunk);
+  const int row0 = tile * kRows;
+  const uint16_t* xrow = p.x + (int64_t)(row0 + rg) * p.K + cg * 8;
+  const int64_t row_step = (int64_t)(4 * WAVES) * p.K;
+
+  constexpr int kRing = 4;                // k blocks of x in flight or in use
+  uint4 xr[kRing][RPT], b[2][VT][STEPS];  // b: two sets of W operands, one in use, one in flight
+  // the products of the leading terms by k parity, all others in an accumulator of their own: shorter chains of roundings
+  floatx16_t lead[NACC][2], rest[NACC];
 #pragma unroll
-      for (int d = 0; d < kEmit; ++d) fetch_x(k0 + d, xe[d]);
+  for (int t = 0; t < NACC; ++t)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) lead[t][0][v] = lead[t][1][v] = rest[t][v] = 0.f;
+  double ss[RPT];
+#pragma unroll
+  for (int u = 0; u < RPT; ++u) ss[u] = 0.0;
+
+  const int vtiles = p.N / 32 * (FP32W ? 2 : 1);
+  const uint4* wlane = p.w + (int64_t)(chunk * WAVES + wave) * VT * 512 + lane;
+  auto fetch_w = [&](int kb, int set, uint4 (&d)[VT][STEPS]) {
+    const uint4* at = wlane + (int64_t)min(kb, kblocks - 1) * vtiles * 512 + set * STEPS * 64;
+#pragma unroll
+    for (int t = 0; t < VT; ++t)
+#pragma unroll
+      for (int j = 0; j < STEPS; ++j) d[t][j] = at[t * 512 + j * 64];
+  };
+  auto fetch_x = [&](int kb, uint4 (&d)[RPT]) {
+#pragma unroll
+    for (int u = 0; u < RPT; ++u) d[u] = *(const uint4*)(xrow + u * row_step + min(kb, kblocks - 1) * kGroup);
+  };
+  const int aj = cg & 7;  // the row position is XORed with the k step as in the kernel above
+  auto produce = [&](int kb, const uint4 (&xk)[RPT]) {
+    const uint4 g = sh.gamma[kb * 16 + cg];
+#pragma unroll
+    for (int u = 0; u < RPT; ++u) {
+      ss[u] += (double)sumsq8(xk[u]);
+      uint4 hi, lo;
+      router_split(xk[u], g, hi, lo);
+      const int slot = (cg >> 3) * 32 + ((rg + u * 4 * WAVES) ^ aj);
+      sh.a[kb & 1][0][aj][slot] = hi;
+      sh.a[kb & 1][1][aj][slot] = lo;
     }
-    const int64_t at = (int64_t)(row0 + rg) * p.K + k0 * kGroup + cg * 8;
-    uint16_t* y = p.y + at;
-    uint8_t* q = p.q + at;
-    float* s = p.s + (int64_t)k0 * p.M + row0 + rg;
+  };
+  auto multiply = [&](int buf, int set, const uint4 (&w)[VT][STEPS]) {
 #pragma unroll
-    for (int d = 0; d < kEmit; ++d) {
-      if (k0 + d < q1) {
-        const uint4 g = sh.gamma[(k0 + d) * 16 + cg];
+    for (int j = 0; j < STEPS; ++j) {
+      const int step = set * STEPS + j;
+      const int slot = (lane & 32) + ((lane & 31) ^ step);
+      const bf16x8_t hi = operand(sh.a[buf][0][step][slot]);
+      const bf16x8_t lo = operand(sh.a[buf][1][step][slot]);
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
-          router_emit<KIND, ROUND>(y + u * half_tile + d * kGroup, q + u * half_tile + d * kGroup,
-                                   s + (int64_t)d * p.M + u * 32, cg == 0, xe[d][u], g, rs[u]);
+      for (int t = 0; t < VT; ++t) {
+        const bf16x8_t wt = operand(w[t][j]);
+        if (!FP32W || t == 0) {
+          floatx16_t& c = lead[FP32W ? 0 : t][step & 1];
+          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(hi, wt, c, 0, 0, 0);
+        } else {
+          rest[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(hi, wt, rest[0], 0, 0, 0);
+        }
+        floatx16_t& c = rest[FP32W ? 0 : t];
+        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lo, wt, c, 0, 0, 0);
+      }
+    }
+  };
+
+#pragma unroll
+  for (int d = 0; d < kRing; ++d) fetch_x(d, xr[d]);
+  fetch_w(0, 0, b[0]);
+  for (int i = tid_x(); i < kblocks * 16; i += 64 * WAVES) sh.gamma[i] = *(const uint4*)(p.gamma + i * 8);
+  __syncthreads();
+  produce(0, xr[0]);
+  fetch_x(kRing, xr[0]);
+  __syncthreads();
+#pragma unroll 1
+  for (int kb = 0; kb < kblocks; kb += kRing) {
+#pragma unroll
+    for (int d = 0; d < kRing; ++d) {
+      if (kb + d < kblocks) {
+#pragma unroll
+        for (int set = 0; set < SETS; ++set) {
+          fetch_w(kb + d + (set + 1) / SETS, (set + 1) % SETS, b[(set + 1) & 1]);
+          multiply(d & 1, set, b[set & 1]);
+        }
+        if (kb + d + 1 < kblocks) {
+          produce(kb + d + 1, xr[(d + 1) % kRing]);
+          fetch_x(kb + d + 1 + kRing, xr[(d + 1) % kRing]);
+        }
+        __syncthreads();
       }
     }
   }
+
+  const int q0 = chunk * kblocks / p.chunks, q1 = (chunk + 1) * kblocks / p.chunks;
+  uint4 xe[8 / RPT][RPT];
+  router_fetch_share(p, row0 + rg, 4 * WAVES, cg, q0, xe);
+  float rs[RPT];
+#pragma unroll
+  for (int u = 0; u < RPT; ++u) {
+    rs[u] = 1.0f / sqrtf((float)row16_sum_d(ss[u]) / (float)p.K + p.eps);
+    const unsigned factor = router_factor(rs[u], xrow + u * row_step, sh.gamma + cg, kblocks);
+    if (cg == 0) {
+      sh.factor[u * 4 * WAVES + rg] = factor;
+      if (chunk == 0) p.rstd[row0 + u * 4 * WAVES + rg] = rs[u];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < NACC; ++t) {
+    const int col = ((chunk * WAVES + wave) * NACC + t) * 32 + (lane & 31);
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      // register v of a 32x32 result holds row (v / 4) * 8 + (lane / 32) * 4 + v % 4, column lane % 32
+      const int row = (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3);
+      p.logits[(int64_t)(row0 + row) * p.N + col] =
+          router_logit((lead[t][0][v] + lead[t][1][v]) + rest[t][v], sh.factor[row]);
+    }
+  }
+  router_emit_share<KIND, ROUND>(p, sh.gamma, row0 + rg, 4 * WAVES, cg, q0, q1, rs, xe);
 }
 
 // ---------------------------------------------------------------------------
@@ -530,6 +692,38 @@ hipError_t launch_pack_router_weight(const void* wr, int weight_fp32, void* wpac
   return hipGetLastError();
 }
 
+struct RouterForm {
+  int rows, cols;  // of a workgroup: rows of x, logits
+};
+
+// which kernel, by the number of workgroups that each would have: fq_policy.hpp
+static RouterForm router_form(int64_t M, int K, int N, bool weight_fp32) {
+  const auto ceil_div = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+  const int64_t tiles = ceil_div(M, kRouterRows);
+  if (M < kRouterRows || tiles * (N / 64) <= Policy::kRouterFewRowsMax) return {kRouterFewRows, 32};
+  const bool narrow = !weight_fp32 && tiles * (N / 64) <= Policy::kRouterNarrowMax;
+  const int cols64 = weight_fp32 || narrow ? 64 : 128;
+  const int cols32 = N % 512 == 0 && !weight_fp32 ? 512 : N % 256 == 0 ? 256 : 128;
+  const int per_cu = cols32 == 128 ? 3 : cols32 == 256 && !weight_fp32 ? 2 : 1;
+  const int64_t rounds64 = ceil_div(tiles * (N / cols64), 256);
+  const int64_t slots = 256 * per_cu, workgroups32 = M / 32 * (N / cols32), rounds32 = ceil_div(workgroups32, slots);
+  const int kblocks = K / kGroup;
+  bool take32;
+  if (per_cu == 1) {
+    // in fifths of a round: one that leaves CUs free is shorter, the others' W arrives faster
+    const int64_t fifths = rounds32 == 1 && rounds64 > 1 ? 3 * slots + 2 * workgroups32 : 5 * slots * rounds32;
+    take32 = (kblocks + 25) * fifths <= 20 * 5 * slots * rounds64 ||
+             (!weight_fp32 && !narrow && kblocks <= Policy::kRouter32ShortK);
+  } else if (weight_fp32) {
+    take32 = (kblocks + 10) * rounds32 <= 12 * rounds64;
+  } else if (cols32 == 256) {
+    take32 = narrow ? kblocks <= Policy::kRouter32ShortK : (kblocks + 12) * rounds32 <= 20 * rounds64;
+  } else {
+    take32 = !narrow && (kblocks + 34) * rounds32 <= 40 * rounds64;
+  }
+  return take32 ? RouterForm{32, cols32} : RouterForm{kRouterRows, cols64};
+}
+
 // the main kernels on a weight already in operand order
 hipError_t launch_rmsnorm_router_quant_packed(const void* x, const void* gamma, const void* wpacked,
                                               int weight_fp32, void* y, float* rstd, float* logits, void* q,
@@ -538,16 +732,20 @@ hipError_t launch_rmsnorm_router_quant_packed(const void* x, const void* gamma, 
   if (M == 0) return hipSuccess;
   RouterArgs p{(const uint16_t*)x, (const uint16_t*)gamma, (const uint4*)wpacked, (uint16_t*)y, rstd, logits,
                (uint8_t*)q, s, (int)M, K, N, 0, eps};
-  const int64_t tiles = (M + kRouterRows - 1) / kRouterRows;
-  const int64_t workgroups = tiles * (N / 64);  // of 64 logits
-  const bool few = M < kRouterRows || workgroups <= Policy::kRouterFewRowsMax;
-  const bool narrow = !weight_fp32 && workgroups <= Policy::kRouterNarrowMax;
-  p.chunks = few ? N / 32 : weight_fp32 || narrow ? N / 64 : N / 128;
-  const dim3 grid((unsigned)((few ? M / kRouterFewRows : tiles) * p.chunks));
+  const RouterForm f = router_form(M, K, N, weight_fp32 != 0);
+  p.chunks = N / f.cols;
+  const dim3 grid((unsigned)((M + f.rows - 1) / f.rows * p.chunks));
+#define FQ_ROUTER_32(KINDV, ROUNDV, FP32V, VTV, WAVESV)                                                              \
+  hipLaunchKernelGGL((rmsnorm_router_quant_32_rows_kernel<KINDV, ROUNDV, FP32V, VTV, WAVESV>), grid,                 \
+                     dim3(64 * WAVESV), 0, stream, p)
 #define FQ_ROUTER_GO(KINDV, ROUNDV, FP32V)                                                                           \
-  if (few)                                                                                                           \
+  if (f.rows == 32) {                                                                                                \
+    if (f.cols == 128) FQ_ROUTER_32(KINDV, ROUNDV, FP32V, FP32V ? 2 : 1, 4);                                         \
+    else if (FP32V || f.cols == 512) FQ_ROUTER_32(KINDV, ROUNDV, FP32V, 2, 8);                                       \
+    else FQ_ROUTER_32(KINDV, ROUNDV, FP32V, FP32V ? 2 : 1, 8);                                                       \
+  } else if (f.rows == kRouterFewRows)                                                                                                  \
     hipLaunchKernelGGL((rmsnorm_router_quant_few_rows_kernel<KINDV, ROUNDV, FP32V>), grid, dim3(512), 0, stream, p); \
-  else if (!FP32V && narrow)                                                                                         \
+  else if (!FP32V && f.cols == 64)                                                                                     \
     hipLaunchKernelGGL((rmsnorm_router_quant_kernel<KINDV, ROUNDV, FP32V, FP32V ? 2 : 1>), grid, dim3(512), 0,       \
                        stream, p);                                                                                   \
   else                                                                                                               \
@@ -572,6 +770,7 @@ hipError_t launch_rmsnorm_router_quant_packed(const void* x, const void* gamma, 
 #undef FQ_ROUTER_WEIGHT
 #undef FQ_ROUTER_ROUND
 #undef FQ_ROUTER_GO
+#undef FQ_ROUTER_32
   return hipGetLastError();
 }
 

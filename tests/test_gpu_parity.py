@@ -557,13 +557,13 @@ def test_block_quant(gpu, M, N, round_scale):
     (8192, 256, 2048, torch.bfloat16), (256, 128, 1536, torch.bfloat16), (128, 512, 4096, torch.bfloat16),
     (384, 384, 7168, torch.bfloat16), (256, 128, 1024, torch.bfloat16), (128, 256, 1024, torch.bfloat16),
     (128, 128, 2048, torch.bfloat16),
-    # an fp32 router weight (what Megatron keeps), as two bf16 planes: register-resident (2N = 256) and streamed forms
+    # an fp32 router weight (what Megatron keeps), as two bf16 planes: workgroups of 64 rows x 64 logits, then of 16 x 32
     (8192, 256, 2048, torch.float32), (256, 128, 2048, torch.float32), (128, 128, 1024, torch.float32),
     (256, 256, 1536, torch.float32),
-    # more than 512 (virtual) columns: one launch per chunk of 512
+    # N that is no power of two, or beyond what a workgroup of any form takes: several column chunks share a row tile
     (256, 1024, 2048, torch.bfloat16), (128, 640, 1536, torch.bfloat16), (128, 384, 2048, torch.float32),
     (128, 1024, 1024, torch.float32),
-    # the widest router the entry point accepts: 16 launches (bf16) / 32 virtual-column chunks (fp32)
+    # the widest router the entry point accepts: more column chunks than k blocks
     (128, 8192, 256, torch.bfloat16), (128, 8192, 128, torch.float32)])
 @pytest.mark.parametrize("round_scale", [False, True])
 def test_rms_norm_fp32_gemm_block_quant(gpu, M, N, K, wdtype, round_scale):
@@ -616,19 +616,10 @@ def test_rms_norm_fp32_gemm_block_quant(gpu, M, N, K, wdtype, round_scale):
     check_quant_pair("router.col", pin[5], pin[6], qt, st, **EXACT)
 
 
-@pytest.mark.parametrize("M,N,K,wdtype", [
-    # 16-row workgroups: the fewest rows, one k block, the most workgroups of 64 x 64 that still take them (80)
-    (32, 128, 128, torch.bfloat16), (2560, 128, 384, torch.bfloat16), (1280, 256, 1152, torch.float32),
-    # 64 x 64: one more than that, the most that take it (256), a last row tile that is half a tile
-    (2624, 128, 640, torch.bfloat16), (8192, 128, 256, torch.bfloat16), (1312, 256, 128, torch.bfloat16),
-    # 64 x 128 and the fp32 form: k blocks of every remainder modulo the ring of four, half a row tile
-    (8224, 128, 128, torch.bfloat16), (8224, 128, 384, torch.bfloat16), (8256, 128, 640, torch.bfloat16),
-    (2144, 256, 256, torch.float32), (1312, 256, 1920, torch.float32), (2048, 384, 896, torch.float32)])
-def test_router_kernel_choice(gpu, M, N, K, wdtype):
-    """Every form of the router kernel at the edges of its range, rows in the 32s that the C interface takes."""
+def check_router(gpu, M, N, K, wdtype, dtype=E4M3, round_scale=False):
+    """One call through the C interface, which takes rows in 32s and both FP8 types, against the oracle."""
     from linghe_amd import _lib
 
-    announce("router kernel choice", M, N, K, wdtype)
     g = gen(25)
     x = (torch.randn(M, K, generator=g) ** 2).to(torch.bfloat16)
     nw = torch.randn(K, generator=g).to(torch.bfloat16)
@@ -639,27 +630,65 @@ def test_router_kernel_choice(gpu, M, N, K, wdtype):
     y = torch.full((M, K), 7.0, dtype=torch.bfloat16, device=gpu)
     rms = torch.full((M,), 7.0, device=gpu)
     logits = torch.full((M, N), 7.0, device=gpu)
-    q = torch.zeros((M, K), dtype=torch.float8_e4m3fn, device=gpu)
+    q = torch.zeros((M, K), dtype=dtype, device=gpu)
     s = torch.full((K // 128, M), 7.0, device=gpu)
     p = _lib.ptr
     _lib.check(_lib.lib.fq_rmsnorm_router_quant_fwd(p(xd), p(nwd), p(rwd), fp32, p(scratch), p(y), p(rms), p(logits),
-                                                    p(q), p(s), M, K, N, 1e-6, 0, _lib.FQ_E4M3, _lib.stream_of(xd)))
+                                                    p(q), p(s), M, K, N, 1e-6, int(round_scale), _lib.fp8_kind(dtype),
+                                                    _lib.stream_of(xd)))
     torch.cuda.synchronize()
-    pin = O.rms_gemm_block_quant_forward(x, nw, rw, rstd=rms.cpu())
     want = 1.0 / torch.sqrt((x.double() ** 2).mean(1) + 1e-6)
     assert float((rms.cpu().double() / want - 1).abs().max()) < 4 * 2.0 ** -23
+    pin = O.rms_gemm_block_quant_forward(x, nw, rw, rstd=rms.cpu())
     assert torch.equal(pin[0].view(torch.int16), y.cpu().view(torch.int16))
-    check_quant_pair("router.row", pin[3], pin[4], q, s, **EXACT)
+    ref = O.rms_norm_and_block_quant_forward(x, nw, round_scale=round_scale, fp8_dtype=dtype, rstd=rms.cpu())
+    check_quant_pair("router.row", ref[0], ref[1], q, s, **EXACT)
     # x * gamma enters exactly, an fp32 weight to 2^-17 of each |w|; fp32 accumulation below 2^-16 of sum |y||w|
     y32 = (x.float() * rms.cpu()[:, None]) * nw.float()
     err = (logits.cpu().double() - y32.double() @ rw.double().t()).abs()
     assert bool((err <= 2.0 ** -16 * (y32.abs().double() @ rw.double().abs().t())).all())
 
 
-# one call of each form of the router kernel: 16-row, 64 x 64, 64 x 128, fp32
-@pytest.mark.parametrize("M,N,K,wdtype", [(128, 128, 640, torch.bfloat16), (2688, 128, 256, torch.bfloat16),
-                                          (8320, 128, 384, torch.bfloat16), (2176, 256, 256, torch.float32),
-                                          (128, 256, 384, torch.float32)])
+@pytest.mark.parametrize("M,N,K,wdtype", [
+    # 16-row workgroups: the fewest rows, one k block, the most workgroups of 64 x 64 that still take them (80)
+    (32, 128, 128, torch.bfloat16), (2560, 128, 384, torch.bfloat16), (1280, 256, 1152, torch.float32),
+    # 64 x 64: one more than that, the most that take it (256), a last row tile that is half a tile
+    (2624, 128, 640, torch.bfloat16), (8192, 128, 256, torch.bfloat16), (1312, 256, 384, torch.bfloat16),
+    # 64 x 128 and the fp32 form: k blocks of every remainder modulo the ring of four, half a row tile
+    (8224, 128, 896, torch.bfloat16), (8224, 128, 1024, torch.bfloat16), (8288, 128, 1152, torch.bfloat16),
+    (4224, 256, 1280, torch.bfloat16),
+    (2144, 256, 256, torch.float32), (1312, 256, 1920, torch.float32), (2048, 384, 896, torch.float32),
+    # 32 rows x 128 logits, one, two and three column chunks; x 256 and x 512: k blocks of every remainder, an odd
+    # number of row tiles, fewer k blocks than chunks
+    (8224, 128, 128, torch.bfloat16), (8224, 128, 384, torch.bfloat16), (8256, 128, 640, torch.bfloat16),
+    (2720, 384, 128, torch.float32), (2720, 128, 256, torch.float32), (6176, 384, 896, torch.bfloat16),
+    (1312, 256, 128, torch.bfloat16), (4128, 256, 1024, torch.bfloat16), (4128, 256, 896, torch.float32),
+    (1376, 1024, 256, torch.float32), (3104, 512, 256, torch.bfloat16), (4128, 512, 640, torch.bfloat16),
+    (2080, 1024, 128, torch.bfloat16)])
+def test_router_kernel_choice(gpu, M, N, K, wdtype):
+    """Every form of the router kernel at the edges of its range."""
+    announce("router kernel choice", M, N, K, wdtype)
+    check_router(gpu, M, N, K, wdtype)
+
+
+# one call of each form and weight type
+@pytest.mark.parametrize("M,N,K,wdtype", [(96, 128, 256, torch.bfloat16), (96, 128, 256, torch.float32),
+                                          (2624, 128, 384, torch.bfloat16), (8224, 128, 896, torch.bfloat16),
+                                          (2144, 256, 384, torch.float32), (8224, 128, 256, torch.bfloat16),
+                                          (2720, 128, 256, torch.float32), (4128, 256, 256, torch.bfloat16),
+                                          (4128, 256, 256, torch.float32), (4128, 512, 256, torch.bfloat16)])
+@pytest.mark.parametrize("dtype,round_scale", [(E4M3, True), (E5M2, False), (E5M2, True)])
+def test_router_forms_fp8_types(gpu, M, N, K, wdtype, dtype, round_scale):
+    announce("router forms, types", M, N, K, wdtype, dtype, round_scale)
+    check_router(gpu, M, N, K, wdtype, dtype, round_scale)
+
+
+# one call of each form of the router kernel: 16-row, 64 x 64, 64 x 128, 64 x 64 fp32, 32 rows x 128, 256 and 512
+@pytest.mark.parametrize("M,N,K,wdtype", [(128, 128, 640, torch.bfloat16), (128, 256, 384, torch.float32),
+                                          (2688, 128, 256, torch.bfloat16), (8320, 128, 896, torch.bfloat16),
+                                          (2176, 256, 256, torch.float32), (8320, 128, 384, torch.bfloat16),
+                                          (2816, 128, 256, torch.float32), (4224, 256, 256, torch.bfloat16),
+                                          (4224, 256, 256, torch.float32), (4224, 512, 256, torch.bfloat16)])
 def test_router_rows_without_a_statistic(gpu, M, N, K, wdtype):
     """Rows whose squares overflow: the statistic is 0, hence y and, for finite values, the logits (zeros, not the NaN
     of overflowed products); an infinity makes the row's logits NaN.  Other rows do not notice."""
