@@ -721,6 +721,8 @@ static RouterForm router_form(int64_t M, int K, int N, bool weight_fp32) {
   } else {
     take32 = !narrow && (kblocks + 34) * rounds32 <= 40 * rounds64;
   }
+  // a launch has less than 2^32 work-items; the 32-row form needs half as many as the others or less
+  take32 |= tiles * (N / cols64) * 512 > (int64_t)UINT32_MAX;
   return take32 ? RouterForm{32, cols32} : RouterForm{kRouterRows, cols64};
 }
 
