@@ -535,7 +535,7 @@ def build_cases(names, dev):
 
     add("next_router", build=router_case)
     add("next_router_packed", build=lambda: router_case(True))
-    # a wide router: more than 512 logits run as one launch per 512 (virtual) columns, x re-read by each
+    # a wide router: the arithmetic, not the bytes, bounds it
     add("next_router_wide", build=lambda: router_case(False, (2048, 2048, 2048), "next_router_wide"))
 
     # ---------------------------------------------------------------- the per-expert tile plan of cfg3's counts

@@ -165,12 +165,15 @@ struct Policy {
 
   // ---- router kernels: hint on the stores of y and the codes
   static constexpr bool kStoreHintRouter = true;
-  // Which router kernel, by the number of workgroups of 64 rows x 64 logits the call has (us of the kernel
-  // alone at K = 2048, few-rows / 64-logit / 128-logit form).  Up to 80 of them, 256 CUs are mostly idle
-  // and the 16-row form spreads the rows further: 1024 x 256 14.8 / 20.0 / 27.2, 2048 x 256 25.5 / 21.0 / 28.0;
-  // fp32 weight: 1024 x 256 19.6 / 23.4, 2048 x 256 36.4 / 24.8.  As long as the 64-logit workgroups fit
-  // the chip at once they halve a workgroup's work: 4096 x 256 46.9 / 23.8 / 30.0, 8192 x 128 48.6 /
-  // 29.9 / 37.1; beyond, the 128-logit form turns x into operands half as often: 8192 x 256 88.7 / 42.2 / 36.3.
+  // Which router kernel, by the number of workgroups of 64 rows x 64 logits the call has; us of the kernel alone, few-rows
+  // / 64-logit / 128-logit form.  Up to 80 of them, 256 CUs are mostly idle and the 16-row form spreads the rows further,
+  // at every K alike: 1024 x 256 (64 of them) x 1024 7.7 / 11.9 / 16.4, x 2048 13.6 / 18.8 / 26.1, x 7168 33.0 / 52.8 /
+  // 74.4; 1536 x 256 (96) x 1024 10.6 / 12.0, x 2048 18.6 / 18.9, x 7168 48.0 / 53.6; 2048 x 256 (128) x 1024 13.2 / 12.3,
+  // x 2048 23.3 / 19.1, x 7168 61.7 / 55.0; fp32 weight (no 128-logit form): 64 of them x 2048 18.5 / 22.0, x 7168 48.6 /
+  // 62.9, 96 x 2048 26.2 / 22.1, x 7168 72.0 / 64.5.  As long as the 64-logit workgroups fit the chip at once they halve
+  // a workgroup's work: 4096 x 256 (256) x 1024 13.1 / 17.2 (64- / 128-logit), x 2048 21.0 / 27.2, x 7168 68.0 / 83.3;
+  // beyond, the 128-logit form turns x into operands half as often: 4224 x 256 (264) x 1024 23.1 / 17.2, x 2048
+  // 37.2 / 27.3, x 7168 114.9 / 81.9.
   static constexpr int kRouterFewRowsMax = 80;
   static constexpr int kRouterNarrowMax = 256;
   // The 32-row form against these two by rounds (workgroups over 256 CUs, and over what the CUs hold): one of its rounds

@@ -17,10 +17,12 @@
 // into the same accumulators.
 //
 // The kernels below share the work out over (row tile, column chunk) pairs; the workgroups of
-// one row tile sit on one XCD (router_tile), so that x comes from memory once and from that
-// XCD's L2 for the other chunks.  Each of them walks all of K for its columns of the logits,
+// one row tile sit on one XCD (router_tile), so that the chunks' walks over K read x from memory
+// once and else from that XCD's L2.  Each of them walks all of K for its columns of the logits,
 // accumulating the row statistic beside it, and then writes y, the codes and the scales for its
-// share of the K / 128 quantisation groups, re-reading that part of x from the L2.
+// share of the K / 128 quantisation groups, re-reading that part of x: from the L2 where the XCD's
+// row tiles and the weight still fit it (8192 x 256 x 2048 fetches 63.6 MB past the L2s where x and one weight per
+// XCD are 42).
 #include "fq_device.hpp"
 #include "fq_launch.h"
 #include "fq_policy.hpp"
@@ -207,9 +209,9 @@ __device__ __forceinline__ bf16x8_t operand(const uint4& v) { return __builtin_b
 // added up through LDS at the end.
 // Bound by instruction issue: per k block about 1000 clocks of matrix instructions and 900 of operand
 // arithmetic on each SIMD, partly on top of each other, and per block of the second part 1600 clocks of
-// normalising and quantising.  us of the kernel (32-row workgroups with all of W each before / now): 4096 x 256 x 4096
-// with an fp32 weight 84 / 53, 8192 x 256 x 2048 bf16 35.8 / 36.3, 4096 x 512 x 4096 bf16 84 / 51,
-// 16384 x 128 x 2048 bf16 62 / 51; with VT = 1 4096 x 256 x 2048 28.8 / 23.8.
+// normalising and quantising.  us of the kernel (former 32-row workgroups with all of W each / these): 4096 x 256 x 4096
+// with an fp32 weight 81 / 48, 8192 x 256 x 2048 bf16 34.3 / 34.3, 4096 x 512 x 4096 bf16 82 / 49,
+// 16384 x 128 x 2048 bf16 59 / 50; with VT = 1 4096 x 256 x 2048 27.3 / 21.1.
 // ---------------------------------------------------------------------------
 constexpr int kRouterRows = 64;
 
@@ -425,7 +427,9 @@ __global__ __launch_bounds__(512) void rmsnorm_router_quant_kernel(RouterArgs p)
 // one for the two planes of an fp32 weight) over all of K; nothing is exchanged at the end.
 // W operands come in sets of half a k block (whole blocks cost 165-175 registers instead of 127 with 256 logits, and the
 // second workgroup on a CU: 16384 x 256 x 1024 36.7 / 33.0 us). Three workgroups fit a CU with 128 logits, two with 256
-// of a bf16 weight, one otherwise.
+// of a bf16 weight, one otherwise. Bound by instruction issue like the kernel above, W read per 32 instead of 64 rows;
+// us of the 64-row form / this: 4224 x 512 x 1024 29.5 / 22.1, 16384 x 256 x 1024 40.0 / 33.5, fp32 4224 x 256 x 1024
+// 26.8 / 21.2.
 // ---------------------------------------------------------------------------
 template <int KIND, bool ROUND, bool FP32W, int VT, int WAVES>
 __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 3 : 2) void rmsnorm_router_quant_32_rows_kernel(RouterArgs p) {
@@ -567,7 +571,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 3 : 2) void rmsnorm_router
 // Few rows: 16 rows x 32 logits per workgroup.  Every wave takes whole k blocks of its own (block
 // number modulo 8) and makes the A operands in its registers, so there is neither an LDS round
 // trip nor a barrier in the walk over K; the eight partial results meet in LDS at the end.
-// Latency bound: 512 x 256 x 2048 24.9 -> 8.8 us, 512 x 256 x 7168 82 -> 19.5 (32-row workgroups before).
+// Latency bound: 512 x 256 x 2048 24.1 -> 8.2 us, 512 x 256 x 7168 82 -> 19.5 (32-row workgroups before).
 // ---------------------------------------------------------------------------
 constexpr int kRouterFewRows = 16;
 
