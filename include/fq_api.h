@@ -207,7 +207,8 @@ int64_t fq_rmsnorm_router_scratch_bytes(int64_t K, int64_t N, int weight_is_fp32
  * The product has fp32-GEMM accuracy: y, and an fp32 weight, enter the matrix
  * cores as two bf16 terms each (16 significant bits; the reference's tl.dot on
  * fp32 operands uses fewer).  weight_scratch: fq_rmsnorm_router_scratch_bytes()
- * bytes the call overwrites (the weight re-ordered for the matrix cores).
+ * bytes the call overwrites (the weight re-ordered for the matrix cores, an fp32
+ * one of the larger calls multiplied by gamma: fq_rmsnorm_router_folds).
  * (output_mode 1 of the reference is fq_rmsnorm_quant_fwd with output_mode 1.) */
 int fq_rmsnorm_router_quant_fwd(const void* x, const void* gamma, const void* route_weight, int weight_is_fp32,
                                 void* weight_scratch, void* y, float* rstd, float* logits, void* q, float* s,
@@ -220,13 +221,19 @@ int fq_rmsnorm_router_quant_fwd(const void* x, const void* gamma, const void* ro
  * fq_pack_router_weight re-orders route_weight [N,K] (bf16, or fp32 split into two bf16
  * planes) into `packed` (fq_rmsnorm_router_scratch_bytes() bytes);
  * fq_rmsnorm_router_quant_fwd_packed is fq_rmsnorm_router_quant_fwd on that buffer, with the
- * weight_is_fp32 it was packed with.  Results are bit-identical to the one-call form. */
+ * weight_is_fp32 it was packed with.  Results are bit-identical to the one-call form, but for the
+ * logits of the calls for which fq_rmsnorm_router_folds() is 1: there the one-call form takes the two
+ * terms of gamma * route_weight, this one those of route_weight (same accuracy, and the one-call
+ * form is the faster one). */
 int fq_pack_router_weight(const void* route_weight, int weight_is_fp32, void* packed, int64_t K, int64_t N,
                           void* stream);
 int fq_rmsnorm_router_quant_fwd_packed(const void* x, const void* gamma, const void* packed_weight,
                                        int weight_is_fp32, void* y, float* rstd, float* logits, void* q, float* s,
                                        int64_t M, int64_t K, int64_t N, float eps, int round_scale, int fp8_kind,
                                        void* stream);
+
+/* 1 where fq_rmsnorm_router_quant_fwd folds gamma into the weight, else 0 */
+int fq_rmsnorm_router_folds(int64_t M, int64_t K, int64_t N, int weight_is_fp32);
 
 /* triton_silu_and_block_quant_forward, linghe/utils/silu.py:279-335.
  * x bf16 [M, 2n] (gate | up).  Outputs as fq_blockwise_quant with N = n. */

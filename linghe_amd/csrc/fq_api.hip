@@ -429,6 +429,10 @@ int fq_rmsnorm_router_quant_fwd(const void* x, const void* gamma, const void* ro
                       fn);
 }
 
+int fq_rmsnorm_router_folds(int64_t M, int64_t K, int64_t N, int weight_is_fp32) {
+  return weight_is_fp32 && fq::router_folds(M, (int)K, (int)N);
+}
+
 int fq_pack_router_weight(const void* route_weight, int weight_is_fp32, void* packed, int64_t K, int64_t N,
                           void* stream) {
   const char* fn = "fq_pack_router_weight";

@@ -94,6 +94,9 @@ hipError_t launch_rmsnorm_router_quant(const void* x, const void* gamma, const v
                                        int64_t M, int K, int N, float eps, int round_scale, int kind,
                                        hipStream_t stream);
 
+// whether that call, with an fp32 weight, multiplies the weight by gamma instead of re-ordering it
+bool router_folds(int64_t M, int K, int N);
+
 // the two halves of launch_rmsnorm_router_quant: re-order the weight (once per weight update),
 // run on the re-ordered weight
 hipError_t launch_pack_router_weight(const void* wr, int weight_fp32, void* wpacked, int K, int N, hipStream_t stream);

@@ -679,6 +679,276 @@ __global__ __launch_bounds__(512) void rmsnorm_router_quant_few_rows_kernel(Rout
   }
 }
 
+// ---------------------------------------------------------------------------
+// An fp32 weight with gamma folded into it:
+//   logits[m, :] = r[m] * sum_k x[m, k] * (gamma[k] * W[:, k])
+// x is an operand as it lies in memory, so the two planes of gamma * W take two products instead of the four of
+// (x * gamma) and W, and no operand arithmetic. What the planes leave of gamma * W is what those of W left of W (below
+// 2^-17 of its size): the logits' error against 64 bits, over 70 inputs of K = 1024 .. 7168, 0.99 of the other form's
+// (2.40-2.51e-6 of the logits' norm against 2.46-2.50). The folding is done on every call, in the place of the re-ordering:
+// it depends on gamma, which a weight re-ordered ahead of the calls does not know.
+//
+// The planes lie as the kernel below reads them: per slab of 64 columns and 32-column tile four k steps of hi, then lo,
+// 64 lanes of 8 columns (16 ks + 8 (lane / 32) .. of row lane % 32). 16 rows of a 128-column block per workgroup, as in
+// the packing kernel.
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void fold_router_weight_kernel(const float* __restrict__ wr,
+                                                                 const uint16_t* __restrict__ gamma,
+                                                                 uint4* __restrict__ folded, int K, int n_halves) {
+  const int kb = wg_x() / n_halves;
+  const int n = (wg_x() - kb * n_halves) * 16 + (tid_x() >> 4);  // row of W
+  const int c = tid_x() & 15;                                    // piece of its 128 columns
+  const float4* src = (const float4*)(wr + (int64_t)n * K + kb * kGroup + c * 8);
+  const float4 a = src[0], b = src[1];
+  float w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w}, g[8], back[8], lo[8];
+  unpack8(*(const uint4*)(gamma + kb * kGroup + c * 8), g);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) w[i] *= g[i];
+  const uint4 hi = pack8_bf16(w);
+  unpack8(hi, back);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) lo[i] = w[i] - back[i];
+  const int slab = kb * 2 + (c >> 3), ks = (c >> 1) & 3;
+  uint4* dst = folded + (((int64_t)slab * (n_halves >> 1) + (n >> 5)) * 4 + ks) * 128 + (c & 1) * 32 + (n & 31);
+  dst[0] = hi;
+  dst[64] = pack8_bf16(lo);
+}
+
+typedef __attribute__((address_space(3))) void lds_void_t;
+
+// 64 rows of a slab of 64 columns from memory into LDS, eight rows an instruction; at: this lane's byte offset in the
+// first and the second eight of 16 rows. With valid = 0 (else K) nothing is read and zeros arrive.
+__device__ __forceinline__ void router_fetch_slab(const uint16_t* x, int valid, int K, int slab, const uint32_t (&at)[2],
+                                                  uint4* slot) {
+  const __amdgpu_buffer_rsrc_t from =
+      __builtin_amdgcn_make_buffer_rsrc((void*)x, 0, kRouterRows * valid * 2, 0x00027000);
+#pragma unroll
+  for (int i = 0; i < kRouterRows / 8; ++i)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (lds_void_t*)(slot + i * 64), 16, at[i & 1],
+                                             slab * 128 + (i >> 1) * 32 * K, 0, 0);
+}
+
+// 64 rows x 64 logits per workgroup of eight waves in two roles. Four multiply, each over every fourth slab of 64 columns
+// for all of the logits, x asked for four slabs ahead and straight into LDS, W one slab ahead into registers; they share
+// nothing until their sums meet at the end, so there is no barrier in the walk over K. The other four normalise and
+// quantise the workgroup's share of the tile's rows meanwhile, so that y and the codes leave while the matrix cores work.
+// Bound by what a CU can load: 1.5 MB at K = 4096 (W 1.0, x 0.5), which takes 20 us by itself (about 75 KB a us and CU;
+// 16 us with x in the L2), beside 15 us of the rows' reads and writes through the same path. Twice the slabs in flight or
+// eight multiplying waves change nothing, 128 x 64 logits leave half of the CUs idle at 4096 rows.
+// us of a call (64- or 32-row form, weight re-ordered / this, weight folded): 4096 x 256 x 4096 51.7 / 37.8,
+// 2048 x 256 x 7168 69.3 / 55.4, 8192 x 256 x 2048 54.8 / 39.8, 4224 x 512 x 1024 41.1 / 27.6, 8192 x 128 x 2048
+// 36.6 / 29.8.
+// ---------------------------------------------------------------------------
+template <int KIND, bool ROUND>
+__global__ __launch_bounds__(512) void rmsnorm_router_quant_folded_kernel(RouterArgs p) {
+  // slabs of x of each multiplying wave, a row's eight pieces XORed with half its number so that reads meet all banks;
+  // afterwards the partial sums of the first and the second 32 rows. Four arrays: the compiler tells the loads into one
+  // from those into another, and a read waits for its own slab only.
+  __shared__ uint4 a0[4][kRouterRows * 8];
+  __shared__ uint4 a1[4][kRouterRows * 8];
+  __shared__ uint4 a2[4][kRouterRows * 8];
+  __shared__ uint4 a3[4][kRouterRows * 8];
+  __shared__ double sq[4][2][kRouterRows];  // squares of a row: by wave and by half of its lanes
+  __shared__ unsigned sfactor[kRouterRows];
+  const int lane = tid_x() & 63;
+  const int wave = uniform32(tid_x() >> 6);
+  const int kblocks = p.K / kGroup;
+  int tile, chunk;
+  router_tile((p.M + kRouterRows - 1) / kRouterRows, p.chunks, tile, chunk);
+  const int row0 = min(tile * kRouterRows, p.M - kRouterRows);
+  const int r = lane & 31, h = lane >> 5;
+
+  if (wave < 4) {
+    // ---- 64 rows x 64 logits over slabs wave, wave + 4, ..
+    const int slabs = kblocks * 2;
+    const int stages = (slabs - wave + 3) >> 2;
+    floatx16_t acc[2][2];
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[rt][t][v] = 0.f;
+    double ss[2] = {0.0, 0.0};
+    if (stages > 0) {
+      const uint4* w = p.w + (int64_t)chunk * 1024;
+      const uint16_t* x = p.x + (int64_t)row0 * p.K;
+      auto slab_of = [&](int s) { return min(wave + 4 * s, slabs - 1); };
+      uint32_t at[2];  // rows 8 i + lane / 8 of 16, in bytes
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int row = 8 * i + (lane >> 3);
+        at[i] = (uint32_t)(row * p.K + (((lane & 7) ^ ((row >> 1) & 7)) * 8)) * 2u;
+      }
+      auto fetch_x = [&](int s, uint4* slot) {
+        router_fetch_slab(x, s < stages ? p.K : 0, p.K, slab_of(s), at, slot);
+      };
+      uint4 b[4][4];  // [k step][tile 0 hi, lo, tile 1 hi, lo]: a set is refilled in place once it was used
+      auto fetch_w = [&](int s, int ks, uint4 (&d)[4]) {
+        const uint4* from = w + ((int64_t)slab_of(s) * (p.N / 32) * 8 + ks * 2) * 64;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) d[t] = from[((t >> 1) * 8 + (t & 1)) * 64 + lane];
+      };
+      fetch_x(0, a0[wave]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_w(0, i, b[i]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      fetch_x(1, a1[wave]);
+      fetch_x(2, a2[wave]);
+      fetch_x(3, a3[wave]);
+      auto load = [&](const uint4* slot, int ks, int rt) {
+        uint32_t lane_at = (uint32_t)(r * 128 + (h ^ ((r >> 1) & 7)) * 16);
+        asm volatile("" : "+v"(lane_at));  // (one register, not one per slot, k step and row tile)
+        return *(const uint4*)((const char*)slot + rt * 4096 + (lane_at ^ (ks * 32)));
+      };
+      uint4 af[2][2];
+      // (the order of loads and products is laid out step by step: the waits count the loads behind the one they are for)
+      auto stage = [&](int s, const uint4* slot, const uint4* next) {
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+#pragma unroll
+          for (int rt = 0; rt < 2; ++rt) af[(ks + 1) & 1][rt] = load(ks < 3 ? slot : next, (ks + 1) & 3, rt);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int rt = 0; rt < 2; ++rt) {
+            const uint4 a = af[ks & 1][rt];
+            ss[rt] += (double)sumsq8(a);
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+              acc[rt][t >> 1] =
+                  __builtin_amdgcn_mfma_f32_32x32x16_bf16(operand(a), operand(b[ks][t]), acc[rt][t >> 1], 0, 0, 0);
+          }
+          fetch_w(s + 1, ks, b[ks]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      };
+#pragma unroll
+      for (int rt = 0; rt < 2; ++rt) af[0][rt] = load(a0[wave], 0, rt);
+      int s = 0;
+#pragma unroll 1
+      for (; s + 3 < stages; s += 4) {
+        stage(s, a0[wave], a1[wave]);
+        fetch_x(s + 4, a0[wave]);
+        __builtin_amdgcn_sched_barrier(0);
+        stage(s + 1, a1[wave], a2[wave]);
+        fetch_x(s + 5, a1[wave]);
+        __builtin_amdgcn_sched_barrier(0);
+        stage(s + 2, a2[wave], a3[wave]);
+        fetch_x(s + 6, a2[wave]);
+        __builtin_amdgcn_sched_barrier(0);
+        stage(s + 3, a3[wave], a0[wave]);
+        fetch_x(s + 7, a3[wave]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (s < stages) stage(s, a0[wave], a1[wave]);
+      if (s + 1 < stages) stage(s + 1, a1[wave], a2[wave]);
+      if (s + 2 < stages) stage(s + 2, a2[wave], a3[wave]);
+      __builtin_amdgcn_s_waitcnt(0);
+    }
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) {
+      sq[wave][h][rt * 32 + r] = ss[rt];
+      floatx4_t* part = (floatx4_t*)(rt == 0 ? a0[wave] : a1[wave]);
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          part[(t * 4 + i) * 64 + lane] =
+              floatx4_t{acc[rt][t][4 * i], acc[rt][t][4 * i + 1], acc[rt][t][4 * i + 2], acc[rt][t][4 * i + 3]};
+    }
+  } else {
+    // ---- statistic, y and codes of this workgroup's share of the tile's rows: four at a time, 16 lanes each
+    constexpr int kHeld = 16, kStep = 4;  // k blocks of a row in registers, worked on together; beyond the last: it again
+    const int cg = lane & 15;
+    const int last = (kblocks - 1) / kHeld;
+#pragma unroll 1
+    for (int batch = chunk * 4 + wave - 4; batch < kRouterRows / 4; batch += p.chunks * 4) {
+      const int row = row0 + batch * 4 + (lane >> 4);
+      const uint16_t* x = p.x + (int64_t)row * p.K + cg * 8;
+      const uint16_t* gamma = p.gamma + cg * 8;
+      uint4 xe[kHeld], ge[2][kStep];
+      auto fetch = [&](int k0) {
+#pragma unroll
+        for (int d = 0; d < kHeld; ++d) xe[d] = *(const uint4*)(x + min(k0 + d, kblocks - 1) * kGroup);
+      };
+      auto fetch_gamma = [&](int k0, uint4 (&g)[kStep]) {
+#pragma unroll
+        for (int d = 0; d < kStep; ++d) g[d] = *(const uint4*)(gamma + min(k0 + d, kblocks - 1) * kGroup);
+      };
+      double ss = 0.0;
+#pragma unroll 1
+      for (int set = 0; set <= last; ++set) {
+        fetch(set * kHeld);
+#pragma unroll
+        for (int d = 0; d < kHeld; ++d) ss += set * kHeld + d < kblocks ? (double)sumsq8(xe[d]) : 0.0;
+      }
+      fetch_gamma(last * kHeld, ge[0]);
+      const float rs = 1.0f / sqrtf((float)row16_sum_d(ss) / (float)p.K + p.eps);
+      if (cg == 0) p.rstd[row] = rs;
+      // the last set, which is in registers, first
+#pragma unroll 1
+      for (int i = 0; i <= last; ++i) {
+        const int k0 = (i == 0 ? last : i - 1) * kHeld;
+        if (i > 0) {
+          fetch(k0);
+          fetch_gamma(k0, ge[0]);
+        }
+#pragma unroll
+        for (int g = 0; g < kHeld / kStep; ++g) {
+          if (k0 + g * kStep < kblocks) {
+            fetch_gamma(k0 + (g + 1) * kStep, ge[(g + 1) & 1]);
+#pragma unroll
+            for (int d = 0; d < kStep; ++d) {
+              const int kb = min(k0 + g * kStep + d, kblocks - 1);
+              const int64_t at = (int64_t)row * p.K + kb * kGroup + cg * 8;
+              router_emit<KIND, ROUND>(p.y + at, p.q + at, p.s + (int64_t)kb * p.M + row, cg == 0, xe[g * kStep + d],
+                                       ge[g & 1][d], rs);
+            }
+          }
+        }
+      }
+    }
+  }
+  __syncthreads();
+
+  // ---- eight lanes a row: its factor
+  {
+    const int row = tid_x() >> 3, part = tid_x() & 7;
+    double total = 0.0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) total += sq[i >> 1][i & 1][row];
+    unsigned factor = __float_as_uint(1.0f / sqrtf((float)total / (float)p.K + p.eps));
+    bool bad = false;
+    if (factor == 0) {
+#pragma unroll 1
+      for (int c = part * 8; c < p.K; c += 64)
+        bad |= router_nonfinite(*(const uint4*)(p.x + (int64_t)(row0 + row) * p.K + c)) ||
+               router_nonfinite(*(const uint4*)(p.gamma + c));
+    }
+    if ((__ballot(bad) >> (lane & 56)) & 0xff) factor = kNanBits;
+    if (part == 0) sfactor[row] = factor;
+  }
+  __syncthreads();
+  const floatx4_t* sums = (const floatx4_t*)(wave < 4 ? &a0[0][0] : &a1[0][0]);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int set = (wave & 3) * 2 + i;  // of eight sets of four rows and 32 columns
+    floatx4_t v = sums[set * 64 + lane];
+#pragma unroll
+    for (int k = 1; k < 4; ++k) v += sums[k * (kRouterRows * 8) + set * 64 + lane];
+    // register e of a 32x32 result holds row (e / 4) * 8 + (lane / 32) * 4 + e % 4, column lane % 32
+    const int row = (wave >> 2) * 32 + (set & 3) * 8 + h * 4;
+    const int col = (chunk * 2 + (set >> 2)) * 32 + r;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      p.logits[(int64_t)(row0 + row + e) * p.N + col] = router_logit(v[e], sfactor[row + e]);
+  }
+}
+
+
 int64_t rmsnorm_router_scratch_bytes(int K, int N, int weight_fp32) {
   return (int64_t)N * K * (weight_fp32 ? 4 : 2);  // the bf16 planes of W in operand order
 }
@@ -728,6 +998,22 @@ static RouterForm router_form(int64_t M, int K, int N, bool weight_fp32) {
   // a launch has less than 2^32 work-items; the 32-row form needs half as many as the others or less
   take32 |= tiles * (N / cols64) * 512 > (int64_t)UINT32_MAX;
   return take32 ? RouterForm{32, cols32} : RouterForm{kRouterRows, cols64};
+}
+
+// An fp32 weight: whether a call folds gamma into it. us of a call re-ordered / folded, number of 64 x 64 workgroups behind
+// the size. Fewer than the few-rows form takes, or half of them: 512 x 256 x 2048 (32) 15.0 / 18.1, 512 x 384 x 2048 (48)
+// 24.0 / 19.5, x 7168 55.7 / 51.0, 1024 x 256 x 1536 (64) 18.3 / 15.4, x 1024 14.1 / 12.7, of which the re-ordering, that a caller
+// may have done ahead, is 2.3. Short K: in one round 4096 x 256 (256) x 384 12.1 / 10.1, x 256 10.9 / 9.6, 4096 x 128 x 384 12.2 / 11.1,
+// x 256 10.5 / 10.9; in more 8192 x 256 (512) x 896 26.5 / 23.7, x 640 20.7 / 20.3, x 384 15.0 / 15.8, 16384 x 256 x 768 44.2 / 41.3,
+// 8192 x 512 x 640 35.8 / 36.9. With 128 logits a workgroup has 32 rows to quantise, its longer part at long K: 8192 x 128
+// (256) x 2048 36.6 / 29.8, x 3072 48.3 / 43.8, 4096 x 128 x 4096 50.2 / 52.6, 6144 x 128 x 5120 68.0 / 72.1.
+bool router_folds(int64_t M, int K, int N) {
+  const int64_t workgroups = (M + kRouterRows - 1) / kRouterRows * (N / 64);
+  if (M < kRouterRows || workgroups * 512 > (int64_t)UINT32_MAX) return false;
+  if (N == 128 && K > 3072) return false;
+  if (workgroups <= Policy::kRouterFewRowsMax)
+    return N > 128 && K >= 1536 && workgroups > Policy::kRouterFewRowsMax / 2;
+  return K >= (workgroups <= 256 ? 384 : 896);
 }
 
 // the main kernels on a weight already in operand order
@@ -785,6 +1071,27 @@ hipError_t launch_rmsnorm_router_quant(const void* x, const void* gamma, const v
                                        int64_t M, int K, int N, float eps, int round_scale, int kind,
                                        hipStream_t stream) {
   if (M == 0) return hipSuccess;
+  if (weight_fp32 && router_folds(M, K, N)) {
+    const int n_halves = N / 16;
+    hipLaunchKernelGGL(fold_router_weight_kernel, dim3((unsigned)((int64_t)n_halves * (K / kGroup))), dim3(256), 0, stream,
+                       (const float*)wr, (const uint16_t*)gamma, (uint4*)wpacked, K, n_halves);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    const RouterArgs p{(const uint16_t*)x, (const uint16_t*)gamma, (const uint4*)wpacked, (uint16_t*)y, rstd, logits,
+                       (uint8_t*)q, s, (int)M, K, N, N / 64, eps};
+    const dim3 grid((unsigned)((M + kRouterRows - 1) / kRouterRows * p.chunks));
+#define FQ_ROUTER_FOLDED(KINDV, ROUNDV) \
+  hipLaunchKernelGGL((rmsnorm_router_quant_folded_kernel<KINDV, ROUNDV>), grid, dim3(512), 0, stream, p)
+    if (kind == kE5M2) {
+      if (round_scale) FQ_ROUTER_FOLDED(kE5M2, true);
+      else FQ_ROUTER_FOLDED(kE5M2, false);
+    } else {
+      if (round_scale) FQ_ROUTER_FOLDED(kE4M3, true);
+      else FQ_ROUTER_FOLDED(kE4M3, false);
+    }
+#undef FQ_ROUTER_FOLDED
+    return hipGetLastError();
+  }
   const hipError_t e = launch_pack_router_weight(wr, weight_fp32, wpacked, K, N, stream);
   if (e != hipSuccess) return e;
   return launch_rmsnorm_router_quant_packed(x, gamma, wpacked, weight_fp32, y, rstd, logits, q, s, M, K, N, eps,

@@ -184,7 +184,9 @@ def triton_rms_norm_fp32_gemm_block_quant_forward(
         packed_route_weight: (keyword-only addition) the result of pack_route_weight(route_weight).
             The kernels read the router weight in matrix-core operand order; without this
             argument it is re-ordered on every call, with it the caller re-orders once per
-            weight update.  Results are identical.
+            weight update.  Results are identical.  (The larger calls with an fp32 weight read
+            route_weight itself: with norm_weight folded into it they are faster than on the
+            packed one.)
 
     Returns:
         - y: rms normed tensor
@@ -227,12 +229,15 @@ def triton_rms_norm_fp32_gemm_block_quant_forward(
             if packed_route_weight is not None:
                 assert packed_route_weight.is_cuda and packed_route_weight.dtype == torch.uint8
                 assert packed_route_weight.numel() == need and packed_route_weight.is_contiguous()
+            if packed_route_weight is not None and (route_weight.data_ptr() % 16 or
+                                                    not _lib.lib.fq_rmsnorm_router_folds(M, K, N, w_fp32)):
                 _lib.check(_lib.lib.fq_rmsnorm_router_quant_fwd_packed(
                     _lib.ptr(x), _lib.ptr(norm_weight), _lib.ptr(packed_route_weight), w_fp32, _lib.ptr(y),
                     _lib.ptr(rms), _lib.ptr(logits), _lib.ptr(x_q), _lib.ptr(x_s), M, K, N, float(eps),
                     int(bool(round_scale)), _lib.FQ_E4M3, _lib.stream_of(x)))
             else:
-                # route_weight re-ordered for the matrix cores (an fp32 weight as two bf16 planes)
+                # route_weight re-ordered for the matrix cores (an fp32 weight as two bf16 planes, in the larger calls
+                # of gamma * route_weight, which depends on both and is made by every call)
                 scratch = torch.empty(need, dtype=torch.uint8, device=device)
                 _lib.check(_lib.lib.fq_rmsnorm_router_quant_fwd(
                     _lib.ptr(x), _lib.ptr(norm_weight), _lib.ptr(route_weight), w_fp32, _lib.ptr(scratch),

@@ -616,7 +616,7 @@ def test_rms_norm_fp32_gemm_block_quant(gpu, M, N, K, wdtype, round_scale):
     check_quant_pair("router.col", pin[5], pin[6], qt, st, **EXACT)
 
 
-def check_router(gpu, M, N, K, wdtype, dtype=E4M3, round_scale=False):
+def check_router(gpu, M, N, K, wdtype, dtype=E4M3, round_scale=False, packed=False):
     """One call through the C interface, which takes rows in 32s and both FP8 types, against the oracle."""
     from linghe_amd import _lib
 
@@ -633,9 +633,12 @@ def check_router(gpu, M, N, K, wdtype, dtype=E4M3, round_scale=False):
     q = torch.zeros((M, K), dtype=dtype, device=gpu)
     s = torch.full((K // 128, M), 7.0, device=gpu)
     p = _lib.ptr
-    _lib.check(_lib.lib.fq_rmsnorm_router_quant_fwd(p(xd), p(nwd), p(rwd), fp32, p(scratch), p(y), p(rms), p(logits),
-                                                    p(q), p(s), M, K, N, 1e-6, int(round_scale), _lib.fp8_kind(dtype),
-                                                    _lib.stream_of(xd)))
+    rest = (p(y), p(rms), p(logits), p(q), p(s), M, K, N, 1e-6, int(round_scale), _lib.fp8_kind(dtype), _lib.stream_of(xd))
+    if packed:
+        _lib.check(_lib.lib.fq_pack_router_weight(p(rwd), fp32, p(scratch), K, N, _lib.stream_of(xd)))
+        _lib.check(_lib.lib.fq_rmsnorm_router_quant_fwd_packed(p(xd), p(nwd), p(scratch), fp32, *rest))
+    else:
+        _lib.check(_lib.lib.fq_rmsnorm_router_quant_fwd(p(xd), p(nwd), p(rwd), fp32, p(scratch), *rest))
     torch.cuda.synchronize()
     want = 1.0 / torch.sqrt((x.double() ** 2).mean(1) + 1e-6)
     assert float((rms.cpu().double() / want - 1).abs().max()) < 4 * 2.0 ** -23
@@ -669,6 +672,24 @@ def test_router_kernel_choice(gpu, M, N, K, wdtype):
     """Every form of the router kernel at the edges of its range."""
     announce("router kernel choice", M, N, K, wdtype)
     check_router(gpu, M, N, K, wdtype)
+
+
+@pytest.mark.parametrize("M,N,K,dtype,round_scale", [
+    # slabs of 64 columns: one or two for each of the four waves, and every remainder modulo the four in flight
+    (2656, 128, 384, E4M3, True), (2624, 128, 512, E4M3, False), (2624, 128, 1024, E5M2, False),
+    (2688, 128, 1152, E4M3, False), (2656, 128, 1280, E4M3, False), (2624, 128, 1792, E4M3, False),
+    # the fewest workgroups, a last row tile that is half a tile, rows of more k blocks than are held, the widest
+    (704, 256, 1536, E4M3, False), (736, 256, 2176, E5M2, True), (672, 256, 8192, E4M3, False),
+    (1120, 384, 4224, E4M3, True), (64, 8192, 384, E4M3, False)])
+def test_router_folded_weight(gpu, M, N, K, dtype, round_scale):
+    """An fp32 weight with gamma folded into it (the error bound is that of the re-ordered one: the two terms leave
+    below 2^-17 of each |gamma * w|), and the same sizes on a weight packed ahead."""
+    from linghe_amd import _lib
+
+    announce("router, folded weight", M, N, K, dtype, round_scale)
+    assert _lib.lib.fq_rmsnorm_router_folds(M, K, N, 1) == 1 and _lib.lib.fq_rmsnorm_router_folds(M, K, N, 0) == 0
+    check_router(gpu, M, N, K, torch.float32, dtype, round_scale)
+    check_router(gpu, M, N, K, torch.float32, dtype, round_scale, packed=True)
 
 
 # one call of each form and weight type
