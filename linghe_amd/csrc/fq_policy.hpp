@@ -187,6 +187,18 @@ struct Policy {
   // k blocks up to which it is ahead in one round of either (4096 x 512 x 128 8.9 / 7.4, x 256 10.0 / 9.6, x 512
   // 12.2 / 13.7; 4096 x 256 x 256 7.7 / 7.4, x 512 9.2 / 9.9)
   static constexpr int kRouter32ShortK = 2;
+  // From this K on the 64-row x 128-logit form of a bf16 weight has its waves in two roles where the logits are whole 256s (N = 128:
+  // 64 rows for four waves to quantise). us 64-row form / two roles: 8192 x 256 x 1024 18.7 / 19.0, x 1280 23.6 / 23.7, x 1536
+  // 26.9 / 25.5, x 2048 34.3 / 32.0, 4224 x 256 x 1280 19.5 / 19.3, x 1536 21.9 / 19.8, x 3072 37.3 / 37.0, 8192 x 512 x 4096
+  // 94.5 / 84.6, 8320 x 128 x 2048 35.8 / 37.5, 4096 x 384 x 3072 35.2 / 38.6, x 4096 48.5 / 47.6. K blocks that do not come
+  // out even over the four multiplying waves, and rows of a few more than the 16 that are held, are carried by 512 logits and
+  // more only: 6144 x 256 x 1664 25.1 / 27.1, x 2176 30.7 / 33.7, 4224 x 256 x 4224 51.4 / 53.2, 8192 x 512 x 2176 60.4 / 57.4, 4224 x
+  // 512 x 3200 70.3 / 62.3.
+  static constexpr int kRouterTwoRolesMinK = 1536;
+  // ... and from this K on it is ahead of the 32-row form too: 16384 x 256 x 1536 45.3 / 48.1 (32-row / two roles), x 2048
+  // 65.4 / 60.2, x 3072 83.8 / 80.5, 8320 x 512 x 1536 60.7 / 50.4, x 2048 73.7 / 63.5, 8192 x 1024 x 1536 65.0 / 70.5, x 2048
+  // 96.6 / 89.2.
+  static constexpr int kRouterTwoRolesAlwaysK = 2048;
 };
 
 }  // namespace fq

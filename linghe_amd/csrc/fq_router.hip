@@ -679,6 +679,248 @@ __global__ __launch_bounds__(512) void rmsnorm_router_quant_few_rows_kernel(Rout
   }
 }
 
+// The role of a wave that multiplies nothing: statistic, y, codes and scales of the tile's rows 4 batch .. 4 batch + 3,
+// then of batch + step and so on, 16 lanes a row.
+template <int KIND, bool ROUND>
+__device__ __forceinline__ void router_rows(const RouterArgs& p, int row0, int batch, int step) {
+  constexpr int kHeld = 16, kStep = 4;  // k blocks of a row in registers, worked on together; beyond the last: it again
+  const int lane = tid_x() & 63, cg = lane & 15, kblocks = p.K / kGroup;
+  const int last = (kblocks - 1) / kHeld;
+#pragma unroll 1
+  for (; batch < kRouterRows / 4; batch += step) {
+    const int row = row0 + batch * 4 + (lane >> 4);
+    const uint16_t* x = p.x + (int64_t)row * p.K + cg * 8;
+    const uint16_t* gamma = p.gamma + cg * 8;
+    uint4 xe[kHeld], ge[2][kStep];
+    auto fetch = [&](int k0) {
+#pragma unroll
+      for (int d = 0; d < kHeld; ++d) xe[d] = *(const uint4*)(x + min(k0 + d, kblocks - 1) * kGroup);
+    };
+    auto fetch_gamma = [&](int k0, uint4 (&g)[kStep]) {
+#pragma unroll
+      for (int d = 0; d < kStep; ++d) g[d] = *(const uint4*)(gamma + min(k0 + d, kblocks - 1) * kGroup);
+    };
+    double ss = 0.0;
+#pragma unroll 1
+    for (int set = 0; set <= last; ++set) {
+      fetch(set * kHeld);
+#pragma unroll
+      for (int d = 0; d < kHeld; ++d) ss += set * kHeld + d < kblocks ? (double)sumsq8(xe[d]) : 0.0;
+    }
+    fetch_gamma(last * kHeld, ge[0]);
+    const float rs = 1.0f / sqrtf((float)row16_sum_d(ss) / (float)p.K + p.eps);
+    if (cg == 0) p.rstd[row] = rs;
+    // the last set, which is in registers, first
+#pragma unroll 1
+    for (int i = 0; i <= last; ++i) {
+      const int k0 = (i == 0 ? last : i - 1) * kHeld;
+      if (i > 0) {
+        fetch(k0);
+        fetch_gamma(k0, ge[0]);
+      }
+#pragma unroll
+      for (int g = 0; g < kHeld / kStep; ++g) {
+        if (k0 + g * kStep < kblocks) {
+          fetch_gamma(k0 + (g + 1) * kStep, ge[(g + 1) & 1]);
+#pragma unroll
+          for (int d = 0; d < kStep; ++d) {
+            const int kb = min(k0 + g * kStep + d, kblocks - 1);
+            const int64_t at = (int64_t)row * p.K + kb * kGroup + cg * 8;
+            router_emit<KIND, ROUND>(p.y + at, p.q + at, p.s + (int64_t)kb * p.M + row, cg == 0, xe[g * kStep + d],
+                                     ge[g & 1][d], rs);
+          }
+        }
+      }
+    }
+  }
+}
+
+// the factors of a tile's rows from the squares that four waves saw of them, eight lanes a row
+__device__ __forceinline__ void router_factors(const RouterArgs& p, int row0, const double (&sq)[4][2][kRouterRows],
+                                               unsigned (&sfactor)[kRouterRows]) {
+  const int lane = tid_x() & 63, row = tid_x() >> 3, part = tid_x() & 7;
+  double total = 0.0;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) total += sq[i >> 1][i & 1][row];
+  unsigned factor = __float_as_uint(1.0f / sqrtf((float)total / (float)p.K + p.eps));
+  bool bad = false;
+  if (factor == 0) {
+#pragma unroll 1
+    for (int c = part * 8; c < p.K; c += 64)
+      bad |= router_nonfinite(*(const uint4*)(p.x + (int64_t)(row0 + row) * p.K + c)) ||
+             router_nonfinite(*(const uint4*)(p.gamma + c));
+  }
+  if ((__ballot(bad) >> (lane & 56)) & 0xff) factor = kNanBits;
+  if (part == 0) sfactor[row] = factor;
+}
+
+typedef __attribute__((address_space(3))) void lds_void_t;
+
+// 64 rows of a k block from memory into LDS, four rows an instruction; at: this lane's byte offset in each four of 16
+// rows. With valid = 0 (else K) nothing is read and zeros arrive.
+__device__ __forceinline__ void router_fetch_block(const uint16_t* x, int valid, int K, int block, const uint32_t (&at)[4],
+                                                   uint4* slot) {
+  const __amdgpu_buffer_rsrc_t from =
+      __builtin_amdgcn_make_buffer_rsrc((void*)x, 0, kRouterRows * valid * 2, 0x00027000);
+#pragma unroll
+  for (int i = 0; i < kRouterRows / 4; ++i)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (lds_void_t*)(slot + i * 64), 16, at[i & 3],
+                                             block * kGroup * 2 + (i >> 2) * 32 * K, 0, 0);
+}
+
+// ---------------------------------------------------------------------------
+// 64 rows x 128 logits of a bf16 weight per workgroup of eight waves in two roles. Four multiply, each over every fourth k
+// block for all of the logits: x comes straight into LDS two blocks ahead, becomes operands in the wave's registers one
+// product group ahead, W half a block ahead; they share nothing until their sums meet at the end. The other four normalise
+// and quantise the workgroup's share of the tile's rows meanwhile (router_rows).
+// Bound by the instructions of the multiplying waves, one on a SIMD: 256 clocks of matrix instructions and about 220 of
+// operand arithmetic per 32 rows x 16 columns x 128 logits, which overlap in part (by themselves 23 us of 32 at
+// 8192 x 256 x 2048; the rows by themselves 17). us of the 64 x 128 kernel above / this: 8192 x 256 x 2048 34.4 / 31.6,
+// x 4096 65.1 / 57.4, x 7168 107.9 / 93.8, 4096 x 512 x 2048 27.3 / 25.0, 3072 x 512 x 1536 20.3 / 16.6, x 4096 43.0 / 38.8;
+// logits' error against 64 bits over 50 inputs 1.00 of that kernel's.
+// ---------------------------------------------------------------------------
+template <int KIND, bool ROUND>
+__global__ __launch_bounds__(512) void rmsnorm_router_quant_two_roles_kernel(RouterArgs p) {
+  // two k blocks of each multiplying wave, a row's 16 pieces XORed with its number; afterwards the partial sums of the first
+  // and the second 32 rows. (Two arrays: the compiler tells the loads into one from those into the other.)
+  __shared__ uint4 a0[4][kRouterRows * 16];
+  __shared__ uint4 a1[4][kRouterRows * 16];
+  __shared__ uint4 sgamma[4][256];          // of the k blocks of a multiplying wave
+  __shared__ double sq[4][2][kRouterRows];  // squares of a row: by wave and by half of its lanes
+  __shared__ unsigned sfactor[kRouterRows];
+  const int lane = tid_x() & 63;
+  const int wave = uniform32(tid_x() >> 6);
+  const int kblocks = p.K / kGroup;
+  int tile, chunk;
+  router_tile((p.M + kRouterRows - 1) / kRouterRows, p.chunks, tile, chunk);
+  const int row0 = min(tile * kRouterRows, p.M - kRouterRows);
+  const int r = lane & 31, h = lane >> 5;
+
+  if (wave < 4) {
+    // ---- 64 rows x 128 logits over k blocks wave, wave + 4, .. (K is 512 or more: every wave has one)
+    const int stages = (kblocks - wave + 3) >> 2;
+    const int vtiles = p.N / 32;
+    const uint4* w = p.w + (int64_t)chunk * 4 * 512;
+    const uint16_t* x = p.x + (int64_t)row0 * p.K;
+    auto block = [&](int s) { return min(wave + 4 * s, kblocks - 1); };
+    u32x4_t g4[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      g4[i] = *(const u32x4_t*)(p.gamma + block(4 * i + (lane >> 4)) * kGroup + (lane & 15) * 8);
+    uint32_t at[4];  // rows 4 i + lane / 16 of 16, in bytes
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = 4 * i + (lane >> 4);
+      at[i] = (uint32_t)(row * p.K + (((lane & 15) ^ row) * 8)) * 2u;
+    }
+    auto fetch_x = [&](int s, uint4* slot) {
+      router_fetch_block(x, s < stages ? p.K : 0, p.K, block(s), at, slot);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    uint4 b[4][4];
+    auto fetch_w = [&](int s, int j, uint4 (&d)[4]) {
+      const uint4* from = w + ((int64_t)block(s) * vtiles * 8 + j) * 64;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) d[t] = from[t * 512 + lane];
+    };
+    floatx16_t acc[2][4];
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[rt][t][v] = 0.f;
+    double ss[2] = {0.0, 0.0};
+    fetch_x(0, a0[wave]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      __builtin_amdgcn_sched_barrier(0);
+      fetch_w(0, j, b[j]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_x(1, a1[wave]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) *(u32x4_t*)&sgamma[wave][i * 64 + lane] = g4[i];
+
+    uint4 hi[2], lo[2], raw[2], gr[2];
+    auto load = [&](const uint4* slot, int j, int rt) {
+      uint32_t lane_at = (uint32_t)(r * 256 + ((8 * h) ^ (r & 15)) * 16);
+      asm volatile("" : "+v"(lane_at));  // (one register, not one per slot, k step and row tile)
+      return *(const uint4*)((const char*)slot + rt * 8192 + (lane_at ^ (j * 16)));
+    };
+    auto gamma_of = [&](int s, int j) { return sgamma[wave][(s & 15) * 16 + 8 * h + j]; };
+    // sixteen groups of products, 32 rows and a k step each: the products of group u, the operands of u + 1, the reads of
+    // u + 2. (Laid out group by group: the waits count the loads behind the one they are for.)
+    auto stage = [&](int s, const uint4* slot, const uint4* next) {
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        const int j = u >> 1, rt = u & 1, j2 = ((u + 2) & 15) >> 1;
+        __builtin_amdgcn_sched_barrier(0);
+        const uint4 raw2 = load(u < 14 ? slot : next, j2, rt);
+        if (rt == 0) gr[(j + 1) & 1] = gamma_of(u < 14 ? s : s + 1, j2);
+        __builtin_amdgcn_sched_barrier(0);
+        const bf16x8_t ah = operand(hi[u & 1]), al = operand(lo[u & 1]);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          floatx16_t& c = acc[rt][t];
+          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, operand(b[j & 3][t]), c, 0, 0, 0);
+          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, operand(b[j & 3][t]), c, 0, 0, 0);
+        }
+        const double squares = (double)sumsq8(raw[(u + 1) & 1]);
+        ss[(u + 1) & 1] += u < 15 || s + 1 < stages ? squares : 0.0;
+        router_split(raw[(u + 1) & 1], gr[((u + 1) >> 1) & 1], hi[(u + 1) & 1], lo[(u + 1) & 1]);
+        raw[u & 1] = raw2;
+        __builtin_amdgcn_sched_barrier(0);
+        if (rt == 1) fetch_w(j < 4 ? s : s + 1, (j + 4) & 7, b[j & 3]);
+      }
+    };
+    raw[0] = load(a0[wave], 0, 0);
+    raw[1] = load(a0[wave], 0, 1);
+    gr[0] = gamma_of(0, 0);
+    ss[0] += (double)sumsq8(raw[0]);
+    router_split(raw[0], gr[0], hi[0], lo[0]);
+#pragma unroll 1
+    for (int s = 0; s + 1 < stages; s += 2) {
+      stage(s, a0[wave], a1[wave]);
+      fetch_x(s + 2, a0[wave]);
+      stage(s + 1, a1[wave], a0[wave]);
+      fetch_x(s + 3, a1[wave]);
+    }
+    if (stages & 1) stage(stages - 1, a0[wave], a1[wave]);
+    __builtin_amdgcn_s_waitcnt(0);
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) {
+      sq[wave][h][rt * 32 + r] = ss[rt];
+      floatx4_t* part = (floatx4_t*)(rt == 0 ? a0[wave] : a1[wave]);
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          part[(t * 4 + i) * 64 + lane] =
+              floatx4_t{acc[rt][t][4 * i], acc[rt][t][4 * i + 1], acc[rt][t][4 * i + 2], acc[rt][t][4 * i + 3]};
+    }
+  } else {
+    router_rows<KIND, ROUND>(p, row0, chunk * 4 + wave - 4, p.chunks * 4);
+  }
+  __syncthreads();
+  router_factors(p, row0, sq, sfactor);
+  __syncthreads();
+  const floatx4_t* sums = (const floatx4_t*)(wave < 4 ? &a0[0][0] : &a1[0][0]);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int set = (wave & 3) * 4 + i;  // of 16 sets of four rows and 32 columns
+    floatx4_t v = sums[set * 64 + lane];
+#pragma unroll
+    for (int k = 1; k < 4; ++k) v += sums[k * (kRouterRows * 16) + set * 64 + lane];
+    // register e of a 32x32 result holds row (e / 4) * 8 + (lane / 32) * 4 + e % 4, column lane % 32
+    const int row = (wave >> 2) * 32 + (set & 3) * 8 + h * 4;
+    const int col = (chunk * 4 + (set >> 2)) * 32 + r;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      p.logits[(int64_t)(row0 + row + e) * p.N + col] = router_logit(v[e], sfactor[row + e]);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // An fp32 weight with gamma folded into it:
 //   logits[m, :] = r[m] * sum_k x[m, k] * (gamma[k] * W[:, k])
@@ -713,8 +955,6 @@ __global__ __launch_bounds__(256) void fold_router_weight_kernel(const float* __
   dst[0] = hi;
   dst[64] = pack8_bf16(lo);
 }
-
-typedef __attribute__((address_space(3))) void lds_void_t;
 
 // 64 rows of a slab of 64 columns from memory into LDS, eight rows an instruction; at: this lane's byte offset in the
 // first and the second eight of 16 rows. With valid = 0 (else K) nothing is read and zeros arrive.
@@ -759,7 +999,7 @@ __global__ __launch_bounds__(512) void rmsnorm_router_quant_folded_kernel(Router
   const int r = lane & 31, h = lane >> 5;
 
   if (wave < 4) {
-    // ---- 64 rows x 64 logits over slabs wave, wave + 4, ..
+    // ---- 64 rows x 64 logits over slabs wave, wave + 4, .. (K is 256 or more: every wave has one)
     const int slabs = kblocks * 2;
     const int stages = (slabs - wave + 3) >> 2;
     floatx16_t acc[2][2];
@@ -770,84 +1010,82 @@ __global__ __launch_bounds__(512) void rmsnorm_router_quant_folded_kernel(Router
 #pragma unroll
         for (int v = 0; v < 16; ++v) acc[rt][t][v] = 0.f;
     double ss[2] = {0.0, 0.0};
-    if (stages > 0) {
-      const uint4* w = p.w + (int64_t)chunk * 1024;
-      const uint16_t* x = p.x + (int64_t)row0 * p.K;
-      auto slab_of = [&](int s) { return min(wave + 4 * s, slabs - 1); };
-      uint32_t at[2];  // rows 8 i + lane / 8 of 16, in bytes
+    const uint4* w = p.w + (int64_t)chunk * 1024;
+    const uint16_t* x = p.x + (int64_t)row0 * p.K;
+    auto slab_of = [&](int s) { return min(wave + 4 * s, slabs - 1); };
+    uint32_t at[2];  // rows 8 i + lane / 8 of 16, in bytes
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int row = 8 * i + (lane >> 3);
-        at[i] = (uint32_t)(row * p.K + (((lane & 7) ^ ((row >> 1) & 7)) * 8)) * 2u;
-      }
-      auto fetch_x = [&](int s, uint4* slot) {
-        router_fetch_slab(x, s < stages ? p.K : 0, p.K, slab_of(s), at, slot);
-      };
-      uint4 b[4][4];  // [k step][tile 0 hi, lo, tile 1 hi, lo]: a set is refilled in place once it was used
-      auto fetch_w = [&](int s, int ks, uint4 (&d)[4]) {
-        const uint4* from = w + ((int64_t)slab_of(s) * (p.N / 32) * 8 + ks * 2) * 64;
-#pragma unroll
-        for (int t = 0; t < 4; ++t) d[t] = from[((t >> 1) * 8 + (t & 1)) * 64 + lane];
-      };
-      fetch_x(0, a0[wave]);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        __builtin_amdgcn_sched_barrier(0);
-        fetch_w(0, i, b[i]);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      fetch_x(1, a1[wave]);
-      fetch_x(2, a2[wave]);
-      fetch_x(3, a3[wave]);
-      auto load = [&](const uint4* slot, int ks, int rt) {
-        uint32_t lane_at = (uint32_t)(r * 128 + (h ^ ((r >> 1) & 7)) * 16);
-        asm volatile("" : "+v"(lane_at));  // (one register, not one per slot, k step and row tile)
-        return *(const uint4*)((const char*)slot + rt * 4096 + (lane_at ^ (ks * 32)));
-      };
-      uint4 af[2][2];
-      // (the order of loads and products is laid out step by step: the waits count the loads behind the one they are for)
-      auto stage = [&](int s, const uint4* slot, const uint4* next) {
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-#pragma unroll
-          for (int rt = 0; rt < 2; ++rt) af[(ks + 1) & 1][rt] = load(ks < 3 ? slot : next, (ks + 1) & 3, rt);
-          __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-          for (int rt = 0; rt < 2; ++rt) {
-            const uint4 a = af[ks & 1][rt];
-            ss[rt] += (double)sumsq8(a);
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-              acc[rt][t >> 1] =
-                  __builtin_amdgcn_mfma_f32_32x32x16_bf16(operand(a), operand(b[ks][t]), acc[rt][t >> 1], 0, 0, 0);
-          }
-          fetch_w(s + 1, ks, b[ks]);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      };
-#pragma unroll
-      for (int rt = 0; rt < 2; ++rt) af[0][rt] = load(a0[wave], 0, rt);
-      int s = 0;
-#pragma unroll 1
-      for (; s + 3 < stages; s += 4) {
-        stage(s, a0[wave], a1[wave]);
-        fetch_x(s + 4, a0[wave]);
-        __builtin_amdgcn_sched_barrier(0);
-        stage(s + 1, a1[wave], a2[wave]);
-        fetch_x(s + 5, a1[wave]);
-        __builtin_amdgcn_sched_barrier(0);
-        stage(s + 2, a2[wave], a3[wave]);
-        fetch_x(s + 6, a2[wave]);
-        __builtin_amdgcn_sched_barrier(0);
-        stage(s + 3, a3[wave], a0[wave]);
-        fetch_x(s + 7, a3[wave]);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      if (s < stages) stage(s, a0[wave], a1[wave]);
-      if (s + 1 < stages) stage(s + 1, a1[wave], a2[wave]);
-      if (s + 2 < stages) stage(s + 2, a2[wave], a3[wave]);
-      __builtin_amdgcn_s_waitcnt(0);
+    for (int i = 0; i < 2; ++i) {
+      const int row = 8 * i + (lane >> 3);
+      at[i] = (uint32_t)(row * p.K + (((lane & 7) ^ ((row >> 1) & 7)) * 8)) * 2u;
     }
+    auto fetch_x = [&](int s, uint4* slot) {
+      router_fetch_slab(x, s < stages ? p.K : 0, p.K, slab_of(s), at, slot);
+    };
+    uint4 b[4][4];  // [k step][tile 0 hi, lo, tile 1 hi, lo]: a set is refilled in place once it was used
+    auto fetch_w = [&](int s, int ks, uint4 (&d)[4]) {
+      const uint4* from = w + ((int64_t)slab_of(s) * (p.N / 32) * 8 + ks * 2) * 64;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) d[t] = from[((t >> 1) * 8 + (t & 1)) * 64 + lane];
+    };
+    fetch_x(0, a0[wave]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      __builtin_amdgcn_sched_barrier(0);
+      fetch_w(0, i, b[i]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_x(1, a1[wave]);
+    fetch_x(2, a2[wave]);
+    fetch_x(3, a3[wave]);
+    auto load = [&](const uint4* slot, int ks, int rt) {
+      uint32_t lane_at = (uint32_t)(r * 128 + (h ^ ((r >> 1) & 7)) * 16);
+      asm volatile("" : "+v"(lane_at));  // (one register, not one per slot, k step and row tile)
+      return *(const uint4*)((const char*)slot + rt * 4096 + (lane_at ^ (ks * 32)));
+    };
+    uint4 af[2][2];
+    // (the order of loads and products is laid out step by step: the waits count the loads behind the one they are for)
+    auto stage = [&](int s, const uint4* slot, const uint4* next) {
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt) af[(ks + 1) & 1][rt] = load(ks < 3 ? slot : next, (ks + 1) & 3, rt);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt) {
+          const uint4 a = af[ks & 1][rt];
+          ss[rt] += (double)sumsq8(a);
+#pragma unroll
+          for (int t = 0; t < 4; ++t)
+            acc[rt][t >> 1] =
+                __builtin_amdgcn_mfma_f32_32x32x16_bf16(operand(a), operand(b[ks][t]), acc[rt][t >> 1], 0, 0, 0);
+        }
+        fetch_w(s + 1, ks, b[ks]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) af[0][rt] = load(a0[wave], 0, rt);
+    int s = 0;
+#pragma unroll 1
+    for (; s + 3 < stages; s += 4) {
+      stage(s, a0[wave], a1[wave]);
+      fetch_x(s + 4, a0[wave]);
+      __builtin_amdgcn_sched_barrier(0);
+      stage(s + 1, a1[wave], a2[wave]);
+      fetch_x(s + 5, a1[wave]);
+      __builtin_amdgcn_sched_barrier(0);
+      stage(s + 2, a2[wave], a3[wave]);
+      fetch_x(s + 6, a2[wave]);
+      __builtin_amdgcn_sched_barrier(0);
+      stage(s + 3, a3[wave], a0[wave]);
+      fetch_x(s + 7, a3[wave]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (s < stages) stage(s, a0[wave], a1[wave]);
+    if (s + 1 < stages) stage(s + 1, a1[wave], a2[wave]);
+    if (s + 2 < stages) stage(s + 2, a2[wave], a3[wave]);
+    __builtin_amdgcn_s_waitcnt(0);
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt) {
       sq[wave][h][rt * 32 + r] = ss[rt];
@@ -860,77 +1098,11 @@ __global__ __launch_bounds__(512) void rmsnorm_router_quant_folded_kernel(Router
               floatx4_t{acc[rt][t][4 * i], acc[rt][t][4 * i + 1], acc[rt][t][4 * i + 2], acc[rt][t][4 * i + 3]};
     }
   } else {
-    // ---- statistic, y and codes of this workgroup's share of the tile's rows: four at a time, 16 lanes each
-    constexpr int kHeld = 16, kStep = 4;  // k blocks of a row in registers, worked on together; beyond the last: it again
-    const int cg = lane & 15;
-    const int last = (kblocks - 1) / kHeld;
-#pragma unroll 1
-    for (int batch = chunk * 4 + wave - 4; batch < kRouterRows / 4; batch += p.chunks * 4) {
-      const int row = row0 + batch * 4 + (lane >> 4);
-      const uint16_t* x = p.x + (int64_t)row * p.K + cg * 8;
-      const uint16_t* gamma = p.gamma + cg * 8;
-      uint4 xe[kHeld], ge[2][kStep];
-      auto fetch = [&](int k0) {
-#pragma unroll
-        for (int d = 0; d < kHeld; ++d) xe[d] = *(const uint4*)(x + min(k0 + d, kblocks - 1) * kGroup);
-      };
-      auto fetch_gamma = [&](int k0, uint4 (&g)[kStep]) {
-#pragma unroll
-        for (int d = 0; d < kStep; ++d) g[d] = *(const uint4*)(gamma + min(k0 + d, kblocks - 1) * kGroup);
-      };
-      double ss = 0.0;
-#pragma unroll 1
-      for (int set = 0; set <= last; ++set) {
-        fetch(set * kHeld);
-#pragma unroll
-        for (int d = 0; d < kHeld; ++d) ss += set * kHeld + d < kblocks ? (double)sumsq8(xe[d]) : 0.0;
-      }
-      fetch_gamma(last * kHeld, ge[0]);
-      const float rs = 1.0f / sqrtf((float)row16_sum_d(ss) / (float)p.K + p.eps);
-      if (cg == 0) p.rstd[row] = rs;
-      // the last set, which is in registers, first
-#pragma unroll 1
-      for (int i = 0; i <= last; ++i) {
-        const int k0 = (i == 0 ? last : i - 1) * kHeld;
-        if (i > 0) {
-          fetch(k0);
-          fetch_gamma(k0, ge[0]);
-        }
-#pragma unroll
-        for (int g = 0; g < kHeld / kStep; ++g) {
-          if (k0 + g * kStep < kblocks) {
-            fetch_gamma(k0 + (g + 1) * kStep, ge[(g + 1) & 1]);
-#pragma unroll
-            for (int d = 0; d < kStep; ++d) {
-              const int kb = min(k0 + g * kStep + d, kblocks - 1);
-              const int64_t at = (int64_t)row * p.K + kb * kGroup + cg * 8;
-              router_emit<KIND, ROUND>(p.y + at, p.q + at, p.s + (int64_t)kb * p.M + row, cg == 0, xe[g * kStep + d],
-                                       ge[g & 1][d], rs);
-            }
-          }
-        }
-      }
-    }
+    router_rows<KIND, ROUND>(p, row0, chunk * 4 + wave - 4, p.chunks * 4);
   }
   __syncthreads();
 
-  // ---- eight lanes a row: its factor
-  {
-    const int row = tid_x() >> 3, part = tid_x() & 7;
-    double total = 0.0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) total += sq[i >> 1][i & 1][row];
-    unsigned factor = __float_as_uint(1.0f / sqrtf((float)total / (float)p.K + p.eps));
-    bool bad = false;
-    if (factor == 0) {
-#pragma unroll 1
-      for (int c = part * 8; c < p.K; c += 64)
-        bad |= router_nonfinite(*(const uint4*)(p.x + (int64_t)(row0 + row) * p.K + c)) ||
-               router_nonfinite(*(const uint4*)(p.gamma + c));
-    }
-    if ((__ballot(bad) >> (lane & 56)) & 0xff) factor = kNanBits;
-    if (part == 0) sfactor[row] = factor;
-  }
+  router_factors(p, row0, sq, sfactor);
   __syncthreads();
   const floatx4_t* sums = (const floatx4_t*)(wave < 4 ? &a0[0][0] : &a1[0][0]);
 #pragma unroll
@@ -967,21 +1139,25 @@ hipError_t launch_pack_router_weight(const void* wr, int weight_fp32, void* wpac
 }
 
 struct RouterForm {
-  int rows, cols;  // of a workgroup: rows of x, logits
+  int rows, cols;          // of a workgroup: rows of x, logits
+  bool two_roles = false;  // 64 x 128 with the multiplying and the quantising waves apart
 };
 
 // which kernel, by the number of workgroups that each would have: fq_policy.hpp
 static RouterForm router_form(int64_t M, int K, int N, bool weight_fp32) {
   const auto ceil_div = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
   const int64_t tiles = ceil_div(M, kRouterRows);
+  const int kblocks = K / kGroup;
   if (M < kRouterRows || tiles * (N / 64) <= Policy::kRouterFewRowsMax) return {kRouterFewRows, 32};
   const bool narrow = !weight_fp32 && tiles * (N / 64) <= Policy::kRouterNarrowMax;
   const int cols64 = weight_fp32 || narrow ? 64 : 128;
+  const bool two_roles = cols64 == 128 && N % 256 == 0 &&
+                         (kblocks % 4 == 0 ? K >= Policy::kRouterTwoRolesMinK
+                                           : N > 256 && K >= Policy::kRouterTwoRolesAlwaysK);
   const int cols32 = N % 512 == 0 && !weight_fp32 ? 512 : N % 256 == 0 ? 256 : 128;
   const int per_cu = cols32 == 128 ? 3 : cols32 == 256 && !weight_fp32 ? 2 : 1;
   const int64_t rounds64 = ceil_div(tiles * (N / cols64), 256);
   const int64_t slots = 256 * per_cu, workgroups32 = M / 32 * (N / cols32), rounds32 = ceil_div(workgroups32, slots);
-  const int kblocks = K / kGroup;
   bool take32;
   if (per_cu == 1) {
     // in fifths of a round: one that leaves CUs free is shorter, the others' W arrives faster
@@ -995,9 +1171,10 @@ static RouterForm router_form(int64_t M, int K, int N, bool weight_fp32) {
   } else {
     take32 = !narrow && (kblocks + 34) * rounds32 <= 40 * rounds64;
   }
+  if (two_roles && K >= Policy::kRouterTwoRolesAlwaysK) take32 = false;
   // a launch has less than 2^32 work-items; the 32-row form needs half as many as the others or less
   take32 |= tiles * (N / cols64) * 512 > (int64_t)UINT32_MAX;
-  return take32 ? RouterForm{32, cols32} : RouterForm{kRouterRows, cols64};
+  return take32 ? RouterForm{32, cols32} : RouterForm{kRouterRows, cols64, two_roles};
 }
 
 // An fp32 weight: whether a call folds gamma into it. us of a call re-ordered / folded, number of 64 x 64 workgroups behind
@@ -1037,6 +1214,8 @@ hipError_t launch_rmsnorm_router_quant_packed(const void* x, const void* gamma, 
     else FQ_ROUTER_32(KINDV, ROUNDV, FP32V, FP32V ? 2 : 1, 8);                                                       \
   } else if (f.rows == kRouterFewRows)                                                                                                  \
     hipLaunchKernelGGL((rmsnorm_router_quant_few_rows_kernel<KINDV, ROUNDV, FP32V>), grid, dim3(512), 0, stream, p); \
+  else if (!FP32V && f.two_roles)                                                                                      \
+    hipLaunchKernelGGL((rmsnorm_router_quant_two_roles_kernel<KINDV, ROUNDV>), grid, dim3(512), 0, stream, p);           \
   else if (!FP32V && f.cols == 64)                                                                                     \
     hipLaunchKernelGGL((rmsnorm_router_quant_kernel<KINDV, ROUNDV, FP32V, FP32V ? 2 : 1>), grid, dim3(512), 0,       \
                        stream, p);                                                                                   \

@@ -661,6 +661,10 @@ def check_router(gpu, M, N, K, wdtype, dtype=E4M3, round_scale=False, packed=Fal
     (8224, 128, 896, torch.bfloat16), (8224, 128, 1024, torch.bfloat16), (8288, 128, 1152, torch.bfloat16),
     (4224, 256, 1280, torch.bfloat16),
     (2144, 256, 256, torch.float32), (1312, 256, 1920, torch.float32), (2048, 384, 896, torch.float32),
+    # 64 x 128 with its waves in two roles: k blocks of every remainder modulo the four waves and the two in flight, half
+    # a row tile, eight chunks, the longest K
+    (4256, 256, 1536, torch.bfloat16), (2112, 512, 2176, torch.bfloat16), (2144, 512, 2304, torch.bfloat16),
+    (1120, 1024, 2432, torch.bfloat16), (4160, 256, 2048, torch.bfloat16), (4128, 256, 8192, torch.bfloat16),
     # 32 rows x 128 logits, one, two and three column chunks; x 256 and x 512: k blocks of every remainder, an odd
     # number of row tiles, fewer k blocks than chunks
     (8224, 128, 128, torch.bfloat16), (8224, 128, 384, torch.bfloat16), (8256, 128, 640, torch.bfloat16),
@@ -697,19 +701,22 @@ def test_router_folded_weight(gpu, M, N, K, dtype, round_scale):
                                           (2624, 128, 384, torch.bfloat16), (8224, 128, 896, torch.bfloat16),
                                           (2144, 256, 384, torch.float32), (8224, 128, 256, torch.bfloat16),
                                           (2720, 128, 256, torch.float32), (4128, 256, 256, torch.bfloat16),
-                                          (4128, 256, 256, torch.float32), (4128, 512, 256, torch.bfloat16)])
+                                          (4128, 256, 256, torch.float32), (4128, 512, 256, torch.bfloat16),
+                                          (4128, 256, 1536, torch.bfloat16)])
 @pytest.mark.parametrize("dtype,round_scale", [(E4M3, True), (E5M2, False), (E5M2, True)])
 def test_router_forms_fp8_types(gpu, M, N, K, wdtype, dtype, round_scale):
     announce("router forms, types", M, N, K, wdtype, dtype, round_scale)
     check_router(gpu, M, N, K, wdtype, dtype, round_scale)
 
 
-# one call of each form of the router kernel: 16-row, 64 x 64, 64 x 128, 64 x 64 fp32, 32 rows x 128, 256 and 512
+# one call of each form of the router kernel: 16-row, 64 x 64, 64 x 128, 64 x 64 fp32, 32 rows x 128, 256 and 512, two
+# roles, folded weight
 @pytest.mark.parametrize("M,N,K,wdtype", [(128, 128, 640, torch.bfloat16), (128, 256, 384, torch.float32),
                                           (2688, 128, 256, torch.bfloat16), (8320, 128, 896, torch.bfloat16),
                                           (2176, 256, 256, torch.float32), (8320, 128, 384, torch.bfloat16),
                                           (2816, 128, 256, torch.float32), (4224, 256, 256, torch.bfloat16),
-                                          (4224, 256, 256, torch.float32), (4224, 512, 256, torch.bfloat16)])
+                                          (4224, 256, 256, torch.float32), (4224, 512, 256, torch.bfloat16),
+                                          (4224, 256, 1536, torch.bfloat16), (2176, 256, 1024, torch.float32)])
 def test_router_rows_without_a_statistic(gpu, M, N, K, wdtype):
     """Rows whose squares overflow: the statistic is 0, hence y and, for finite values, the logits (zeros, not the NaN
     of overflowed products); an infinity makes the row's logits NaN.  Other rows do not notice."""
