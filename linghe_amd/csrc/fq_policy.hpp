@@ -111,31 +111,26 @@ struct Policy {
   // 16-byte chunks per lane, matrix and step in the bf16 SwiGLU backward (three matrices are read):
   // 29.0 / 30.4 / 28.7 / 35.5 us with 2 / 3 / 4 / 8 at 8192 x 4096
   static constexpr int kSwigluBwdRowsUnroll = 4;
-  // the wide-row (three or four waves per row) RMSNorm + row-wise quant kernel loads the next row while it works on
-  // the current one (122 instead of 84 registers): 68.5 -> 65.5 us at 16384 x 7168
-  static constexpr bool kPrefetchRowQuantWide = true;
-  // Workgroups of that kernel's launch (us at n with: one per row / 4 / 16 looping per CU).  One per row as far as these:
-  // the hardware hands them out as others finish, while looping ones leave most of the chip idle in the last
-  // round of few (2000 x 4096 7.4 / 8.5 / 7.4, 5000 x 4096 14.2 / 15.8 / 20.5, 5000 x 7168 22.6 / 23.5 / 32.7,
-  // 8192 x 7168 34.1 / 34.2 / 35.4).
-  static constexpr int kRowQuantWideRowPerWg = 8192;
-  // Beyond, 16 looping per CU where their last round is full, that is idle for at most M / 12 rows (12000 x 4096
-  // 28.1 / 31.1 / 28.8, 16384 x 2176 26.7 / 29.8 / 25.9, 16384 x 5120 50.8 / 48.6 / 47.2, 50000 x 2176
-  // 74.7 / 80.9 / 70.7), else still one per row up to 4096 columns (9000 x 3072 17.9 / 20.3 / 23.6, 10000 x 4096
-  // 24.3 / 26.7 / 28.5, 18000 x 4096 42.1 / 46.3 / 45.4).
-  static constexpr int kRowQuantWideWgsPerCu = 16;
-  static constexpr int kRowQuantWideIdleShare = 12;
-  // Rows of three chunks a thread (4096 < n <= 6144; five workgroups on a CU) turn to looping earlier, and to 4 per CU
-  // where 16 do not come out even (6001 x 5120 21.5 / 21.8 / 26.4, 7000 x 4224 23.4 / 22.5 / 24.7, 8192 x 4608
-  // 27.4 / 25.7 / 26.6, 9000 x 5120 29.8 / 29.0 / 35.8, 10000 x 4608 31.7 / 31.0 / 35.6, 14000 x 5632 45.6 / 45.2 / 49.5).
-  static constexpr int kRowQuantThreeChunksRowPerWg = 6144;
-  // Four chunks a thread (n > 6144): exactly the four workgroups that a CU holds (16384 x 7168: 64.0 / 65.4 / 64.8 /
-  // 64.6 / 68.0 with 4 / 5 / 6 / 8 / 12).
-  static constexpr int kRowQuantFewLoopingPerCu = 4;
-  // up to 3072 columns (two chunks on 192 threads) three waves share a row: with four, a quarter and more of the
-  // lanes repeat the row's last chunk (us four / three waves, one workgroup per row: 1500 x 3072 5.89 / 5.79,
-  // 3001 x 2560 8.43 / 7.93, 8192 x 3072 19.0 / 17.9; three chunks on 192 are behind: 3001 x 3584 9.1 / 10.3)
-  static constexpr int kRowQuantThreeWavesMax = 3072;
+  // RMSNorm + row-wise quant of more than 2048 columns (us 2 / 3 / 4 chunks a thread, one row at once). Up to so many
+  // rows (n <= 3072, <= 6144, above) two chunks a thread: 1 x 7168 2.56 / 2.82 / 2.94, 256 x 5120 3.40 / 3.57 / 3.73,
+  // 1500 x 2560 5.12 / 5.47 / 5.70, 700 x 5632 5.46 / 5.33 / 5.81, 1500 x 6656 9.09 / 9.35 / 9.09. Beyond, what leaves
+  // few lanes without a chunk: 3001 x 2560 7.48 / 7.42 / 7.80, 3001 x 4096 9.72 / 10.2 / 9.88, 4104 x 4608
+  // 15.3 / 13.8 / 14.2, 3001 x 5632 14.0 / 12.6 / 12.8, 4104 x 6656 20.3 / 20.2 / 18.9.
+  static constexpr int kRowQuantTwoChunksNarrow = 2000, kRowQuantTwoChunks = 512, kRowQuantTwoChunksWide = 1500;
+  // Up to so many rows one at once, then two (us one / two): 7000 x 3072 15.0 / 15.4, 8192 x 2560 14.9 / 14.8,
+  // 16384 x 3584 35.7 / 33.0, 4104 x 5120 15.3 / 15.4, 6000 x 5120 21.0 / 20.0, 12288 x 5632 41.0 / 39.3, 6000 x 7168
+  // 26.8 / 26.8, 16384 x 7168 66.1 / 62.4.
+  static constexpr int kRowQuantOneRowNarrow = 8000, kRowQuantOneRow = 4500, kRowQuantOneRowWide = 6500;
+  // Workgroups that load the next row while they work on the current one stay where they are ahead (us so / the other
+  // kernel). 4096 and more than 7168 columns beyond 1024 rows, one row each up to 8192 rows (7000 x 4096 18.8 / 19.2,
+  // 4104 x 8064 20.8 / 21.8, 1500 x 8192 9.8 / 10.1, 8192 38.0 / 40.1), then the widest 4 per CU (16384 69.7 / 72.7).
+  // 4096 < n <= 6144 for two to four rows per CU (513 x 4608 4.26 / 4.38, 1024 x 6144 6.37 / 6.58; 1500 8.57 / 8.34).
+  // 4096 and 6144 columns beyond 8192 rows by 16 looping per CU where their last round is full, that is idle for at most
+  // M / 24 rows (16384 x 4096 38.3 / 39.4, 12288 x 6144 41.1 / 41.9; one row each 12000 x 4096 28.1, looping 28.8).
+  static constexpr int kRowQuantAhead = 1024, kRowQuantAheadThree = 1100;
+  static constexpr int kRowQuantLoopingMin = 8192, kRowQuantIdleShare = 24;
+  static constexpr int kRowQuantLoopingPerCu = 16, kRowQuantLooping8192 = 4;
+  static constexpr bool kPrefetchRowQuantWide = true;  // (they load a row ahead: 68.5 -> 65.5 us at 16384 x 7168)
   // the same in the wide-row RMSNorm backward with one chunk per thread (2048 < n <= 4096: 70.4 -> 66.9 us at
   // 16384 x 3072, 78.5 -> 76.4 at 16384 x 4096); with two chunks the second register set spills
   static constexpr bool kPrefetchRowBwdWide = true;

@@ -241,6 +241,68 @@ __global__ __launch_bounds__(T) void rmsnorm_fwd_kernel(const uint16_t* __restri
 }
 
 // ---------------------------------------------------------------------------
+// forward, quantising, rows of more than 2048 columns: T threads of NC chunks have ROWS rows at once and are done
+// (T * NC covers the row). Against looping workgroups that load a row ahead, nothing is kept but the rows and gamma
+// (52-80 registers instead of 75-122), so that a CU holds more of them, and the hardware hands them out as others
+// finish. Bound by memory; us before / now: 4104 x 5120 16.4 / 15.3, 8192 x 4608 26.8 / 24.4, 16384 x 3584 37.2 / 33.0,
+// x 4608 48.2 / 41.7, x 7168 65.7 / 62.4 (352 MB: 5.4 / 5.6 TB/s), 1 x 7168 3.3 / 2.6.
+// ---------------------------------------------------------------------------
+template <int T, int NC, int ROWS, int KIND, bool ROUND>
+__global__ __launch_bounds__(T) void rmsnorm_quant_rows_kernel(const uint16_t* __restrict__ x,
+                                                               const uint16_t* __restrict__ gamma,
+                                                               uint8_t* __restrict__ q, float* __restrict__ scale,
+                                                               float* __restrict__ rstd, int64_t M, int n, float eps) {
+  __shared__ double red[ROWS][T / 64];
+  const int tid = tid_x();
+  // one contiguous eighth of the rows per XCD, as in the kernel above
+  const int G = (int)n_wg_x(), per = (G + 7) >> 3;
+  const int xcd = (int)wg_x() & 7, slot = (int)wg_x() >> 3;
+  const int full = (G & 7) ? (G & 7) : 8;
+  const int64_t row0 = (int64_t)(xcd < full ? xcd * per + slot : full * per + (xcd - full) * (per - 1) + slot) * ROWS;
+  uint4 raw[ROWS][NC], gm[NC];
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i)
+    load_row_clamped<T, NC, Policy::kLoadHintRows>(x + (ROWS == 1 || row0 + i < M ? row0 + i : M - 1) * n, n,
+                                                   raw[i]);
+  load_row_clamped<T, NC>(gamma, n, gm);
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) {
+    const double ss = wave_sum_d(sumsq_live<T, NC>(raw[i], n));
+    if ((tid & 63) == 0) red[i][tid >> 6] = ss;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) {
+    const int64_t row = row0 + i;
+    if (ROWS > 1 && row >= M) return;
+    double ss = red[i][0];
+#pragma unroll
+    for (int w = 1; w < T / 64; ++w) ss += red[i][w];
+    const float r = rstd_from_sumsq((float)ss, n, eps);
+    if (tid == 0) rstd[row] = r;
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+      const int c = tid + k * T;
+      float a[8], w[8], y[8], m = 0.f;
+      unpack8(raw[i][k], a);
+      unpack8(gm[k], w);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        y[j] = (a[j] * r) * w[j];
+        m = fmaxf(m, fabsf(y[j]));
+      }
+      m = row16_max(m);
+      const float sc = make_scale<KIND, ROUND>(m);
+      const uint2 pk = quantize8<KIND, ROUND>(y, make_quantum<ROUND>(sc));
+      if (c * 8 < n) {
+        store8<false>(q + row * n + c * 8, pk);  // (ordinary stores, as above for wide rows)
+        if ((c & 15) == 0) scale[(int64_t)(c >> 4) * M + row] = sc;
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // statistic only (the first pass of RMSNorm + quant, output_mode 2): one wave per
 // row, eight 16-byte loads per lane in flight, nothing kept.  Few registers, so a
 // CU holds its 32 waves and a 16384-row input is two rows per wave with no tail.
@@ -620,14 +682,60 @@ static void pick_row_shape(int n, int T, int& nchunk) {
   FQ_ROW_CASE(64, 13, __VA_ARGS__) FQ_ROW_CASE(64, 14, __VA_ARGS__) FQ_ROW_CASE(64, 15, __VA_ARGS__) \
   FQ_ROW_CASE(64, 16, __VA_ARGS__) { return hipErrorInvalidValue; }
 
-// workgroups of the wide-row RMSNorm + row-wise quant kernel; chunks: 16-byte pieces of a row per thread of 256
-static int64_t row_quant_wide_workgroups(int64_t M, int chunks) {
-  if (M <= (chunks == 3 ? Policy::kRowQuantThreeChunksRowPerWg : Policy::kRowQuantWideRowPerWg)) return M;
-  const int64_t few = 256 * Policy::kRowQuantFewLoopingPerCu, looping = 256 * Policy::kRowQuantWideWgsPerCu;
-  if (chunks == 4) return few;
+// Rows of more than 2048 columns, quantising form: workgroups of the kernel that loops over rows, 0 for the other one
+static int64_t row_quant_looping(int64_t M, int n) {
+  const int64_t looping = 256 * Policy::kRowQuantLoopingPerCu;
   const int64_t idle = (M + looping - 1) / looping * looping - M;
-  if (idle * Policy::kRowQuantWideIdleShare <= M) return looping;
-  return chunks == 3 ? few : M;  // M < looping * kRowQuantWideIdleShare here
+  const bool even = M > Policy::kRowQuantLoopingMin && idle * Policy::kRowQuantIdleShare <= M;
+  if (n == 4096) return M <= Policy::kRowQuantAhead ? 0 : even ? looping : M;
+  if (n > 4096 && n <= 6144 && M > Policy::kRowQuantTwoChunks && M <= Policy::kRowQuantAheadThree) return M;
+  if (n == 6144) return even ? looping : 0;
+  if (n <= 7168 || M <= Policy::kRowQuantAhead) return 0;
+  return M <= Policy::kRowQuantLoopingMin ? M : 256 * Policy::kRowQuantLooping8192;
+}
+
+template <int KIND, bool ROUND>
+static void launch_row_quant_wide(const uint16_t* x, const uint16_t* gamma, uint8_t* q, float* scale, float* rstd,
+                                  int64_t M, int n, float eps, hipStream_t stream) {
+#define FQ_ROW_QUANT_LOOPING(NC)                                                                                 \
+  hipLaunchKernelGGL((rmsnorm_fwd_kernel<256, NC, false, 1, KIND, ROUND>), dim3((unsigned)looping), dim3(256),   \
+                     0, stream, x, gamma, (void*)q, scale, rstd, M, n, eps, 1)
+#define FQ_ROW_QUANT(T, NC, ROWS)                                                                                \
+  hipLaunchKernelGGL((rmsnorm_quant_rows_kernel<T, NC, ROWS, KIND, ROUND>),                                      \
+                     dim3((unsigned)((M + ROWS - 1) / ROWS)), dim3(T), 0, stream, x, gamma, q, scale, rstd, M, n, eps)
+#define FQ_ROW_QUANT_ROWS(T, NC) \
+  if (two) FQ_ROW_QUANT(T, NC, 2); else FQ_ROW_QUANT(T, NC, 1)
+  if (const int64_t looping = row_quant_looping(M, n)) {
+    if (n == 4096) FQ_ROW_QUANT_LOOPING(2);
+    else if (n <= 6144) FQ_ROW_QUANT_LOOPING(3);
+    else FQ_ROW_QUANT_LOOPING(4);
+    return;
+  }
+  const bool two = M > (n <= 3072   ? Policy::kRowQuantOneRowNarrow
+                        : n <= 6144 ? Policy::kRowQuantOneRow
+                                    : Policy::kRowQuantOneRowWide);
+  const int few = n <= 3072   ? Policy::kRowQuantTwoChunksNarrow
+                  : n <= 6144 ? Policy::kRowQuantTwoChunks
+                              : Policy::kRowQuantTwoChunksWide;
+  if (M <= few) {
+    if (n <= 3072) FQ_ROW_QUANT(192, 2, 1);
+    else if (n <= 4096) FQ_ROW_QUANT(256, 2, 1);
+    else if (n <= 6144) FQ_ROW_QUANT(384, 2, 1);
+    else FQ_ROW_QUANT(512, 2, 1);
+  } else if (n <= 3072) {
+    FQ_ROW_QUANT_ROWS(128, 3);
+  } else if (n <= 4096) {
+    FQ_ROW_QUANT_ROWS(256, 2);
+  } else if (n <= 4608) {
+    FQ_ROW_QUANT_ROWS(192, 3);
+  } else if (n <= 6144) {
+    FQ_ROW_QUANT_ROWS(256, 3);
+  } else {
+    FQ_ROW_QUANT_ROWS(256, 4);
+  }
+#undef FQ_ROW_QUANT_ROWS
+#undef FQ_ROW_QUANT
+#undef FQ_ROW_QUANT_LOOPING
 }
 
 hipError_t launch_rmsnorm_fwd(const void* x, const void* gamma, void* out, float* scale, float* rstd, int64_t M,
@@ -656,25 +764,17 @@ hipError_t launch_rmsnorm_fwd(const void* x, const void* gamma, void* out, float
   } else if (!quant) {
     if (reuse_rstd) { FQ_LAUNCH_FWD(true, 0, kE4M3, false) } else { FQ_LAUNCH_FWD(false, 0, kE4M3, false) }
   } else if (n > 2048) {
-    // wide rows, quantising form: four waves per row (a wave per row needs up to ~230 registers), three
-    // where two chunks a thread still cover the row with them
-    const int nc4 = (n / 8 + 255) / 256;
-    const dim3 grid4((unsigned)row_quant_wide_workgroups(M, nc4));
-#define FQ_LAUNCH_FWD4(T, NC, KINDV, ROUNDV)                                                                   \
-  hipLaunchKernelGGL((rmsnorm_fwd_kernel<T, NC, false, 1, KINDV, ROUNDV>), grid4, dim3(T), 0, stream,           \
-                     (const uint16_t*)x, (const uint16_t*)gamma, out, scale, rstd, M, n, eps, rows_per_wg)
-#define FQ_LAUNCH_FWD4_NC(KINDV, ROUNDV) \
-  if (n <= Policy::kRowQuantThreeWavesMax) { FQ_LAUNCH_FWD4(192, 2, KINDV, ROUNDV); }                          \
-  else if (nc4 == 2) { FQ_LAUNCH_FWD4(256, 2, KINDV, ROUNDV); }                                                \
-  else if (nc4 == 3) { FQ_LAUNCH_FWD4(256, 3, KINDV, ROUNDV); }                                                \
-  else { FQ_LAUNCH_FWD4(256, 4, KINDV, ROUNDV); }
+#define FQ_ROW_QUANT_WIDE(KINDV, ROUNDV)                                                                         \
+  launch_row_quant_wide<KINDV, ROUNDV>((const uint16_t*)x, (const uint16_t*)gamma, (uint8_t*)out, scale, rstd,   \
+                                       M, n, eps, stream)
     if (kind == kE5M2) {
-      if (round_scale) { FQ_LAUNCH_FWD4_NC(kE5M2, true) } else { FQ_LAUNCH_FWD4_NC(kE5M2, false) }
+      if (round_scale) FQ_ROW_QUANT_WIDE(kE5M2, true);
+      else FQ_ROW_QUANT_WIDE(kE5M2, false);
     } else {
-      if (round_scale) { FQ_LAUNCH_FWD4_NC(kE4M3, true) } else { FQ_LAUNCH_FWD4_NC(kE4M3, false) }
+      if (round_scale) FQ_ROW_QUANT_WIDE(kE4M3, true);
+      else FQ_ROW_QUANT_WIDE(kE4M3, false);
     }
-#undef FQ_LAUNCH_FWD4_NC
-#undef FQ_LAUNCH_FWD4
+#undef FQ_ROW_QUANT_WIDE
   } else if (kind == kE5M2) {
     if (round_scale) { FQ_LAUNCH_FWD(false, 1, kE5M2, true) } else { FQ_LAUNCH_FWD(false, 1, kE5M2, false) }
   } else {

@@ -286,7 +286,15 @@ def test_rmsnorm_and_block_quant(gpu, M, N, round_scale):
 @pytest.mark.parametrize("M,N", [(1, 2176), (8200, 2176), (37, 3072), (4099, 3072), (8195, 3200), (5, 6272), (8195, 6272),
                                  # 16 looping per CU (last round full), four, and one more or fewer row than either takes
                                  (12288, 2176), (12289, 2176), (11343, 3200), (11342, 3200), (6144, 4224), (6145, 4224),
-                                 (8192, 4224)])
+                                 (8192, 4224),
+                                 # the narrowest and widest of each number of threads and chunks, one row at once and
+                                 # two (an even and an odd number of rows), one row more or fewer than each takes
+                                 (2000, 3072), (2001, 2176), (8000, 3072), (8001, 2176), (37, 3200), (4501, 3968),
+                                 (513, 4224), (4500, 4608), (4501, 4224), (512, 6144), (4502, 5888), (1500, 8064),
+                                 (1501, 6272), (6501, 7168),
+                                 # a row ahead: one row each, 4 per CU and 16 (and 4096 columns with an idle last round)
+                                 (513, 4736), (1100, 6144), (1101, 6144), (1025, 7296), (1024, 4096), (1025, 4096),
+                                 (8193, 8192), (8193, 4096), (12288, 6144), (12289, 4096), (12200, 4096)])
 def test_rmsnorm_rows_only_wide(gpu, M, N):
     from linghe_amd.utils.norm import triton_rms_norm_and_block_quant_forward as fn
 
