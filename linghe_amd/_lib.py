@@ -95,13 +95,12 @@ class _MissingModule:
                           "`python -m linghe_amd.build`. There is no fallback path.") from self._cause
 
 
-try:  # outputs and launch of the row-wise quantisers in one native call
+try:  # outputs and launch of an entry point in one native call
     from . import _fq_torch as native
 except ImportError as e:
     native = _MissingModule(e)
 else:
-    native.bind(*(ctypes.cast(getattr(lib, name), _P).value
-                  for name in ("fq_rmsnorm_quant_fwd", "fq_swiglu_quant_fwd", "fq_group_quant", "fq_last_error")))
+    native.bind(*(ctypes.cast(getattr(lib, name), _P).value for name in native.FUNCTIONS))
 
 
 def check(rc: int) -> None:

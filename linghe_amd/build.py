@@ -78,8 +78,9 @@ def build_library(extra_flags=(), verbose: bool = False, csrc: str = CSRC, out: 
         try:
             build_host_module()
         except RuntimeError as e:
-            raise RuntimeError(f"{out} is built and serves every call but the row-wise quantisers; "
-                               f"the host module is not (it needs torch's and Python's headers): {e}") from e
+            raise RuntimeError(f"{out} is built and serves the callers of the C interface; the host module, which "
+                               f"the Python entry points launch through and which needs torch's and Python's "
+                               f"headers, is not: {e}") from e
     return out
 
 

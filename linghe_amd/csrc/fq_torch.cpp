@@ -1,27 +1,43 @@
-// The outputs and the launch of the row-wise quantisers in one native call.
+// The outputs and the launch of an entry point in one native call.
 //
-// A decode step's kernels run 2.2-3.7 us each, and a Python wrapper that allocates its two to five outputs
-// with torch.empty and calls the library through ctypes takes 12 us: what bounds a small call is the host.
-// The wrappers keep their checks in Python and hand over here; allocation goes through the dispatcher as
-// torch.empty does (same allocator, pools and modes) and the interpreter lock is released meanwhile.
+// A small call's kernels run 2-5 us each, and a Python wrapper that allocates its two to seven outputs with torch.empty
+// and calls the library through ctypes takes 7-13 us (more where it adds up the tokens of 256 experts): what bounds a
+// small call is the host. The wrappers keep their checks in Python and hand over here; allocation goes through the
+// dispatcher as torch.empty does (same allocator, pools and modes) and the interpreter lock is released meanwhile.
 // The kernel library is the one that _lib.py loaded: bind() takes its functions' addresses, there is no
 // link-time dependency that could bring a second one into the process.
-// RMSNorm + group + SwiGLU quantiser, three calls: 36.8 -> 21.7 us on 32 rows of 2048, 36.8 -> 23.9 on 3001 of 4096.
+// us through ctypes / here, back to back: RMSNorm + group + SwiGLU quantiser on 32 rows of 2048 36.8 / 21.7; SwiGLU +
+// quant forward and backward 768 x 1408 18.4 / 14.3; activation and weight of a linear layer, 336 x 3584 and 1152 x 3584,
+// 18.4 / 11.4; bf16 RMSNorm and SwiGLU, forward and backward, 480 x 2944 / 512 37.6 / 28.4; gather + pad + quant and
+// per-expert quant, 642 tokens to 8 of 16 experts, 28.5 / 21.5; per-expert SwiGLU, 1152 tokens to 2 of 64, with a plan
+// 46.2 / 37.1; router 256 x 1152, 384 logits 20.4 / 14.3.
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <ATen/ATen.h>
 #include <pybind11/pybind11.h>
 
+#include <cstdlib>
+#include <iterator>
+#include <vector>
+
 #include "../../include/fq_api.h"
 
 namespace {
 
+// the library's functions that are called here
+#define FQ_FUNCTIONS(F)                                                                                              \
+  F(rmsnorm_fwd) F(rmsnorm_bwd) F(rmsnorm_bwd_num_partials) F(rmsnorm_quant_fwd) F(rmsnorm_router_quant_fwd)         \
+  F(rmsnorm_router_quant_fwd_packed) F(swiglu_fwd) F(swiglu_bwd) F(swiglu_quant_fwd) F(swiglu_quant_bwd)             \
+  F(batched_swiglu_quant_fwd) F(batched_swiglu_quant_fwd_planned) F(batched_swiglu_quant_bwd)                        \
+  F(batched_swiglu_quant_bwd_planned) F(group_quant) F(block_quant) F(blockwise_quant) F(batched_blockwise_quant)    \
+  F(batched_blockwise_quant_planned) F(batched_pad_permute_quant) F(batched_pad_permute_quant_planned)               \
+  F(expert_plan_shape) F(last_error)
+
 struct {
-  decltype(&fq_rmsnorm_quant_fwd) rmsnorm_quant_fwd = nullptr;
-  decltype(&fq_swiglu_quant_fwd) swiglu_quant_fwd = nullptr;
-  decltype(&fq_group_quant) group_quant = nullptr;
-  decltype(&fq_last_error) last_error = nullptr;
+#define FQ_MEMBER(name) decltype(&fq_##name) name = nullptr;
+  FQ_FUNCTIONS(FQ_MEMBER)
+#undef FQ_MEMBER
 } lib;
 
 at::ScalarType dtype_of(PyObject* o) {
@@ -34,8 +50,6 @@ int64_t int_of(PyObject* o) {
   if (v == -1 && PyErr_Occurred()) throw python_error();
   return v;
 }
-
-void* stream_of(PyObject* o) { return reinterpret_cast<void*>(static_cast<intptr_t>(int_of(o))); }
 
 // the tensor behind an argument; undefined for None
 at::Tensor tensor_or_none(PyObject* o) {
@@ -54,23 +68,69 @@ void check(int rc) {
   TORCH_CHECK(rc == 0, "libfq_gfx950 error ", rc, ": ", lib.last_error());
 }
 
-void need_args(Py_ssize_t n, Py_ssize_t want) { TORCH_CHECK(n == want, "expected ", want, " arguments, got ", n); }
+float* floats(const at::Tensor& t) { return static_cast<float*>(data(t)); }
 
-void need_lib() { TORCH_CHECK(lib.last_error, "bind() was not called"); }
-
-template <typename F>
-F function_at(PyObject* o) {
-  const int64_t address = int_of(o);
-  TORCH_CHECK(address != 0, "a function's address is 0");
-  return reinterpret_cast<F>(static_cast<intptr_t>(address));
+// the numbers of an iterable, each through int(); of a size that sums of a million of them cannot overflow
+std::vector<int64_t> ints_of(PyObject* o) {
+  const auto items = pybind11::reinterpret_steal<pybind11::object>(PySequence_Tuple(o));
+  if (!items) throw python_error();
+  std::vector<int64_t> values(static_cast<size_t>(PyTuple_GET_SIZE(items.ptr())));
+  for (size_t i = 0; i < values.size(); ++i) {
+    PyObject* item = PyTuple_GET_ITEM(items.ptr(), static_cast<Py_ssize_t>(i));
+    if (PyLong_CheckExact(item)) {
+      values[i] = int_of(item);
+    } else {
+      const auto number = pybind11::reinterpret_steal<pybind11::object>(PyNumber_Long(item));
+      if (!number) throw python_error();
+      values[i] = int_of(number.ptr());
+    }
+    TORCH_CHECK(std::abs(values[i]) < (int64_t{1} << 40), values[i], " rows of one expert");
+  }
+  return values;
 }
 
-// (fq_rmsnorm_quant_fwd, fq_swiglu_quant_fwd, fq_group_quant, fq_last_error): addresses in the loaded library
+// the arguments of a call, one after the other
+class Args {
+ public:
+  Args(PyObject* const* a, Py_ssize_t n, Py_ssize_t want) : a_(a) {
+    TORCH_CHECK(n == want, "expected ", want, " arguments, got ", n);
+    TORCH_CHECK(lib.last_error, "bind() was not called");
+  }
+  at::Tensor tensor() { return tensor_or_none(*a_++); }
+  int64_t integer() { return int_of(*a_++); }
+  int flag() { return static_cast<int>(integer()); }
+  std::vector<int64_t> integers() { return ints_of(*a_++); }
+  void* address() { return reinterpret_cast<void*>(static_cast<intptr_t>(integer())); }
+  at::ScalarType dtype() { return dtype_of(*a_++); }
+  float real() {
+    const double v = PyFloat_AsDouble(*a_++);
+    if (v == -1.0 && PyErr_Occurred()) throw python_error();
+    return static_cast<float>(v);
+  }
+
+ private:
+  PyObject* const* a_;
+};
+
+template <typename F>
+void set_function(F& f, PyObject* o) {
+  const int64_t address = int_of(o);
+  TORCH_CHECK(address != 0, "a function's address is 0");
+  f = reinterpret_cast<F>(static_cast<intptr_t>(address));
+}
+
+// the addresses in the loaded library of the functions that FUNCTIONS names, in its order
 PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   HANDLE_TH_ERRORS
-  need_args(n_args, 4);
-  lib = {function_at<decltype(&fq_rmsnorm_quant_fwd)>(a[0]), function_at<decltype(&fq_swiglu_quant_fwd)>(a[1]),
-         function_at<decltype(&fq_group_quant)>(a[2]), function_at<decltype(&fq_last_error)>(a[3])};
+  decltype(lib) bound;
+  Py_ssize_t i = 0;
+#define FQ_SET(name)                                             \
+  TORCH_CHECK(i < n_args, "bind() misses the address of fq_" #name); \
+  set_function(bound.name, a[i++]);
+  FQ_FUNCTIONS(FQ_SET)
+#undef FQ_SET
+  TORCH_CHECK(i == n_args, "bind() expected ", i, " addresses, got ", n_args);
+  lib = bound;
   Py_RETURN_NONE;
   END_HANDLE_TH_ERRORS
 }
@@ -91,20 +151,60 @@ PyObject* wrap(const std::initializer_list<at::Tensor>& outs) {
   return tuple;
 }
 
+// (x, gamma, out, rms, M, n, eps, reuse rms, stream): out and rms are allocated where None is given
+PyObject* rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+  HANDLE_TH_ERRORS
+  Args in(a, n_args, 9);
+  const at::Tensor x = in.tensor(), gamma = in.tensor();
+  at::Tensor out = in.tensor(), rms = in.tensor();
+  const int64_t M = in.integer(), n = in.integer();
+  const float eps = in.real();
+  const int reuse = in.flag();
+  void* stream = in.address();
+  {
+    pybind11::gil_scoped_release no_gil;
+    if (!out.defined()) out = at::empty_like(x);
+    if (!rms.defined()) rms = empty(x, at::kFloat, {M});
+    if (M > 0) check(lib.rmsnorm_fwd(data(x), data(gamma), data(out), floats(rms), M, n, eps, reuse, stream));
+  }
+  return wrap({out, rms});
+  END_HANDLE_TH_ERRORS
+}
+
+// (dy, x, gamma, rms, dx, M, n, eps, stream): dx is allocated where None is given
+PyObject* rmsnorm_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+  HANDLE_TH_ERRORS
+  Args in(a, n_args, 9);
+  const at::Tensor dy = in.tensor(), x = in.tensor(), gamma = in.tensor(), rms = in.tensor();
+  at::Tensor dx = in.tensor(), dgamma;
+  const int64_t M = in.integer(), n = in.integer();
+  const float eps = in.real();
+  void* stream = in.address();
+  {
+    pybind11::gil_scoped_release no_gil;
+    if (!dx.defined()) dx = at::empty_like(x);
+    dgamma = empty(gamma, at::kFloat, {n});
+    const int64_t n_partials = lib.rmsnorm_bwd_num_partials(M, n);
+    const at::Tensor partials = empty(gamma, at::kFloat, {n_partials, n});
+    check(lib.rmsnorm_bwd(data(dy), data(x), data(gamma), floats(rms), data(dx), floats(dgamma), floats(partials),
+                          n_partials, M, n, eps, stream));
+  }
+  return wrap({dx, dgamma});
+  END_HANDLE_TH_ERRORS
+}
+
 // (x, gamma, out, scale, rms, eps, round_scale, output_mode, fp8 dtype, kind, stream): out, scale and rms are
 // allocated where None is given and the mode writes them
 PyObject* rmsnorm_quant(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   HANDLE_TH_ERRORS
-  need_args(n_args, 11);
-  need_lib();
-  const at::Tensor x = tensor_or_none(a[0]), gamma = tensor_or_none(a[1]);
-  at::Tensor out = tensor_or_none(a[2]), scale = tensor_or_none(a[3]), rms = tensor_or_none(a[4]), qt, st;
-  const double eps = PyFloat_AsDouble(a[5]);
-  if (eps == -1.0 && PyErr_Occurred()) throw python_error();
-  const int round = static_cast<int>(int_of(a[6])), mode = static_cast<int>(int_of(a[7]));
-  const at::ScalarType fp8 = dtype_of(a[8]);
-  const int kind = static_cast<int>(int_of(a[9]));
-  void* stream = stream_of(a[10]);
+  Args in(a, n_args, 11);
+  const at::Tensor x = in.tensor(), gamma = in.tensor();
+  at::Tensor out = in.tensor(), scale = in.tensor(), rms = in.tensor(), qt, st;
+  const float eps = in.real();
+  const int round = in.flag(), mode = in.flag();
+  const at::ScalarType fp8 = in.dtype();
+  const int kind = in.flag();
+  void* stream = in.address();
   {
     pybind11::gil_scoped_release no_gil;
     const int64_t M = x.size(0), n = x.size(1);
@@ -117,25 +217,102 @@ PyObject* rmsnorm_quant(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     if (!rms.defined()) rms = empty(x, at::kFloat, {M});
     if (M > 0)
       check(lib.rmsnorm_quant_fwd(data(x), data(gamma), mode != 1 ? data(out) : nullptr,
-                                  static_cast<float*>(mode != 1 ? data(scale) : nullptr),
-                                  static_cast<float*>(data(rms)), data(qt), static_cast<float*>(data(st)), M, n,
-                                  static_cast<float>(eps), round, mode, kind, stream));
+                                  mode != 1 ? floats(scale) : nullptr, floats(rms), data(qt), floats(st), M, n, eps,
+                                  round, mode, kind, stream));
   }
   return wrap({out, scale, rms, qt, st});
+  END_HANDLE_TH_ERRORS
+}
+
+// (x, gamma, route_weight, packed weight or None, weight is fp32, scratch bytes, rms, output_mode, eps, round_scale,
+// stream): rms is allocated where None is given
+PyObject* rmsnorm_router_quant(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+  HANDLE_TH_ERRORS
+  Args in(a, n_args, 11);
+  const at::Tensor x = in.tensor(), gamma = in.tensor(), weight = in.tensor(), packed = in.tensor();
+  const int fp32 = in.flag();
+  const int64_t scratch_bytes = in.integer();
+  at::Tensor rms = in.tensor(), y, logits, q, s, qt, st;
+  const int mode = in.flag();
+  const float eps = in.real();
+  const int round = in.flag();
+  void* stream = in.address();
+  {
+    pybind11::gil_scoped_release no_gil;
+    const int64_t M = x.size(0), K = x.size(1), N = weight.size(0);
+    y = empty(x, x.scalar_type(), {M, K});
+    if (!rms.defined()) rms = empty(x, at::kFloat, {M});
+    logits = empty(x, at::kFloat, {M, N});
+    q = empty(x, at::kFloat8_e4m3fn, {M, K});
+    s = empty(x, at::kFloat, {K / 128, M});
+    qt = empty(x, at::kFloat8_e4m3fn, {K, M});
+    st = empty(x, at::kFloat, {M / 128, K});
+    if (M > 0 && mode == 1) {
+      check(lib.rmsnorm_quant_fwd(data(x), data(gamma), nullptr, nullptr, floats(rms), data(qt), floats(st), M, K, eps,
+                                  round, 1, FQ_E4M3, stream));
+    } else if (M > 0 && packed.defined()) {
+      check(lib.rmsnorm_router_quant_fwd_packed(data(x), data(gamma), data(packed), fp32, data(y), floats(rms),
+                                                floats(logits), data(q), floats(s), M, K, N, eps, round, FQ_E4M3,
+                                                stream));
+    } else if (M > 0) {
+      // route_weight re-ordered for the matrix cores (an fp32 weight as two bf16 planes, in the larger calls of
+      // gamma * route_weight, which depends on both and is made by every call)
+      const at::Tensor scratch = empty(x, at::kByte, {scratch_bytes});
+      check(lib.rmsnorm_router_quant_fwd(data(x), data(gamma), data(weight), fp32, data(scratch), data(y), floats(rms),
+                                         floats(logits), data(q), floats(s), M, K, N, eps, round, FQ_E4M3, stream));
+    }
+  }
+  return wrap({y, rms, logits, q, s, qt, st});
+  END_HANDLE_TH_ERRORS
+}
+
+// (x, weight or None, weight is bf16, out, stream): out is allocated where None is given
+PyObject* swiglu(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+  HANDLE_TH_ERRORS
+  Args in(a, n_args, 5);
+  const at::Tensor x = in.tensor(), weight = in.tensor();
+  const int wbf16 = in.flag();
+  at::Tensor out = in.tensor();
+  void* stream = in.address();
+  {
+    pybind11::gil_scoped_release no_gil;
+    const int64_t M = x.size(0), n = x.size(1) / 2;
+    if (!out.defined()) out = empty(x, x.scalar_type(), {M, n});
+    check(lib.swiglu_fwd(data(x), data(weight), wbf16, data(out), M, n, stream));
+  }
+  return THPVariable_Wrap(out);
+  END_HANDLE_TH_ERRORS
+}
+
+// (g, x, weight or None, weight is bf16, stream)
+PyObject* swiglu_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+  HANDLE_TH_ERRORS
+  Args in(a, n_args, 5);
+  const at::Tensor g = in.tensor(), x = in.tensor(), weight = in.tensor();
+  const int wbf16 = in.flag();
+  void* stream = in.address();
+  at::Tensor dx, dw;
+  {
+    pybind11::gil_scoped_release no_gil;
+    const int64_t M = x.size(0), N = x.size(1);
+    if (weight.defined()) dw = empty(x, weight.scalar_type(), weight.sizes());
+    dx = empty(x, x.scalar_type(), {M, N});
+    check(lib.swiglu_bwd(data(g), data(x), data(weight), wbf16, data(dx), data(dw), M, N / 2, stream));
+  }
+  return wrap({dx, dw});
   END_HANDLE_TH_ERRORS
 }
 
 // (x, out, scale, round_scale, output_mode, fp8 dtype, kind, stream)
 PyObject* swiglu_quant(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   HANDLE_TH_ERRORS
-  need_args(n_args, 8);
-  need_lib();
-  const at::Tensor x = tensor_or_none(a[0]);
-  at::Tensor out = tensor_or_none(a[1]), scale = tensor_or_none(a[2]), qt, st;
-  const int round = static_cast<int>(int_of(a[3])), mode = static_cast<int>(int_of(a[4]));
-  const at::ScalarType fp8 = dtype_of(a[5]);
-  const int kind = static_cast<int>(int_of(a[6]));
-  void* stream = stream_of(a[7]);
+  Args in(a, n_args, 8);
+  const at::Tensor x = in.tensor();
+  at::Tensor out = in.tensor(), scale = in.tensor(), qt, st;
+  const int round = in.flag(), mode = in.flag();
+  const at::ScalarType fp8 = in.dtype();
+  const int kind = in.flag();
+  void* stream = in.address();
   {
     pybind11::gil_scoped_release no_gil;
     const int64_t M = x.size(0), n = x.size(1) / 2;
@@ -144,43 +321,317 @@ PyObject* swiglu_quant(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     qt = empty(x, fp8, {n, M});
     st = empty(x, at::kFloat, {(M + 127) / 128, n});
     if (M > 0)
-      check(lib.swiglu_quant_fwd(data(x), data(out), static_cast<float*>(data(scale)), data(qt),
-                                 static_cast<float*>(data(st)), M, n, round, mode, kind, stream));
+      check(lib.swiglu_quant_fwd(data(x), data(out), floats(scale), data(qt), floats(st), M, n, round, mode, kind,
+                                 stream));
   }
   return wrap({out, scale, qt, st});
+  END_HANDLE_TH_ERRORS
+}
+
+// (g, x, round_scale, fp8 dtype, kind, stream)
+PyObject* swiglu_quant_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+  HANDLE_TH_ERRORS
+  Args in(a, n_args, 6);
+  const at::Tensor g = in.tensor(), x = in.tensor();
+  const int round = in.flag();
+  const at::ScalarType fp8 = in.dtype();
+  const int kind = in.flag();
+  void* stream = in.address();
+  at::Tensor q, s, qt, st;
+  {
+    pybind11::gil_scoped_release no_gil;
+    const int64_t M = x.size(0), N = x.size(1);
+    q = empty(x, fp8, {M, N});
+    s = empty(x, at::kFloat, {N / 128, M});
+    qt = empty(x, fp8, {N, M});
+    st = empty(x, at::kFloat, {(M + 127) / 128, N});
+    if (M > 0)
+      check(lib.swiglu_quant_bwd(data(g), data(x), data(q), floats(s), data(qt), floats(st), M, N / 2, round, kind,
+                                 stream));
+  }
+  return wrap({q, s, qt, st});
+  END_HANDLE_TH_ERRORS
+}
+
+// (x, weight, weight is bf16, counts, counts are int64, plan's table or None, plan's shape, blocks, out, scale,
+// round_scale, output_mode, fp8 dtype, kind, stream): out and scale are allocated where None is given
+PyObject* batched_swiglu_quant(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+  HANDLE_TH_ERRORS
+  Args in(a, n_args, 15);
+  const at::Tensor x = in.tensor(), weight = in.tensor();
+  const int wbf16 = in.flag();
+  const at::Tensor counts = in.tensor();
+  const int i64 = in.flag();
+  const at::Tensor plan = in.tensor();
+  const int64_t* shape = static_cast<const int64_t*>(in.address());
+  const int64_t blocks = in.integer();
+  at::Tensor out = in.tensor(), scale = in.tensor(), qt, st;
+  const int round = in.flag(), mode = in.flag();
+  const at::ScalarType fp8 = in.dtype();
+  const int kind = in.flag();
+  void* stream = in.address();
+  {
+    pybind11::gil_scoped_release no_gil;
+    const int64_t M = x.size(0), n = x.size(1) / 2;
+    if (!out.defined()) out = empty(x, fp8, {M, n});
+    if (!scale.defined()) scale = empty(x, at::kFloat, {M, n / 128});
+    qt = empty(x, fp8, {M, n});
+    st = empty(x, at::kFloat, {blocks, n});
+    if (M > 0 && plan.defined())
+      check(lib.batched_swiglu_quant_fwd_planned(data(x), data(weight), wbf16, data(plan), shape, data(out),
+                                                 floats(scale), data(qt), floats(st), M, n, round, mode, kind, stream));
+    else if (M > 0)
+      check(lib.batched_swiglu_quant_fwd(data(x), data(weight), wbf16, data(counts), i64,
+                                         static_cast<int>(counts.size(0)), blocks, data(out), floats(scale), data(qt),
+                                         floats(st), M, n, round, mode, kind, stream));
+  }
+  return wrap({out, scale, qt, st});
+  END_HANDLE_TH_ERRORS
+}
+
+// (g, x, weight, weight is bf16, dw, counts, counts are int64, plan's table or None, plan's shape, blocks, round_scale,
+// fp8 dtype, kind, stream): dw is allocated where None is given
+PyObject* batched_swiglu_quant_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+  HANDLE_TH_ERRORS
+  Args in(a, n_args, 14);
+  const at::Tensor g = in.tensor(), x = in.tensor(), weight = in.tensor();
+  const int wbf16 = in.flag();
+  at::Tensor dw = in.tensor(), q, s, qt, st;
+  const at::Tensor counts = in.tensor();
+  const int i64 = in.flag();
+  const at::Tensor plan = in.tensor();
+  const int64_t* shape = static_cast<const int64_t*>(in.address());
+  const int64_t blocks = in.integer();
+  const int round = in.flag();
+  const at::ScalarType fp8 = in.dtype();
+  const int kind = in.flag();
+  void* stream = in.address();
+  {
+    pybind11::gil_scoped_release no_gil;
+    const int64_t M = x.size(0), N = x.size(1), n = N / 2;
+    q = empty(x, fp8, {M, N});
+    s = empty(x, at::kFloat, {M, N / 128});
+    qt = empty(x, fp8, {M, N});
+    st = empty(x, at::kFloat, {blocks, N});
+    if (!dw.defined()) dw = at::empty_like(weight);
+    if (blocks != 0) {
+      const at::Tensor partials = empty(x, at::kFloat, {M, n / 128});
+      if (plan.defined())
+        check(lib.batched_swiglu_quant_bwd_planned(data(g), data(x), data(weight), wbf16, data(plan), shape, data(q),
+                                                   floats(s), data(dw), data(qt), floats(st), floats(partials), M, n,
+                                                   round, kind, stream));
+      else
+        check(lib.batched_swiglu_quant_bwd(data(g), data(x), data(weight), wbf16, data(counts), i64,
+                                           static_cast<int>(counts.size(0)), blocks, data(q), floats(s), data(dw),
+                                           data(qt), floats(st), floats(partials), M, n, round, kind, stream));
+    }
+  }
+  return wrap({q, s, dw, qt, st});
   END_HANDLE_TH_ERRORS
 }
 
 // (x, round_scale, fp8 dtype, kind, stream)
 PyObject* group_quant(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   HANDLE_TH_ERRORS
-  need_args(n_args, 5);
-  need_lib();
-  const at::Tensor x = tensor_or_none(a[0]);
+  Args in(a, n_args, 5);
+  const at::Tensor x = in.tensor();
   at::Tensor q, s;
-  const int round = static_cast<int>(int_of(a[1]));
-  const at::ScalarType fp8 = dtype_of(a[2]);
-  const int kind = static_cast<int>(int_of(a[3]));
-  void* stream = stream_of(a[4]);
+  const int round = in.flag();
+  const at::ScalarType fp8 = in.dtype();
+  const int kind = in.flag();
+  void* stream = in.address();
   {
     pybind11::gil_scoped_release no_gil;
     const int64_t M = x.size(0), n = x.size(1);
     q = empty(x, fp8, {M, n});
     s = empty(x, at::kFloat, {M, n / 128});
-    if (M > 0) check(lib.group_quant(data(x), data(q), static_cast<float*>(data(s)), M, n, round, kind, stream));
+    if (M > 0) check(lib.group_quant(data(x), data(q), floats(s), M, n, round, kind, stream));
   }
   return wrap({q, s});
   END_HANDLE_TH_ERRORS
 }
 
-#define FQ_FAST(f) reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(f))
-PyMethodDef methods[] = {{"bind", FQ_FAST(bind), METH_FASTCALL, nullptr},
-                         {"rmsnorm_quant", FQ_FAST(rmsnorm_quant), METH_FASTCALL, nullptr},
-                         {"swiglu_quant", FQ_FAST(swiglu_quant), METH_FASTCALL, nullptr},
-                         {"group_quant", FQ_FAST(group_quant), METH_FASTCALL, nullptr},
+// (x, round_scale, fp8 dtype, kind, stream)
+PyObject* block_quant(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+  HANDLE_TH_ERRORS
+  Args in(a, n_args, 5);
+  const at::Tensor x = in.tensor();
+  at::Tensor q, s;
+  const int round = in.flag();
+  const at::ScalarType fp8 = in.dtype();
+  const int kind = in.flag();
+  void* stream = in.address();
+  {
+    pybind11::gil_scoped_release no_gil;
+    const int64_t M = x.size(0), n = x.size(1);
+    q = empty(x, fp8, {M, n});
+    s = empty(x, at::kFloat, {M / 128, n / 128});
+    check(lib.block_quant(data(x), data(q), floats(s), M, n, round, kind, stream));
+  }
+  return wrap({q, s});
+  END_HANDLE_TH_ERRORS
+}
+
+// (x, round_scale, output_mode, fp8 dtype, kind, stream)
+PyObject* blockwise_quant(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+  HANDLE_TH_ERRORS
+  Args in(a, n_args, 6);
+  const at::Tensor x = in.tensor();
+  at::Tensor q, s, qt, st;
+  const int round = in.flag(), mode = in.flag();
+  const at::ScalarType fp8 = in.dtype();
+  const int kind = in.flag();
+  void* stream = in.address();
+  {
+    pybind11::gil_scoped_release no_gil;
+    const int64_t M = x.size(0), n = x.size(1);
+    q = empty(x, fp8, {M, n});
+    s = empty(x, at::kFloat, {n / 128, M});
+    qt = empty(x, fp8, {n, M});
+    st = empty(x, at::kFloat, {(M + 127) / 128, n});
+    if (M > 0)
+      check(lib.blockwise_quant(data(x), data(q), floats(s), data(qt), floats(st), M, n, round, mode, kind, stream));
+  }
+  return wrap({q, s, qt, st});
+  END_HANDLE_TH_ERRORS
+}
+
+// (x, counts, counts are int64, plan's table or None, plan's shape, blocks, round_scale, fp8 dtype, kind, stream)
+PyObject* batched_blockwise_quant(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+  HANDLE_TH_ERRORS
+  Args in(a, n_args, 10);
+  const at::Tensor x = in.tensor(), counts = in.tensor();
+  const int i64 = in.flag();
+  const at::Tensor plan = in.tensor();
+  const int64_t* shape = static_cast<const int64_t*>(in.address());
+  const int64_t blocks = in.integer();
+  const int round = in.flag();
+  const at::ScalarType fp8 = in.dtype();
+  const int kind = in.flag();
+  void* stream = in.address();
+  at::Tensor q, s, qt, st;
+  {
+    pybind11::gil_scoped_release no_gil;
+    const int64_t M = x.size(0), n = x.size(1);
+    q = empty(x, fp8, {M, n});
+    s = empty(x, at::kFloat, {M * n / 128});
+    qt = empty(x, fp8, {M * n});
+    st = empty(x, at::kFloat, {blocks * n});
+    if (M > 0 && plan.defined())
+      check(lib.batched_blockwise_quant_planned(data(x), data(plan), shape, data(q), floats(s), data(qt), floats(st), M,
+                                                n, round, kind, stream));
+    else if (M > 0)
+      check(lib.batched_blockwise_quant(data(x), data(counts), i64, static_cast<int>(counts.size(0)), blocks, data(q),
+                                        floats(s), data(qt), floats(st), M, n, round, kind, stream));
+  }
+  return wrap({q, s, qt, st});
+  END_HANDLE_TH_ERRORS
+}
+
+// (x, counts, counts are int64, plan's table or None, plan's shape, blocks, indices, probs or None, probs are bf16,
+// launch, round_scale, fp8 dtype, kind, stream); launch 0: the outputs alone
+PyObject* batched_pad_permute_quant(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+  HANDLE_TH_ERRORS
+  Args in(a, n_args, 14);
+  const at::Tensor x = in.tensor(), counts = in.tensor();
+  const int i64 = in.flag();
+  const at::Tensor plan = in.tensor();
+  const int64_t* shape = static_cast<const int64_t*>(in.address());
+  const int64_t blocks = in.integer();
+  const at::Tensor indices = in.tensor(), probs = in.tensor();
+  const int pbf16 = in.flag(), launch = in.flag(), round = in.flag();
+  const at::ScalarType fp8 = in.dtype();
+  const int kind = in.flag();
+  void* stream = in.address();
+  at::Tensor q, s, qt, st, prob_out;
+  {
+    pybind11::gil_scoped_release no_gil;
+    const int64_t m = x.size(0), n = x.size(1), M = indices.size(0);
+    const int experts = static_cast<int>(counts.size(0));
+    q = empty(x, fp8, {M, n});
+    s = empty(x, at::kFloat, {M, n / 128});
+    qt = empty(x, fp8, {M, n});
+    st = empty(x, at::kFloat, {blocks, n});
+    if (probs.defined()) prob_out = empty(x, probs.scalar_type(), {M});
+    if (launch && plan.defined())
+      check(lib.batched_pad_permute_quant_planned(data(x), data(plan), shape, experts, data(indices), data(probs),
+                                                  pbf16, data(prob_out), data(q), floats(s), data(qt), floats(st), m, M,
+                                                  n, round, kind, stream));
+    else if (launch)
+      check(lib.batched_pad_permute_quant(data(x), data(counts), i64, experts, blocks, data(indices), data(probs),
+                                          pbf16, data(prob_out), data(q), floats(s), data(qt), floats(st), m, M, n,
+                                          round, kind, stream));
+  }
+  return wrap({q, s, qt, st, prob_out});
+  END_HANDLE_TH_ERRORS
+}
+
+// (tokens per expert) -> (128-row blocks, rows with every expert's rounded up to 16)
+PyObject* expert_blocks(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(n_args == 1, "expected 1 argument, got ", n_args);
+  int64_t blocks = 0, padded = 0;
+  for (const int64_t c : ints_of(a[0])) {
+    blocks += (c + 127) >> 7;  // (below zero rounded as Python's // does)
+    padded += ((c + 15) >> 4) * 16;
+  }
+  PyObject* pair = Py_BuildValue("(LL)", static_cast<long long>(blocks), static_cast<long long>(padded));
+  if (!pair) throw python_error();
+  return pair;
+  END_HANDLE_TH_ERRORS
+}
+
+// (tokens per expert, pad, address of the plan's shape)
+PyObject* expert_plan_shape(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+  HANDLE_TH_ERRORS
+  Args in(a, n_args, 3);
+  const std::vector<int64_t> counts = in.integers();
+  const int pad = in.flag();
+  int64_t* shape = static_cast<int64_t*>(in.address());
+  const int64_t none = 0;
+  check(lib.expert_plan_shape(counts.empty() ? &none : counts.data(), static_cast<int>(counts.size()), pad, shape));
+  Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
+}
+
+#define FQ_METHOD(f) {#f, reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(f)), METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {FQ_METHOD(bind),
+                         FQ_METHOD(rmsnorm),
+                         FQ_METHOD(rmsnorm_bwd),
+                         FQ_METHOD(rmsnorm_quant),
+                         FQ_METHOD(rmsnorm_router_quant),
+                         FQ_METHOD(swiglu),
+                         FQ_METHOD(swiglu_bwd),
+                         FQ_METHOD(swiglu_quant),
+                         FQ_METHOD(swiglu_quant_bwd),
+                         FQ_METHOD(batched_swiglu_quant),
+                         FQ_METHOD(batched_swiglu_quant_bwd),
+                         FQ_METHOD(group_quant),
+                         FQ_METHOD(block_quant),
+                         FQ_METHOD(blockwise_quant),
+                         FQ_METHOD(batched_blockwise_quant),
+                         FQ_METHOD(batched_pad_permute_quant),
+                         FQ_METHOD(expert_blocks),
+                         FQ_METHOD(expert_plan_shape),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_fq_torch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace
 
-extern "C" PyObject* PyInit__fq_torch() { return PyModule_Create(&module); }
+extern "C" PyObject* PyInit__fq_torch() {
+  PyObject* m = PyModule_Create(&module);
+#define FQ_NAME(name) "fq_" #name,
+  const char* const names[] = {FQ_FUNCTIONS(FQ_NAME)};
+#undef FQ_NAME
+  PyObject* functions = m ? PyTuple_New(static_cast<Py_ssize_t>(std::size(names))) : nullptr;
+  for (Py_ssize_t i = 0; functions && i < static_cast<Py_ssize_t>(std::size(names)); ++i) {
+    PyObject* name = PyUnicode_FromString(names[i]);
+    if (!name) Py_CLEAR(functions);
+    else PyTuple_SET_ITEM(functions, i, name);
+  }
+  if (!functions || PyModule_AddObject(m, "FUNCTIONS", functions) < 0) {
+    Py_XDECREF(functions);
+    Py_CLEAR(m);
+  }
+  return m;
+}

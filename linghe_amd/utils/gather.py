@@ -5,6 +5,8 @@ extension (the reference always emits e4m3fn).
 """
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from .. import _lib
@@ -38,22 +40,16 @@ def triton_batch_block_pad_permute_with_indices(
     n_experts = token_count_per_expert.size(0)
     M = indices.shape[0]
     device = xs.device
-    x_q = torch.empty((M, N), device=device, dtype=fp8_dtype)
-    x_scale = torch.empty((M, N // 128), device=device, dtype=torch.float32)
-    blocks = sum((int(c) + 127) // 128 for c in splits)
-    xt_q = torch.empty((M, N), device=device, dtype=fp8_dtype)
-    xt_scale = torch.empty((blocks, N), device=device, dtype=torch.float32)
-    prob_output = None
-    if probs is not None:
-        prob_output = torch.empty((M,), device=device, dtype=probs.dtype)
+    blocks, padded = _lib.native.expert_blocks(splits)
+    counts = token_count_per_expert
     if m == 0 or M == 0:
-        return x_q, x_scale, xt_q, xt_scale, prob_output
-    padded = sum((int(c) + 15) // 16 * 16 for c in splits)
+        with _lib.on_device(device):
+            return _lib.native.batched_pad_permute_quant(xs, counts, 0, None, 0, blocks, indices, probs, 0, 0, 0,
+                                                         fp8_dtype, 0, _lib.stream_of(xs))
     assert M == padded, f"indices holds {M} entries, the counts rounded up to 16 add up to {padded}"
     if indices.dtype != torch.int32:
         raise TypeError(f"indices must be int32, got {indices.dtype}")
     assert indices.is_contiguous() and token_count_per_expert.is_contiguous()
-    counts = token_count_per_expert
     if counts.dtype == torch.int64:
         is64 = 1
     elif counts.dtype == torch.int32:
@@ -67,18 +63,12 @@ def triton_batch_block_pad_permute_with_indices(
             pbf16 = 1
         elif probs.dtype != torch.float32:
             raise TypeError(f"probs must be float32 or bfloat16, got {probs.dtype}")
+    table, shape = None, 0
     if plan is not None:
         if plan.blocks != blocks or plan.pad != 16 or plan.table.device != device:
             raise ValueError("plan does not belong to these splits / this layout (pad=16) / this device")
-        with _lib.on_device(device):
-            _lib.check(_lib.lib.fq_batched_pad_permute_quant_planned(
-                _lib.ptr(xs), _lib.ptr(plan.table), plan.shape, n_experts, _lib.ptr(indices), _lib.ptr(probs), pbf16,
-                _lib.ptr(prob_output), _lib.ptr(x_q), _lib.ptr(x_scale), _lib.ptr(xt_q), _lib.ptr(xt_scale), m, M, N,
-                int(bool(round_scale)), _lib.fp8_kind(fp8_dtype), _lib.stream_of(xs)))
-        return x_q, x_scale, xt_q, xt_scale, prob_output
+        table, shape = plan.table, ctypes.addressof(plan.shape)
     with _lib.on_device(device):
-        _lib.check(_lib.lib.fq_batched_pad_permute_quant(
-            _lib.ptr(xs), _lib.ptr(counts), is64, n_experts, blocks, _lib.ptr(indices),
-            _lib.ptr(probs), pbf16, _lib.ptr(prob_output), _lib.ptr(x_q), _lib.ptr(x_scale), _lib.ptr(xt_q),
-            _lib.ptr(xt_scale), m, M, N, int(bool(round_scale)), _lib.fp8_kind(fp8_dtype), _lib.stream_of(xs)))
-    return x_q, x_scale, xt_q, xt_scale, prob_output
+        return _lib.native.batched_pad_permute_quant(xs, counts, is64, table, shape, blocks, indices, probs, pbf16, 1,
+                                                     int(bool(round_scale)), fp8_dtype, _lib.fp8_kind(fp8_dtype),
+                                                     _lib.stream_of(xs))

@@ -45,16 +45,11 @@ def triton_rms_norm_forward(x, weight, eps=1e-6, out=None, rms=None):
     _check_hidden(n)
     _lib.require_device_bf16(x, "x")
     _lib.require_device_bf16(weight, "weight")
-    if out is None:
+    if out is None and type(x) is not torch.Tensor:  # (a subclass may have its own)
         out = torch.empty_like(x)
-    reuse = rms is not None
-    if not reuse:
-        rms = torch.empty((M,), device=x.device, dtype=torch.float32)
-    if M > 0:
-        with _lib.on_device(x.device):
-            _lib.check(_lib.lib.fq_rmsnorm_fwd(_lib.ptr(x), _lib.ptr(weight), _lib.ptr(out), _lib.ptr(rms),
-                                               M, n, float(eps), int(reuse), _lib.stream_of(x)))
-    return out, rms
+    with _lib.on_device(x.device):
+        new = _lib.native.rmsnorm(x, weight, out, rms, M, n, float(eps), int(rms is not None), _lib.stream_of(x))
+    return new[0] if out is None else out, new[1] if rms is None else rms
 
 
 def triton_rms_norm_backward(grad_output, x, w, eps=1e-6, rms=None):
@@ -71,15 +66,10 @@ def triton_rms_norm_backward(grad_output, x, w, eps=1e-6, rms=None):
     _lib.require_device_bf16(grad_output, "grad_output")
     _lib.require_device_bf16(w, "w")
     assert x.is_contiguous() and w.is_contiguous()
-    dx = torch.empty_like(x)
-    dw = torch.empty((n,), dtype=torch.float32, device=w.device)
-    n_part = int(_lib.lib.fq_rmsnorm_bwd_num_partials(M, n))
-    tmp_dw = torch.empty((n_part, n), dtype=torch.float32, device=w.device)
+    dx = None if type(x) is torch.Tensor else torch.empty_like(x)  # (a subclass may have its own)
     with _lib.on_device(x.device):
-        _lib.check(_lib.lib.fq_rmsnorm_bwd(_lib.ptr(grad_output), _lib.ptr(x), _lib.ptr(w), _lib.ptr(rms),
-                                           _lib.ptr(dx), _lib.ptr(dw), _lib.ptr(tmp_dw), n_part, M, n,
-                                           float(eps), _lib.stream_of(x)))
-    return dx, dw
+        new = _lib.native.rmsnorm_bwd(grad_output, x, w, rms, dx, M, n, float(eps), _lib.stream_of(x))
+    return new if dx is None else (dx, new[1])
 
 
 def triton_rms_norm_and_block_quant_forward(
@@ -207,44 +197,22 @@ def triton_rms_norm_fp32_gemm_block_quant_forward(
     _lib.require_device_bf16(x, "x")
     _lib.require_device_bf16(norm_weight, "norm_weight")
     device = x.device
-    y = torch.empty(M, K, dtype=x.dtype, device=device)
     if rms is None:
         assert output_mode == 0
-        rms = torch.empty(M, dtype=torch.float32, device=device)
-    logits = torch.empty(M, N, dtype=torch.float32, device=device)
-    x_q = torch.empty((M, K), device=device, dtype=torch.float8_e4m3fn)
-    x_s = torch.empty((K // 128, M), device=device, dtype=torch.float32)
-    xt_q = torch.empty((K, M), device=device, dtype=torch.float8_e4m3fn)
-    xt_s = torch.empty((M // 128, K), device=device, dtype=torch.float32)
-    if M == 0:
-        return y, rms, logits, x_q, x_s, xt_q, xt_s
+    w_fp32, need, packed = 0, 0, None
+    if output_mode == 0 and M > 0:
+        if route_weight.dtype not in (torch.bfloat16, torch.float32):
+            raise TypeError(f"route_weight must be bfloat16 or float32, got {route_weight.dtype}")
+        if not route_weight.is_cuda:
+            raise RuntimeError("route_weight must live on the GPU: the HIP kernels are the only implementation")
+        w_fp32 = int(route_weight.dtype == torch.float32)
+        need = int(_lib.lib.fq_rmsnorm_router_scratch_bytes(K, N, w_fp32))
+        if packed_route_weight is not None:
+            assert packed_route_weight.is_cuda and packed_route_weight.dtype == torch.uint8
+            assert packed_route_weight.numel() == need and packed_route_weight.is_contiguous()
+            if route_weight.data_ptr() % 16 or not _lib.lib.fq_rmsnorm_router_folds(M, K, N, w_fp32):
+                packed = packed_route_weight
     with _lib.on_device(device):
-        if output_mode == 0:
-            if route_weight.dtype not in (torch.bfloat16, torch.float32):
-                raise TypeError(f"route_weight must be bfloat16 or float32, got {route_weight.dtype}")
-            if not route_weight.is_cuda:
-                raise RuntimeError("route_weight must live on the GPU: the HIP kernels are the only implementation")
-            w_fp32 = int(route_weight.dtype == torch.float32)
-            need = int(_lib.lib.fq_rmsnorm_router_scratch_bytes(K, N, w_fp32))
-            if packed_route_weight is not None:
-                assert packed_route_weight.is_cuda and packed_route_weight.dtype == torch.uint8
-                assert packed_route_weight.numel() == need and packed_route_weight.is_contiguous()
-            if packed_route_weight is not None and (route_weight.data_ptr() % 16 or
-                                                    not _lib.lib.fq_rmsnorm_router_folds(M, K, N, w_fp32)):
-                _lib.check(_lib.lib.fq_rmsnorm_router_quant_fwd_packed(
-                    _lib.ptr(x), _lib.ptr(norm_weight), _lib.ptr(packed_route_weight), w_fp32, _lib.ptr(y),
-                    _lib.ptr(rms), _lib.ptr(logits), _lib.ptr(x_q), _lib.ptr(x_s), M, K, N, float(eps),
-                    int(bool(round_scale)), _lib.FQ_E4M3, _lib.stream_of(x)))
-            else:
-                # route_weight re-ordered for the matrix cores (an fp32 weight as two bf16 planes, in the larger calls
-                # of gamma * route_weight, which depends on both and is made by every call)
-                scratch = torch.empty(need, dtype=torch.uint8, device=device)
-                _lib.check(_lib.lib.fq_rmsnorm_router_quant_fwd(
-                    _lib.ptr(x), _lib.ptr(norm_weight), _lib.ptr(route_weight), w_fp32, _lib.ptr(scratch),
-                    _lib.ptr(y), _lib.ptr(rms), _lib.ptr(logits), _lib.ptr(x_q), _lib.ptr(x_s), M, K, N, float(eps),
-                    int(bool(round_scale)), _lib.FQ_E4M3, _lib.stream_of(x)))
-        else:
-            _lib.check(_lib.lib.fq_rmsnorm_quant_fwd(
-                _lib.ptr(x), _lib.ptr(norm_weight), None, None, _lib.ptr(rms), _lib.ptr(xt_q), _lib.ptr(xt_s),
-                M, K, float(eps), int(bool(round_scale)), 1, _lib.FQ_E4M3, _lib.stream_of(x)))
-    return y, rms, logits, x_q, x_s, xt_q, xt_s
+        new = _lib.native.rmsnorm_router_quant(x, norm_weight, route_weight, packed, w_fp32, need, rms, output_mode,
+                                               float(eps), int(bool(round_scale)), _lib.stream_of(x))
+    return new if rms is None else (new[0], rms, *new[2:])

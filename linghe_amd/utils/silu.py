@@ -5,13 +5,11 @@ keyword-only extension (the reference always emits e4m3fn).
 """
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from .. import _lib
-
-
-def _blocks_of(splits) -> int:
-    return sum((int(c) + 127) // 128 for c in splits)
 
 
 class ExpertPlan:
@@ -39,12 +37,8 @@ def build_expert_plan(counts: torch.Tensor, splits, pad: int = 1) -> ExpertPlan:
     """counts: device int32/int64 [n_experts]; splits: the same numbers as a python list;
     pad: 1 for the layouts with the experts back to back (SwiGLU, blockwise quantiser), 16 for
     gather + pad + quant (every expert's region of the outputs rounded up to 16 rows)."""
-    import ctypes
-
-    n = len(splits)
-    host = (ctypes.c_int64 * max(n, 1))(*[int(c) for c in splits])
     shape = (ctypes.c_int64 * 5)()
-    _lib.check(_lib.lib.fq_expert_plan_shape(host, n, pad, shape))
+    _lib.native.expert_plan_shape(splits, pad, ctypes.addressof(shape))
     nbytes = int(_lib.lib.fq_expert_plan_bytes(shape))
     table = torch.empty((max(nbytes, 16),), device=counts.device, dtype=torch.uint8)
     if shape[0]:
@@ -72,6 +66,14 @@ def _counts_flag(counts: torch.Tensor) -> int:
     raise TypeError(f"counts must be int32 or int64, got {counts.dtype}")
 
 
+def _tiles_of(plan, blocks: int, counts: torch.Tensor, device):
+    """Where the native call finds its tiles: counts and their flag, or a plan's table and the address of its shape."""
+    if plan is None:
+        return counts, _counts_flag(counts), None, 0
+    _check_plan(plan, blocks, device)
+    return None, 0, plan.table, ctypes.addressof(plan.shape)
+
+
 def _weight_flag(weight: torch.Tensor) -> int:
     if weight.dtype == torch.float32:
         return 0
@@ -94,16 +96,13 @@ def triton_weighted_silu_forward(x, weight=None, out=None, asm=False):
     _lib.require_device_bf16(x, "x")
     M, N = x.shape
     assert N % 256 == 0
-    if out is None:
-        out = torch.empty((M, N // 2), device=x.device, dtype=x.dtype)
     wflag = 0
     if weight is not None:
         assert weight.is_contiguous() and weight.numel() == M
         wflag = _weight_flag(weight)
     with _lib.on_device(x.device):
-        _lib.check(_lib.lib.fq_swiglu_fwd(_lib.ptr(x), _lib.ptr(weight), wflag, _lib.ptr(out), M, N // 2,
-                                          _lib.stream_of(x)))
-    return out
+        new = _lib.native.swiglu(x, weight, wflag, out, _lib.stream_of(x))
+    return new if out is None else out
 
 
 def triton_weighted_silu_backward(g, x, weight=None):
@@ -124,16 +123,12 @@ def triton_weighted_silu_backward(g, x, weight=None):
     M, N = x.shape
     assert N % 256 == 0
     assert g.shape == (M, N // 2)
-    dw, wflag = None, 0
+    wflag = 0
     if weight is not None:
         assert weight.is_contiguous() and weight.numel() == M
         wflag = _weight_flag(weight)
-        dw = torch.empty(weight.shape, device=x.device, dtype=weight.dtype)
-    dx = torch.empty((M, N), device=x.device, dtype=x.dtype)
     with _lib.on_device(x.device):
-        _lib.check(_lib.lib.fq_swiglu_bwd(_lib.ptr(g), _lib.ptr(x), _lib.ptr(weight), wflag, _lib.ptr(dx),
-                                          _lib.ptr(dw), M, N // 2, _lib.stream_of(x)))
-    return dx, dw
+        return _lib.native.swiglu_bwd(g, x, weight, wflag, _lib.stream_of(x))
 
 
 def triton_silu_and_block_quant_forward(
@@ -190,17 +185,9 @@ def triton_silu_and_block_quant_backward(g, x, round_scale=False, *, fp8_dtype=t
     _lib.require_device_bf16(x, "x")
     _lib.require_device_bf16(g, "g")
     device = x.device
-    dx = torch.empty((M, N), device=device, dtype=fp8_dtype)
-    dx_scale = torch.empty((N // 128, M), device=device, dtype=torch.float32)
-    transpose_dx = torch.empty((N, M), device=device, dtype=fp8_dtype)
-    transpose_dx_scale = torch.empty(((M + 127) // 128, N), device=device, dtype=torch.float32)
-    if M > 0:
-        with _lib.on_device(device):
-            _lib.check(_lib.lib.fq_swiglu_quant_bwd(
-                _lib.ptr(g), _lib.ptr(x), _lib.ptr(dx), _lib.ptr(dx_scale), _lib.ptr(transpose_dx),
-                _lib.ptr(transpose_dx_scale), M, n, int(bool(round_scale)), _lib.fp8_kind(fp8_dtype),
-                _lib.stream_of(x)))
-    return dx, dx_scale, transpose_dx, transpose_dx_scale
+    with _lib.on_device(device):
+        return _lib.native.swiglu_quant_bwd(g, x, int(bool(round_scale)), fp8_dtype,
+                                            _lib.fp8_kind(fp8_dtype) if M else 0, _lib.stream_of(x))
 
 
 def triton_batch_weighted_silu_and_block_quant_forward(
@@ -238,36 +225,20 @@ def triton_batch_weighted_silu_and_block_quant_forward(
     _lib.require_device_bf16(x, "x")
     M, N = x.shape
     n = N // 2
-    n_experts = counts.shape[0]
     assert N <= 8192
     assert n % 128 == 0 and N == 2 * n
     assert output_mode in (0, 1, 2)
     assert weight.numel() == M
     device = x.device
-    if out is None:
-        out = torch.empty((M, n), device=device, dtype=fp8_dtype)
-    if scale is None:
-        scale = torch.empty((M, n // 128), device=device, dtype=torch.float32)
-    blocks = _blocks_of(splits)
-    transpose_output = torch.empty((M, n), device=device, dtype=fp8_dtype)
-    transpose_scale = torch.empty((blocks, n), device=device, dtype=torch.float32)
-    if M == 0:
-        return out, scale, transpose_output, transpose_scale
-    if plan is not None:
-        _check_plan(plan, blocks, device)
-        with _lib.on_device(device):
-            _lib.check(_lib.lib.fq_batched_swiglu_quant_fwd_planned(
-                _lib.ptr(x), _lib.ptr(weight), _weight_flag(weight), _lib.ptr(plan.table), plan.shape,
-                _lib.ptr(out), _lib.ptr(scale), _lib.ptr(transpose_output), _lib.ptr(transpose_scale), M, n,
-                int(bool(round_scale)), output_mode, _lib.fp8_kind(fp8_dtype), _lib.stream_of(x)))
-        return out, scale, transpose_output, transpose_scale
+    blocks, _ = _lib.native.expert_blocks(splits)
+    tiles, wflag, kind = (None, 0, None, 0), 0, 0
+    if M > 0:
+        tiles = _tiles_of(plan, blocks, counts, device)
+        wflag, kind = _weight_flag(weight), _lib.fp8_kind(fp8_dtype)
     with _lib.on_device(device):
-        _lib.check(_lib.lib.fq_batched_swiglu_quant_fwd(
-            _lib.ptr(x), _lib.ptr(weight), _weight_flag(weight), _lib.ptr(counts), _counts_flag(counts),
-            n_experts, blocks, _lib.ptr(out), _lib.ptr(scale), _lib.ptr(transpose_output),
-            _lib.ptr(transpose_scale), M, n, int(bool(round_scale)), output_mode,
-            _lib.fp8_kind(fp8_dtype), _lib.stream_of(x)))
-    return out, scale, transpose_output, transpose_scale
+        new = _lib.native.batched_swiglu_quant(x, weight, wflag, *tiles, blocks, out, scale, int(bool(round_scale)),
+                                               output_mode, fp8_dtype, kind, _lib.stream_of(x))
+    return new[0] if out is None else out, new[1] if scale is None else scale, new[2], new[3]
 
 
 def triton_batch_weighted_silu_and_block_quant_backward(
@@ -285,7 +256,6 @@ def triton_batch_weighted_silu_and_block_quant_backward(
     """
     M, N = x.shape
     n = N // 2
-    n_expert = counts.shape[0]
     assert n % 128 == 0
     assert g.is_contiguous()
     assert x.is_contiguous() and weight.is_contiguous()
@@ -293,28 +263,13 @@ def triton_batch_weighted_silu_and_block_quant_backward(
     _lib.require_device_bf16(x, "x")
     _lib.require_device_bf16(g, "g")
     device = x.device
-    dx = torch.empty((M, N), device=device, dtype=fp8_dtype)
-    dx_scale = torch.empty((M, N // 128), device=device, dtype=torch.float32)
-    s = _blocks_of(splits)
-    transpose_dx = torch.empty((M, N), device=device, dtype=fp8_dtype)
-    transpose_dx_scale = torch.empty((s, N), device=device, dtype=torch.float32)
-    dw = torch.empty_like(weight)
-    if s == 0:
-        return dx, dx_scale, dw, transpose_dx, transpose_dx_scale
-    dws = torch.empty((M, n // 128), device=device, dtype=torch.float32)
-    if plan is not None:
-        _check_plan(plan, s, device)
-        with _lib.on_device(device):
-            _lib.check(_lib.lib.fq_batched_swiglu_quant_bwd_planned(
-                _lib.ptr(g), _lib.ptr(x), _lib.ptr(weight), _weight_flag(weight), _lib.ptr(plan.table), plan.shape,
-                _lib.ptr(dx), _lib.ptr(dx_scale), _lib.ptr(dw), _lib.ptr(transpose_dx),
-                _lib.ptr(transpose_dx_scale), _lib.ptr(dws), M, n, int(bool(round_scale)),
-                _lib.fp8_kind(fp8_dtype), _lib.stream_of(x)))
-        return dx, dx_scale, dw, transpose_dx, transpose_dx_scale
+    blocks, _ = _lib.native.expert_blocks(splits)
+    dw = None if type(weight) is torch.Tensor else torch.empty_like(weight)  # (a subclass may have its own)
+    tiles, wflag, kind = (None, 0, None, 0), 0, 0
+    if blocks != 0:
+        tiles = _tiles_of(plan, blocks, counts, device)
+        wflag, kind = _weight_flag(weight), _lib.fp8_kind(fp8_dtype)
     with _lib.on_device(device):
-        _lib.check(_lib.lib.fq_batched_swiglu_quant_bwd(
-            _lib.ptr(g), _lib.ptr(x), _lib.ptr(weight), _weight_flag(weight), _lib.ptr(counts),
-            _counts_flag(counts), n_expert, s, _lib.ptr(dx), _lib.ptr(dx_scale), _lib.ptr(dw),
-            _lib.ptr(transpose_dx), _lib.ptr(transpose_dx_scale), _lib.ptr(dws), M, n,
-            int(bool(round_scale)), _lib.fp8_kind(fp8_dtype), _lib.stream_of(x)))
-    return dx, dx_scale, dw, transpose_dx, transpose_dx_scale
+        new = _lib.native.batched_swiglu_quant_bwd(g, x, weight, wflag, dw, *tiles, blocks, int(bool(round_scale)),
+                                                   fp8_dtype, kind, _lib.stream_of(x))
+    return new if dw is None else (new[0], new[1], dw, new[3], new[4])

@@ -12,6 +12,7 @@ import sys
 import textwrap
 
 import pytest
+import torch
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HEADER = os.path.join(ROOT, "include", "fq_api.h")
@@ -352,3 +353,23 @@ def test_build_needs_one_compiler(monkeypatch):
     B.build_library()
     assert len(commands) == len(B.SOURCES) + 2
     assert {c[0] for c in commands} == {B._hipcc()}
+
+
+@pytest.mark.parametrize("splits", [[], [0], [1, 15, 16, 17, 0, 127, 128, 129], (5, -1, -16, -129), [True, 2.9, "7"],
+                                    torch.tensor([3, 200]), range(300)])
+def test_expert_blocks_are_those_of_the_counts(splits):
+    """Any iterable of what int() takes; 128-row blocks and rows in units of 16, rounded as Python's // rounds."""
+    from linghe_amd import _lib
+
+    want = [int(c) for c in splits]
+    assert _lib.native.expert_blocks(splits) == (sum((c + 127) // 128 for c in want),
+                                                 sum((c + 15) // 16 * 16 for c in want))
+
+
+@pytest.mark.parametrize("splits,error", [(5, TypeError), ([None], TypeError), (["a"], ValueError),
+                                          ([1 << 40], RuntimeError), ([1 << 70], OverflowError)])
+def test_expert_blocks_refuses(splits, error):
+    from linghe_amd import _lib
+
+    with pytest.raises(error):
+        _lib.native.expert_blocks(splits)

@@ -277,3 +277,33 @@ def test_entry_points_under_graph_capture(gpu):
         for k, (a, b) in enumerate(zip(want, got)):
             assert torch.equal(a, b), (rep, k)
         _ = (src.float() * 2).sum().item()  # eager work between the replays
+
+
+class OwnTensor(torch.Tensor):
+    pass
+
+
+@pytest.mark.parametrize("M", [0, 128])
+def test_given_and_own_outputs(gpu, M):
+    """Buffers that the caller gives are those that come back; what takes its type from an input keeps it; no rows."""
+    from linghe_amd.utils.norm import triton_rms_norm_backward, triton_rms_norm_forward
+    from linghe_amd.utils.silu import (triton_batch_weighted_silu_and_block_quant_backward,
+                                       triton_weighted_silu_backward, triton_weighted_silu_forward)
+
+    x, h = (torch.randn(M, n, device=gpu).bfloat16() for n in (256, 512))
+    gamma, w = torch.ones(256, device=gpu).bfloat16(), torch.rand(M, 1, device=gpu)
+    out, rms = torch.empty_like(x), torch.empty(M, device=gpu)
+    y, r = triton_rms_norm_forward(x, gamma)
+    assert y.shape == x.shape and r.shape == (M,)
+    rms.copy_(r)
+    got = triton_rms_norm_forward(x, gamma, out=out, rms=rms)
+    assert got[0] is out and got[1] is rms and torch.equal(out, y)
+    assert triton_weighted_silu_forward(h, w, out=out) is out and triton_weighted_silu_forward(h).shape == x.shape
+    dh, dw = triton_weighted_silu_backward(x, h, w.view(-1))
+    assert dh.shape == h.shape and dw.shape == (M,) and triton_weighted_silu_backward(x, h)[1] is None
+    own = x.as_subclass(OwnTensor)
+    assert type(triton_rms_norm_forward(own, gamma)[0]) is OwnTensor
+    assert type(triton_rms_norm_backward(x, own, gamma, rms=rms)[0]) is OwnTensor
+    counts = torch.tensor([M, 0], device=gpu)
+    new = triton_batch_weighted_silu_and_block_quant_backward(x, h, w.as_subclass(OwnTensor), counts, [M, 0])
+    assert type(new[2]) is OwnTensor and new[2].shape == (M, 1) and new[4].shape == (M // 128, 512)
