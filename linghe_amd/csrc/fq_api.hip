@@ -294,8 +294,7 @@ int fq_rmsnorm_fwd(const void* x, const void* gamma, void* out, float* rstd, int
 }
 
 int64_t fq_rmsnorm_bwd_num_partials(int64_t M, int64_t n) {
-  (void)n;
-  return fq::rmsnorm_bwd_partials(M);
+  return fq::rmsnorm_bwd_partials(M, n);
 }
 
 int fq_rmsnorm_bwd(const void* dy, const void* x, const void* gamma, const float* rstd, void* dx, float* dgamma,
@@ -304,7 +303,7 @@ int fq_rmsnorm_bwd(const void* dy, const void* x, const void* gamma, const float
   int rc = check_norm_shape(fn, M, n);
   if (rc) return rc;
   FQ_REQUIRE(dgamma, FQ_ERR_ARG, "%s: dgamma is NULL", fn);
-  FQ_REQUIRE(n_partials == fq::rmsnorm_bwd_partials(M), FQ_ERR_SHAPE,
+  FQ_REQUIRE(n_partials == fq::rmsnorm_bwd_partials(M, n), FQ_ERR_SHAPE,
              "%s: n_partials must equal fq_rmsnorm_bwd_num_partials(M, n)", fn);
   if (M > 0) {  // with no rows only dgamma is touched (it is zeroed); the row kernel is not launched
     FQ_REQUIRE(dy && x && gamma && dx && dgamma_partials, FQ_ERR_ARG, "%s: NULL pointer", fn);
@@ -322,7 +321,7 @@ int fq_rmsnorm_bwd_noalloc(const void* dy, const void* x, const void* gamma, con
   int rc = check_norm_shape(fn, M, n);
   if (rc) return rc;
   FQ_REQUIRE(dgamma, FQ_ERR_ARG, "%s: dgamma is NULL", fn);
-  const int64_t need = fq::rmsnorm_bwd_partials(M) * n * (int64_t)sizeof(float);
+  const int64_t need = fq::rmsnorm_bwd_partials(M, n) * n * (int64_t)sizeof(float);
   FQ_REQUIRE(need <= fq::rmsnorm_bwd_static_scratch_bytes(), FQ_ERR_SHAPE,
              "%s: %lld bytes of dgamma partials exceed the library's fixed %lld-byte scratch array", fn,
              (long long)need, (long long)fq::rmsnorm_bwd_static_scratch_bytes());

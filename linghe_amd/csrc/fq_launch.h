@@ -64,7 +64,7 @@ hipError_t launch_rmsnorm_fwd(const void* x, const void* gamma, void* out, float
                               int n, float eps, int reuse_rstd, int quant, int round_scale, int kind,
                               hipStream_t stream);
 
-int64_t rmsnorm_bwd_partials(int64_t M);
+int64_t rmsnorm_bwd_partials(int64_t M, int64_t n);
 
 hipError_t launch_rmsnorm_bwd(const void* dy, const void* x, const void* gamma, const float* rstd, void* dx,
                               float* dgamma, float* dg_part, int64_t n_partials, int64_t M, int n, float eps,

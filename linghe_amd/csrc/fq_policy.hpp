@@ -131,6 +131,13 @@ struct Policy {
   static constexpr int kRowQuantLoopingMin = 8192, kRowQuantIdleShare = 24;
   static constexpr int kRowQuantLoopingPerCu = 16, kRowQuantLooping8192 = 4;
   static constexpr bool kPrefetchRowQuantWide = true;  // (they load a row ahead: 68.5 -> 65.5 us at 16384 x 7168)
+  // Rows of a workgroup of the RMSNorm backward where 512 workgroups are not reached. It writes one partial row of
+  // dgamma and walks its rows one after the other, so that eight each (before) left most of the chip idle. Up to 2048
+  // columns one row for each of the four waves (us 8 / 4 / 1 rows: 32 x 2048 7.7 / 6.4 / 6.8, 512 x 2048 8.8 / 7.4 /
+  // 9.2, 1024 x 640 7.2 / 6.3 / 7.0). Wider rows take the whole workgroup: one workgroup per CU up to 1024 rows, then
+  // three rows each (8 / 4 / 3 / 2 / 1 rows: 32 x 7168 16.2 / 10.3 / 9.3 / 7.9 / 6.7, 512 x 2944 13.8 / 9.8 / 8.5 / 8.5 /
+  // 9.7, 1024 x 4096 15.7 / 12.3 / 13.0 / 13.3 / 13.3, 1448 x 5120 20.2 / 18.2 / 18.0 / 18.4 / 18.3).
+  static constexpr int kRowBwdRowsNarrow = 4, kRowBwdOnePerCu = 1024, kRowBwdRowsWide = 3;
   // the same in the wide-row RMSNorm backward with one chunk per thread (2048 < n <= 4096: 70.4 -> 66.9 us at
   // 16384 x 3072, 78.5 -> 76.4 at 16384 x 4096); with two chunks the second register set spills
   static constexpr bool kPrefetchRowBwdWide = true;

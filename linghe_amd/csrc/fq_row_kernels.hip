@@ -577,7 +577,7 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_wave_kernel(const uint16_t* _
 }
 
 // dgamma[c] = sum_p part[p, c] in a fixed order: 32 strided slices of p, each
-// summed sequentially (loads issued eight ahead), then combined 0..31.
+// summed by eights (loads issued eight ahead), then combined in pairs.
 // 32 columns per workgroup of 1024 threads: bound by the trips to memory of a slice, two at 512
 // partial rows; with 64 columns and 16 slices four, on half the CUs.  us of the whole backward,
 // 64 / 32 / 16 columns: 1000 x 2048 10.8 / 10.0 / 9.7, 4096 x 1024 10.9 / 10.4 / 10.8, 8192 x 2048
@@ -585,6 +585,15 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_wave_kernel(const uint16_t* _
 // Up to 16 partial rows (128 rows of the matrix) 64 columns and 16 slices: the sum over 32 slices, most of them empty,
 // is the longer chain (32 / 64 columns, 1 x 1024 4.78 / 4.58, 64 x 1024 6.11 / 5.88, 9 x 512 5.09 / 4.84).
 constexpr int kColsumFewPartials = 16;
+// (in pairs, then pairs of pairs: one partial row a workgroup makes many of them, and a chain rounds once for each)
+template <int N>
+__device__ __forceinline__ float pairwise_sum(float (&v)[N]) {
+#pragma unroll
+  for (int h = N / 2; h > 0; h /= 2)
+#pragma unroll
+    for (int k = 0; k < h; ++k) v[k] += v[k + h];
+  return v[0];
+}
 template <int kCols>
 __global__ __launch_bounds__(1024) void colsum_kernel(const float* __restrict__ part, float* __restrict__ out,
                                                       int P, int n) {
@@ -601,18 +610,27 @@ __global__ __launch_bounds__(1024) void colsum_kernel(const float* __restrict__ 
       float v[8];
 #pragma unroll
       for (int u = 0; u < 8; ++u) v[u] = src[(int64_t)(p + u * kSlices) * n];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) acc += v[u];
+      acc += pairwise_sum(v);
     }
-    for (; p < P; p += kSlices) acc += src[(int64_t)p * n];
+    if (p + kSlices < P) {  // what is left, at once too: one after the other they are a chain of trips to memory
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 7; ++u) v[u] = src[(int64_t)(p + u * kSlices < P ? p + u * kSlices : p) * n];
+#pragma unroll
+      for (int u = 1; u < 7; ++u) v[u] = p + u * kSlices < P ? v[u] : 0.f;
+      v[7] = 0.f;
+      acc += pairwise_sum(v);
+    } else if (p < P) {
+      acc += src[(int64_t)p * n];
+    }
   }
   red[slice][lane] = acc;
   __syncthreads();
   if (slice == 0 && col < n) {
-    float tot = red[0][lane];
+    float v[kSlices];
 #pragma unroll
-    for (int k = 1; k < kSlices; ++k) tot += red[k][lane];
-    out[col] = tot;
+    for (int k = 0; k < kSlices; ++k) v[k] = red[k][lane];
+    out[col] = pairwise_sum(v);
   }
 }
 
@@ -788,10 +806,14 @@ bool rmsnorm_passes_by_xcd(int64_t M, int n) {
   return M % kGroup == 0 && M * n * 2 <= (int64_t)Policy::kRmsnormByXcdMaxBytes;
 }
 
-int64_t rmsnorm_bwd_partials(int64_t M) {
+int64_t rmsnorm_bwd_partials(int64_t M, int64_t n) {
   // one partial row of dgamma per workgroup; 512 workgroups (two per CU) at most
-  const int64_t min_rows = 8;
-  int64_t p = (M + min_rows - 1) / min_rows;
+  int64_t rows = Policy::kRowBwdRowsNarrow;  // a workgroup
+  if (n > 2048)  // (up to 8 rows one workgroup adds them all: apart each product of dgamma would be rounded by itself)
+    rows = M <= 8 ? 8 : M <= Policy::kRowBwdOnePerCu ? (M + 255) / 256 : Policy::kRowBwdRowsWide;
+  else if (M <= 8)
+    rows = 8;
+  int64_t p = (M + rows - 1) / rows;
   if (p > 512) p = 512;
   if (p < 1) p = 1;
   return p;
@@ -884,7 +906,7 @@ hipError_t static_scratch_ptr(const void* device_ptr, float** out) {
 
 hipError_t launch_rmsnorm_bwd_static(const void* dy, const void* x, const void* gamma, const float* rstd, void* dx,
                                      float* dgamma, int64_t M, int n, float eps, hipStream_t stream) {
-  const int64_t P = rmsnorm_bwd_partials(M);
+  const int64_t P = rmsnorm_bwd_partials(M, n);
   if (P > kStaticPartialRows || n > kStaticPartialWidth) return hipErrorInvalidValue;
   float* part = nullptr;
   const hipError_t err = static_scratch_ptr(dgamma, &part);

@@ -7,10 +7,10 @@
 // The kernel library is the one that _lib.py loaded: bind() takes its functions' addresses, there is no
 // link-time dependency that could bring a second one into the process.
 // us through ctypes / here, back to back: RMSNorm + group + SwiGLU quantiser on 32 rows of 2048 36.8 / 21.7; SwiGLU +
-// quant forward and backward 768 x 1408 18.4 / 14.3; activation and weight of a linear layer, 336 x 3584 and 1152 x 3584,
-// 18.4 / 11.4; bf16 RMSNorm and SwiGLU, forward and backward, 480 x 2944 / 512 37.6 / 28.4; gather + pad + quant and
-// per-expert quant, 642 tokens to 8 of 16 experts, 28.5 / 21.5; per-expert SwiGLU, 1152 tokens to 2 of 64, with a plan
-// 46.2 / 37.1; router 256 x 1152, 384 logits 20.4 / 14.3.
+// quant forward and backward 768 x 1408 18.4 / 14.3; activation 336 x 3584 and weight of a linear layer 18.4 / 11.4;
+// bf16 RMSNorm and SwiGLU, forward and backward, 480 x 2944 / 512 37.6 / 28.4; gather + pad + quant and per-expert
+// quant, 642 tokens to 8 of 16 experts, 28.5 / 21.5; per-expert SwiGLU, 1152 tokens to 2 of 64, with a plan 46.2 / 37.1;
+// router 256 x 1152, 384 logits 20.4 / 14.3.
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>

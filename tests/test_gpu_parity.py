@@ -281,6 +281,26 @@ def test_rmsnorm_and_block_quant(gpu, M, N, round_scale):
     check_quant_pair("rms.pinned.col", p_ref[3], p_ref[4], qt2, st2, **EXACT)
 
 
+# one partial row of dgamma a workgroup: few and many rows of each width's rule, uneven last rounds of the sum over them
+@pytest.mark.parametrize("M,n", [(1, 640), (31, 640), (132, 2048), (1025, 1408), (2049, 2048), (2, 2056), (31, 2056),
+                                 (33, 7168), (256, 4096), (257, 4104), (1024, 2944), (1025, 2944), (1537, 5120)])
+def test_rmsnorm_bwd_partials(gpu, M, n):
+    from linghe_amd.utils.norm import triton_rms_norm_backward
+
+    g = gen(M + n)
+    x, dy, w = randn_bf16(g, M, n), randn_bf16(g, M, n), gamma_bf16(g, n)
+    dx, dw = triton_rms_norm_backward(dy.to(gpu), x.to(gpu), w.to(gpu))
+    x, dy, w = x.double(), dy.double(), w.double()
+    r = torch.rsqrt(x.pow(2).mean(1, keepdim=True) + 1e-6)
+    terms = dy * x * r
+    # a term's factor r holds 3 roundings, its product and sum 2 more, and no sum is longer than 16 + log2(512) of them
+    assert ((dw.cpu().double() - terms.sum(0)).abs() <= 30 * 2.0**-24 * terms.abs().sum(0)).all()
+    part = r**3 * (dy * x * w).sum(1, keepdim=True) / n
+    big = (r * dy * w).abs() + r**3 * (dy * x * w).abs().sum(1, keepdim=True) / n * x.abs()
+    assert ((dx.cpu().double() - (r * dy * w - part * x)).abs() <= 2.0**-8 * (r * dy * w - part * x).abs()
+            + (n / 8 + 16) * 2.0**-24 * big).all()
+
+
 # ------------------------------------------------------------------ SwiGLU
 # three and four waves per row: the narrowest and widest of each, one workgroup per row and looping ones
 @pytest.mark.parametrize("M,N", [(1, 2176), (8200, 2176), (37, 3072), (4099, 3072), (8195, 3200), (5, 6272), (8195, 6272),
