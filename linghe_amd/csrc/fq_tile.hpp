@@ -498,8 +498,8 @@ __device__ __forceinline__ void load_counts(const void* counts, int is_i64, int 
 // with the loads of up to sixteen steps in flight together: no LDS, no barrier, and every
 // thread of the workgroup ends with the same answer.  (A workgroup-wide scan with three
 // barriers cost 13 % of the batched SwiGLU forward, one wave scanning for the others 6 %.)
-// A workgroup beyond the last tile (the launch is sized for one workgroup per 128 x 128 tile,
-// packing needs fewer) or counts that disagree with the host's yield expert = -1.
+// A workgroup beyond the last tile (the launch is sized for the most that counts of so many rows and blocks can need,
+// scan_workgroups) or counts that disagree with the host's yield expert = -1.
 // `wg` is the tile's number in that order; which workgroup takes which number is the caller's
 // choice (resolve_tile: grid order, or runs of neighbouring row blocks per XCD).  Numbering the
 // tiles so that every XCD works on one contiguous eighth of the REAL tiles needs their number

@@ -59,3 +59,31 @@ def test_pad_permute_packing_boundaries(gpu, ncb):
     check_quant_pair("packed.gather.row", ref[0], ref[1], q.view(-1), s.view(-1), **EXACT)
     check_quant_pair("packed.gather.col", ref[2], ref[3], qt.view(-1), st.view(-1), **EXACT)
     assert torch.equal(p.cpu(), ref[4])
+
+
+# counts for which the launch that scans them is smaller than one workgroup per tile: whole, half and quarter blocks at the
+# least rows that make one (the size is then just enough), at the most, and mixed with empty experts
+@pytest.mark.parametrize("counts", [[65] * 9, [33] * 9, [1] * 70, [64] * 5, [32] * 5, [65, 33, 1] * 7, [1] * 40 + [200],
+                                    [0, 130, 0, 1, 2, 66, 34, 0] * 4, [300] + [3] * 90], ids=lambda c: f"{len(c)}x{c[0]}")
+@pytest.mark.parametrize("ncb", [1, 3, 4, 7])
+def test_scanning_launch_has_a_workgroup_for_every_tile(gpu, counts, ncb):
+    from linghe_amd.quant.block import triton_batch_blockwise_quant
+    from linghe_amd.utils.silu import (build_expert_plan, triton_batch_weighted_silu_and_block_quant_backward as bwd,
+                                       triton_batch_weighted_silu_and_block_quant_forward as fwd)
+
+    announce("scanning launch size", len(counts), ncb)
+    x = randn_bf16(gen(ncb), sum(counts), 128 * ncb)
+    ref = O.batch_blockwise_quant(x, counts, False)
+    cnt = torch.tensor(counts, dtype=torch.int64, device=gpu)
+    q, s, qt, st = triton_batch_blockwise_quant(x.to(gpu), cnt, counts)
+    torch.cuda.synchronize()
+    check_quant_pair("scan.row", ref[0], ref[1], q, s, **EXACT)
+    check_quant_pair("scan.col", ref[2], ref[3], qt, st, **EXACT)
+    # the SwiGLU kernels, against the launch of exactly the workgroups that have a tile
+    g = gen(90 + ncb)
+    h, dy = randn_bf16(g, sum(counts), 256 * ncb).to(gpu), randn_bf16(g, sum(counts), 128 * ncb).to(gpu)
+    w = torch.randn(sum(counts), 1, generator=g).to(gpu)
+    plan = build_expert_plan(cnt, counts)
+    for fn, args in ((fwd, (h, w)), (bwd, (dy, h, w))):
+        for a, b in zip(fn(*args, cnt, counts), fn(*args, cnt, counts, plan=plan)):
+            assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
