@@ -2,21 +2,27 @@
 //
 // A small call's kernels run 2-5 us each, and a Python wrapper that allocates its two to seven outputs with torch.empty
 // and calls the library through ctypes takes 7-13 us (more where it adds up the tokens of 256 experts): what bounds a
-// small call is the host. The wrappers keep their checks in Python and hand over here; allocation goes through the
-// dispatcher as torch.empty does (same allocator, pools and modes) and the interpreter lock is released meanwhile.
+// small call is the host. The wrappers keep their checks in Python and hand over here; the device is made current here, the outputs
+// come from torch's allocator (Outputs) and the interpreter lock is released meanwhile.
 // The kernel library is the one that _lib.py loaded: bind() takes its functions' addresses, there is no
 // link-time dependency that could bring a second one into the process.
-// us through ctypes / here, back to back: RMSNorm + group + SwiGLU quantiser on 32 rows of 2048 36.8 / 21.7; SwiGLU +
-// quant forward and backward 768 x 1408 18.4 / 14.3; activation 336 x 3584 and weight of a linear layer 18.4 / 11.4;
-// bf16 RMSNorm and SwiGLU, forward and backward, 480 x 2944 / 512 37.6 / 28.4; gather + pad + quant and per-expert
-// quant, 642 tokens to 8 of 16 experts, 28.5 / 21.5; per-expert SwiGLU, 1152 tokens to 2 of 64, with a plan 46.2 / 37.1;
-// router 256 x 1152, 384 logits 20.4 / 14.3.
+// us through ctypes / here with outputs through the dispatcher and the device guard in Python / now, back to back: RMSNorm + group +
+// SwiGLU quantiser on 32 rows of 2048 36.8 / 19.4 / 15.5; activation 528 x 3456 and weight of a linear layer - / 12.4 / 9.8;
+// RMSNorm + quant 624 x 1024 - / 10.7 / 8.7; row-wise and then transposed 384 x 1536 - / 14.2 / 11.2; bf16 RMSNorm and SwiGLU,
+// forward and backward, 640 x 1024 / 768 - / 28.8 / 23.7; gather + pad + quant and per-expert quant, 486 tokens to 2 of 128
+// experts, - / 18.7 / 16.8 (the kernels' time). One call: group quantiser 6.6 / 5.2, a tile plan of 64 experts 7.8 (ctypes) / 4.8.
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <ATen/ATen.h>
+#include <ATen/EmptyTensor.h>
+#include <ATen/detail/CUDAHooksInterface.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <pybind11/pybind11.h>
 
+#include <algorithm>
 #include <iterator>
 #include <vector>
 
@@ -27,11 +33,12 @@ namespace {
 // the library's functions that are called here
 #define FQ_FUNCTIONS(F)                                                                                              \
   F(rmsnorm_fwd) F(rmsnorm_bwd) F(rmsnorm_bwd_num_partials) F(rmsnorm_quant_fwd) F(rmsnorm_router_quant_fwd)         \
-  F(rmsnorm_router_quant_fwd_packed) F(rmsnorm_router_quant_fwd_folded) F(swiglu_fwd) F(swiglu_bwd) F(swiglu_quant_fwd) F(swiglu_quant_bwd)             \
+  F(rmsnorm_router_quant_fwd_packed) F(rmsnorm_router_quant_fwd_folded) F(swiglu_fwd) F(swiglu_bwd)                  \
+  F(swiglu_quant_fwd) F(swiglu_quant_bwd)                                                                            \
   F(batched_swiglu_quant_fwd) F(batched_swiglu_quant_fwd_planned) F(batched_swiglu_quant_bwd)                        \
   F(batched_swiglu_quant_bwd_planned) F(group_quant) F(block_quant) F(blockwise_quant) F(batched_blockwise_quant)    \
   F(batched_blockwise_quant_planned) F(batched_pad_permute_quant) F(batched_pad_permute_quant_planned)               \
-  F(expert_plan_shape) F(last_error)
+  F(expert_plan_shape) F(expert_plan_bytes) F(build_expert_plan) F(last_error)
 
 struct {
 #define FQ_MEMBER(name) decltype(&fq_##name) name = nullptr;
@@ -57,9 +64,40 @@ at::Tensor tensor_or_none(PyObject* o) {
   return THPVariable_Unpack(o);
 }
 
-at::Tensor empty(const at::Tensor& like, at::ScalarType type, at::IntArrayRef sizes) {
-  return at::empty(sizes, at::TensorOptions().dtype(type).device(like.device()));
-}
+// The device of a call's first tensor made the current one, and tensors on it. They are made as at::empty makes them behind
+// the dispatcher (0.65 us of a call for each output, 0.25 without it), unless something could be listening there: a mode, a
+// transform, a tracer, or the fill of new memory that deterministic algorithms ask for.
+class Outputs {
+ public:
+  explicit Outputs(const at::Tensor& x)
+      : on_(x.device()),
+        device_(x.device()),
+        plain_(x.is_cuda() && !c10::impl::TorchDispatchModeTLS::any_modes_set() &&
+               (c10::impl::tls_local_dispatch_key_set().included_ - c10::default_included_set).empty() &&
+               !at::globalContext().deterministicAlgorithms()) {}
+
+  at::Tensor empty(const at::Tensor& like, at::ScalarType type, at::IntArrayRef sizes) const {
+    if (!plain_ || like.device() != device_)
+      return at::empty(sizes, at::TensorOptions().dtype(type).device(like.device()));
+    return at::detail::empty_generic(sizes, at::detail::getCUDAHooks().getCUDADeviceAllocator(),
+                                     c10::DispatchKeySet(c10::DispatchKey::CUDA), type, std::nullopt);
+  }
+
+  // of the type, sizes and strides of t
+  at::Tensor empty_like(const at::Tensor& t) const {
+    int64_t stride = 1;
+    for (int64_t d = t.dim() - 1; d >= 0; --d) {  // (a contiguous tensor may have any stride where its size is 1)
+      if (t.stride(d) != stride) return at::empty_like(t);
+      stride *= std::max<int64_t>(t.size(d), 1);
+    }
+    return empty(t, t.scalar_type(), t.sizes());
+  }
+
+ private:
+  c10::DeviceGuard on_;
+  c10::Device device_;
+  bool plain_;
+};
 
 void* data(const at::Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 
@@ -161,10 +199,11 @@ PyObject* rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   const float eps = in.real();
   const int reuse = in.flag();
   void* stream = in.address();
+  const Outputs outputs(x);
   {
     pybind11::gil_scoped_release no_gil;
-    if (!out.defined()) out = at::empty_like(x);
-    if (!rms.defined()) rms = empty(x, at::kFloat, {M});
+    if (!out.defined()) out = outputs.empty_like(x);
+    if (!rms.defined()) rms = outputs.empty(x, at::kFloat, {M});
     if (M > 0) check(lib.rmsnorm_fwd(data(x), data(gamma), data(out), floats(rms), M, n, eps, reuse, stream));
   }
   return wrap({out, rms});
@@ -180,12 +219,13 @@ PyObject* rmsnorm_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   const int64_t M = in.integer(), n = in.integer();
   const float eps = in.real();
   void* stream = in.address();
+  const Outputs outputs(x);
   {
     pybind11::gil_scoped_release no_gil;
-    if (!dx.defined()) dx = at::empty_like(x);
-    dgamma = empty(gamma, at::kFloat, {n});
+    if (!dx.defined()) dx = outputs.empty_like(x);
+    dgamma = outputs.empty(gamma, at::kFloat, {n});
     const int64_t n_partials = lib.rmsnorm_bwd_num_partials(M, n);
-    const at::Tensor partials = empty(gamma, at::kFloat, {n_partials, n});
+    const at::Tensor partials = outputs.empty(gamma, at::kFloat, {n_partials, n});
     check(lib.rmsnorm_bwd(data(dy), data(x), data(gamma), floats(rms), data(dx), floats(dgamma), floats(partials),
                           n_partials, M, n, eps, stream));
   }
@@ -205,16 +245,17 @@ PyObject* rmsnorm_quant(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   const at::ScalarType fp8 = in.dtype();
   const int kind = in.flag();
   void* stream = in.address();
+  const Outputs outputs(x);
   {
     pybind11::gil_scoped_release no_gil;
     const int64_t M = x.size(0), n = x.size(1);
     if (mode != 1) {
-      if (!out.defined()) out = empty(x, fp8, {M, n});
-      if (!scale.defined()) scale = empty(x, at::kFloat, {n / 128, M});
+      if (!out.defined()) out = outputs.empty(x, fp8, {M, n});
+      if (!scale.defined()) scale = outputs.empty(x, at::kFloat, {n / 128, M});
     }
-    qt = empty(x, fp8, {n, M});
-    st = empty(x, at::kFloat, {(M + 127) / 128, n});
-    if (!rms.defined()) rms = empty(x, at::kFloat, {M});
+    qt = outputs.empty(x, fp8, {n, M});
+    st = outputs.empty(x, at::kFloat, {(M + 127) / 128, n});
+    if (!rms.defined()) rms = outputs.empty(x, at::kFloat, {M});
     if (M > 0)
       check(lib.rmsnorm_quant_fwd(data(x), data(gamma), mode != 1 ? data(out) : nullptr,
                                   mode != 1 ? floats(scale) : nullptr, floats(rms), data(qt), floats(st), M, n, eps,
@@ -238,16 +279,17 @@ PyObject* rmsnorm_router_quant(PyObject*, PyObject* const* a, Py_ssize_t n_args)
   const float eps = in.real();
   const int round = in.flag();
   void* stream = in.address();
+  const Outputs outputs(x);
   {
     pybind11::gil_scoped_release no_gil;
     const int64_t M = x.size(0), K = x.size(1);
-    y = empty(x, x.scalar_type(), {M, K});
-    if (!rms.defined()) rms = empty(x, at::kFloat, {M});
-    logits = empty(x, at::kFloat, {M, N});
-    q = empty(x, at::kFloat8_e4m3fn, {M, K});
-    s = empty(x, at::kFloat, {K / 128, M});
-    qt = empty(x, at::kFloat8_e4m3fn, {K, M});
-    st = empty(x, at::kFloat, {M / 128, K});
+    y = outputs.empty(x, x.scalar_type(), {M, K});
+    if (!rms.defined()) rms = outputs.empty(x, at::kFloat, {M});
+    logits = outputs.empty(x, at::kFloat, {M, N});
+    q = outputs.empty(x, at::kFloat8_e4m3fn, {M, K});
+    s = outputs.empty(x, at::kFloat, {K / 128, M});
+    qt = outputs.empty(x, at::kFloat8_e4m3fn, {K, M});
+    st = outputs.empty(x, at::kFloat, {M / 128, K});
     if (M > 0 && mode == 1) {
       check(lib.rmsnorm_quant_fwd(data(x), data(gamma), nullptr, nullptr, floats(rms), data(qt), floats(st), M, K, eps,
                                   round, 1, FQ_E4M3, stream));
@@ -257,13 +299,13 @@ PyObject* rmsnorm_router_quant(PyObject*, PyObject* const* a, Py_ssize_t n_args)
                                                 stream));
     } else if (M > 0 && form == 2) {
       // the two planes of gamma * weight, which every call makes
-      const at::Tensor scratch = empty(x, at::kByte, {scratch_bytes});
+      const at::Tensor scratch = outputs.empty(x, at::kByte, {scratch_bytes});
       check(lib.rmsnorm_router_quant_fwd_folded(data(x), data(gamma), data(weight), data(scratch), data(y), floats(rms),
                                                 floats(logits), data(q), floats(s), M, K, N, eps, round, FQ_E4M3,
                                                 stream));
     } else if (M > 0) {
       // the weight re-ordered for the matrix cores (an fp32 weight as two bf16 planes)
-      const at::Tensor scratch = empty(x, at::kByte, {scratch_bytes});
+      const at::Tensor scratch = outputs.empty(x, at::kByte, {scratch_bytes});
       check(lib.rmsnorm_router_quant_fwd(data(x), data(gamma), data(weight), fp32, data(scratch), data(y), floats(rms),
                                          floats(logits), data(q), floats(s), M, K, N, eps, round, FQ_E4M3, stream));
     }
@@ -280,10 +322,11 @@ PyObject* swiglu(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   const int wbf16 = in.flag();
   at::Tensor out = in.tensor();
   void* stream = in.address();
+  const Outputs outputs(x);
   {
     pybind11::gil_scoped_release no_gil;
     const int64_t M = x.size(0), n = x.size(1) / 2;
-    if (!out.defined()) out = empty(x, x.scalar_type(), {M, n});
+    if (!out.defined()) out = outputs.empty(x, x.scalar_type(), {M, n});
     check(lib.swiglu_fwd(data(x), data(weight), wbf16, data(out), M, n, stream));
   }
   return THPVariable_Wrap(out);
@@ -297,12 +340,13 @@ PyObject* swiglu_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   const at::Tensor g = in.tensor(), x = in.tensor(), weight = in.tensor();
   const int wbf16 = in.flag();
   void* stream = in.address();
+  const Outputs outputs(x);
   at::Tensor dx, dw;
   {
     pybind11::gil_scoped_release no_gil;
     const int64_t M = x.size(0), N = x.size(1);
-    if (weight.defined()) dw = empty(x, weight.scalar_type(), weight.sizes());
-    dx = empty(x, x.scalar_type(), {M, N});
+    if (weight.defined()) dw = outputs.empty(x, weight.scalar_type(), weight.sizes());
+    dx = outputs.empty(x, x.scalar_type(), {M, N});
     check(lib.swiglu_bwd(data(g), data(x), data(weight), wbf16, data(dx), data(dw), M, N / 2, stream));
   }
   return wrap({dx, dw});
@@ -319,13 +363,14 @@ PyObject* swiglu_quant(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   const at::ScalarType fp8 = in.dtype();
   const int kind = in.flag();
   void* stream = in.address();
+  const Outputs outputs(x);
   {
     pybind11::gil_scoped_release no_gil;
     const int64_t M = x.size(0), n = x.size(1) / 2;
-    if (!out.defined()) out = empty(x, fp8, {M, n});
-    if (!scale.defined()) scale = empty(x, at::kFloat, {n / 128, M});
-    qt = empty(x, fp8, {n, M});
-    st = empty(x, at::kFloat, {(M + 127) / 128, n});
+    if (!out.defined()) out = outputs.empty(x, fp8, {M, n});
+    if (!scale.defined()) scale = outputs.empty(x, at::kFloat, {n / 128, M});
+    qt = outputs.empty(x, fp8, {n, M});
+    st = outputs.empty(x, at::kFloat, {(M + 127) / 128, n});
     if (M > 0)
       check(lib.swiglu_quant_fwd(data(x), data(out), floats(scale), data(qt), floats(st), M, n, round, mode, kind,
                                  stream));
@@ -343,14 +388,15 @@ PyObject* swiglu_quant_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   const at::ScalarType fp8 = in.dtype();
   const int kind = in.flag();
   void* stream = in.address();
+  const Outputs outputs(x);
   at::Tensor q, s, qt, st;
   {
     pybind11::gil_scoped_release no_gil;
     const int64_t M = x.size(0), N = x.size(1);
-    q = empty(x, fp8, {M, N});
-    s = empty(x, at::kFloat, {N / 128, M});
-    qt = empty(x, fp8, {N, M});
-    st = empty(x, at::kFloat, {(M + 127) / 128, N});
+    q = outputs.empty(x, fp8, {M, N});
+    s = outputs.empty(x, at::kFloat, {N / 128, M});
+    qt = outputs.empty(x, fp8, {N, M});
+    st = outputs.empty(x, at::kFloat, {(M + 127) / 128, N});
     if (M > 0)
       check(lib.swiglu_quant_bwd(data(g), data(x), data(q), floats(s), data(qt), floats(st), M, N / 2, round, kind,
                                  stream));
@@ -376,13 +422,14 @@ PyObject* batched_swiglu_quant(PyObject*, PyObject* const* a, Py_ssize_t n_args)
   const at::ScalarType fp8 = in.dtype();
   const int kind = in.flag();
   void* stream = in.address();
+  const Outputs outputs(x);
   {
     pybind11::gil_scoped_release no_gil;
     const int64_t M = x.size(0), n = x.size(1) / 2;
-    if (!out.defined()) out = empty(x, fp8, {M, n});
-    if (!scale.defined()) scale = empty(x, at::kFloat, {M, n / 128});
-    qt = empty(x, fp8, {M, n});
-    st = empty(x, at::kFloat, {blocks, n});
+    if (!out.defined()) out = outputs.empty(x, fp8, {M, n});
+    if (!scale.defined()) scale = outputs.empty(x, at::kFloat, {M, n / 128});
+    qt = outputs.empty(x, fp8, {M, n});
+    st = outputs.empty(x, at::kFloat, {blocks, n});
     if (M > 0 && plan.defined())
       check(lib.batched_swiglu_quant_fwd_planned(data(x), data(weight), wbf16, data(plan), shape, data(out),
                                                  floats(scale), data(qt), floats(st), M, n, round, mode, kind, stream));
@@ -412,16 +459,17 @@ PyObject* batched_swiglu_quant_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_a
   const at::ScalarType fp8 = in.dtype();
   const int kind = in.flag();
   void* stream = in.address();
+  const Outputs outputs(x);
   {
     pybind11::gil_scoped_release no_gil;
     const int64_t M = x.size(0), N = x.size(1), n = N / 2;
-    q = empty(x, fp8, {M, N});
-    s = empty(x, at::kFloat, {M, N / 128});
-    qt = empty(x, fp8, {M, N});
-    st = empty(x, at::kFloat, {blocks, N});
-    if (!dw.defined()) dw = at::empty_like(weight);
+    q = outputs.empty(x, fp8, {M, N});
+    s = outputs.empty(x, at::kFloat, {M, N / 128});
+    qt = outputs.empty(x, fp8, {M, N});
+    st = outputs.empty(x, at::kFloat, {blocks, N});
+    if (!dw.defined()) dw = outputs.empty_like(weight);
     if (blocks != 0) {
-      const at::Tensor partials = empty(x, at::kFloat, {M, n / 128});
+      const at::Tensor partials = outputs.empty(x, at::kFloat, {M, n / 128});
       if (plan.defined())
         check(lib.batched_swiglu_quant_bwd_planned(data(g), data(x), data(weight), wbf16, data(plan), shape, data(q),
                                                    floats(s), data(dw), data(qt), floats(st), floats(partials), M, n,
@@ -446,11 +494,12 @@ PyObject* group_quant(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   const at::ScalarType fp8 = in.dtype();
   const int kind = in.flag();
   void* stream = in.address();
+  const Outputs outputs(x);
   {
     pybind11::gil_scoped_release no_gil;
     const int64_t M = x.size(0), n = x.size(1);
-    q = empty(x, fp8, {M, n});
-    s = empty(x, at::kFloat, {M, n / 128});
+    q = outputs.empty(x, fp8, {M, n});
+    s = outputs.empty(x, at::kFloat, {M, n / 128});
     if (M > 0) check(lib.group_quant(data(x), data(q), floats(s), M, n, round, kind, stream));
   }
   return wrap({q, s});
@@ -467,11 +516,12 @@ PyObject* block_quant(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   const at::ScalarType fp8 = in.dtype();
   const int kind = in.flag();
   void* stream = in.address();
+  const Outputs outputs(x);
   {
     pybind11::gil_scoped_release no_gil;
     const int64_t M = x.size(0), n = x.size(1);
-    q = empty(x, fp8, {M, n});
-    s = empty(x, at::kFloat, {M / 128, n / 128});
+    q = outputs.empty(x, fp8, {M, n});
+    s = outputs.empty(x, at::kFloat, {M / 128, n / 128});
     check(lib.block_quant(data(x), data(q), floats(s), M, n, round, kind, stream));
   }
   return wrap({q, s});
@@ -488,13 +538,14 @@ PyObject* blockwise_quant(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   const at::ScalarType fp8 = in.dtype();
   const int kind = in.flag();
   void* stream = in.address();
+  const Outputs outputs(x);
   {
     pybind11::gil_scoped_release no_gil;
     const int64_t M = x.size(0), n = x.size(1);
-    q = empty(x, fp8, {M, n});
-    s = empty(x, at::kFloat, {n / 128, M});
-    qt = empty(x, fp8, {n, M});
-    st = empty(x, at::kFloat, {(M + 127) / 128, n});
+    q = outputs.empty(x, fp8, {M, n});
+    s = outputs.empty(x, at::kFloat, {n / 128, M});
+    qt = outputs.empty(x, fp8, {n, M});
+    st = outputs.empty(x, at::kFloat, {(M + 127) / 128, n});
     if (M > 0)
       check(lib.blockwise_quant(data(x), data(q), floats(s), data(qt), floats(st), M, n, round, mode, kind, stream));
   }
@@ -515,14 +566,15 @@ PyObject* batched_blockwise_quant(PyObject*, PyObject* const* a, Py_ssize_t n_ar
   const at::ScalarType fp8 = in.dtype();
   const int kind = in.flag();
   void* stream = in.address();
+  const Outputs outputs(x);
   at::Tensor q, s, qt, st;
   {
     pybind11::gil_scoped_release no_gil;
     const int64_t M = x.size(0), n = x.size(1);
-    q = empty(x, fp8, {M, n});
-    s = empty(x, at::kFloat, {M * n / 128});
-    qt = empty(x, fp8, {M * n});
-    st = empty(x, at::kFloat, {blocks * n});
+    q = outputs.empty(x, fp8, {M, n});
+    s = outputs.empty(x, at::kFloat, {M * n / 128});
+    qt = outputs.empty(x, fp8, {M * n});
+    st = outputs.empty(x, at::kFloat, {blocks * n});
     if (M > 0 && plan.defined())
       check(lib.batched_blockwise_quant_planned(data(x), data(plan), shape, data(q), floats(s), data(qt), floats(st), M,
                                                 n, round, kind, stream));
@@ -549,16 +601,17 @@ PyObject* batched_pad_permute_quant(PyObject*, PyObject* const* a, Py_ssize_t n_
   const at::ScalarType fp8 = in.dtype();
   const int kind = in.flag();
   void* stream = in.address();
+  const Outputs outputs(x);
   at::Tensor q, s, qt, st, prob_out;
   {
     pybind11::gil_scoped_release no_gil;
     const int64_t m = x.size(0), n = x.size(1), M = indices.size(0);
     const int experts = static_cast<int>(counts.size(0));
-    q = empty(x, fp8, {M, n});
-    s = empty(x, at::kFloat, {M, n / 128});
-    qt = empty(x, fp8, {M, n});
-    st = empty(x, at::kFloat, {blocks, n});
-    if (probs.defined()) prob_out = empty(x, probs.scalar_type(), {M});
+    q = outputs.empty(x, fp8, {M, n});
+    s = outputs.empty(x, at::kFloat, {M, n / 128});
+    qt = outputs.empty(x, fp8, {M, n});
+    st = outputs.empty(x, at::kFloat, {blocks, n});
+    if (probs.defined()) prob_out = outputs.empty(x, probs.scalar_type(), {M});
     if (launch && plan.defined())
       check(lib.batched_pad_permute_quant_planned(data(x), data(plan), shape, experts, data(indices), data(probs),
                                                   pbf16, data(prob_out), data(q), floats(s), data(qt), floats(st), m, M,
@@ -587,16 +640,32 @@ PyObject* expert_blocks(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   END_HANDLE_TH_ERRORS
 }
 
-// (tokens per expert, pad, address of the plan's shape)
-PyObject* expert_plan_shape(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+// (counts, counts are int64 (-1: of another type), tokens per expert, pad, address of the plan's shape, stream) -> the plan's
+// table, None where there are rows and the counts are of another type
+PyObject* expert_plan(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   HANDLE_TH_ERRORS
-  Args in(a, n_args, 3);
-  const std::vector<int64_t> counts = in.integers();
+  Args in(a, n_args, 6);
+  const at::Tensor counts = in.tensor();
+  const int i64 = in.flag();
+  const std::vector<int64_t> tokens = in.integers();
   const int pad = in.flag();
   int64_t* shape = static_cast<int64_t*>(in.address());
+  void* stream = in.address();
   const int64_t none = 0;
-  check(lib.expert_plan_shape(counts.empty() ? &none : counts.data(), static_cast<int>(counts.size()), pad, shape));
-  Py_RETURN_NONE;
+  check(lib.expert_plan_shape(tokens.empty() ? &none : tokens.data(), static_cast<int>(tokens.size()), pad, shape));
+  const int64_t bytes = std::max<int64_t>(lib.expert_plan_bytes(shape), 16);
+  if (shape[0] == 0)
+    return THPVariable_Wrap(at::empty({bytes}, at::TensorOptions().dtype(at::kByte).device(counts.device())));
+  if (i64 < 0) Py_RETURN_NONE;
+  TORCH_CHECK_VALUE(counts.is_cuda(), "Expected a cuda device, but got: ", counts.device());
+  const Outputs outputs(counts);
+  at::Tensor table;
+  {
+    pybind11::gil_scoped_release no_gil;
+    table = outputs.empty(counts, at::kByte, {bytes});
+    check(lib.build_expert_plan(data(counts), i64, static_cast<int>(counts.size(0)), shape, data(table), stream));
+  }
+  return THPVariable_Wrap(table);
   END_HANDLE_TH_ERRORS
 }
 
@@ -618,7 +687,7 @@ PyMethodDef methods[] = {FQ_METHOD(bind),
                          FQ_METHOD(batched_blockwise_quant),
                          FQ_METHOD(batched_pad_permute_quant),
                          FQ_METHOD(expert_blocks),
-                         FQ_METHOD(expert_plan_shape),
+                         FQ_METHOD(expert_plan),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_fq_torch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -26,9 +26,7 @@ def triton_block_quant(x, block_size=128, round_scale=False, *, fp8_dtype=torch.
     M, N = x.size()
     assert M % 128 == 0 and N % 128 == 0
     _lib.require_device_bf16(x, "x")
-    with _lib.on_device(x.device):
-        return _lib.native.block_quant(x, int(bool(round_scale)), fp8_dtype, _lib.fp8_kind(fp8_dtype),
-                                       _lib.stream_of(x))
+    return _lib.native.block_quant(x, int(bool(round_scale)), fp8_dtype, _lib.fp8_kind(fp8_dtype), _lib.stream_of(x))
 
 
 def triton_blockwise_quant(x, round_scale=False, output_mode=2, *, fp8_dtype=torch.float8_e4m3fn):
@@ -50,9 +48,8 @@ def triton_blockwise_quant(x, round_scale=False, output_mode=2, *, fp8_dtype=tor
     assert N % 128 == 0
     assert output_mode in (0, 1, 2)
     _lib.require_device_bf16(x, "x")
-    with _lib.on_device(x.device):
-        return _lib.native.blockwise_quant(x, int(bool(round_scale)), output_mode, fp8_dtype,
-                                           _lib.fp8_kind(fp8_dtype) if M else 0, _lib.stream_of(x))
+    return _lib.native.blockwise_quant(x, int(bool(round_scale)), output_mode, fp8_dtype,
+                                       _lib.fp8_kind(fp8_dtype) if M else 0, _lib.stream_of(x))
 
 
 def triton_batch_blockwise_quant(xs, token_count_per_expert, splits, round_scale=False, *,
@@ -87,6 +84,5 @@ def triton_batch_blockwise_quant(xs, token_count_per_expert, splits, round_scale
         elif counts.dtype != torch.int32:
             raise TypeError(f"token_count_per_expert must be int32 or int64, got {counts.dtype}")
         kind = _lib.fp8_kind(fp8_dtype)
-    with _lib.on_device(device):
-        return _lib.native.batched_blockwise_quant(xs, counts, is64, table, shape, blocks, int(bool(round_scale)),
-                                                   fp8_dtype, kind, _lib.stream_of(xs))
+    return _lib.native.batched_blockwise_quant(xs, counts, is64, table, shape, blocks, int(bool(round_scale)),
+                                               fp8_dtype, kind, _lib.stream_of(xs))

@@ -27,5 +27,4 @@ def triton_group_quant(x, dtype=torch.float8_e4m3fn, group_size=128, round_scale
     _lib.require_device_bf16(x, "x")
     assert dtype in (torch.float8_e4m3fn, torch.float8_e5m2)
     kind = _lib.FQ_E4M3 if dtype == torch.float8_e4m3fn else _lib.FQ_E5M2_MAX448
-    with _lib.on_device(x.device):
-        return _lib.native.group_quant(x, int(bool(round_scale)), dtype, kind, _lib.stream_of(x))
+    return _lib.native.group_quant(x, int(bool(round_scale)), dtype, kind, _lib.stream_of(x))

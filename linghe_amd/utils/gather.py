@@ -43,9 +43,8 @@ def triton_batch_block_pad_permute_with_indices(
     blocks, padded = _lib.native.expert_blocks(splits)
     counts = token_count_per_expert
     if m == 0 or M == 0:
-        with _lib.on_device(device):
-            return _lib.native.batched_pad_permute_quant(xs, counts, 0, None, 0, blocks, indices, probs, 0, 0, 0,
-                                                         fp8_dtype, 0, _lib.stream_of(xs))
+        return _lib.native.batched_pad_permute_quant(xs, counts, 0, None, 0, blocks, indices, probs, 0, 0, 0,
+                                                     fp8_dtype, 0, _lib.stream_of(xs))
     assert M == padded, f"indices holds {M} entries, the counts rounded up to 16 add up to {padded}"
     if indices.dtype != torch.int32:
         raise TypeError(f"indices must be int32, got {indices.dtype}")
@@ -68,7 +67,6 @@ def triton_batch_block_pad_permute_with_indices(
         if plan.blocks != blocks or plan.pad != 16 or plan.table.device != device:
             raise ValueError("plan does not belong to these splits / this layout (pad=16) / this device")
         table, shape = plan.table, ctypes.addressof(plan.shape)
-    with _lib.on_device(device):
-        return _lib.native.batched_pad_permute_quant(xs, counts, is64, table, shape, blocks, indices, probs, pbf16, 1,
-                                                     int(bool(round_scale)), fp8_dtype, _lib.fp8_kind(fp8_dtype),
-                                                     _lib.stream_of(xs))
+    return _lib.native.batched_pad_permute_quant(xs, counts, is64, table, shape, blocks, indices, probs, pbf16, 1,
+                                                 int(bool(round_scale)), fp8_dtype, _lib.fp8_kind(fp8_dtype),
+                                                 _lib.stream_of(xs))

@@ -47,8 +47,7 @@ def triton_rms_norm_forward(x, weight, eps=1e-6, out=None, rms=None):
     _lib.require_device_bf16(weight, "weight")
     if out is None and type(x) is not torch.Tensor:  # (a subclass may have its own)
         out = torch.empty_like(x)
-    with _lib.on_device(x.device):
-        new = _lib.native.rmsnorm(x, weight, out, rms, M, n, float(eps), int(rms is not None), _lib.stream_of(x))
+    new = _lib.native.rmsnorm(x, weight, out, rms, M, n, float(eps), int(rms is not None), _lib.stream_of(x))
     return new[0] if out is None else out, new[1] if rms is None else rms
 
 
@@ -67,8 +66,7 @@ def triton_rms_norm_backward(grad_output, x, w, eps=1e-6, rms=None):
     _lib.require_device_bf16(w, "w")
     assert x.is_contiguous() and w.is_contiguous()
     dx = None if type(x) is torch.Tensor else torch.empty_like(x)  # (a subclass may have its own)
-    with _lib.on_device(x.device):
-        new = _lib.native.rmsnorm_bwd(grad_output, x, w, rms, dx, M, n, float(eps), _lib.stream_of(x))
+    new = _lib.native.rmsnorm_bwd(grad_output, x, w, rms, dx, M, n, float(eps), _lib.stream_of(x))
     return new if dx is None else (dx, new[1])
 
 
@@ -113,7 +111,6 @@ def triton_rms_norm_and_block_quant_forward(
     assert output_mode in (0, 1, 2)
     _lib.require_device_bf16(x, "x")
     _lib.require_device_bf16(weight, "weight")
-    device = x.device
     kind = _lib.fp8_kind(fp8_dtype)
 
     # a given rms is an input in mode 1; in mode 2 it is ignored and recomputed, as in the reference
@@ -122,9 +119,8 @@ def triton_rms_norm_and_block_quant_forward(
     elif output_mode == 1:
         assert rms is not None
     # the transposed buffers are always allocated, as in the reference
-    with _lib.on_device(device):
-        return _lib.native.rmsnorm_quant(x, weight, out, scale, rms if output_mode == 1 else None, float(eps),
-                                         int(bool(round_scale)), output_mode, fp8_dtype, kind, _lib.stream_of(x))
+    return _lib.native.rmsnorm_quant(x, weight, out, scale, rms if output_mode == 1 else None, float(eps),
+                                     int(bool(round_scale)), output_mode, fp8_dtype, kind, _lib.stream_of(x))
 
 
 def pack_route_weight(route_weight: torch.Tensor) -> torch.Tensor:
@@ -198,7 +194,6 @@ def triton_rms_norm_fp32_gemm_block_quant_forward(
     _check_hidden(K)
     _lib.require_device_bf16(x, "x")
     _lib.require_device_bf16(norm_weight, "norm_weight")
-    device = x.device
     if rms is None:
         assert output_mode == 0
     weight, form, w_fp32, need = route_weight, 0, 0, 0
@@ -220,7 +215,6 @@ def triton_rms_norm_fp32_gemm_block_quant_forward(
                 weight, form = weight.view(-1)[planes:], 2
         if form == 2:
             need = int(_lib.lib.fq_rmsnorm_router_folded_scratch_bytes(K, N))
-    with _lib.on_device(device):
-        new = _lib.native.rmsnorm_router_quant(x, norm_weight, weight, N, form, w_fp32, need, rms, output_mode,
-                                               float(eps), int(bool(round_scale)), _lib.stream_of(x))
+    new = _lib.native.rmsnorm_router_quant(x, norm_weight, weight, N, form, w_fp32, need, rms, output_mode,
+                                           float(eps), int(bool(round_scale)), _lib.stream_of(x))
     return new if rms is None else (new[0], rms, *new[2:])

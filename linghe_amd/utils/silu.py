@@ -12,6 +12,9 @@ import torch
 from .. import _lib
 
 
+_PlanShape = ctypes.c_int64 * 5
+
+
 class ExpertPlan:
     """Device-side table of the 128-row blocks of one set of per-expert counts.
 
@@ -37,15 +40,12 @@ def build_expert_plan(counts: torch.Tensor, splits, pad: int = 1) -> ExpertPlan:
     """counts: device int32/int64 [n_experts]; splits: the same numbers as a python list;
     pad: 1 for the layouts with the experts back to back (SwiGLU, blockwise quantiser), 16 for
     gather + pad + quant (every expert's region of the outputs rounded up to 16 rows)."""
-    shape = (ctypes.c_int64 * 5)()
-    _lib.native.expert_plan_shape(splits, pad, ctypes.addressof(shape))
-    nbytes = int(_lib.lib.fq_expert_plan_bytes(shape))
-    table = torch.empty((max(nbytes, 16),), device=counts.device, dtype=torch.uint8)
-    if shape[0]:
-        with _lib.on_device(counts.device):
-            _lib.check(_lib.lib.fq_build_expert_plan(
-                _lib.ptr(counts), _counts_flag(counts), counts.shape[0], shape, _lib.ptr(table),
-                _lib.stream_of(counts)))
+    shape = _PlanShape()
+    flag = 1 if counts.dtype == torch.int64 else 0 if counts.dtype == torch.int32 else -1
+    table = _lib.native.expert_plan(counts, flag, splits, pad, ctypes.addressof(shape),
+                                     _lib.stream_of(counts) if counts.is_cuda else 0)
+    if table is None:
+        _counts_flag(counts)  # raises
     return ExpertPlan(table, shape)
 
 
@@ -100,8 +100,7 @@ def triton_weighted_silu_forward(x, weight=None, out=None, asm=False):
     if weight is not None:
         assert weight.is_contiguous() and weight.numel() == M
         wflag = _weight_flag(weight)
-    with _lib.on_device(x.device):
-        new = _lib.native.swiglu(x, weight, wflag, out, _lib.stream_of(x))
+    new = _lib.native.swiglu(x, weight, wflag, out, _lib.stream_of(x))
     return new if out is None else out
 
 
@@ -127,8 +126,7 @@ def triton_weighted_silu_backward(g, x, weight=None):
     if weight is not None:
         assert weight.is_contiguous() and weight.numel() == M
         wflag = _weight_flag(weight)
-    with _lib.on_device(x.device):
-        return _lib.native.swiglu_bwd(g, x, weight, wflag, _lib.stream_of(x))
+    return _lib.native.swiglu_bwd(g, x, weight, wflag, _lib.stream_of(x))
 
 
 def triton_silu_and_block_quant_forward(
@@ -156,10 +154,8 @@ def triton_silu_and_block_quant_forward(
     n = N // 2
     assert output_mode in (0, 1, 2)
     assert n % 128 == 0 and N == 2 * n
-    device = x.device
-    with _lib.on_device(device):
-        return _lib.native.swiglu_quant(x, out, scale, int(bool(round_scale)), output_mode, fp8_dtype,
-                                        _lib.fp8_kind(fp8_dtype) if M else 0, _lib.stream_of(x))
+    return _lib.native.swiglu_quant(x, out, scale, int(bool(round_scale)), output_mode, fp8_dtype,
+                                    _lib.fp8_kind(fp8_dtype) if M else 0, _lib.stream_of(x))
 
 
 def triton_silu_and_block_quant_backward(g, x, round_scale=False, *, fp8_dtype=torch.float8_e4m3fn):
@@ -184,10 +180,8 @@ def triton_silu_and_block_quant_backward(g, x, round_scale=False, *, fp8_dtype=t
     assert g.shape == (M, n)
     _lib.require_device_bf16(x, "x")
     _lib.require_device_bf16(g, "g")
-    device = x.device
-    with _lib.on_device(device):
-        return _lib.native.swiglu_quant_bwd(g, x, int(bool(round_scale)), fp8_dtype,
-                                            _lib.fp8_kind(fp8_dtype) if M else 0, _lib.stream_of(x))
+    return _lib.native.swiglu_quant_bwd(g, x, int(bool(round_scale)), fp8_dtype,
+                                        _lib.fp8_kind(fp8_dtype) if M else 0, _lib.stream_of(x))
 
 
 def triton_batch_weighted_silu_and_block_quant_forward(
@@ -235,9 +229,8 @@ def triton_batch_weighted_silu_and_block_quant_forward(
     if M > 0:
         tiles = _tiles_of(plan, blocks, counts, device)
         wflag, kind = _weight_flag(weight), _lib.fp8_kind(fp8_dtype)
-    with _lib.on_device(device):
-        new = _lib.native.batched_swiglu_quant(x, weight, wflag, *tiles, blocks, out, scale, int(bool(round_scale)),
-                                               output_mode, fp8_dtype, kind, _lib.stream_of(x))
+    new = _lib.native.batched_swiglu_quant(x, weight, wflag, *tiles, blocks, out, scale, int(bool(round_scale)),
+                                           output_mode, fp8_dtype, kind, _lib.stream_of(x))
     return new[0] if out is None else out, new[1] if scale is None else scale, new[2], new[3]
 
 
@@ -269,7 +262,6 @@ def triton_batch_weighted_silu_and_block_quant_backward(
     if blocks != 0:
         tiles = _tiles_of(plan, blocks, counts, device)
         wflag, kind = _weight_flag(weight), _lib.fp8_kind(fp8_dtype)
-    with _lib.on_device(device):
-        new = _lib.native.batched_swiglu_quant_bwd(g, x, weight, wflag, dw, *tiles, blocks, int(bool(round_scale)),
-                                                   fp8_dtype, kind, _lib.stream_of(x))
+    new = _lib.native.batched_swiglu_quant_bwd(g, x, weight, wflag, dw, *tiles, blocks, int(bool(round_scale)),
+                                               fp8_dtype, kind, _lib.stream_of(x))
     return new if dw is None else (new[0], new[1], dw, new[3], new[4])
