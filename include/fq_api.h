@@ -214,6 +214,11 @@ int fq_rmsnorm_router_quant_fwd(const void* x, const void* gamma, const void* ro
                                 int64_t M, int64_t K, int64_t N, float eps, int round_scale, int fp8_kind,
                                 void* stream);
 
+/* In how many slices of K fq_rmsnorm_router_quant_fwd and its packed form work on a call whose row tiles and
+ * logits leave most of the GPU without work, 0 where they do not.  Such a call reads route_weight as it is and leaves
+ * weight_scratch alone; it is two launches, the first of which leaves partial sums in y and q. */
+int fq_rmsnorm_router_slices(int64_t M, int64_t K, int64_t N, int weight_is_fp32);
+
 /* The two halves of fq_rmsnorm_router_quant_fwd, for callers that keep the re-ordered weight
  * between weight updates (the reference re-reads route_weight on every call,
  * linghe/utils/norm.py:736-784; a router weight changes once per optimiser step).
@@ -229,8 +234,9 @@ int fq_rmsnorm_router_quant_fwd_packed(const void* x, const void* gamma, const v
                                        void* stream);
 
 /* fq_rmsnorm_router_quant_fwd of an fp32 route_weight with gamma multiplied into the weight, for the
- * sizes where that is the faster form: fq_rmsnorm_router_folds() is 1 (always 0 for a bf16 weight);
- * other sizes are refused.  Two terms of gamma * route_weight stand for the two of route_weight, but
+ * sizes where that is faster than one launch of fq_rmsnorm_router_quant_fwd: fq_rmsnorm_router_folds() is 1
+ * (always 0 for a bf16 weight); other sizes are refused.  (Where fq_rmsnorm_router_slices() is not 0 that
+ * form is faster still.)  Two terms of gamma * route_weight stand for the two of route_weight, but
  * for blocks of 64 logits and 64 columns where they would lose more or leave the range of bf16, so
  * the logits differ from those of the other forms by rounding.  scratch:
  * fq_rmsnorm_router_folded_scratch_bytes() bytes the call overwrites (gamma may change from call to

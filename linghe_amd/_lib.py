@@ -47,6 +47,7 @@ SIGNATURES = {
     "fq_pack_router_weight": [_P, _I, _P, _L, _L, _P],
     "fq_rmsnorm_router_quant_fwd_packed": [_P, _P, _P, _I, _P, _P, _P, _P, _P, _L, _L, _L, _F, _I, _I, _P],
     "fq_rmsnorm_router_folds": [_L, _L, _L, _I],
+    "fq_rmsnorm_router_slices": [_L, _L, _L, _I],
     "fq_rmsnorm_router_quant_fwd_folded": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _L, _L, _L, _F, _I, _I, _P],
     "fq_swiglu_quant_fwd": [_P, _P, _P, _P, _P, _L, _L, _I, _I, _I, _P],
     "fq_swiglu_quant_bwd": [_P, _P, _P, _P, _P, _P, _L, _L, _I, _I, _P],

@@ -432,6 +432,11 @@ int fq_rmsnorm_router_folds(int64_t M, int64_t K, int64_t N, int weight_is_fp32)
   return weight_is_fp32 && fq::router_folds(M, (int)K, (int)N);
 }
 
+int fq_rmsnorm_router_slices(int64_t M, int64_t K, int64_t N, int weight_is_fp32) {
+  if (M <= 0 || K <= 0 || N <= 0 || K > 8192 || N > 8192) return 0;
+  return fq::router_slices(M, (int)K, (int)N, weight_is_fp32 != 0);
+}
+
 int64_t fq_rmsnorm_router_folded_scratch_bytes(int64_t K, int64_t N) {
   if (K <= 0 || N <= 0 || K > 8192 || N > 8192) return 0;
   return fq::rmsnorm_router_folded_scratch_bytes((int)K, (int)N);

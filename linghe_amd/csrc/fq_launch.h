@@ -94,6 +94,9 @@ hipError_t launch_rmsnorm_router_quant(const void* x, const void* gamma, const v
                                        int64_t M, int K, int N, float eps, int round_scale, int kind,
                                        hipStream_t stream);
 
+// slices of K in which these work on a call of few row tiles and logits, 0 for the others
+int router_slices(int64_t M, int K, int N, bool weight_fp32);
+
 // the same for an fp32 weight, gamma multiplied into it; only where router_folds()
 bool router_folds(int64_t M, int K, int N);
 int64_t rmsnorm_router_folded_scratch_bytes(int K, int N);

@@ -23,6 +23,7 @@
 // share of the K / 128 quantisation groups, re-reading that part of x: from the L2 where the XCD's
 // row tiles and the weight still fit it (8192 x 256 x 2048 fetched 63.6 MB past the L2s where x and one weight per
 // XCD are 42; 49.9 with quantising waves of their own, which do so beside the products).
+#include <algorithm>
 #include <type_traits>
 
 #include "fq_device.hpp"
@@ -1222,6 +1223,206 @@ __global__ __launch_bounds__(512) void rmsnorm_router_quant_folded_kernel(Router
 }
 
 
+// ---------------------------------------------------------------------------
+// Calls whose row tiles and logits leave most of the chip without work, in two launches: the products over slices of K, as many
+// as the chip has room for, then per row the sum over the slices, the statistic, y, codes and scales. What a slice leaves of a
+// row's logits (fp32) lies in the row's own y and, where that is full, its own codes, which the second kernel reads before it
+// writes them: no scratch, and the weight needs no re-ordering of its own ahead.
+// 64 rows x 64 logits of a slice per workgroup of four waves. Per slab of 64 columns the threads turn x into its two operand
+// terms and an fp32 weight into its two planes, in LDS, two slabs of both on their way; a wave multiplies 32 rows by 32 logits.
+// PACKED: the weight in operand order (pack_router_weight), the same values and order of products.
+// Bound by the operand arithmetic and LDS traffic of a slab (about 700 clocks each, of 500 of matrix instructions) with two or
+// three workgroups on a CU to overlap them, and by two launches' latencies. us of the kernels, few-rows or 64-row form with its
+// re-ordering of the weight / products + rows: 640 x 256 x 4608 fp32 6.8 + 32.8 / 16.2 + 7.5, 512 x 256 x 7168 bf16 5.9 + 19.6 / 11.9
+// + 7.5, 1024 x 512 x 4096 bf16 6.0 + 31.3 / 18.9 + 8.1. A k step for each wave (operands read from LDS once) 17.8 for the 16.2,
+// operands loaded into registers in lane order, without LDS, 20.7.
+// ---------------------------------------------------------------------------
+struct RouterSliceArgs {
+  RouterArgs a;
+  int slices, y_slices;  // of which lie in y
+};
+__device__ __forceinline__ float* router_slice(const RouterSliceArgs& p, int64_t row, int slice) {
+  uint8_t* in_y = (uint8_t*)(p.a.y + row * p.a.K) + (int64_t)slice * p.a.N * 4;
+  uint8_t* in_q = p.a.q + row * p.a.K + (int64_t)(slice - p.y_slices) * p.a.N * 4;
+  return (float*)(slice < p.y_slices ? in_y : in_q);
+}
+
+template <bool FP32W, bool PACKED>
+__global__ __launch_bounds__(256) void router_slices_kernel(RouterSliceArgs p) {
+  constexpr int P = FP32W ? 2 : 1;  // planes of W
+  __shared__ uint4 sa[2][2][2][4][64];  // [buffer][hi, lo][32 rows][k step][lane slot]
+  __shared__ uint4 sb[2][P][2][4][64];  // [buffer][plane][32 logits][k step][lane slot]
+  const RouterArgs& a = p.a;
+  const int tid = (int)tid_x(), lane = tid & 63;
+  const int wave = uniform32(tid >> 6);
+  const int c = tid & 7, r = tid >> 3;  // piece of eight columns of a slab, row (and r + 32)
+  const int slice = (int)wg_x() % p.slices, tile = (int)wg_x() / p.slices;  // (with eight slices an XCD has its own part of K)
+  const int col_tiles = a.N / 64;
+  const int tile_m = tile / col_tiles, tile_n = tile - tile_m * col_tiles;
+  const int row0 = min(tile_m * kRouterRows, a.M - kRouterRows);  // (rows that do not fill a tile are worked on twice)
+  const int slabs = a.K / 64;
+  const int first = slice * slabs / p.slices, last = (slice + 1) * slabs / p.slices - 1;
+  struct Set {
+    u32x4_t x[2], g, w[2][P];  // w: of logits r and r + 32, raw fp32 or planes
+  } set[2];
+  // 16 bytes at `at` of one of three arrays; nothing is read beyond the slice's last slab
+  const int vtiles = a.N / 32 * P;
+  const uint8_t* const w_base = (const uint8_t*)a.w + (PACKED ? (int64_t)tile_n * 2 * P * 8192 : (int64_t)tile_n * 64 * a.K * (P * 2));
+  const uint32_t w_bytes = PACKED ? (uint32_t)((a.K / kGroup - 1) * vtiles + 2 * P) * 8192u : 64u * a.K * (P * 2);
+  const uint32_t x_at = (uint32_t)(r * a.K + c * 8) * 2u, w_at = PACKED ? c * 1024u + r * 16u : x_at * P;
+  auto load = [&](const void* base, uint32_t bytes, bool valid, uint32_t at, uint32_t from) {
+    return __builtin_amdgcn_raw_buffer_load_b128(
+        __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, valid ? bytes : 0, 0x00027000), at, from, 0);
+  };
+  auto fetch = [&](int slab, Set& d) {
+    const bool valid = slab <= last;
+    const uint32_t k = (uint32_t)slab * 64u, pitch = 64u * a.K;  // of 32 rows of x
+#pragma unroll
+    for (int u = 0; u < 2; ++u) d.x[u] = load(a.x + (int64_t)row0 * a.K, 2 * pitch, valid, x_at, u * pitch + k * 2);
+    d.g = load(a.gamma, a.K * 2, valid, c * 16u, k * 2);
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int v = 0; v < P; ++v)
+        d.w[u][v] = PACKED ? load(w_base, w_bytes, valid, w_at, ((k >> 7) * vtiles + u * P + v) * 8192u + (k & 64) * 8u)
+                           : load(w_base, w_bytes, valid, w_at + v * 16u, (u * pitch + k * 2) * P);
+  };
+  auto words = [](const u32x4_t& v) { return make_uint4(v[0], v[1], v[2], v[3]); };
+  // (the position is XORed with the piece so that the eight lanes of a row write to different banks)
+  const int slot = (c & 1) * 32 + (r ^ c), step = c >> 1;
+  auto produce = [&](int buf, const Set& d) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      uint4 hi, lo;
+      router_split(words(d.x[u]), words(d.g), hi, lo);
+      sa[buf][0][u][step][slot] = hi;
+      sa[buf][1][u][step][slot] = lo;
+      if constexpr (FP32W && !PACKED) {
+        float w[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) w[i] = __uint_as_float(d.w[u][i >> 2 & (P - 1)][i & 3]);
+        router_planes(w, hi, lo);
+        sb[buf][0][u][step][slot] = hi;
+        sb[buf][P - 1][u][step][slot] = lo;
+      } else {
+#pragma unroll
+        for (int v = 0; v < P; ++v) sb[buf][v][u][step][slot] = words(d.w[u][v]);
+      }
+    }
+  };
+  // the products of the leading terms apart from the others: shorter chains of roundings
+  floatx16_t lead, rest;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) lead[v] = rest[v] = 0.f;
+  const int rt = wave & 1, ct = wave >> 1;
+  auto multiply = [&](int buf) {
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      const int at = (lane & 32) + ((lane & 31) ^ (2 * ks + (lane >> 5)));
+      const bf16x8_t hi = operand(sa[buf][0][rt][ks][at]), lo = operand(sa[buf][1][rt][ks][at]);
+      const bf16x8_t w = operand(sb[buf][0][ct][ks][at]);
+      lead = __builtin_amdgcn_mfma_f32_32x32x16_bf16(hi, w, lead, 0, 0, 0);
+      rest = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lo, w, rest, 0, 0, 0);
+      if constexpr (FP32W) {
+        const bf16x8_t wl = operand(sb[buf][P - 1][ct][ks][at]);
+        rest = __builtin_amdgcn_mfma_f32_32x32x16_bf16(hi, wl, rest, 0, 0, 0);
+        rest = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lo, wl, rest, 0, 0, 0);
+      }
+    }
+  };
+  fetch(first, set[0]);
+  fetch(first + 1, set[1]);
+  auto one = [&](int slab, int u) {
+    produce(u, set[u]);
+    fetch(slab + 2, set[u]);
+    __syncthreads();
+    multiply(u);
+    __builtin_amdgcn_sched_barrier(0);  // (the next slab is not waited for earlier)
+  };
+  int slab = first;
+#pragma unroll 1
+  for (; slab < last; slab += 2) {  // (no branch inside: the waits count the loads behind the one they are for)
+    one(slab, 0);
+    one(slab + 1, 1);
+  }
+  if (slab == last) one(slab, 0);
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    // register v of a 32x32 result holds row (v / 4) * 8 + (lane / 32) * 4 + v % 4, column lane % 32
+    const int row = row0 + rt * 32 + (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3);
+    router_slice(p, row, slice)[tile_n * 64 + ct * 32 + (lane & 31)] = lead[v] + rest[v];
+  }
+}
+
+constexpr int kRouterSliceLogits = 1024;  // at most: four of a row for each of 256 threads
+template <int NC, int KIND, bool ROUND>
+__global__ __launch_bounds__(256) void router_finish_kernel(RouterSliceArgs p) {
+  __shared__ double red[4];
+  __shared__ unsigned nonfinite;
+  const RouterArgs& a = p.a;
+  const int tid = (int)tid_x();
+  const int64_t row = wg_x();
+  const int last = (a.K >> 3) - 1;
+  uint4 raw[NC], gm[NC];
+#pragma unroll
+  for (int k = 0; k < NC; ++k) raw[k] = *(const uint4*)(a.x + row * a.K + min(tid + k * 256, last) * 8);
+#pragma unroll
+  for (int k = 0; k < NC; ++k) gm[k] = *(const uint4*)(a.gamma + min(tid + k * 256, last) * 8);
+  float sum[kRouterSliceLogits / 256];
+#pragma unroll
+  for (int i = 0; i < kRouterSliceLogits / 256; ++i) {
+    sum[i] = 0.f;
+    const int n = tid + i * 256;
+    if (n < a.N) {
+#pragma unroll 1
+      for (int s0 = 0; s0 < p.slices; s0 += 8) {
+        float part[8];
+#pragma unroll
+        for (int s = 0; s < 8; ++s) part[s] = router_slice(p, row, min(s0 + s, p.slices - 1))[n];
+#pragma unroll
+        for (int s = 0; s < 8; ++s) sum[i] += s0 + s < p.slices ? part[s] : 0.f;
+      }
+    }
+  }
+  double ss = 0.0;
+#pragma unroll
+  for (int k = 0; k < NC; ++k) {
+    const float squares = sumsq8(raw[k]);
+    ss += (double)(tid + k * 256 <= last ? squares : 0.f);
+  }
+  ss = wave_sum_d(ss);
+  if ((tid & 63) == 0) red[tid >> 6] = ss;
+  if (tid == 0) nonfinite = 0;
+  // the slices are in registers before any of the row's y and codes is written over them
+#pragma unroll
+  for (int i = 0; i < kRouterSliceLogits / 256; ++i) asm volatile("" : "+v"(sum[i]));
+  __syncthreads();
+  const float r = 1.0f / sqrtf((float)(((red[0] + red[1]) + red[2]) + red[3]) / (float)a.K + a.eps);
+  unsigned factor = __float_as_uint(r);
+  if (factor == 0) {  // workgroup-uniform
+    bool bad = false;
+#pragma unroll
+    for (int k = 0; k < NC; ++k) bad |= router_nonfinite(raw[k]) || router_nonfinite(gm[k]);
+    if (bad) nonfinite = 1;
+    __syncthreads();
+    if (nonfinite) factor = kNanBits;
+  }
+  if (tid == 0) a.rstd[row] = r;
+#pragma unroll
+  for (int i = 0; i < kRouterSliceLogits / 256; ++i) {
+    const int n = tid + i * 256;
+    if (n < a.N) a.logits[row * a.N + n] = router_logit(sum[i], factor);
+  }
+#pragma unroll
+  for (int k = 0; k < NC; ++k) {
+    const int c = tid + k * 256;  // 16 lanes have a group, all of them or none a place in the row
+    if (c <= last)
+      router_emit<KIND, ROUND>(a.y + row * a.K + c * 8, a.q + row * a.K + c * 8, a.s + (int64_t)(c >> 4) * a.M + row,
+                               (c & 15) == 0, raw[k], gm[k], r);
+  }
+}
+
+
 int64_t rmsnorm_router_folded_scratch_bytes(int K, int N) {
   return (int64_t)N * K * 4 + (int64_t)(N / 64) * (K / 64) * 4;  // two bf16 planes, a word per block of 64 x 64
 }
@@ -1298,6 +1499,52 @@ bool router_folds(int64_t M, int K, int N) {
   return K >= (workgroups <= 256 ? 384 : 896);
 }
 
+// Slices of K of the two-launch form, 0 where a call takes another one: as many as make 256 workgroups of 64 x 64 (512 where
+// there are more than 64 row and column tiles), as fit into y and the codes, at most 16; fewer than three leave the chip idle
+// still. us of a call on a weight as it is, other forms / slices (number of tiles behind the size). bf16: 1024 x 256 (64) x 1536
+// 14.7 / 14.2, x 2048 17.6 / 15.3, x 4096 26.4 / 20.3, x 7168 37.7 / 27.1, 512 x 256 (32) x 4096 17.5 / 14.6, 2048 x 256 (128) x 2048
+// 22.5 / 21.2, x 4096 37.1 / 27.8, 1024 x 512 (128) x 7168 54.5 / 36.5, 4096 x 128 (128) x 4096 45.1 / 35.8, 2560 x 256 (160) x 2048
+// 22.9 / 23.8, x 4096 38.5 / 34.3, 1664 x 512 (208) x 3328 32.7 / 33.3 (a weight re-ordered ahead saves the others 4-6, and more
+// than 64 tiles of K = 2048 are level then). fp32, of which the larger fold gamma in one launch more: 512 x 256 x 1024
+// 14.2 / 13.7, 640 x 256 (40) x 4608 39.4 / 23.6, 512 x 512 (64) x 2048 22.6 / 19.2, x 7168 53.4 / 34.4, 1024 x 256 x 1024 15.7 / 14.3,
+// x 4096 30.9 / 24.7, 1536 x 256 (96) x 4096 31.1 / 34.6, 2048 x 256 x 7168 55.4 / 58.1; with 128 logits, which fold late,
+// 2048 x 128 (64) x 2048 23.5 / 18.3, 4096 x 128 (128) x 2048 24.0 / 27.9, x 4096 48.6 / 45.2, x 7168 83.1 / 70.1. Two slices or one:
+// 128 x 512 x 1536 fp32 16.3 / 25.4, 512 x 512 x 1024 bf16 14.2 / 16.5.
+int router_slices(int64_t M, int K, int N, bool weight_fp32) {
+  if (M < kRouterRows || N > kRouterSliceLogits) return 0;
+  const int64_t tiles = (M + kRouterRows - 1) / kRouterRows * (N / 64);
+  const int most = weight_fp32 ? (N == 128 && K >= 4096 ? 128 : K >= 1024 ? 64 : 0)
+                               : (K >= 4096 ? 160 : K >= 2560 ? 128 : K >= 2048 ? 64 : 0);
+  if (tiles > most) return 0;
+  const int64_t fill = ((tiles <= 64 ? 256 : 512) + tiles - 1) / tiles;
+  const int slices = (int)std::min<int64_t>({fill, K / (2 * N) + K / (4 * N), K / 128, 16});
+  return slices >= 3 ? slices : 0;
+}
+
+template <bool FP32W, bool PACKED>
+static hipError_t launch_router_slices(const RouterArgs& a, int slices, int round_scale, int kind, hipStream_t stream) {
+  const RouterSliceArgs p{a, slices, std::min(slices, a.K / (2 * a.N))};
+  const int64_t tiles = (int64_t)(a.M + kRouterRows - 1) / kRouterRows * (a.N / 64);
+  hipLaunchKernelGGL((router_slices_kernel<FP32W, PACKED>), dim3((unsigned)(tiles * slices)), dim3(256), 0, stream, p);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+#define FQ_FINISH(NCV, KINDV, ROUNDV) \
+  hipLaunchKernelGGL((router_finish_kernel<NCV, KINDV, ROUNDV>), dim3((unsigned)a.M), dim3(256), 0, stream, p)
+#define FQ_FINISH_NC(KINDV, ROUNDV)                    \
+  if (a.K <= 2048) FQ_FINISH(1, KINDV, ROUNDV);        \
+  else if (a.K <= 4096) FQ_FINISH(2, KINDV, ROUNDV);   \
+  else if (a.K <= 6144) FQ_FINISH(3, KINDV, ROUNDV);   \
+  else FQ_FINISH(4, KINDV, ROUNDV);
+  if (kind == kE5M2) {
+    if (round_scale) { FQ_FINISH_NC(kE5M2, true) } else { FQ_FINISH_NC(kE5M2, false) }
+  } else {
+    if (round_scale) { FQ_FINISH_NC(kE4M3, true) } else { FQ_FINISH_NC(kE4M3, false) }
+  }
+#undef FQ_FINISH_NC
+#undef FQ_FINISH
+  return hipGetLastError();
+}
+
 // the main kernels on a weight already in operand order
 hipError_t launch_rmsnorm_router_quant_packed(const void* x, const void* gamma, const void* wpacked,
                                               int weight_fp32, void* y, float* rstd, float* logits, void* q,
@@ -1306,6 +1553,9 @@ hipError_t launch_rmsnorm_router_quant_packed(const void* x, const void* gamma, 
   if (M == 0) return hipSuccess;
   RouterArgs p{(const uint16_t*)x, (const uint16_t*)gamma, (const uint4*)wpacked, (uint16_t*)y, rstd, logits,
                (uint8_t*)q, s, (int)M, K, N, 0, eps};
+  if (const int slices = router_slices(M, K, N, weight_fp32 != 0))
+    return weight_fp32 ? launch_router_slices<true, true>(p, slices, round_scale, kind, stream)
+                       : launch_router_slices<false, true>(p, slices, round_scale, kind, stream);
   const RouterForm f = router_form(M, K, N, weight_fp32 != 0);
   p.chunks = N / f.cols;
   const dim3 grid((unsigned)((M + f.rows - 1) / f.rows * p.chunks));
@@ -1379,6 +1629,12 @@ hipError_t launch_rmsnorm_router_quant(const void* x, const void* gamma, const v
                                        int64_t M, int K, int N, float eps, int round_scale, int kind,
                                        hipStream_t stream) {
   if (M == 0) return hipSuccess;
+  if (const int slices = router_slices(M, K, N, weight_fp32 != 0)) {  // (the weight as it is)
+    const RouterArgs p{(const uint16_t*)x, (const uint16_t*)gamma, (const uint4*)wr, (uint16_t*)y, rstd, logits,
+                       (uint8_t*)q, s, (int)M, K, N, 0, eps};
+    return weight_fp32 ? launch_router_slices<true, false>(p, slices, round_scale, kind, stream)
+                       : launch_router_slices<false, false>(p, slices, round_scale, kind, stream);
+  }
   const hipError_t e = launch_pack_router_weight(wr, weight_fp32, wpacked, K, N, stream);
   if (e != hipSuccess) return e;
   return launch_rmsnorm_router_quant_packed(x, gamma, wpacked, weight_fp32, y, rstd, logits, q, s, M, K, N, eps,

@@ -203,7 +203,8 @@ def triton_rms_norm_fp32_gemm_block_quant_forward(
         if not route_weight.is_cuda:
             raise RuntimeError("route_weight must live on the GPU: the HIP kernels are the only implementation")
         w_fp32 = int(route_weight.dtype == torch.float32)
-        folds = w_fp32 and _lib.lib.fq_rmsnorm_router_folds(M, K, N, w_fp32)
+        sliced = _lib.lib.fq_rmsnorm_router_slices(M, K, N, w_fp32)
+        folds = w_fp32 and not sliced and _lib.lib.fq_rmsnorm_router_folds(M, K, N, w_fp32)
         planes = int(_lib.lib.fq_rmsnorm_router_scratch_bytes(K, N, w_fp32))
         need, form = planes, 2 if folds else 0
         if packed_route_weight is not None:
