@@ -24,7 +24,9 @@ struct Policy {
   // (M or a per-expert count that is not a multiple of 16) are where the hint on the transposed
   // stores costs most: the SwiGLU forward takes 100 instead of 70 us at 16300 x 3584 with it (and
   // gains 3 % at 8192 x 2048), so it keeps the hint on the row-wise codes only; the RMSNorm tile
-  // kernel gains 18 % from it on aligned rows and loses 8 % on unaligned ones.
+  // kernel gains 18 % from it on rows that start on lines and loses on others, which go out in pieces from two row blocks that
+  // an L2 would merge: 14160 x 5120 46.0 us without / 68.9 with it, 9104 x 4096 24.2 / 32.3, 14160 x 5632 49.8 / 66.0; rows on half
+  // lines are level (14144 x 4096 36.7 / 36.6, 4160 x 2048 8.5 / 7.7).
   static constexpr int kStoreHintBlockwise = 0;
   static constexpr int kStoreHintBlockwiseBatched = 1;
   // ... and with its tiles read from a plan, numbered so that neighbouring row blocks share an XCD, the row-wise
@@ -83,6 +85,11 @@ struct Policy {
   static constexpr bool kPlanPackedFirstSiluBwd = false;
   static constexpr bool kPlanPackedFirstBlockwise = true;
   static constexpr bool kPlanPackedFirstPermute = false;  // 43.8 / 43.3 us first / last (33040 x 2048 gathered from 16384 rows)
+  // One matrix, M no multiple of 128: neighbouring row blocks share lines of the transposed rows, which one L2 merges and two
+  // write out twice. In grid order a column block stays on its XCD where their number is a multiple of 8; elsewhere every XCD
+  // takes an eighth of the tiles counted column block after column block. us of the tile kernel in grid order / so: RMSNorm
+  // 15935 x 5248 62.8 / 52.8, 8120 x 2176 14.8 / 11.8, 3046 x 1408 7.4 / 6.8, 6537 x 768 7.7 / 7.2, 1303 x 6272 8.4 / 7.7, plain
+  // quantiser 9040 x 3968 31.4 / 27.6, 4720 x 6528 27.8 / 25.4, 6256 x 2944 17.6 / 17.2, 15216 x 640 10.6 / 10.7.
   // row blocks per run that an XCD works on (xcd_runs; 0: every eighth tile).  Same sizes, planned launches with
   // 0 / 2 / 4 / 8 / 16: SwiGLU forward 43.4 / 41.2 / 40.8 / 40.7 / 40.8 us, backward 76.5 / 76.1 / 75.5 / 75.3 / 76.2,
   // blockwise quantiser 30.9 / 30.3 / 29.9 / 29.9 / 29.8.  Launches that scan the counts, 0 / 2 / 4 / 8: forward

@@ -86,12 +86,13 @@ __device__ __forceinline__ int xcd_runs(int id, int total, int chunk) {
 // faster with it at 16384 x 7168 and slower below ~2000 tiles or with narrow rows, the
 // per-expert SwiGLU backward 5 % faster; gather+pad+quant 18 % slower, the blockwise
 // quantisers 5-9 %, the forward SwiGLU kernels 2-4 %), so the caller decides.
+// 2 = the same eighths of the tiles taken column block after column block (fq_policy.hpp).
 template <bool BATCHED>
 __device__ __forceinline__ TileGeom resolve_tile(int64_t M, int ncb, int64_t out_w, const BatchArgs& b,
                                                  int remap = 0) {
   TileGeom g;
   int id = wg_x();
-  if (remap == 1) {  // workgroup-uniform
+  if (remap) {  // workgroup-uniform
     const int G = (int)n_wg_x();
     const int per = (G + 7) >> 3;
     const int xcd = id & 7, slot = id >> 3;
@@ -102,8 +103,15 @@ __device__ __forceinline__ TileGeom resolve_tile(int64_t M, int ncb, int64_t out
   g.kc_shift = 0;
   g.n_sub = 1;
   if constexpr (!BATCHED) {
-    const int rbk = id / ncb;
-    g.cb = id - rbk * ncb;
+    int rbk;
+    if (remap == 2) {  // column block after column block
+      const int rbs = (int)((M + kGroup - 1) / kGroup);
+      g.cb = id / rbs;
+      rbk = id - g.cb * rbs;
+    } else {
+      rbk = id / ncb;
+      g.cb = id - rbk * ncb;
+    }
     g.row0 = (int64_t)rbk * kGroup;
     const int64_t left = M - g.row0;
     g.rows_valid = left < kGroup ? (int)left : kGroup;

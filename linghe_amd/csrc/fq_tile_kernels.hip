@@ -16,12 +16,13 @@ namespace fq {
 // ---------------------------------------------------------------------------
 // PLANNED: the per-expert form with its tiles read from a plan (same code; another cache policy,
 // because its tile numbering lets an XCD's L2 merge the partial lines of the transposed codes)
-template <int KIND, bool ROUND, int MODE, bool BATCHED, bool PLANNED = false>
+// BY_COLUMNS: one matrix in the order of shared_lines_remap (a kernel of its own: the choice costs the other 0.1 us)
+template <int KIND, bool ROUND, int MODE, bool BATCHED, bool PLANNED = false, bool BY_COLUMNS = false>
 __global__ __launch_bounds__(2048 / (BATCHED ? Policy::kRowsPerThreadBlockwiseBatched : Policy::kRowsPerThreadBlockwise))
 void blockwise_quant_kernel(const uint16_t* __restrict__ x, OutPtrs out, int64_t M, int N, BatchArgs batch) {
   constexpr int RPT = BATCHED ? Policy::kRowsPerThreadBlockwiseBatched : Policy::kRowsPerThreadBlockwise;
   __shared__ TileShared<RPT> sh;
-  const TileGeom g = resolve_tile<BATCHED>(M, N / kGroup, N, batch);
+  const TileGeom g = resolve_tile<BATCHED>(M, N / kGroup, N, batch, BY_COLUMNS ? 2 : 0);
   if (!g.valid) return;
   uint4 raw[RPT];
   constexpr bool LDNT = BATCHED ? Policy::kLoadHintBlockwiseBatched : Policy::kLoadHintBlockwise;
@@ -111,10 +112,10 @@ __global__ __launch_bounds__(256) void pad_permute_quant_kernel(const uint16_t* 
 // ALL_FULL: single matrix with M a multiple of 128 (see quantize_tiles)
 template <int KIND, bool ROUND, int MODE, bool BATCHED, bool WEIGHTED, bool ALL_FULL>
 __global__ __launch_bounds__(2048 / Policy::kRowsPerThreadSiluFwd) void silu_quant_fwd_kernel(const uint16_t* __restrict__ x, RowWeight weight,
-                                                             OutPtrs out, int64_t M, int n, BatchArgs batch) {
+                                                             OutPtrs out, int64_t M, int n, int remap, BatchArgs batch) {
   constexpr int RPT = Policy::kRowsPerThreadSiluFwd;
   __shared__ TileShared<RPT> sh;
-  const TileGeom g = resolve_tile<BATCHED>(M, n / kGroup, n, batch);
+  const TileGeom g = resolve_tile<BATCHED>(M, n / kGroup, n, batch, BATCHED || ALL_FULL ? 0 : remap);
   if (!g.valid) return;
   const int64_t ld = 2 * (int64_t)n;
   uint4 r1[RPT], r2[RPT];
@@ -440,6 +441,9 @@ __global__ __launch_bounds__(1024) void expert_plan_kernel(const void* __restric
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
+// Order of the tiles of one matrix whose transposed rows share lines between row blocks (M no multiple of 128): fq_policy.hpp
+static int shared_lines_remap(int64_t M, int ncb, int mode) { return mode != 0 && M % kGroup != 0 && ncb % 8 != 0 ? 2 : 0; }
+
 static BatchArgs batch_args(const void* counts, int counts_i64, int n_experts, const void* plan,
                             const PlanShape* ps, bool packed_first, int xcd_rows_scan,
                             int xcd_rows_planned = Policy::kXcdRowsPlanned) {
@@ -491,6 +495,7 @@ hipError_t launch_blockwise_quant(const void* x, void* q, float* s, void* qt, fl
                                   const PlanShape* ps) {
   OutPtrs out{(uint8_t*)q, s, (uint8_t*)qt, st};
   const BatchArgs b = batch_args(counts, counts_i64, n_experts, plan, ps, Policy::kPlanPackedFirstBlockwise, 0);
+  const bool by_columns = !counts && !plan && shared_lines_remap(M, N / kGroup, mode);
   const int64_t tiles = plan ? plan_workgroups(ps->unpacked, ps->packed2, ps->packed4, N / kGroup)
                         : counts ? scan_workgroups(M, row_blocks, N / kGroup) : row_blocks * (N / kGroup);
   if (tiles == 0) return hipSuccess;
@@ -502,8 +507,9 @@ hipError_t launch_blockwise_quant(const void* x, void* q, float* s, void* qt, fl
       FQ_DISPATCH_MODE(mode, MD,
         FQ_DISPATCH_BOOL(batched, B,
           FQ_DISPATCH_BOOL(plan != nullptr, P,
-            hipLaunchKernelGGL((blockwise_quant_kernel<K, R, MD, B || P, P>), grid, block, 0, stream,
-                               (const uint16_t*)x, out, M, N, b);)))))
+            FQ_DISPATCH_BOOL(by_columns, C,
+              hipLaunchKernelGGL((blockwise_quant_kernel<K, R, MD, B || P, P, C && !(B || P)>), grid, block, 0, stream,
+                                 (const uint16_t*)x, out, M, N, b);))))))
   return hipGetLastError();
 }
 
@@ -533,6 +539,7 @@ hipError_t launch_silu_quant_fwd(const void* x, const void* weight, int weight_b
                                  hipStream_t stream, const void* plan, const PlanShape* ps) {
   OutPtrs out{(uint8_t*)q, s, (uint8_t*)qt, st};
   const BatchArgs b = batch_args(counts, counts_i64, n_experts, plan, ps, Policy::kPlanPackedFirstSiluFwd, 0);
+  const int remap = shared_lines_remap(M, n / kGroup, mode);
   if (mode == 0 && !counts && !plan && !weight && silu_quant_rows_per_team(M, n) > 0)
     return launch_silu_quant_rows(x, q, s, M, n, round_scale, kind, stream);
   RowWeight w{weight, weight_bf16};
@@ -550,7 +557,7 @@ hipError_t launch_silu_quant_fwd(const void* x, const void* weight, int weight_b
           FQ_DISPATCH_BOOL(weighted, W,
             FQ_DISPATCH_BOOL(all_full, AF,
               hipLaunchKernelGGL((silu_quant_fwd_kernel<K, R, MD, B, W, AF && !B>), grid, block, 0, stream,
-                                 (const uint16_t*)x, w, out, M, n, b);))))))
+                                 (const uint16_t*)x, w, out, M, n, remap, b);))))))
   return hipGetLastError();
 }
 
@@ -590,11 +597,13 @@ hipError_t launch_rmsnorm_quant_tile(const void* x, const void* gamma, const flo
   const int64_t tiles = ((M + kGroup - 1) / kGroup) * (n / kGroup);
   if (tiles == 0) return hipSuccess;
   const dim3 grid((unsigned)tiles), block(2048 / Policy::kRowsPerThreadRmsnorm);
-  // transposed rows start every M bytes: off 16-byte boundaries their stores go out plain
-  const bool aligned_rows = M % 16 == 0;
+  // transposed rows start every M bytes: where they share lines their stores go out plain
+  const bool aligned_rows = M % 64 == 0;
   // XCD remap (see resolve_tile): wide rows and several waves of workgroups
   // ... and, behind the statistic pass, wherever that pass handed out the rows by XCD
-  const int remap = (aligned_rows && n >= 4096 && tiles >= 3072) || (mode == 2 && rmsnorm_passes_by_xcd(M, n));
+  const int shared = shared_lines_remap(M, n / kGroup, mode);
+  const int remap = shared ? shared
+                    : (aligned_rows && n >= 4096 && tiles >= 3072) || (mode == 2 && rmsnorm_passes_by_xcd(M, n));
   // raised priority until the loads are out: only when the whole launch is resident at once (four
   // workgroups per CU of a 256-CU device; more tiles than that arrive in generations)
   const int first = Policy::kStartPriorityRmsnorm && tiles <= 1024;

@@ -8,7 +8,7 @@ import torch
 
 from oracle import fq_oracle as O
 from tests.helpers import announce, check_quant_pair, gen, randn_bf16
-from tests.test_gpu_parity import EXACT, _batched_case
+from tests.test_gpu_parity import EXACT, FUSED, _batched_case
 
 pytestmark = pytest.mark.gpu
 
@@ -87,3 +87,36 @@ def test_scanning_launch_has_a_workgroup_for_every_tile(gpu, counts, ncb):
     for fn, args in ((fwd, (h, w)), (bwd, (dy, h, w))):
         for a, b in zip(fn(*args, cnt, counts), fn(*args, cnt, counts, plan=plan)):
             assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
+# column blocks that do not come in eights: every XCD takes an eighth of the tiles, column block after column block; fewer tiles
+# than XCDs, eighths that end inside a column block, a last row block of the fewest rows
+@pytest.mark.parametrize("M", [16, 144, 1040, 2160])
+@pytest.mark.parametrize("ncb", [1, 3, 7, 9])
+def test_tiles_of_shared_lines(gpu, M, ncb):
+    from linghe_amd.quant.block import triton_blockwise_quant
+    from linghe_amd.utils.norm import triton_rms_norm_and_block_quant_forward
+    from linghe_amd.utils.silu import triton_silu_and_block_quant_forward
+
+    announce("tiles of shared lines", M, ncb)
+    n, g = 128 * ncb, gen(100 + ncb)
+    x, w, h = randn_bf16(g, M, n), randn_bf16(g, n), randn_bf16(g, M, 2 * n)
+    for mode in (2, 1):
+        q, s, qt, st = triton_blockwise_quant(x.to(gpu), output_mode=mode)
+        torch.cuda.synchronize()
+        ref = O.batch_blockwise_quant(x, [M], False)
+        if mode == 2:
+            check_quant_pair("shared.row", ref[0], ref[1], q.view(-1), s.view(-1), **EXACT)
+        check_quant_pair("shared.col", ref[2], ref[3], qt.view(-1), st.view(-1), **EXACT)
+    for rows in (M, M - 1):  # transposed rows that start anywhere
+        a = x[:rows].contiguous()
+        q, s, rms, qt, st = triton_rms_norm_and_block_quant_forward(a.to(gpu), w.to(gpu))
+        torch.cuda.synchronize()
+        ref = O.rms_norm_and_block_quant_forward(a, w, rstd=rms.cpu())
+        check_quant_pair("shared.rms.row", ref[0], ref[1], q, s, **EXACT)
+        check_quant_pair("shared.rms.col", ref[3], ref[4], qt, st, **EXACT)
+        q, s, qt, st = triton_silu_and_block_quant_forward(h[:rows].contiguous().to(gpu))
+        torch.cuda.synchronize()
+        ref = O.silu_and_block_quant_forward(h[:rows].contiguous())
+        check_quant_pair("shared.silu.row", ref[0], ref[1], q, s, **FUSED)
+        check_quant_pair("shared.silu.col", ref[2], ref[3], qt, st, **FUSED)
