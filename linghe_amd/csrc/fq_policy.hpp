@@ -17,8 +17,10 @@ struct Policy {
   // gather+pad+quant 75 -> 55 us, RMSNorm+quant after the statistic pass 25 -> 21 us
   // (8192 x 2048) and 146 -> 122 us (16384 x 7168).  The SwiGLU backward is 3-7 % slower when its
   // transposed stores carry it; the plain blockwise quantiser takes none (13.2 us at 8192 x 2048
-  // against 14.2-16.1 with any), its per-expert form the transposed stores only (31.5 us against
-  // 39.2 without, 32.7 with the row-wise codes only and 36.3 with both); the RMSNorm tile kernel
+  // against 14.2-16.1 with any), its per-expert form the row-wise codes only, so that an L2 merges the pieces of lines that two
+  // row blocks share (us with none / the transposed stores / the row-wise ones / both: 33040 x 2048 in 32 experts 53.4 / 50.0 / 46.8 /
+  // 57.2, 16000 x 4096 in 16 53.2 / 53.1 / 45.8 / 62.7, 16000 x 7168 in 64 104.9 / 122.0 / 90.2 / 124.5, 28500 x 1408 in 128 33.3 / 33.1 /
+  // 32.2 / 36.4, 65536 x 1024 in 256 55.7 / 53.6 / 51.0 / -; with a plan 65536 x 512 in 256 33.2 / 29.8 / 27.8 / 33.5); the RMSNorm tile kernel
   // with the statistic given (transposed output only, x read once: nothing to protect) none
   // (16384 x 7168: 66.6 -> 59.5 us).  Transposed rows that do not start on 16-byte boundaries
   // (M or a per-expert count that is not a multiple of 16) are where the hint on the transposed
@@ -28,11 +30,7 @@ struct Policy {
   // an L2 would merge: 14160 x 5120 46.0 us without / 68.9 with it, 9104 x 4096 24.2 / 32.3, 14160 x 5632 49.8 / 66.0; rows on half
   // lines are level (14144 x 4096 36.7 / 36.6, 4160 x 2048 8.5 / 7.7).
   static constexpr int kStoreHintBlockwise = 0;
-  static constexpr int kStoreHintBlockwiseBatched = 1;
-  // ... and with its tiles read from a plan, numbered so that neighbouring row blocks share an XCD, the row-wise
-  // codes only (the L2 then merges the partial lines of the transposed ones): 65536 x 512 in 256 experts
-  // 33.2 / 29.8 / 27.8 / 33.5 us with 0 / 1 / 2 / 3
-  static constexpr int kStoreHintBlockwisePlanned = 2;
+  static constexpr int kStoreHintBlockwiseBatched = 2;
   static constexpr int kStoreHintPermute = 3;
   static constexpr int kStoreHintSiluFwd = 2;        // both layouts, single matrix
   static constexpr int kStoreHintSiluFwdRows = 2;    // row-wise layout only

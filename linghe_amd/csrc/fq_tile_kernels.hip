@@ -14,10 +14,8 @@ namespace fq {
 // ---------------------------------------------------------------------------
 // plain blockwise quant
 // ---------------------------------------------------------------------------
-// PLANNED: the per-expert form with its tiles read from a plan (same code; another cache policy,
-// because its tile numbering lets an XCD's L2 merge the partial lines of the transposed codes)
 // BY_COLUMNS: one matrix in the order of shared_lines_remap (a kernel of its own: the choice costs the other 0.1 us)
-template <int KIND, bool ROUND, int MODE, bool BATCHED, bool PLANNED = false, bool BY_COLUMNS = false>
+template <int KIND, bool ROUND, int MODE, bool BATCHED, bool BY_COLUMNS>
 __global__ __launch_bounds__(2048 / (BATCHED ? Policy::kRowsPerThreadBlockwiseBatched : Policy::kRowsPerThreadBlockwise))
 void blockwise_quant_kernel(const uint16_t* __restrict__ x, OutPtrs out, int64_t M, int N, BatchArgs batch) {
   constexpr int RPT = BATCHED ? Policy::kRowsPerThreadBlockwiseBatched : Policy::kRowsPerThreadBlockwise;
@@ -26,8 +24,7 @@ void blockwise_quant_kernel(const uint16_t* __restrict__ x, OutPtrs out, int64_t
   if (!g.valid) return;
   uint4 raw[RPT];
   constexpr bool LDNT = BATCHED ? Policy::kLoadHintBlockwiseBatched : Policy::kLoadHintBlockwise;
-  constexpr int NT = PLANNED ? Policy::kStoreHintBlockwisePlanned
-                     : BATCHED ? Policy::kStoreHintBlockwiseBatched : Policy::kStoreHintBlockwise;
+  constexpr int NT = BATCHED ? Policy::kStoreHintBlockwiseBatched : Policy::kStoreHintBlockwise;
   constexpr bool LEAN = BATCHED || Policy::kLeanBlockwise;
   const TilePart<RPT> tp = tile_part<RPT>(g);
   load_rows<RPT, LDNT, LEAN>(x + g.row0 * N + (int64_t)(g.cb + tp.asub) * kGroup, N, tp.rows, raw, tp.sl.rgl);
@@ -506,10 +503,9 @@ hipError_t launch_blockwise_quant(const void* x, void* q, float* s, void* qt, fl
     FQ_DISPATCH_BOOL(round_scale, R,
       FQ_DISPATCH_MODE(mode, MD,
         FQ_DISPATCH_BOOL(batched, B,
-          FQ_DISPATCH_BOOL(plan != nullptr, P,
-            FQ_DISPATCH_BOOL(by_columns, C,
-              hipLaunchKernelGGL((blockwise_quant_kernel<K, R, MD, B || P, P, C && !(B || P)>), grid, block, 0, stream,
-                                 (const uint16_t*)x, out, M, N, b);))))))
+          FQ_DISPATCH_BOOL(by_columns, C,
+            hipLaunchKernelGGL((blockwise_quant_kernel<K, R, MD, B, C && !B>), grid, block, 0, stream, (const uint16_t*)x,
+                               out, M, N, b);)))))
   return hipGetLastError();
 }
 
