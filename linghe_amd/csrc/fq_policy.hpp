@@ -87,7 +87,11 @@ struct Policy {
   // write out twice. In grid order a column block stays on its XCD where their number is a multiple of 8; elsewhere every XCD
   // takes an eighth of the tiles counted column block after column block. us of the tile kernel in grid order / so: RMSNorm
   // 15935 x 5248 62.8 / 52.8, 8120 x 2176 14.8 / 11.8, 3046 x 1408 7.4 / 6.8, 6537 x 768 7.7 / 7.2, 1303 x 6272 8.4 / 7.7, plain
-  // quantiser 9040 x 3968 31.4 / 27.6, 4720 x 6528 27.8 / 25.4, 6256 x 2944 17.6 / 17.2, 15216 x 640 10.6 / 10.7.
+  // quantiser 9040 x 3968 31.4 / 27.6, 4720 x 6528 27.8 / 25.4.
+  // The plain quantiser, with the least work in a tile, only from so many tiles on; us of a call with a weight's quantiser: 14800 x 1920
+  // (1740 tiles) 29.4 / 26.9, x 1664 (1508) 25.2 / 24.3, x 1408 (1276) 20.75 / 20.96, x 1152 (1044) 20.4 / 19.8, x 896 (812) 16.0 / 15.6,
+  // x 768 (696) 14.0 / 14.3, x 640 (580) 13.75 / 13.96, 6000 x 1920 (705) 14.55 / 14.69: up to 1276 it goes either way
+  static constexpr int kBlockwiseByColumnsTiles = 1408;
   // row blocks per run that an XCD works on (xcd_runs; 0: every eighth tile).  Same sizes, planned launches with
   // 0 / 2 / 4 / 8 / 16: SwiGLU forward 43.4 / 41.2 / 40.8 / 40.7 / 40.8 us, backward 76.5 / 76.1 / 75.5 / 75.3 / 76.2,
   // blockwise quantiser 30.9 / 30.3 / 29.9 / 29.9 / 29.8.  Launches that scan the counts, 0 / 2 / 4 / 8: forward

@@ -492,7 +492,8 @@ hipError_t launch_blockwise_quant(const void* x, void* q, float* s, void* qt, fl
                                   const PlanShape* ps) {
   OutPtrs out{(uint8_t*)q, s, (uint8_t*)qt, st};
   const BatchArgs b = batch_args(counts, counts_i64, n_experts, plan, ps, Policy::kPlanPackedFirstBlockwise, 0);
-  const bool by_columns = !counts && !plan && shared_lines_remap(M, N / kGroup, mode);
+  const bool by_columns = !counts && !plan && row_blocks * (N / kGroup) >= Policy::kBlockwiseByColumnsTiles &&
+                          shared_lines_remap(M, N / kGroup, mode);
   const int64_t tiles = plan ? plan_workgroups(ps->unpacked, ps->packed2, ps->packed4, N / kGroup)
                         : counts ? scan_workgroups(M, row_blocks, N / kGroup) : row_blocks * (N / kGroup);
   if (tiles == 0) return hipSuccess;

@@ -120,3 +120,19 @@ def test_tiles_of_shared_lines(gpu, M, ncb):
         ref = O.silu_and_block_quant_forward(h[:rows].contiguous())
         check_quant_pair("shared.silu.row", ref[0], ref[1], q, s, **FUSED)
         check_quant_pair("shared.silu.col", ref[2], ref[3], qt, st, **FUSED)
+
+
+# the plain quantiser takes that order from 1408 tiles on: 1404 and 1413 of them, the last row block of 112 rows
+@pytest.mark.parametrize("M", [19952, 20080])
+def test_plain_tiles_of_shared_lines(gpu, M):
+    from linghe_amd.quant.block import triton_blockwise_quant
+
+    announce("plain tiles of shared lines", M)
+    x = randn_bf16(gen(M), M, 128 * 9)
+    ref = O.batch_blockwise_quant(x, [M], False)
+    for mode in (2, 1):
+        q, s, qt, st = triton_blockwise_quant(x.to(gpu), output_mode=mode)
+        torch.cuda.synchronize()
+        if mode == 2:
+            check_quant_pair("shared.row", ref[0], ref[1], q.view(-1), s.view(-1), **EXACT)
+        check_quant_pair("shared.col", ref[2], ref[3], qt.view(-1), st.view(-1), **EXACT)
