@@ -215,7 +215,7 @@ int fq_rmsnorm_router_quant_fwd(const void* x, const void* gamma, const void* ro
                                 void* stream);
 
 /* In how many slices of K fq_rmsnorm_router_quant_fwd and its packed form work on a call whose row tiles and
- * logits leave most of the GPU without work, 0 where they do not.  Such a call reads route_weight as it is and leaves
+ * logits leave most of the GPU without work, 0 where they do not (and for sizes that they refuse).  Such a call reads route_weight as it is and leaves
  * weight_scratch alone; it is two launches, the first of which leaves partial sums in y and q. */
 int fq_rmsnorm_router_slices(int64_t M, int64_t K, int64_t N, int weight_is_fp32);
 

@@ -433,7 +433,8 @@ int fq_rmsnorm_router_folds(int64_t M, int64_t K, int64_t N, int weight_is_fp32)
 }
 
 int fq_rmsnorm_router_slices(int64_t M, int64_t K, int64_t N, int weight_is_fp32) {
-  if (M <= 0 || K <= 0 || N <= 0 || K > 8192 || N > 8192) return 0;
+  // what the entry points refuse takes no form
+  if (M <= 0 || M % 32 != 0 || K <= 0 || K % 128 != 0 || K > 8192 || N <= 0 || N % 128 != 0 || N > 8192) return 0;
   return fq::router_slices(M, (int)K, (int)N, weight_is_fp32 != 0);
 }
 

@@ -96,6 +96,11 @@ def test_c_side_validation_without_gpu():
     assert folded(*[None] * 9, 32, 4096, 256, 1e-6, 0, 0, None) == -2 and b"folds" in L.fq_last_error()
     assert folded(*[None] * 9, 4096, 4096, 256, 1e-6, 0, 0, None) == -1 and b"NULL" in L.fq_last_error()
     assert folded(*[None] * 9, 4096, 4096, 200, 1e-6, 0, 0, None) == -2 and b"router" in L.fq_last_error()
+    # slices of K: 0 for what the entry points refuse, also where a tile of 64 logits does not fit
+    slices = L.fq_rmsnorm_router_slices
+    assert [slices(*size, 0) for size in ((128, 4096, 32), (128, 4096, 1), (128, 4096, 200), (100, 4096, 256),
+                                          (128, 4100, 256), (0, 4096, 256), (128, 16384, 256), (-128, 4096, 256))] == [0] * 8
+    assert slices(128, 4096, 256, 0) > 0 and slices(128, 4096, 256, 1) > 0
     # the no-work kernel's variants: chunks per lane 4 / 8 / 16 only, order 0..3
     assert L.fq_stream_rw_variant(None, 0, None, 0, None, 4, 0, 0, 0, 0, None) == -1          # no sink
     assert L.fq_stream_rw_variant(None, 16, None, 0, None, 5, 0, 0, 0, 0, None) == -1
