@@ -24,6 +24,7 @@
 // row tiles and the weight still fit it (8192 x 256 x 2048 fetched 63.6 MB past the L2s where x and one weight per
 // XCD are 42; 49.9 with quantising waves of their own, which do so beside the products).
 #include <algorithm>
+#include <climits>
 #include <type_traits>
 
 #include "fq_device.hpp"
@@ -1499,26 +1500,53 @@ bool router_folds(int64_t M, int K, int N) {
   return K >= (workgroups <= 256 ? 384 : 896);
 }
 
-// Slices of K of the two-launch form, 0 where a call takes another one: as many as make 256 workgroups of 64 x 64 (512 where
-// there are more than 64 row and column tiles), as fit into y and the codes, at most 16; fewer than three leave the chip idle
-// still. us of a call on a weight as it is, other forms / slices (number of tiles behind the size). bf16: 1024 x 256 (64) x 1536
-// 14.7 / 14.2, x 2048 17.6 / 15.3, x 4096 26.4 / 20.3, x 7168 37.7 / 27.1, 512 x 256 (32) x 4096 17.5 / 14.6, 2048 x 256 (128) x 2048
-// 22.5 / 21.2, x 4096 37.1 / 27.8, 1024 x 512 (128) x 7168 54.5 / 36.5, 4096 x 128 (128) x 4096 45.1 / 35.8, 2560 x 256 (160) x 2048
-// 22.9 / 23.8, x 4096 38.5 / 34.3, 1664 x 512 (208) x 3328 32.7 / 33.3 (a weight re-ordered ahead saves the others 4-6, and more
-// than 64 tiles of K = 2048 are level then). fp32, of which the larger fold gamma in one launch more: 512 x 256 x 1024
-// 14.2 / 13.7, 640 x 256 (40) x 4608 39.4 / 23.6, 512 x 512 (64) x 2048 22.6 / 19.2, x 7168 53.4 / 34.4, 1024 x 256 x 1024 15.7 / 14.3,
-// x 4096 30.9 / 24.7, 1536 x 256 (96) x 4096 31.1 / 34.6, 2048 x 256 x 7168 55.4 / 58.1; with 128 logits, which fold late,
-// 2048 x 128 (64) x 2048 23.5 / 18.3, 4096 x 128 (128) x 2048 24.0 / 27.9, x 4096 48.6 / 45.2, x 7168 83.1 / 70.1. Two slices or one:
-// 128 x 512 x 1536 fp32 16.3 / 25.4, 512 x 512 x 1024 bf16 14.2 / 16.5.
+// Slices of K of the two-launch form, 0 where a call takes another one: as many as make no more than 256 workgroups of 64 x 64
+// (512 where there are more than 64 row and column tiles), as fit into y and the codes, at most 16. A few workgroups more are a
+// round more (us, packed weight: 384 x 256 (24 tiles) x 4096 fp32 10 slices 14.9 / 11 17.2, 768 x 256 (48) x 4096 fp32 5
+// 19.3 / 6 23.0, 1536 x 256 (96) x 4096 5 23.9 / 6 26.0). Fewer than three leave the chip idle still.
+// A weight packed ahead takes the form that the weight as it is takes (same results, bit by bit), and packing it saves the
+// other forms a launch. So the lines up to 64 tiles lie where the few-rows kernel alone is at most a few percent ahead (once,
+// 320 x 384 x 3840, 12). It needs one round of workgroups up to 32 tiles and two up to 64. us of a packed call few-rows / slices,
+// [of a call on the weight as it is], sizes that take the slices; then sizes that do not:
+// up to 32 tiles, 128 logits, bf16: 128 x 128 (4) x 2048 8.7 / 8.3, 512 x 128 (16) x 3200 11.5 / 11.6, 640 x 128 (20) x 3328
+// 11.7 / 12.1, 1024 x 128 (32) x 3840 13.7 / 14.0 [16.6 / 14.0], x 7168 21.7 / 18.9; 512 x 128 x 2048 9.1 / 10.1 [11.6 / 9.9],
+// 1024 x 128 x 3072 10.7 / 12.6. fp32: 256 x 128 (8) x 2048 10.3 / 9.7, 512 x 128 x 2048 10.5 / 10.9 [14.2 / 10.7], 640 x 128 x
+// 2560 11.6 / 12.5, 1024 x 128 x 3328 14.0 / 15.0 [18.2 / 15.0]; 512 x 128 x 1536 8.3 / 10.8, 1024 x 128 x 2048 11.1 / 11.7.
+// ... more logits, bf16: 256 x 256 (16) x 3328 10.6 / 10.9, 512 x 256 (32) x 3840 12.4 / 12.6, x 4096 12.9 / 12.7 [17.1 / 12.6], x
+// 7168 19.7 / 17.0, 256 x 512 (32) x 4096 (six slices) 13.0 / 13.5 [19.4 / 13.5], 320 x 384 (30) x 4096 13.0 / 14.1 [18.4 / 14.2],
+// 128 x 1024 (32) x 7168 (four) 22.3 / 22.8 [30.6 / 22.6]; 512 x 256 x 2048 8.7 / 10.6 [11.8 / 10.5], x 3584 11.6 / 12.3 [15.5 / 12.1],
+// 256 x 512 x 3584 (four) 11.2 / 14.6, 128 x 1024 x 4096 (three) 15.9 / 18.9 [23.3 / 18.7]. fp32: 256 x 256 x 3072 11.9 / 12.6
+// [18.0 / 12.6], 512 x 256 x 3328 13.3 / 14.0 [19.5 / 13.9], x 4096 17.3 / 14.8, 256 x 512 x 3584 (four) 18.0 / 18.2 [24.8 / 18.7],
+// 128 x 1024 x 4096 (three) 25.8 / 24.5; 512 x 256 x 1024 6.6 / 11.6 [10.3 / 11.6], x 3072 12.0 / 13.2 [18.2 / 13.2], 128 x 512 x 2048
+// (three) 10.7 / 15.0.
+// 33 to 64 tiles, bf16: 1024 x 256 (64) x 2048 14.0 / 13.0, x 3072 15.2 / 15.8 [19.5 / 15.8], 640 x 384 (60) x 3072 14.5 / 15.6
+// [19.3 / 15.6], 512 x 512 (64) x 2304 (three) 14.1 / 14.8 [18.7 / 14.9]; x 2560 (three) 14.0 / 15.6. fp32: 2048 x 128 (64) x 1280
+// 13.3 / 13.7, x 2048 19.9 / 16.3, 384 x 512 (48) x 2048 (three) 19.3 / 16.7; 2048 x 128 x 1024 11.8 / 12.9, 512 x 384 (48) x 1536
+// (three) 13.4 / 14.3.
+// Beyond, on the weight as it is, other forms / slices: 2048 x 256 (128) x 2048 22.5 / 21.2 (level with a packed weight), x 3072
+// 30.5 / 22.2, 2560 x 256 (160) x 2048 22.9 / 23.8, x 4096 37.6 / 32.3, 1664 x 512 (208) x 3328 32.7 / 33.3; fp32, which fold gamma
+// there, 4096 x 128 (128) x 2048 24.0 / 27.9, x 4096 52.7 / 42.8, 1536 x 256 (96) x 4096 31.1 / 34.6.
 int router_slices(int64_t M, int K, int N, bool weight_fp32) {
   if (M < kRouterRows || N > kRouterSliceLogits) return 0;
   const int64_t tiles = (M + kRouterRows - 1) / kRouterRows * (N / 64);
-  const int most = weight_fp32 ? (N == 128 && K >= 4096 ? 128 : K >= 1024 ? 64 : 0)
-                               : (K >= 4096 ? 160 : K >= 2560 ? 128 : K >= 2048 ? 64 : 0);
+  const int most = weight_fp32 ? (N == 128 && K >= 4096 ? 128 : 64) : (K >= 4096 ? 160 : K >= 2560 ? 128 : 64);
   if (tiles > most) return 0;
-  const int64_t fill = ((tiles <= 64 ? 256 : 512) + tiles - 1) / tiles;
-  const int slices = (int)std::min<int64_t>({fill, K / (2 * N) + K / (4 * N), K / 128, 16});
-  return slices >= 3 ? slices : 0;
+  const int64_t fill = (tiles <= 64 ? 256 : 512) / tiles;
+  const int slices = (int)std::min<int64_t>({fill, K / (2 * N) + K / (4 * N), 16});
+  if (slices < 3) return 0;
+  int from = 0;  // least K
+  if (tiles <= 32) {
+    if (slices < 6 && weight_fp32) from = slices >= 4 && tiles >= 16 ? 3584 : tiles > 16 ? 3840 : INT_MAX;
+    else if (slices < 6) from = slices >= 4 && tiles > 16 ? 6144 : INT_MAX;
+    else if (weight_fp32 && N == 128) from = tiles <= 8 ? 1792 : tiles <= 20 ? 2048 : 3328;
+    else if (weight_fp32) from = N == 256 && tiles > 16 ? 3328 : 3072;
+    else if (N == 128) from = tiles <= 8 ? 2048 : tiles <= 16 ? 3200 : tiles <= 20 ? 3328 : 3840;
+    else if (K < 4608 && K > (K < 4096 ? 550 : 700) * slices) from = INT_MAX;  // slices that are too long
+    else from = tiles <= 16 ? 3328 : 3840;
+  } else if (tiles <= 64) {
+    from = weight_fp32 ? (slices >= 4 ? 1280 : 1792) : slices >= 4 || K <= 2304 ? 2048 : 3584;
+  }
+  return K >= from ? slices : 0;
 }
 
 template <bool FP32W, bool PACKED>

@@ -4,6 +4,7 @@ points keep the reference's signatures, and host-side argument checks fire
 before anything reaches a device."""
 import ctypes
 import inspect
+import itertools
 import os
 import re
 import shutil
@@ -101,6 +102,13 @@ def test_c_side_validation_without_gpu():
     assert [slices(*size, 0) for size in ((128, 4096, 32), (128, 4096, 1), (128, 4096, 200), (100, 4096, 256),
                                           (128, 4100, 256), (0, 4096, 256), (128, 16384, 256), (-128, 4096, 256))] == [0] * 8
     assert slices(128, 4096, 256, 0) > 0 and slices(128, 4096, 256, 1) > 0
+    # ... and where the one launch of a packed weight, whose results are those of the weight as it is, takes less
+    assert [slices(*size) for size in ((512, 2048, 256, 0), (256, 3584, 512, 0), (128, 4096, 1024, 0), (512, 2560, 512, 0),
+                                       (512, 1024, 256, 1), (512, 3072, 256, 1), (1024, 2048, 128, 1))] == [0] * 7
+    # whole rounds of workgroups
+    for M, N, K, fp32 in itertools.product(range(64, 2625, 32), (128, 256, 384, 512, 640, 1024), range(1024, 8193, 512), (0, 1)):
+        tiles = -(-M // 64) * (N // 64)
+        assert slices(M, K, N, fp32) * tiles <= (256 if tiles <= 64 else 512), (M, N, K, fp32)
     # the no-work kernel's variants: chunks per lane 4 / 8 / 16 only, order 0..3
     assert L.fq_stream_rw_variant(None, 0, None, 0, None, 4, 0, 0, 0, 0, None) == -1          # no sink
     assert L.fq_stream_rw_variant(None, 16, None, 0, None, 5, 0, 0, 0, 0, None) == -1
