@@ -207,7 +207,8 @@ int64_t fq_rmsnorm_router_scratch_bytes(int64_t K, int64_t N, int weight_is_fp32
  * The product has fp32-GEMM accuracy: y, and an fp32 weight, enter the matrix
  * cores as two bf16 terms each (16 significant bits; the reference's tl.dot on
  * fp32 operands uses fewer).  weight_scratch: fq_rmsnorm_router_scratch_bytes()
- * bytes the call overwrites (the weight re-ordered for the matrix cores).
+ * bytes the call overwrites (the weight re-ordered for the matrix cores); 16 do
+ * where fq_rmsnorm_router_slices() is not 0.
  * (output_mode 1 of the reference is fq_rmsnorm_quant_fwd with output_mode 1.) */
 int fq_rmsnorm_router_quant_fwd(const void* x, const void* gamma, const void* route_weight, int weight_is_fp32,
                                 void* weight_scratch, void* y, float* rstd, float* logits, void* q, float* s,
@@ -215,8 +216,9 @@ int fq_rmsnorm_router_quant_fwd(const void* x, const void* gamma, const void* ro
                                 void* stream);
 
 /* In how many slices of K fq_rmsnorm_router_quant_fwd and its packed form work on a call whose row tiles and
- * logits leave most of the GPU without work, 0 where they do not (and for sizes that they refuse).  Such a call reads route_weight as it is and leaves
- * weight_scratch alone; it is two launches, the first of which leaves partial sums in y and q. */
+ * logits leave most of the GPU without work, 0 where they do not (and for sizes that they refuse).  Such a call reads
+ * route_weight as it is and leaves weight_scratch alone, which may then be of 16 bytes; it is two launches, the first of
+ * which leaves partial sums in y and q. */
 int fq_rmsnorm_router_slices(int64_t M, int64_t K, int64_t N, int weight_is_fp32);
 
 /* The two halves of fq_rmsnorm_router_quant_fwd, for callers that keep the re-ordered weight

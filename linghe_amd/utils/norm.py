@@ -206,7 +206,7 @@ def triton_rms_norm_fp32_gemm_block_quant_forward(
         sliced = _lib.lib.fq_rmsnorm_router_slices(M, K, N, w_fp32)
         folds = w_fp32 and not sliced and _lib.lib.fq_rmsnorm_router_folds(M, K, N, w_fp32)
         planes = int(_lib.lib.fq_rmsnorm_router_scratch_bytes(K, N, w_fp32))
-        need, form = planes, 2 if folds else 0
+        need, form = 16 if sliced else planes, 2 if folds else 0  # (slices leave the scratch alone)
         if packed_route_weight is not None:
             weight, form = packed_route_weight, 1
             assert weight.is_cuda and weight.dtype == torch.uint8 and weight.is_contiguous()
