@@ -203,9 +203,7 @@ def triton_rms_norm_fp32_gemm_block_quant_forward(
         if not route_weight.is_cuda:
             raise RuntimeError("route_weight must live on the GPU: the HIP kernels are the only implementation")
         w_fp32 = int(route_weight.dtype == torch.float32)
-        sliced = _lib.lib.fq_rmsnorm_router_slices(M, K, N, w_fp32)
-        folds = w_fp32 and not sliced and _lib.lib.fq_rmsnorm_router_folds(M, K, N, w_fp32)
-        planes = int(_lib.lib.fq_rmsnorm_router_scratch_bytes(K, N, w_fp32))
+        sliced, folds, planes, folded = _lib.native.router_sizes(M, K, N, w_fp32)
         need, form = 16 if sliced else planes, 2 if folds else 0  # (slices leave the scratch alone)
         if packed_route_weight is not None:
             weight, form = packed_route_weight, 1
@@ -215,7 +213,7 @@ def triton_rms_norm_fp32_gemm_block_quant_forward(
             if folds and weight.numel() > planes:
                 weight, form = weight.view(-1)[planes:], 2
         if form == 2:
-            need = int(_lib.lib.fq_rmsnorm_router_folded_scratch_bytes(K, N))
+            need = folded
     new = _lib.native.rmsnorm_router_quant(x, norm_weight, weight, N, form, w_fp32, need, rms, output_mode,
                                            float(eps), int(bool(round_scale)), _lib.stream_of(x))
     return new if rms is None else (new[0], rms, *new[2:])

@@ -64,6 +64,18 @@ def test_argument_types_match_header():
     assert _lib.lib.fq_rmsnorm_bwd_num_partials.restype is ctypes.c_int64
 
 
+def test_router_sizes_are_those_of_the_library():
+    """What the Python entry point asks of the host module is what the C interface answers."""
+    from linghe_amd import _lib
+
+    L = _lib.lib
+    for M, K, N, fp32 in itertools.product((32, 128, 1024, 4096), (256, 2048, 4096, 8192), (128, 256, 1024, 8192), (0, 1)):
+        slices = L.fq_rmsnorm_router_slices(M, K, N, fp32)
+        assert _lib.native.router_sizes(M, K, N, fp32) == (
+            slices, 0 if slices else L.fq_rmsnorm_router_folds(M, K, N, fp32), L.fq_rmsnorm_router_scratch_bytes(K, N, fp32),
+            L.fq_rmsnorm_router_folded_scratch_bytes(K, N))
+
+
 def test_c_side_validation_without_gpu():
     """Shape / flag errors are reported by return code before any HIP call."""
     from linghe_amd import _lib
