@@ -17,6 +17,7 @@
 #include <ATen/ATen.h>
 #include <ATen/EmptyTensor.h>
 #include <ATen/detail/CUDAHooksInterface.h>
+#include <ATen/record_function.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
@@ -68,7 +69,7 @@ at::Tensor tensor_or_none(PyObject* o) {
 
 // The device of a call's first tensor made the current one, and tensors on it. They are made as at::empty makes them behind
 // the dispatcher (0.65 us of a call for each output, 0.25 without it), unless something could be listening there: a mode, a
-// transform, a tracer, or the fill of new memory that deterministic algorithms ask for.
+// transform, a tracer, an observer of operators (a profiler), or the fill of new memory that deterministic algorithms ask for.
 class Outputs {
  public:
   explicit Outputs(const at::Tensor& x)
@@ -76,7 +77,7 @@ class Outputs {
         device_(x.device()),
         plain_(x.is_cuda() && !c10::impl::TorchDispatchModeTLS::any_modes_set() &&
                (c10::impl::tls_local_dispatch_key_set().included_ - c10::default_included_set).empty() &&
-               !at::globalContext().deterministicAlgorithms()) {}
+               !at::hasCallbacks() && !at::globalContext().deterministicAlgorithms()) {}
 
   at::Tensor empty(const at::Tensor& like, at::ScalarType type, at::IntArrayRef sizes) const {
     if (!plain_ || like.device() != device_)

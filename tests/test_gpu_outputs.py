@@ -59,6 +59,16 @@ def test_outputs_in_every_state_of_torch(gpu, name):
             assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
 
 
+@pytest.mark.parametrize("name", ["group", "norm", "norm_bwd", "swiglu", "plan"])
+def test_a_profiler_sees_the_outputs(gpu, name):
+    announce("outputs, profiler", name)
+    call = _calls(gpu)[name]
+    outs = len(call())
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU], acc_events=True) as seen:
+        call()
+    assert sum(e.name == "aten::empty" for e in seen.events()) >= outs
+
+
 def test_deterministic_algorithms_fill_what_is_not_written(gpu):
     call = _calls(gpu)["swiglu"]
     torch.use_deterministic_algorithms(True)
