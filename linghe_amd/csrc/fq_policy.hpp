@@ -92,6 +92,13 @@ struct Policy {
   // (1740 tiles) 29.4 / 26.9, x 1664 (1508) 25.2 / 24.3, x 1408 (1276) 20.75 / 20.96, x 1152 (1044) 20.4 / 19.8, x 896 (812) 16.0 / 15.6,
   // x 768 (696) 14.0 / 14.3, x 640 (580) 13.75 / 13.96, 6000 x 1920 (705) 14.55 / 14.69: up to 1276 it goes either way
   static constexpr int kBlockwiseByColumnsTiles = 1408;
+  // The SwiGLU forward from so many tiles on, and where rows don't start on half lines. us of the kernel, both layouts [transposed
+  // only], grid order / by columns: 3001 x 1408 (264 tiles) 10.4 / 10.3 [9.3 / 9.0], 5000 x 3200 (1000) 21.9 / 20.5 [21.6 / 19.9],
+  // 8120 x 2176 (1088) 25.8 / 24.3, 14800 x 1920 (1740) 36.9 / 34.1 [40.3 / 37.1], 16336 x 5248 (5248) 97.4 / 94.8 [135 / 104]; 1040 x
+  // 1408 (99) 6.57 / 6.75, 2160 x 1408 (187) 7.41 / 7.56; half lines: 4160 x 2944 15.8 / 16.3 [13.1 / 13.4], 14144 x 1664 27.3 / 28.7
+  // [24.6 / 25.2], x 3456 53.1 / 55.3 [51.6 / 52.7], but 16320 x 2944 56.1 / 54.0 [59.3 / 49.5], where rows start 16 KB apart but
+  // for one half line. At 9 row blocks and 513 to 567 tiles it loses up to 8 % (1040 x 7552 13.2 / 13.8).
+  static constexpr int kSiluByColumnsTiles = 256;
   // row blocks per run that an XCD works on (xcd_runs; 0: every eighth tile).  Same sizes, planned launches with
   // 0 / 2 / 4 / 8 / 16: SwiGLU forward 43.4 / 41.2 / 40.8 / 40.7 / 40.8 us, backward 76.5 / 76.1 / 75.5 / 75.3 / 76.2,
   // blockwise quantiser 30.9 / 30.3 / 29.9 / 29.9 / 29.8.  Launches that scan the counts, 0 / 2 / 4 / 8: forward

@@ -536,7 +536,8 @@ hipError_t launch_silu_quant_fwd(const void* x, const void* weight, int weight_b
                                  hipStream_t stream, const void* plan, const PlanShape* ps) {
   OutPtrs out{(uint8_t*)q, s, (uint8_t*)qt, st};
   const BatchArgs b = batch_args(counts, counts_i64, n_experts, plan, ps, Policy::kPlanPackedFirstSiluFwd, 0);
-  const int remap = shared_lines_remap(M, n / kGroup, mode);
+  const int remap = M % 64 != 0 && row_blocks * (n / kGroup) >= Policy::kSiluByColumnsTiles
+                        ? shared_lines_remap(M, n / kGroup, mode) : 0;
   if (mode == 0 && !counts && !plan && !weight && silu_quant_rows_per_team(M, n) > 0)
     return launch_silu_quant_rows(x, q, s, M, n, round_scale, kind, stream);
   RowWeight w{weight, weight_bf16};

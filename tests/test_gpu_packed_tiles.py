@@ -122,6 +122,23 @@ def test_tiles_of_shared_lines(gpu, M, ncb):
         check_quant_pair("shared.silu.col", ref[2], ref[3], qt, st, **FUSED)
 
 
+# the SwiGLU forward takes that order from 256 tiles on: 252, 255 and 289 of them, rows that start anywhere, and rows on half lines,
+# which stay in grid order
+@pytest.mark.parametrize("M,ncb", [(2683, 12), (2160, 15), (2160, 17), (2159, 17), (2112, 17)])
+def test_silu_tiles_of_shared_lines(gpu, M, ncb):
+    from linghe_amd.utils.silu import triton_silu_and_block_quant_forward
+
+    announce("SwiGLU tiles of shared lines", M, ncb)
+    h = randn_bf16(gen(M + ncb), M, 256 * ncb)
+    ref = O.silu_and_block_quant_forward(h)
+    for mode in (2, 1):
+        q, s, qt, st = triton_silu_and_block_quant_forward(h.to(gpu), output_mode=mode)
+        torch.cuda.synchronize()
+        if mode == 2:
+            check_quant_pair("shared.silu.row", ref[0], ref[1], q, s, **FUSED)
+        check_quant_pair("shared.silu.col", ref[2], ref[3], qt, st, **FUSED)
+
+
 # the plain quantiser takes that order from 1408 tiles on: 1404 and 1413 of them, the last row block of 112 rows
 @pytest.mark.parametrize("M", [19952, 20080])
 def test_plain_tiles_of_shared_lines(gpu, M):
