@@ -88,6 +88,13 @@ struct Policy {
   // takes an eighth of the tiles counted column block after column block. us of the tile kernel in grid order / so: RMSNorm
   // 15935 x 5248 62.8 / 52.8, 8120 x 2176 14.8 / 11.8, 3046 x 1408 7.4 / 6.8, 6537 x 768 7.7 / 7.2, 1303 x 6272 8.4 / 7.7, plain
   // quantiser 9040 x 3968 31.4 / 27.6, 4720 x 6528 27.8 / 25.4.
+  // RMSNorm with both outputs, rows on half lines, 4096 columns and 3072 tiles or more: eighths of the tiles in grid order (us of
+  // a call, so / by columns: 11328 x 5504 64.7 / 68.7, 15040 x 5504 84.2 / 90.0, 12352 x 4992 63.7 / 65.7, 14144 x 6528 91.8 / 94.2,
+  // 18496 x 6016 109.6 / 112.3, 16320 x 5248 92.1 / 86.9 and 84.7 / 88.9; fewer tiles 8256 x 3456 31.9 / 31.2, 4160 x 5248
+  // 26.8 / 26.2).
+  // Column blocks in eights: rows that share lines anywhere take grid order at all sizes. us of the transposed output, statistic
+  // given, eighths / grid order: 14352 x 4096 38.9 / 36.8, x 6144 55.1 / 51.0, x 7168 63.1 / 58.4, x 8192 78.1 / 63.5, x 5120 45.0 / 44.0,
+  // but within 80 rows of 16384 16400 x 4096 42.2 / 42.7, 16336 x 5120 47.5 / 51.2, 16464 x 7168 68.5 / 72.9 (x 8192 90.5 / 78.6).
   // The plain quantiser, with the least work in a tile, only from so many tiles on; us of a call with a weight's quantiser: 14800 x 1920
   // (1740 tiles) 29.4 / 26.9, x 1664 (1508) 25.2 / 24.3, x 1408 (1276) 20.75 / 20.96, x 1152 (1044) 20.4 / 19.8, x 896 (812) 16.0 / 15.6,
   // x 768 (696) 14.0 / 14.3, x 640 (580) 13.75 / 13.96, 6000 x 1920 (705) 14.55 / 14.69: up to 1276 it goes either way

@@ -599,9 +599,10 @@ hipError_t launch_rmsnorm_quant_tile(const void* x, const void* gamma, const flo
   const bool aligned_rows = M % 64 == 0;
   // XCD remap (see resolve_tile): wide rows and several waves of workgroups
   // ... and, behind the statistic pass, wherever that pass handed out the rows by XCD
-  const int shared = shared_lines_remap(M, n / kGroup, mode);
-  const int remap = shared ? shared
-                    : (aligned_rows && n >= 4096 && tiles >= 3072) || (mode == 2 && rmsnorm_passes_by_xcd(M, n));
+  const bool wide = aligned_rows && n >= 4096 && tiles >= 3072;
+  // (with both outputs rows on half lines pass the L2s by)
+  const int shared = mode == 2 && wide ? 0 : shared_lines_remap(M, n / kGroup, mode);
+  const int remap = shared ? shared : wide || (mode == 2 && rmsnorm_passes_by_xcd(M, n));
   // raised priority until the loads are out: only when the whole launch is resident at once (four
   // workgroups per CU of a 256-CU device; more tiles than that arrive in generations)
   const int first = Policy::kStartPriorityRmsnorm && tiles <= 1024;

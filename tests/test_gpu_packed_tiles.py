@@ -139,6 +139,24 @@ def test_silu_tiles_of_shared_lines(gpu, M, ncb):
         check_quant_pair("shared.silu.col", ref[2], ref[3], qt, st, **FUSED)
 
 
+# RMSNorm with both outputs, rows on half lines: eighths of the tiles in grid order from 4096 columns and 3072 tiles on, 3087 of
+# them here, by column blocks below, and with the transposed output alone at all sizes
+@pytest.mark.parametrize("M,n", [(6208, 8064), (2112, 4224), (6208, 896)])
+def test_rmsnorm_tiles_on_half_lines(gpu, M, n):
+    from linghe_amd.utils.norm import triton_rms_norm_and_block_quant_forward as fn
+
+    announce("RMSNorm tiles on half lines", M, n)
+    g = gen(M + n)
+    x, w = randn_bf16(g, M, n), randn_bf16(g, n)
+    q, s, rms, qt, st = fn(x.to(gpu), w.to(gpu))
+    qt1, st1 = fn(x.to(gpu), w.to(gpu), rms=rms, output_mode=1)[3:]
+    torch.cuda.synchronize()
+    ref = O.rms_norm_and_block_quant_forward(x, w, rstd=rms.cpu())
+    check_quant_pair("half.rms.row", ref[0], ref[1], q, s, **EXACT)
+    check_quant_pair("half.rms.col", ref[3], ref[4], qt, st, **EXACT)
+    assert torch.equal(qt1.view(torch.uint8), qt.view(torch.uint8)) and torch.equal(st1, st)
+
+
 # the plain quantiser takes that order from 1408 tiles on: 1404 and 1413 of them, the last row block of 112 rows
 @pytest.mark.parametrize("M", [19952, 20080])
 def test_plain_tiles_of_shared_lines(gpu, M):
