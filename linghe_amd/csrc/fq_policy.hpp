@@ -95,6 +95,10 @@ struct Policy {
   // Column blocks in eights: rows that share lines anywhere take grid order at all sizes. us of the transposed output, statistic
   // given, eighths / grid order: 14352 x 4096 38.9 / 36.8, x 6144 55.1 / 51.0, x 7168 63.1 / 58.4, x 8192 78.1 / 63.5, x 5120 45.0 / 44.0,
   // but within 80 rows of 16384 16400 x 4096 42.2 / 42.7, 16336 x 5120 47.5 / 51.2, 16464 x 7168 68.5 / 72.9 (x 8192 90.5 / 78.6).
+  // One block of columns more or less than a multiple of 16384: rows start 32 KB apart but for 256 bytes, and a walk down a column
+  // block is the slower one. us in grid order / by columns: plain quantiser 1040 x 32640 36.2 / 45.0, 2064 x 16256 36.8 / 40.5, 4112 x
+  // 16512 56.8 / 68.5 (transposed only 46.3 / 54.4), but 4112 x 16128 54.4 / 50.3, x 16640 56.0 / 53.0, 4112 x 8064 35.8 / 34.0, 2064 x
+  // 24448 51.2 / 47.2; SwiGLU forward 2064 x 16256 43.2 / 51.9, 528 x 32640 24.9 / 29.1, but 2064 x 16128 42.9 / 39.6.
   // The plain quantiser, with the least work in a tile, only from so many tiles on; us of a call with a weight's quantiser: 14800 x 1920
   // (1740 tiles) 29.4 / 26.9, x 1664 (1508) 25.2 / 24.3, x 1408 (1276) 20.75 / 20.96, x 1152 (1044) 20.4 / 19.8, x 896 (812) 16.0 / 15.6,
   // x 768 (696) 14.0 / 14.3, x 640 (580) 13.75 / 13.96, 6000 x 1920 (705) 14.55 / 14.69: up to 1276 it goes either way

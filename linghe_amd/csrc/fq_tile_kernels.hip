@@ -439,7 +439,10 @@ __global__ __launch_bounds__(1024) void expert_plan_kernel(const void* __restric
 // launchers
 // ---------------------------------------------------------------------------
 // Order of the tiles of one matrix whose transposed rows share lines between row blocks (M no multiple of 128): fq_policy.hpp
-static int shared_lines_remap(int64_t M, int ncb, int mode) { return mode != 0 && M % kGroup != 0 && ncb % 8 != 0 ? 2 : 0; }
+static int shared_lines_remap(int64_t M, int ncb, int mode) {
+  const bool around_16k = (ncb + 1) % 128 <= 2;  // columns, in blocks of 128
+  return mode != 0 && M % kGroup != 0 && ncb % 8 != 0 && !around_16k ? 2 : 0;
+}
 
 static BatchArgs batch_args(const void* counts, int counts_i64, int n_experts, const void* plan,
                             const PlanShape* ps, bool packed_first, int xcd_rows_scan,

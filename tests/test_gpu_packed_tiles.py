@@ -123,8 +123,8 @@ def test_tiles_of_shared_lines(gpu, M, ncb):
 
 
 # the SwiGLU forward takes that order from 256 tiles on: 252, 255 and 289 of them, rows that start anywhere, and rows on half lines,
-# which stay in grid order
-@pytest.mark.parametrize("M,ncb", [(2683, 12), (2160, 15), (2160, 17), (2159, 17), (2112, 17)])
+# and widths next to a multiple of 16384 columns, which stay in grid order
+@pytest.mark.parametrize("M,ncb", [(2683, 12), (2160, 15), (2160, 17), (2159, 17), (2112, 17), (272, 127)])
 def test_silu_tiles_of_shared_lines(gpu, M, ncb):
     from linghe_amd.utils.silu import triton_silu_and_block_quant_forward
 
@@ -157,13 +157,14 @@ def test_rmsnorm_tiles_on_half_lines(gpu, M, n):
     assert torch.equal(qt1.view(torch.uint8), qt.view(torch.uint8)) and torch.equal(st1, st)
 
 
-# the plain quantiser takes that order from 1408 tiles on: 1404 and 1413 of them, the last row block of 112 rows
-@pytest.mark.parametrize("M", [19952, 20080])
-def test_plain_tiles_of_shared_lines(gpu, M):
+# the plain quantiser takes that order from 1408 tiles on: 1404 and 1413 of them, the last row block of 112 rows; widths next to
+# a multiple of 16384 columns, which stay in grid order, and one further off
+@pytest.mark.parametrize("M,ncb", [(19952, 9), (20080, 9), (1424, 127), (1424, 129), (1424, 126)])
+def test_plain_tiles_of_shared_lines(gpu, M, ncb):
     from linghe_amd.quant.block import triton_blockwise_quant
 
-    announce("plain tiles of shared lines", M)
-    x = randn_bf16(gen(M), M, 128 * 9)
+    announce("plain tiles of shared lines", M, ncb)
+    x = randn_bf16(gen(M), M, 128 * ncb)
     ref = O.batch_blockwise_quant(x, [M], False)
     for mode in (2, 1):
         q, s, qt, st = triton_blockwise_quant(x.to(gpu), output_mode=mode)
