@@ -1311,10 +1311,11 @@ __global__ __launch_bounds__(256) void router_slices_kernel(RouterSliceArgs p) {
       }
     }
   };
-  // the products of the leading terms apart from the others: shorter chains of roundings
-  floatx16_t lead, rest;
+  // the products of the leading terms apart from the others, and those of even k steps from those of odd ones: shorter chains
+  // of roundings
+  floatx16_t lead[2], rest;
 #pragma unroll
-  for (int v = 0; v < 16; ++v) lead[v] = rest[v] = 0.f;
+  for (int v = 0; v < 16; ++v) lead[0][v] = lead[1][v] = rest[v] = 0.f;
   const int rt = wave & 1, ct = wave >> 1;
   auto multiply = [&](int buf) {
 #pragma unroll
@@ -1322,7 +1323,7 @@ __global__ __launch_bounds__(256) void router_slices_kernel(RouterSliceArgs p) {
       const int at = (lane & 32) + ((lane & 31) ^ (2 * ks + (lane >> 5)));
       const bf16x8_t hi = operand(sa[buf][0][rt][ks][at]), lo = operand(sa[buf][1][rt][ks][at]);
       const bf16x8_t w = operand(sb[buf][0][ct][ks][at]);
-      lead = __builtin_amdgcn_mfma_f32_32x32x16_bf16(hi, w, lead, 0, 0, 0);
+      lead[ks & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(hi, w, lead[ks & 1], 0, 0, 0);
       rest = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lo, w, rest, 0, 0, 0);
       if constexpr (FP32W) {
         const bf16x8_t wl = operand(sb[buf][P - 1][ct][ks][at]);
@@ -1351,7 +1352,7 @@ __global__ __launch_bounds__(256) void router_slices_kernel(RouterSliceArgs p) {
   for (int v = 0; v < 16; ++v) {
     // register v of a 32x32 result holds row (v / 4) * 8 + (lane / 32) * 4 + v % 4, column lane % 32
     const int row = row0 + rt * 32 + (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3);
-    router_slice(p, row, slice)[tile_n * 64 + ct * 32 + (lane & 31)] = lead[v] + rest[v];
+    router_slice(p, row, slice)[tile_n * 64 + ct * 32 + (lane & 31)] = (lead[0][v] + lead[1][v]) + rest[v];
   }
 }
 
