@@ -18,7 +18,8 @@
 //
 // The kernels below share the work out over (row tile, column chunk) pairs; the workgroups of
 // one row tile sit on one XCD (router_tile), so that the chunks' walks over K read x from memory
-// once and else from that XCD's L2.  Each of them walks all of K for its columns of the logits,
+// once and else from that XCD's L2.  But for the calls of few tiles, whose workgroups take a slice of K each and leave the
+// rows to a second kernel (router_slices), each of them walks all of K for its columns of the logits,
 // accumulating the row statistic beside it, and then writes y, the codes and the scales for its
 // share of the K / 128 quantisation groups, re-reading that part of x: from the L2 where the XCD's
 // row tiles and the weight still fit it (8192 x 256 x 2048 fetched 63.6 MB past the L2s where x and one weight per
@@ -1232,11 +1233,11 @@ __global__ __launch_bounds__(512) void rmsnorm_router_quant_folded_kernel(Router
 // 64 rows x 64 logits of a slice per workgroup of four waves. Per slab of 64 columns the threads turn x into its two operand
 // terms and an fp32 weight into its two planes, in LDS, two slabs of both on their way; a wave multiplies 32 rows by 32 logits.
 // PACKED: the weight in operand order (pack_router_weight), the same values and order of products.
-// Bound by the operand arithmetic and LDS traffic of a slab (about 700 clocks each, of 500 of matrix instructions) with two or
-// three workgroups on a CU to overlap them, and by two launches' latencies. us of the kernels, few-rows or 64-row form with its
-// re-ordering of the weight / products + rows: 640 x 256 x 4608 fp32 6.8 + 32.8 / 16.2 + 7.5, 512 x 256 x 7168 bf16 5.9 + 19.6 / 11.9
-// + 7.5, 1024 x 512 x 4096 bf16 6.0 + 31.3 / 18.9 + 8.1. A k step for each wave (operands read from LDS once) 17.8 for the 16.2,
-// operands loaded into registers in lane order, without LDS, 20.7.
+// Bound by the operand arithmetic and LDS traffic of a slab (about 700 clocks each, of 500 of matrix instructions), which one
+// workgroup on a CU overlaps little (two from 65 tiles on), and by two launches' latencies. us of the kernels, few-rows or 64-row form
+// with its re-ordering of the weight / products + rows: 640 x 256 x 4608 fp32 6.8 + 32.8 / 15.0 + 5.6, 512 x 256 x 7168 bf16 5.9 + 19.6 /
+// 12.9 + 6.3, 1024 x 512 x 4096 bf16 6.0 + 31.3 / 19.3 + 8.5. With six slices for the first (16.2) a k step for each
+// wave (operands read from LDS once) took 17.8, operands loaded into registers in lane order, without LDS, 20.7.
 // ---------------------------------------------------------------------------
 struct RouterSliceArgs {
   RouterArgs a;
@@ -1492,6 +1493,8 @@ static RouterForm router_form(int64_t M, int K, int N, bool weight_fp32) {
 // 11.3 / 11.5; in more 8192 x 256 (512) x 896 26.2 / 25.1, x 768 23.8 / 23.5, x 640 20.6 / 22.1, 8192 x 512 x 896 44.3 / 42.7.
 // With 128 logits a workgroup has 32 rows to quantise: 4096 x 128 x 768 15.7 / 15.7, x 1024 18.2 / 16.4, x 4096 48.5 / 40.6,
 // 12288 x 128 x 896 27.3 / 28.6, x 1024 30.6 / 29.3, 8192 x 128 x 8192 126.9 / 122.5.
+// (The Python entry point folds where there are no slices of K: of the calls of 41 to 64 workgroups those of a K below 1792 that
+// makes three slices, and of more than 1024 logits.)
 bool router_folds(int64_t M, int K, int N) {
   const int64_t workgroups = (M + kRouterRows - 1) / kRouterRows * (N / 64);
   if (M < kRouterRows || workgroups * 512 > (int64_t)UINT32_MAX) return false;

@@ -173,7 +173,8 @@ def triton_rms_norm_fp32_gemm_block_quant_forward(
             1: only output transposed quantizatino tensor (rms must be given)
         packed_route_weight: (keyword-only addition) the result of pack_route_weight(route_weight).
             The kernels read the router weight in matrix-core operand order; without this
-            argument it is re-ordered on every call, with it the caller re-orders once per
+            argument it is re-ordered on every call (but for calls of few rows and logits with a long K, which read
+            it as it is and gain nothing by packing), with it the caller re-orders once per
             weight update, and route_weight itself is not read.  Results are identical.
 
     Returns:
